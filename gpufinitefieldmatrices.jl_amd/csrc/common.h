@@ -242,7 +242,7 @@ struct TuneEntry {
     double ms = 0.0;    // measured time of the winner
 };
 
-constexpr int WS_COUNT = 21;
+constexpr int WS_COUNT = 22;
 
 struct modp_ctx {
     int device = 0;
@@ -260,10 +260,11 @@ struct modp_ctx {
     std::vector<KernelTiming> timings;
     std::vector<hipEvent_t> event_pool;
     hipEvent_t slots[16] = {nullptr};
-    // table of modular inverses for the current elimination modulus
+    // table of small modular inverses for the current elimination modulus
     uint32_t *invtab = nullptr;
     int64_t invtab_p = 0;
-    size_t invtab_cap = 0;
+    // steps of the elimination panels so far (64 a panel): their exchange tags
+    uint32_t panel_tag = 0;
     // autotuner: MODP_TUNE_OFF / _CACHED / _ON_MISS and its cache
     int tune_mode = 0;
     std::map<TuneKey, TuneEntry> tune_cache;
@@ -302,7 +303,8 @@ enum {
     WS_INV_U = 17,     // matrix inverse: PLUQ factors
     WS_INV_L = 18,
     WS_PERM = 19,      // lines moved by a permutation
-    WS_GPOS = 20       // row positions of the W-resident elimination panel
+    WS_GPOS = 20,      // row positions of the W-resident elimination panel
+    WS_PANEL = 21      // exchange area of the elimination panels on one XCD
 };
 
 // error plumbing: every internal function returns a modp_status

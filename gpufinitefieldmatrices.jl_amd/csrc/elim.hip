@@ -11,14 +11,14 @@
 // src/CuModMatrix/rref_lu_pluq/pluq_kernels.jl:90-142, one pivot per host
 // iteration with a host round-trip each; here one launch factors a whole
 // panel):
-//   for each inner panel of w columns (w*rows-per-thread <= 64 registers):
-//     k_panel    one 512-thread workgroup holds the panel in registers; per
+//   for each inner panel of w <= 32 columns:
+//     k_panel    (elim_panel.h) the panel in registers, one row per lane; per
 //                column: wave64 argmax by DPP with lowest-row tie-break,
-//                cross-wave through LDS, the pivot's inverse from a table (or
-//                extended Euclid), and the rank-1 update of the remaining
-//                panel columns; rows move only at the end, by a row map, and
+//                across waves through LDS or one XCD's L2, the pivot's
+//                inverse, and the rank-1 update of the remaining panel
+//                columns; rows move only at the end, by a row map, and
 //                the old values of the moved rows in the block's other
-//                columns are staged.  Above 32 x 512 rows k_panel_g does the
+//                columns are staged.  Above 16,384 rows k_panel_g does the
 //                same with the panel left in W (any row count).
 //     k_update   the block's other columns: the row map, and right of the
 //                panel the triangular solve with L11 (rows of U) and the
@@ -30,451 +30,14 @@
 
 #include <type_traits>
 
-#include "common.h"
+#include "elim_panel.h"
 
 namespace {
 
-// compile-time loop: f(integral_constant<int, J>) for J = B .. E-1
-template <int B, int E> struct Unroll {
-    template <class F> __device__ __forceinline__ static void run(F &f)
-    {
-        f(std::integral_constant<int, B>{});
-        Unroll<B + 1, E>::run(f);
-    }
-};
-template <int E> struct Unroll<E, E> {
-    template <class F> __device__ __forceinline__ static void run(F &) {}
-};
-
 constexpr int NBO = 128;  // outer block width (K of the trailing GEMM)
 
-struct PanelCtl {
-    int npiv;    // pivots found
-    int status;  // 0 all columns consumed, 1 zero column (pluq stop),
-                 // 2 rows exhausted, 3 pivot not invertible
-    int ncols;   // panel columns consumed
-    int nmap;    // entries of the row gather map
-    int kr0;     // first row of the panel
-};
-
-constexpr int PT = 512;  // threads of the panel workgroup (8 waves, 256-VGPR budget)
-
-typedef int v2i_e __attribute__((ext_vector_type(2)));
-typedef int v4i_e __attribute__((ext_vector_type(4)));
-
-// VW consecutive int32 from a VW-aligned address, one vector load
-template <int VW> __device__ __forceinline__ void load_rows(const int32_t *p, int32_t *x)
-{
-    if constexpr (VW == 4) {
-        const v4i_e t = *reinterpret_cast<const v4i_e *>(p);
-        x[0] = t[0]; x[1] = t[1]; x[2] = t[2]; x[3] = t[3];
-    } else if constexpr (VW == 2) {
-        const v2i_e t = *reinterpret_cast<const v2i_e *>(p);
-        x[0] = t[0]; x[1] = t[1];
-    } else {
-        x[0] = p[0];
-    }
-}
-
-// VW consecutive rows of one column; x[e * stride] is row e
-template <int VW> __device__ __forceinline__ void store_rows(int32_t *p, const int32_t *x, int stride)
-{
-    if constexpr (VW == 4) {
-        *reinterpret_cast<v4i_e *>(p) = v4i_e{x[0], x[stride], x[2 * stride], x[3 * stride]};
-    } else if constexpr (VW == 2) {
-        *reinterpret_cast<v2i_e *>(p) = v2i_e{x[0], x[stride]};
-    } else {
-        p[0] = x[0];
-    }
-}
-
-template <bool SMALL> __device__ __forceinline__ uint32_t mulmod_t(uint32_t a, uint32_t b, const ModP &mp)
-{
-    if (SMALL) {
-        // p < 2^16: operands and quotient fit 24 bits, so the full-rate
-        // 24-bit multiplier gives the exact 32-bit products
-        const uint32_t x = __umul24(a, b);
-        const uint32_t q = (uint32_t)((float)x * mp.pinvf);
-        int32_t r = (int32_t)(x - __umul24(q, mp.p32));
-        r += r < 0 ? (int32_t)mp.p32 : 0;
-        r -= r >= (int32_t)mp.p32 ? (int32_t)mp.p32 : 0;
-        return (uint32_t)r;
-    }
-    return (uint32_t)dmod((double)a * (double)b, mp);
-}
-
-// x mod p for exact integers |x| <= 2^51: fl(x * pinv) is within
-// |x| 2^-52 / p <= 1/(2p) of x/p, so q = rint(.) is within 1/2 + 1/(2p) < 1 of
-// x/p, r = x - q p is exact with |r| < p, and one fix-up brings it to [0,p).
-__device__ __forceinline__ double dmod_near(double x, const ModP &mp)
-{
-    const double r = fma(-rint(x * mp.pinv), mp.pd, x);
-    return r < 0.0 ? r + mp.pd : r;
-}
-
-__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
-
-// Pivot-search keys: larger key = larger residue, then lower position.
-template <bool SMALL> struct PivKey;
-template <> struct PivKey<true> {
-    typedef uint32_t T;  // residue < 2^16 in bits 30..15, 0x7fff - position below
-    static __device__ __forceinline__ T make(uint32_t v, int pos) { return (v << 15) | (uint32_t)(0x7fff - pos); }
-    static __device__ __forceinline__ uint32_t val(T k) { return k >> 15; }
-    static __device__ __forceinline__ int pos(T k) { return 0x7fff - (int)(k & 0x7fffu); }
-};
-template <> struct PivKey<false> {
-    typedef uint64_t T;
-    static __device__ __forceinline__ T make(uint32_t v, int pos) { return ((uint64_t)v << 32) | (uint32_t)(0x7fffffff - pos); }
-    static __device__ __forceinline__ uint32_t val(T k) { return (uint32_t)(k >> 32); }
-    static __device__ __forceinline__ int pos(T k) { return 0x7fffffff - (int)(uint32_t)k; }
-};
-
-// Panel factorisation: one 512-thread workgroup, the panel W[kr0:m, c0:c0+w]
-// in registers (thread t owns local rows t + 512*q) as exact integers in
-// FP64.  Each rank-1 update is one FMA: for p < 2^16 every product is below
-// 2^32, so up to 2^21 updates stay exact below 2^53 and only the pivot
-// column and the pivot row are reduced (lazy reduction); larger p reduce
-// after every update.
-//
-// One barrier per column: every wave finds its best candidate (largest
-// residue, then lowest position) with DPP, and the lane holding it publishes
-// that row, its index and its inverse in LDS before the barrier (double
-// buffered by column parity); after the barrier all threads pick the winner
-// among the waves and already have its row.  Rows never move: each row
-// carries its current position (the reference's swap of positions pc and
-// Ip), a row chosen as pivot is frozen with its normalised U row kept in
-// LDS, and at the end every row is written to its final position.
-template <int RPT, int NBW, bool SMALL>
-__global__ __launch_bounds__(PT) void k_panel(int32_t *__restrict__ W, int64_t ldw, int m, int kr0_in, int c0,
-                                              int w, ModP mp, int ple, const uint32_t *__restrict__ invtab,
-                                              int32_t *__restrict__ ipiv, int32_t *__restrict__ pivval,
-                                              int32_t *__restrict__ pivinv, int32_t *__restrict__ pivcol,
-                                              int32_t *__restrict__ colmap, int32_t *__restrict__ map_dst,
-                                              int32_t *__restrict__ map_src, PanelCtl *__restrict__ ctl,
-                                              int *__restrict__ abort, int KC, int FAR, int32_t *__restrict__ stage,
-                                              int *__restrict__ cursor)
-{
-    constexpr int NW = PT / 64;
-    if (abort && *abort) {
-        // an earlier panel of this block stopped: nothing to do
-        if (threadIdx.x == 0) {
-            ctl->npiv = 0;
-            ctl->status = 4;
-            ctl->ncols = 0;
-            ctl->nmap = 0;
-            ctl->kr0 = kr0_in;
-        }
-        return;
-    }
-    // the first row comes from the device cursor when the previous panel's
-    // pivot count is not known to the host (lu, rref)
-    const int kr0 = cursor ? *cursor : kr0_in;
-    typedef PivKey<SMALL> K;
-    typedef typename K::T key_t;
-    __shared__ key_t s_key[2][NW];
-    __shared__ double s_crow[2][NW][NBW];        // candidate rows (unreduced)
-    __shared__ uint32_t s_cinv[2][NW];
-    __shared__ int s_cidx[2][NW];                // candidate local row index
-    __shared__ uint32_t s_U[NBW][NBW];
-    __shared__ int s_pcol[NBW];
-    // per pivot: source position, value, inverse; per column: pivot or -1
-    // (kept in LDS during the steps, written out at the end)
-    __shared__ int s_ip[NBW], s_pv[NBW], s_pi[NBW], s_cmap[NBW];
-    __shared__ int s_cnt;
-    __shared__ int s_msrc[2 * NBW];  // source row of each row-map entry
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int rows = m - kr0;
-    // Rows are read as VW-row vectors from the VW-aligned row kra <= kr0:
-    // register row q of this thread is panel row rowi(q) (negative for the
-    // sh rows above kr0, which only pad the first vector).  kra + RPT * PT >= m
-    // because the host sizes RPT from m.
-    constexpr int VW = RPT < 4 ? RPT : 4;
-    const int kra = kr0 & ~(VW - 1), sh = kr0 - kra;
-    auto rowi = [&](int q) { return VW * tid + (q % VW) + (q / VW) * (VW * PT) - sh; };
-    double v[RPT][NBW];
-    int pos[RPT];
-    uint32_t pivmask = 0;
-#pragma unroll
-    for (int g = 0; g < RPT / VW; ++g) {
-        const int64_t base = (int64_t)kra + VW * tid + g * (VW * PT);  // first row of the vector
-#pragma unroll
-        for (int j = 0; j < NBW; ++j) {
-            int32_t x[VW];
-#pragma unroll
-            for (int e = 0; e < VW; ++e) x[e] = 0;
-            if (j < w && base < ldw) load_rows<VW>(W + base + (int64_t)(c0 + j) * ldw, x);
-#pragma unroll
-            for (int e = 0; e < VW; ++e) {
-                const int i = rowi(g * VW + e);
-                // rows above kr0 keep their (final) values: the in-place
-                // stores at the end write them back unchanged
-                v[g * VW + e][j] = i < rows ? (double)x[e] : 0.0;
-            }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < RPT; ++q) pos[q] = rowi(q);
-    if (tid == 0) s_cnt = 0;
-
-    // rows that exist (bit q: register row q is a panel row)
-    uint32_t live = 0;
-#pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-        const int i = rowi(q);
-        if (i >= 0 && i < rows) live |= 1u << q;
-    }
-    int pc = 0, status = 0, consumed = w, par = 0;
-    bool active = true;
-    // One step per panel column, unrolled at compile time so that v[][jc]
-    // is a register.  Every step runs, also after the panel has stopped or
-    // past its width, with a zero update: the step is straight-line code,
-    // so the register array is never copied between branches.  Per-thread
-    // work is kept to the rows the thread owns: the pivot row is published
-    // unreduced, and its reduction and normalisation are spread over the
-    // lanes (lane j handles column j) and broadcast back with readlane.
-    auto step = [&](auto JC) __attribute__((always_inline)) {
-        constexpr int jc = decltype(JC)::value;
-        const bool run = active && jc < w && pc < rows;
-        if (active && jc < w && pc >= rows) {
-            status = 2;
-            consumed = jc;
-            active = false;
-        }
-        // this thread's best row among those not yet pivots; column jc is
-        // final after this step, so it is reduced here once and for all
-        const uint32_t elig = run ? live & ~pivmask : 0u;
-        key_t mine = 0;
-        int mq = 0;
-#pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            if (SMALL) v[q][jc] = dmod_near(v[q][jc], mp);
-            // selects, not branches: keys of rows that are not eligible are 0
-            const key_t k = ((elig >> q) & 1u) ? K::make((uint32_t)v[q][jc], pos[q]) : (key_t)0;
-            const bool better = k > mine;
-            mine = better ? k : mine;
-            mq = better ? q : mq;
-        }
-        // every lane fetches the inverse of its own candidate before the wave
-        // reduction, so the table load overlaps it
-        const uint32_t myinv = (invtab && K::val(mine) != 0) ? invtab[K::val(mine)] : 0u;
-        const key_t wbest = wave_max(mine);
-        // the lane holding the wave's candidate (keys are unique) publishes
-        // its index and inverse; its register row is made wave-uniform, so
-        // the row is published through a scalar branch per register row
-        // rather than a per-lane select over all of them
-        const uint64_t wmask = __ballot(mine == wbest && K::val(wbest) != 0);
-        if (wmask) {
-            const int wl = (int)__builtin_ctzll(wmask);
-            const int wq = __builtin_amdgcn_readlane(mq, wl);
-            if (lane == wl) {
-                s_cinv[par][wave] = invtab ? myinv : modinv_fast(K::val(wbest), mp);
-                s_cidx[par][wave] = rowi(mq);
-            }
-            // one divergent branch (the winning lane), then scalar branches
-            // on the wave-uniform register row
-            auto publish = [&](auto Q) __attribute__((always_inline)) {
-                constexpr int q = decltype(Q)::value;
-                if (wq == q) {
-#pragma unroll
-                    for (int j = 0; j < NBW; ++j)
-                        if (j > jc) s_crow[par][wave][j] = v[q][j];
-                    // keeps the cases' stores apart: merged, they would
-                    // become one store of an indexed (scratch) register row
-                    asm volatile("" ::: "memory");
-                }
-            };
-            if (lane == wl) Unroll<0, RPT>::run(publish);
-        }
-        if (lane == 0) s_key[par][wave] = wbest;
-        __syncthreads();
-        key_t best = s_key[par][0];
-        int bw = 0;
-#pragma unroll
-        for (int x = 1; x < NW; ++x) {
-            const key_t k = s_key[par][x];
-            if (k > best) { best = k; bw = x; }
-        }
-        bw = uniform(bw);
-        const int cp = par;
-        par ^= 1;
-        const uint32_t V = (uint32_t)uniform((int)K::val(best));
-        const int Ip = uniform(K::pos(best));
-        const uint32_t inv = V != 0 ? (uint32_t)uniform((int)s_cinv[cp][bw]) : 0u;
-        const int wrow = V != 0 ? uniform(s_cidx[cp][bw]) : -1;
-        const bool piv = run && V != 0 && inv != 0;
-        if (run && V == 0) {
-            if (ple) {
-                if (tid == 0) s_cmap[jc] = -1;
-            } else {
-                status = 1;
-                consumed = jc;
-                active = false;
-            }
-        }
-        if (run && V != 0 && inv == 0) {
-            status = 3;
-            consumed = jc;
-            active = false;
-        }
-        // positions: the winner moves to pc, the row at pc moves to Ip
-        if (piv) {
-#pragma unroll
-            for (int q = 0; q < RPT; ++q) {
-                const bool win = rowi(q) == wrow;
-                pivmask |= win ? 1u << q : 0u;
-                pos[q] = win ? pc : (pos[q] == pc ? Ip : pos[q]);
-            }
-        }
-        // normalised pivot row: lane j reduces and scales column j, wave 0
-        // keeps it for the output, readlane hands every lane the values
-        uint32_t ul = 0;
-        if (piv && lane > jc && lane < NBW) {
-            const double x = s_crow[cp][bw][lane];
-            const uint32_t r = (uint32_t)(SMALL ? dmod_near(x, mp) : x);
-            ul = mulmod_t<SMALL>(r, inv, mp);
-            if (wave == 0) s_U[pc][lane] = ul;
-        }
-        double u[NBW];
-#pragma unroll
-        for (int j = 0; j < NBW; ++j) u[j] = j > jc ? (double)(uint32_t)__builtin_amdgcn_readlane((int)ul, j) : 0.0;
-        // rank-1 update of the rows that are not pivots (a zero update when
-        // this step found no pivot)
-        const uint32_t upd = live & ~pivmask;
-#pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            const double l = ((upd >> q) & 1u) ? v[q][jc] : 0.0;
-#pragma unroll
-            for (int j = 0; j < NBW; ++j)
-                if (j > jc) {
-                    v[q][j] = fma(-l, u[j], v[q][j]);
-                    if (!SMALL) v[q][j] = dmod(v[q][j], mp);
-                }
-        }
-        if (piv && tid == 0) {
-            s_ip[pc] = Ip;
-            s_pv[pc] = (int)V;
-            s_pi[pc] = (int)inv;
-            s_pcol[pc] = jc;
-            s_cmap[jc] = pc;
-        }
-        pc += piv ? 1 : 0;
-    };
-    Unroll<0, NBW>::run(step);
-    __syncthreads();
-
-    // Row gather map: positions 0..pc-1 first, in order, then every other
-    // row that moved.
-#pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-        const int i = rowi(q);
-        if (i >= 0 && i < rows) {
-            const int dst = kr0 + pos[q];
-            if (pos[q] < pc) {
-                map_dst[pos[q]] = dst;
-                map_src[pos[q]] = kr0 + i;
-                s_msrc[pos[q]] = kr0 + i;
-            } else if (pos[q] != i) {
-                const int e = pc + atomicAdd(&s_cnt, 1);
-                map_dst[e] = dst;
-                map_src[e] = kr0 + i;
-                s_msrc[e] = kr0 + i;
-            }
-        }
-    }
-    __syncthreads();
-    // The old values of every moved row in the block's other columns go to
-    // the stage (stage[e + 64 ci], ci counting the block columns left of the
-    // panel, then those right of it) for the update kernel; the loads are
-    // issued here and stored after the panel's own stores.
-    constexpr int SPT = (2 * NBW * NBO + PT - 1) / PT;
-    const int nmap_all = pc + s_cnt, ncol_other = (FAR - KC) - w, nstage = nmap_all * ncol_other;
-    int32_t sv[SPT];
-#pragma unroll
-    for (int k = 0; k < SPT; ++k) {
-        const int idx = tid + k * PT;
-        if (idx < nstage) {
-            const int e = idx % nmap_all, ci = idx / nmap_all;
-            const int c = ci < c0 - KC ? KC + ci : KC + ci + w;
-            sv[k] = W[(int64_t)s_msrc[e] + (int64_t)c * ldw];
-        }
-    }
-
-    // Every row to its final position, in two passes: first every row is
-    // stored in place with one vector store per VW rows and column (no
-    // per-row branches), then, once those stores are complete, the rows
-    // that moved and the pivot rows (1 at the pivot column, the normalised
-    // U row after it) overwrite their destinations.  The rows that moved
-    // leave exactly the positions that other moved rows fill, so every
-    // in-place value that is wrong is overwritten.
-    {
-        // the values are converted first and the stores issued back to back
-        // (full-width panels need no per-column test)
-        const int64_t basev = (int64_t)kra + VW * tid;
-        int32_t out[RPT][NBW];
-#pragma unroll
-        for (int q = 0; q < RPT; ++q)
-#pragma unroll
-            for (int j = 0; j < NBW; ++j) out[q][j] = (int32_t)(uint32_t)v[q][j];
-#pragma unroll
-        for (int g = 0; g < RPT / VW; ++g) {
-            const int64_t base = basev + g * (VW * PT);
-            int32_t *pg = W + base + (int64_t)c0 * ldw;
-            if (base + VW <= (int64_t)m) {
-                if (w == NBW) {
-#pragma unroll
-                    for (int j = 0; j < NBW; ++j) store_rows<VW>(pg + (int64_t)j * ldw, &out[g * VW][j], NBW);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < NBW; ++j)
-                        if (j < w) store_rows<VW>(pg + (int64_t)j * ldw, &out[g * VW][j], NBW);
-                }
-            }
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-        const int i = rowi(q);
-        const bool pv = (pivmask >> q) & 1u;
-        const bool tail = i >= 0 && i < rows && kra + VW * tid + (q / VW) * (VW * PT) + VW > m;
-        if (i >= 0 && i < rows && (pv || pos[q] != i || tail)) {
-            const int64_t dst = (int64_t)kr0 + pos[q];
-            const int k = pos[q], jk = pv ? s_pcol[k] : NBW;
-#pragma unroll
-            for (int j = 0; j < NBW; ++j)
-                if (j < w)
-                    W[dst + (int64_t)(c0 + j) * ldw] =
-                        (int32_t)(j < jk ? (uint32_t)v[q][j] : (j == jk ? 1u : s_U[k][j]));
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < SPT; ++k) {
-        const int idx = tid + k * PT;
-        if (idx < nstage) stage[idx % nmap_all + 64 * (idx / nmap_all)] = sv[k];
-    }
-    if (tid < pc) {
-        ipiv[kr0 + tid] = kr0 + s_ip[tid];
-        pivval[kr0 + tid] = s_pv[tid];
-        pivinv[kr0 + tid] = s_pi[tid];
-        pivcol[kr0 + tid] = c0 + s_pcol[tid];
-    }
-    if (tid < w) colmap[tid] = tid < consumed ? s_cmap[tid] : -1;
-    if (tid == 0) {
-        ctl->npiv = pc;
-        ctl->status = status;
-        ctl->ncols = consumed;
-        ctl->nmap = pc + s_cnt;
-        ctl->kr0 = kr0;
-        if (cursor) *cursor = kr0 + pc;
-        if (abort && status != 0) *abort = 1;
-    }
-}
-
 // Panel factorisation for any number of rows (the register panel holds at
-// most 32 x 512 rows and its small-prime key 2^15 positions): the same
-// outputs as k_panel from one 1024-thread workgroup that keeps the panel in
+// most 16,384 and its keys 2^15 positions): the same outputs as k_panel from one 1024-thread workgroup that keeps the panel in
 // W.  Thread t owns local rows t + 1024 q and is the only thread that reads
 // or writes them during the column steps; a row's current position (the
 // reference's swap of positions pc and Ip) is kept in gpos[row], the row at
@@ -489,10 +52,9 @@ __global__ __launch_bounds__(PT) void k_panel(int32_t *__restrict__ W, int64_t l
 constexpr int GPT = 1024, GNBW = 16;
 template <int NBW>
 __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_t ldw, int m, int kr0_in, int c0,
-                                                 int w, ModP mp, int ple, const uint32_t *__restrict__ invtab,
-                                                 int32_t *__restrict__ ipiv, int32_t *__restrict__ pivval,
-                                                 int32_t *__restrict__ pivinv, int32_t *__restrict__ pivcol,
-                                                 int32_t *__restrict__ colmap, int32_t *__restrict__ map_dst,
+                                                 int w, ModP mp, int ple, int32_t *__restrict__ ipiv,
+                                                 int32_t *__restrict__ pivval, int32_t *__restrict__ pivinv,
+                                                 int32_t *__restrict__ pivcol, int32_t *__restrict__ map_dst,
                                                  int32_t *__restrict__ map_src, PanelCtl *__restrict__ ctl,
                                                  int *__restrict__ abort, int KC, int FAR, int32_t *__restrict__ stage,
                                                  int *__restrict__ cursor, int32_t *__restrict__ gpos,
@@ -515,7 +77,7 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
     __shared__ uint32_t s_cinv[NW];
     __shared__ uint32_t s_crow[NW][NBW];
     __shared__ uint32_t s_U[NBW][NBW];
-    __shared__ int s_ip[NBW], s_pv[NBW], s_pi[NBW], s_pcol[NBW], s_cmap[NBW];
+    __shared__ int s_ip[NBW], s_pv[NBW], s_pi[NBW], s_pcol[NBW];
     __shared__ int s_msrc[2 * NBW], s_mdst[2 * NBW];
     __shared__ uint32_t s_mv[2 * NBW][NBW];
     __shared__ int s_cnt;
@@ -559,7 +121,7 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
             const uint32_t V = (uint32_t)(mine >> 32);
             s_key[wave] = mine;
             s_row[wave] = mrow;
-            s_cinv[wave] = invtab ? invtab[V] : modinv_fast(V, mp);
+            s_cinv[wave] = modinv_fast(V, mp);
             for (int j = jc + 1; j < NBW; ++j) s_crow[wave][j] = j < w ? (uint32_t)P[mrow + (int64_t)j * ldw] : 0u;
         }
         if (lane == 0 && wbest == 0) s_key[wave] = 0;
@@ -579,9 +141,7 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
         const int wrow = V != 0 ? s_row[bw] : -1;
         const bool piv = run && V != 0 && inv != 0;
         if (run && V == 0) {
-            if (ple) {
-                if (tid == 0) s_cmap[jc] = -1;
-            } else {
+            if (!ple) {
                 status = 1;
                 consumed = jc;
                 active = false;
@@ -604,7 +164,6 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
                 s_pv[pc] = (int)V;
                 s_pi[pc] = (int)inv;
                 s_pcol[pc] = jc;
-                s_cmap[jc] = pc;
             }
             if (tid > jc && tid < NBW) s_U[pc][tid] = tid < w ? mulmod(s_crow[bw][tid], inv, mp) : 0u;
         }
@@ -672,7 +231,6 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
         pivinv[kr0 + tid] = s_pi[tid];
         pivcol[kr0 + tid] = c0 + s_pcol[tid];
     }
-    if (tid < w) colmap[tid] = tid < consumed ? s_cmap[tid] : -1;
     if (tid == 0) {
         ctl->npiv = pc;
         ctl->status = status;
@@ -1062,25 +620,6 @@ __global__ __launch_bounds__(256) void k_trsm_upper_unit(int32_t *__restrict__ W
     }
 }
 
-template <int RPT, int NBW>
-int launch_panel(modp_ctx *ctx, int32_t *W, int64_t ldw, int m, int kr0, int c0, int w, const ModP &mp, int ple,
-                 const uint32_t *invtab, int32_t *ipiv, int32_t *pivval, int32_t *pivinv, int32_t *pivcol,
-                 int32_t *colmap, int32_t *map_dst, int32_t *map_src, PanelCtl *ctl, int *abort, int KC, int FAR,
-                 int32_t *stage, int *cursor)
-{
-    TimedLaunch tl(ctx, "elim_panel");
-    const size_t shm = 0;
-    if (mp.small)
-        k_panel<RPT, NBW, true><<<1, PT, shm, ctx->stream>>>(W, ldw, m, kr0, c0, w, mp, ple, invtab, ipiv, pivval,
-                                                            pivinv, pivcol, colmap, map_dst, map_src, ctl, abort,
-                                                            KC, FAR, stage, cursor);
-    else
-        k_panel<RPT, NBW, false><<<1, PT, shm, ctx->stream>>>(W, ldw, m, kr0, c0, w, mp, ple, invtab, ipiv, pivval,
-                                                             pivinv, pivcol, colmap, map_dst, map_src, ctl, abort,
-                                                             KC, FAR, stage, cursor);
-    return hip_check(ctx, hipGetLastError(), "k_panel launch");
-}
-
 unsigned grid_for(int64_t total, int64_t cap = 16384)
 {
     int64_t b = (total + 255) / 256;
@@ -1093,38 +632,27 @@ int64_t rup(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 
 __global__ void k_set_int(int *p, int v) { *p = v; }
 
-__global__ void k_inv_table(uint32_t *__restrict__ t, ModP mp)
+// t[a] = a^{-1} mod p for a < n, 0 where there is none
+__global__ void k_inv_table(uint32_t *__restrict__ t, int n, ModP mp)
 {
-    for (int64_t a = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; a < mp.p; a += (int64_t)gridDim.x * blockDim.x)
-        t[a] = a == 0 ? 0u : modinv((uint32_t)a, mp);
+    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a < n) t[a] = a > 0 && a < mp.p ? modinv((uint32_t)a, mp) : 0u;
 }
 
-// Inverses of every residue for p <= 2^22 (at most 16 MB), built once per
-// modulus and kept in the context: the panel's pivot inverse becomes one load.
+// Inverses of the residues below PINV, from which the panels make every other
+// inverse; built once per modulus and kept in the context.
 const uint32_t *inverse_table(modp_ctx *ctx, const ModP &mp, int *st)
 {
-    if (mp.p > ((int64_t)1 << 22)) return nullptr;
     if (ctx->invtab && ctx->invtab_p == mp.p) return ctx->invtab;
-    const size_t need = sizeof(uint32_t) * (size_t)mp.p;
-    if (ctx->invtab_cap < need) {
-        if (ctx->invtab) {
-            hipError_t e = hipStreamSynchronize(ctx->stream);
-            const hipError_t ef = hipFree(ctx->invtab);
-            ctx->invtab = nullptr;
-            ctx->invtab_cap = 0;
-            if (e == hipSuccess) e = ef;
-            if (e != hipSuccess) { *st = hip_check(ctx, e, "inverse table release"); return nullptr; }
-        }
-        hipError_t e = hipMalloc(&ctx->invtab, need);
+    if (!ctx->invtab) {
+        hipError_t e = hipMalloc(&ctx->invtab, sizeof(uint32_t) * PINV);
         if (e != hipSuccess) { *st = hip_check(ctx, e, "inverse table"); return nullptr; }
-        ctx->invtab_cap = need;
     }
-    k_inv_table<<<grid_for(mp.p, 4096), 256, 0, ctx->stream>>>(ctx->invtab, mp);
+    k_inv_table<<<PINV / 256, 256, 0, ctx->stream>>>(ctx->invtab, PINV, mp);
     if (hipGetLastError() != hipSuccess) { *st = MODP_ERR_DEVICE; return nullptr; }
     ctx->invtab_p = mp.p;
     return ctx->invtab;
 }
-
 
 }  // namespace
 
@@ -1144,35 +672,23 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     if (m > (int64_t)1 << 30)
         return set_error(ctx, MODP_ERR_DIM, "elimination supports at most 2^30 rows (got %lld)", (long long)m);
 
-    // Panel shape of an outer block starting at row KR: the fewest rows per
-    // thread that hold every row from KR's 4-aligned row down (the panel
-    // kernel reads 4-row vectors from kr0 & ~3 >= KR & ~3), and the panel
-    // width for that many rows per thread (rows per thread x width <= 64
-    // registers; widths measured at 2048 and 4096 rows).  Late blocks have
-    // fewer rows, so their panels are shorter and wider.
-    const char *wenv = getenv("MODP_PANEL_W");
-    const int want_w = wenv ? atoi(wenv) : 0;
+    // Panels of an outer block starting at row KR by the rows left: the register
+    // panel of one workgroup (256 rows: one wave per SIMD) or of one XCD, the
+    // W-resident panel beyond 16,384 rows.  Mod 65521 a 32-column panel takes
+    // 37 us on one workgroup and 49 us on an XCD, whatever its rows (one
+    // workgroup with 512 rows, two waves per SIMD: 58 us).
     // MODP_PANEL_GLOBAL=1 sends every panel to the W-resident kernel (used
     // to compare the two panel kernels at sizes both handle)
     const char *genv = getenv("MODP_PANEL_GLOBAL");
     const bool force_global = genv && atoi(genv) != 0;
-    auto panel_shape = [&](int64_t KR, int *RPT, int *NBW) {
-        const int64_t need = m - (KR & ~(int64_t)3);
-        if (force_global || need > (int64_t)32 * PT) {
-            // more rows than the register panel holds: W-resident panel
-            *RPT = 0;
-            *NBW = GNBW;
-            return;
-        }
-        int r = 1;
-        while ((int64_t)r * PT < need) r *= 2;
-        int wd = r == 1 ? 32 : (r == 2 ? 16 : (r <= 8 ? 8 : 2));
-        // tuning override among the instantiated panel widths
-        if ((r <= 2 && (want_w == 16 || want_w == 32)) || (r == 4 && (want_w == 8 || want_w == 16)) ||
-            (r == 8 && (want_w == 4 || want_w == 8)))
-            wd = want_w;
-        *RPT = r;
-        *NBW = wd;
+    // the cycles that a workgroup of a panel on one XCD waits for the others to
+    // start before the panel is left to the W-resident kernel
+    // (MODP_PANEL_PATIENCE sets it: 0 makes every such panel give up)
+    const char *penv = getenv("MODP_PANEL_PATIENCE");
+    const long long patience = penv ? atoll(penv) : 50000000LL;
+    bool gave_up = false;  // in the previous outer block
+    auto panel_width = [&](int64_t KR) {
+        return force_global || gave_up || m - KR > PMULTI ? GNBW : PNW;
     };
 
     int st = MODP_OK;
@@ -1181,34 +697,52 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     if (!W) return st;
     // pivot arrays, per-panel control blocks and row gather maps of one outer block
     const size_t npv = (size_t)mn + 64;
-    const size_t piv_bytes = sizeof(int32_t) * (4 * npv + 64 + 2 * MAXPAN * 64) + sizeof(PanelCtl) * MAXPAN + 256 +
+    const size_t piv_bytes = sizeof(int32_t) * (4 * npv + 2 * MAXPAN * 64) + sizeof(PanelCtl) * MAXPAN + 512 +
                              sizeof(int32_t) * 64 * NBO;
     int32_t *piv = (int32_t *)ws_get(ctx, WS_PIV, piv_bytes, &st);
     if (!piv) return st;
     int32_t *ipiv = piv, *pivval = piv + npv, *pivinv = piv + 2 * npv, *pivcol = piv + 3 * npv;
-    int32_t *colmap = piv + 4 * npv;
-    int32_t *bmap_dst = colmap + 64, *bmap_src = bmap_dst + MAXPAN * 64;
+    int32_t *bmap_dst = piv + 4 * npv, *bmap_src = bmap_dst + MAXPAN * 64;
     PanelCtl *bctl = (PanelCtl *)(bmap_src + MAXPAN * 64);
     int *flag = (int *)(bctl + MAXPAN);
-    int32_t *stage = (int32_t *)(flag + 64);  // moved rows' old values, 64 x NBO
-    int *cursor = flag + 2;                   // first row of the next panel (lu, rref)
+    int *abort_flag = flag + 1;
+    int *cursor = flag + 2;                         // first row of the next panel (lu, rref)
+    uint32_t *arrive = (uint32_t *)(flag + 4);      // one word per panel of the block
+    int32_t *stage = (int32_t *)(arrive + MAXPAN);  // moved rows' old values, 64 x NBO
     int32_t *Ubig = (int32_t *)ws_get(ctx, WS_UBUF, sizeof(int32_t) * (size_t)NBO * (size_t)(n + 1), &st);
     if (!Ubig) return st;
     // row positions of the W-resident panel (position of each row, row at
     // each position)
     int32_t *gpos = nullptr, *grow = nullptr;
-    if (force_global || m > (int64_t)32 * PT) {
+    if (force_global || m > PSINGLE) {
         gpos = (int32_t *)ws_get(ctx, WS_GPOS, sizeof(int32_t) * 2 * (size_t)m, &st);
         if (!gpos) return st;
         grow = gpos + m;
     }
     PanelCtl *hctl = (PanelCtl *)pinned_get(ctx, sizeof(PanelCtl) * (MAXPAN + 1) + 64, &st);
     if (!hctl) return st;
-    int *abort_flag = flag + 1;
 
     MODP_TRY(util_convert(ctx, kind, m, n, A, lda, EK_I32, W, ldw, mp));
-    const uint32_t *invtab = inverse_table(ctx, mp, &st);
+    const uint32_t *invs = inverse_table(ctx, mp, &st);
     if (st != MODP_OK) return st;
+    // exchange area of the panels on one XCD: its words are recognised by
+    // tags that count the context's panels, so old ones are cleared only when
+    // the 17 bits of a key's tag (the 32 of a residue's) have been through
+    PanelExchange *xch = nullptr;
+    if (!force_global && m > PSINGLE) {
+        const bool fresh = !ctx->ws[WS_PANEL];
+        xch = (PanelExchange *)ws_get(ctx, WS_PANEL, sizeof(PanelExchange), &st);
+        if (!xch) return st;
+        if (fresh) ctx->panel_tag = 0;
+    }
+    auto next_tag = [&](uint32_t *t) -> int {
+        if ((ctx->panel_tag & 0x1ffffu) == 0)
+            HIP_TRY(ctx, hipMemsetAsync(xch, 0, ctx->panel_tag == 0 ? sizeof(PanelExchange) : sizeof(xch->key),
+                                        ctx->stream));
+        *t = ctx->panel_tag;
+        ctx->panel_tag += 64;
+        return MODP_OK;
+    };
 
     auto gemm_sub = [&](int64_t r0, int64_t rows, int64_t ca, int64_t cols, int64_t kcol, int64_t K,
                         const int32_t *Ub, int use_form, const int *skip) -> int {
@@ -1230,39 +764,47 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     const int big_form = form != MODP_FORM_AUTO ? form
                          : (m >= 1024 && n >= 1024) ? MODP_FORM_LIMB_I8 : choose_form(m, n, NBO, p);
 
-    // panel t of the current outer block at (rj, cj), width w
-    auto launch_panel_t = [&](int RPT, int NBW, int t, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w,
-                              int *abort, int *cursor) -> int {
+    // panel t of the current outer block at (rj, cj), width w; it has at most
+    // m - rj rows
+    auto launch_panel_t = [&](int width, int t, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w, int *abort,
+                              int *cursor) -> int {
         if (t >= MAXPAN) return set_error(ctx, MODP_ERR_DEVICE, "more than %d panels in an outer block", MAXPAN);
         int32_t *mdst = bmap_dst + t * 64, *msrc = bmap_src + t * 64;
         PanelCtl *pctl = bctl + t;
-        if (RPT == 0) {
-            TimedLaunch tl(ctx, "elim_panel");
-            k_panel_g<GNBW><<<1, GPT, 0, ctx->stream>>>(W, ldw, (int)m, (int)rj, (int)cj, (int)w, mp, ple, invtab, ipiv,
-                                                        pivval, pivinv, pivcol, colmap, mdst, msrc, pctl, abort,
+        TimedLaunch tl(ctx, "elim_panel");
+        if (width == GNBW) {
+            k_panel_g<GNBW><<<1, GPT, 0, ctx->stream>>>(W, ldw, (int)m, (int)rj, (int)cj, (int)w, mp, ple, ipiv,
+                                                        pivval, pivinv, pivcol, mdst, msrc, pctl, abort,
                                                         (int)KC, (int)FAR, stage, cursor, gpos, grow);
             return hip_check(ctx, hipGetLastError(), "k_panel_g launch");
         }
-        const int key = RPT * 100 + NBW;
-#define LAUNCH_PANEL(R_, W_) \
-    case R_ * 100 + W_: \
-        return launch_panel<R_, W_>(ctx, W, ldw, (int)m, (int)rj, (int)cj, (int)w, mp, ple, invtab, ipiv, pivval, \
-                                    pivinv, pivcol, colmap, mdst, msrc, pctl, abort, (int)KC, (int)FAR, stage, cursor);
-        switch (key) {
-            LAUNCH_PANEL(1, 16)
-            LAUNCH_PANEL(1, 32)
-            LAUNCH_PANEL(2, 16)
-            LAUNCH_PANEL(2, 32)
-            LAUNCH_PANEL(4, 8)
-            LAUNCH_PANEL(4, 16)
-            LAUNCH_PANEL(8, 4)
-            LAUNCH_PANEL(8, 8)
-            LAUNCH_PANEL(16, 2)
-            LAUNCH_PANEL(32, 2)
-        default:
-            return set_error(ctx, MODP_ERR_ARG, "no panel kernel for %d rows/thread x %d columns", RPT, NBW);
+        PanelArgs a = {};
+        a.W = W; a.ldw = ldw; a.m = (int)m; a.kr0 = (int)rj; a.c0 = (int)cj; a.w = (int)w; a.ple = ple;
+        a.KC = (int)KC; a.FAR = (int)FAR; a.mp = mp; a.invs = invs;
+        a.ipiv = ipiv; a.pivval = pivval; a.pivinv = pivinv; a.pivcol = pivcol;
+        a.map_dst = mdst; a.map_src = msrc; a.stage = stage; a.ctl = pctl; a.abort = abort; a.cursor = cursor;
+        const int mode = mp.small ? 0 : mp.p <= ((int64_t)1 << 24) ? 1 : 2;
+        if (m - rj <= PSINGLE) {
+            if (mode == 0) k_panel<false, 0><<<1, PSINGLE, 0, ctx->stream>>>(a);
+            else if (mode == 1) k_panel<false, 1><<<1, PSINGLE, 0, ctx->stream>>>(a);
+            else k_panel<false, 2><<<1, PSINGLE, 0, ctx->stream>>>(a);
+            return hip_check(ctx, hipGetLastError(), "k_panel launch");
         }
-#undef LAUNCH_PANEL
+        a.x = xch;
+        a.arrive = arrive + t;
+        a.G = (int)((m - rj + 255) / 256);
+        a.patience = patience;
+        MODP_TRY(next_tag(&a.tag));
+        const unsigned grid = 8 * (a.G - 1) + 1;
+        if (mode == 0) k_panel<true, 0><<<grid, 256, 0, ctx->stream>>>(a);
+        else if (mode == 1) k_panel<true, 1><<<grid, 256, 0, ctx->stream>>>(a);
+        else k_panel<true, 2><<<grid, 256, 0, ctx->stream>>>(a);
+        return hip_check(ctx, hipGetLastError(), "k_panel launch");
+    };
+    // abort flag, cursor and arrival words of a block
+    auto block_begin = [&]() -> int {
+        return hip_check(ctx, hipMemsetAsync(abort_flag, 0, (size_t)((char *)(arrive + MAXPAN) - (char *)abort_flag),
+                                             ctx->stream), "block flags");
     };
     // the rest of the outer block after panel t: its row moves, and right
     // of the panel the rows of U and the rank-npiv update below the pivots
@@ -1323,15 +865,15 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         if (nbo > NBO) nbo = NBO;
         if (nbo < 0) nbo = 0;  // pluq: only moved zero columns remain
         const int64_t FAR = KC + nbo;
-        int RPT, NBW;
-        panel_shape(KR, &RPT, &NBW);
+        const int NBW = panel_width(KR);
+        gave_up = false;
         bool stop_zero = false;
         if (!ple && nbo > 0) {
             // pluq: every panel of the block is enqueued assuming it finds a
             // pivot in each column; a panel that meets a zero column raises
             // the abort flag, which turns the rest of the block into no-ops,
             // and the block is completed from the host after one sync
-            HIP_TRY(ctx, hipMemsetAsync(abort_flag, 0, sizeof(int), ctx->stream));
+            MODP_TRY(block_begin());
             std::vector<int64_t> pr, pcj, pw;
             for (int64_t cj = KC; cj < FAR;) {
                 const int64_t rj = KR + (cj - KC);
@@ -1345,7 +887,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             const int np = (int)pr.size();
             int64_t Pfull = 0;
             for (int t = 0; t < np; ++t) {
-                MODP_TRY(launch_panel_t(RPT, NBW, t, KC, FAR, pr[t], pcj[t], pw[t], abort_flag, nullptr));
+                MODP_TRY(launch_panel_t(NBW, t, KC, FAR, pr[t], pcj[t], pw[t], abort_flag, nullptr));
                 MODP_TRY(update_t(t, KC, FAR, pr[t], pcj[t], pw[t], abort_flag));
                 Pfull += pw[t];
             }
@@ -1366,6 +908,9 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 if (hctl[ts].status == 3)
                     return set_error(ctx, MODP_ERR_NOT_INVERTIBLE,
                                      "pivot has no inverse modulo %lld (modulus not prime)", (long long)p);
+                if (hctl[ts].status == 6)
+                    return set_error(ctx, MODP_ERR_DEVICE, "an elimination panel's exchange did not end");
+                gave_up = hctl[ts].status == 5;
                 const int64_t npiv = hctl[ts].npiv;
                 int64_t P = 0;
                 for (int t = 0; t < ts; ++t) P += pw[t];
@@ -1385,7 +930,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             // runs out of rows (or meets a pivot without inverse) raises the
             // abort flag, which turns the rest of the block into no-ops, and
             // the host reads the outcome once per block.
-            HIP_TRY(ctx, hipMemsetAsync(abort_flag, 0, sizeof(int), ctx->stream));
+            MODP_TRY(block_begin());
             k_set_int<<<1, 1, 0, ctx->stream>>>(cursor, (int)KR);
             HIP_TRY(ctx, hipGetLastError());
             std::vector<int64_t> pcj, pw;
@@ -1395,7 +940,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             }
             const int np = (int)pcj.size();
             for (int t = 0; t < np; ++t) {
-                MODP_TRY(launch_panel_t(RPT, NBW, t, KC, FAR, KR, pcj[t], pw[t], abort_flag, cursor));
+                MODP_TRY(launch_panel_t(NBW, t, KC, FAR, KR, pcj[t], pw[t], abort_flag, cursor));
                 MODP_TRY(update_t(t, KC, FAR, KR, pcj[t], pw[t], abort_flag));
             }
             HIP_TRY(ctx, hipMemcpyAsync(hctl, bctl, sizeof(PanelCtl) * np, hipMemcpyDeviceToHost, ctx->stream));
@@ -1409,6 +954,9 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 if (pc.status == 3)
                     return set_error(ctx, MODP_ERR_NOT_INVERTIBLE,
                                      "pivot has no inverse modulo %lld (modulus not prime)", (long long)p);
+                if (pc.status == 6)
+                    return set_error(ctx, MODP_ERR_DEVICE, "an elimination panel's exchange did not end");
+                gave_up = pc.status == 5;
                 P += pc.npiv;
                 consumed += pc.ncols;
                 if (pc.status != 0) {
