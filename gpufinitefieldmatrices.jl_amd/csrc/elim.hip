@@ -745,7 +745,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     };
 
     auto gemm_sub = [&](int64_t r0, int64_t rows, int64_t ca, int64_t cols, int64_t kcol, int64_t K,
-                        const int32_t *Ub, int use_form, const int *skip) -> int {
+                        const int32_t *Ub, const int *skip) -> int {
         if (rows <= 0 || cols <= 0 || K <= 0) return MODP_OK;
         GemmArgs g;
         g.m = rows; g.n = cols; g.k = K;
@@ -755,15 +755,10 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         g.epi = EPI_SUB;
         g.mp = mp;
         g.skip = skip;
+        const int use_form = form != MODP_FORM_AUTO ? form : choose_form(rows, cols, K, p);
         if (use_form == MODP_FORM_LIMB_I8) return gemm_limb_i8(ctx, g);
         return gemm_plain_f64(ctx, g);
     };
-    // the trailing updates have K = 128, below the general limb threshold,
-    // but at 1024 x 1024 and beyond the limb form's split passes are paid
-    // back (4096^2 PLUQ: 17.6 ms limb vs 19.0 ms plain)
-    const int big_form = form != MODP_FORM_AUTO ? form
-                         : (m >= 1024 && n >= 1024) ? MODP_FORM_LIMB_I8 : choose_form(m, n, NBO, p);
-
     // panel t of the current outer block at (rj, cj), width w; it has at most
     // m - rj rows
     auto launch_panel_t = [&](int width, int t, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w, int *abort,
@@ -851,7 +846,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             HIP_TRY(ctx, hipGetLastError());
         }
         const int64_t rbeg = KR + P;
-        return gemm_sub(rbeg, m - rbeg, FAR, n - FAR, KC, consumed, Ubig + (FAR - KC) * NBO, big_form, skip);
+        return gemm_sub(rbeg, m - rbeg, FAR, n - FAR, KC, consumed, Ubig + (FAR - KC) * NBO, skip);
     };
 
     std::vector<int64_t> col_stack;
@@ -1074,8 +1069,6 @@ int elim_rref(modp_ctx *ctx, int form, int kind, int64_t m, int64_t n, const voi
     if (rank > 1) {
         int32_t *G = (int32_t *)ws_get(ctx, WS_SCRATCH, sizeof(int32_t) * (size_t)(rank + 64) * 64, &st);
         if (!G) return st;
-        const int bform = form != MODP_FORM_AUTO ? form
-                          : (m >= 1024 && n >= 1024) ? MODP_FORM_LIMB_I8 : MODP_FORM_PLAIN_F64;
         for (int64_t i1 = rank; i1 > 0;) {
             const int64_t i0 = i1 > 64 ? i1 - 64 : 0;
             const int nb = (int)(i1 - i0);
@@ -1098,6 +1091,7 @@ int elim_rref(modp_ctx *ctx, int form, int kind, int64_t m, int64_t n, const voi
                 g.C = W + cs * ldw; g.ldc = ldw; g.kc = EK_I32;
                 g.epi = EPI_SUB;
                 g.mp = mp;
+                const int bform = form != MODP_FORM_AUTO ? form : choose_form(g.m, g.n, g.k, p);
                 if (bform == MODP_FORM_LIMB_I8 && nb >= 64) MODP_TRY(gemm_limb_i8(ctx, g));
                 else MODP_TRY(gemm_plain_f64(ctx, g));
             }

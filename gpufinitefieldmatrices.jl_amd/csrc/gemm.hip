@@ -13,6 +13,8 @@
 // Both forms can cut K into slices that run concurrently (blockIdx.y) and are
 // summed mod p afterwards, for products whose output grid alone leaves CUs
 // idle.
+#include <algorithm>
+
 #include "gemm_limb.h"
 #include "gemm_tile.h"
 
@@ -40,6 +42,69 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64(int64_t m, int64_t n, int64
     __shared__ F64Smem<BM, BN> sm;
     gemm_f64_tile<TA, TB, TC, BM, BN, EPI, RED>(m, n, klen, A + kb * lda, lda, B + kb, ldb, C + blockIdx.y * cslice,
                                                 ldc, mp, rq, tm * BM, tn * BN, sm);
+}
+
+// The plain form of a small product: one workgroup per 16 x 16 block of C,
+// its four waves taking a quarter of K each and their residues summed in LDS.
+// Such a product is bound by latency, so there are no LDS stages and no
+// barriers before the sum: a wave loads the MFMA fragments of eight k4-steps
+// straight from the operands (16 runs of 16 rows of A, 16 columns of B), all
+// before it uses one.  The block is computed transposed, so a lane holds one
+// row.  48 x 40 x 56 mod 11: 8.6 -> 3.5 us (64 x 64 tiles in stages of 16 k).
+template <typename T, typename TC, int EPI>
+__global__ __launch_bounds__(256) void k_gemm_f64_small(int64_t m, int64_t n, int64_t k, const T *__restrict__ A,
+                                                        int64_t lda, const T *__restrict__ B, int64_t ldb,
+                                                        TC *__restrict__ C, int64_t ldc, ModP mp, int R,
+                                                        const int *__restrict__ skip)
+{
+    if (skip && *skip) return;
+    constexpr int U = 8;
+    __shared__ double part[4][16][17];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t mt = (m + 15) / 16;
+    const int64_t r0 = (blockIdx.x % mt) * 16, c0 = (blockIdx.x / mt) * 16;
+    const int64_t kq = (k + 15) / 16 * 4;  // a wave's share of K, in whole k4-steps
+    const int64_t kbeg = wave * kq, kend = min(k, kbeg + kq);
+    const int64_t row = r0 + (lane & 15), col = c0 + (lane & 15);
+    const bool row_ok = row < m, col_ok = col < n;
+    const T *a = A + (row_ok ? row : 0), *b = B + (col_ok ? col : 0) * ldb;
+    const int q = lane >> 4;
+    v4d acc = {0.0, 0.0, 0.0, 0.0};
+    int cnt = 0;
+    for (int64_t k0 = kbeg; k0 < kend; k0 += 4 * U) {
+        T xa[U], xb[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t kk = min(k0 + 4 * u + q, k - 1);
+            xa[u] = a[kk * lda];
+            xb[u] = b[kk];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool in = k0 + 4 * u + q < kend;
+            const double fa = in && row_ok ? bal_of<T>(xa[u], mp) : 0.0;
+            const double fb = in && col_ok ? bal_of<T>(xb[u], mp) : 0.0;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(fb, fa, acc, 0, 0, 0);
+            if (++cnt == R) {
+                cnt = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] = fma(-rint(acc[e] * mp.pinv), mp.pd, acc[e]);
+            }
+        }
+    }
+    // lane: row lane % 16, columns lane / 16 + 4 e
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        part[wave][q + 4 * e][lane & 15] = fma(-rint(acc[e] * mp.pinv), mp.pd, acc[e]);
+    __syncthreads();
+    const int rl = tid & 15, cl = tid >> 4;
+    const double s = part[0][cl][rl] + part[1][cl][rl] + part[2][cl][rl] + part[3][cl][rl];
+    if (r0 + rl < m && c0 + cl < n) {
+        uint32_t v = (uint32_t)dmod(s, mp);
+        TC *dst = C + (r0 + rl) + (c0 + cl) * ldc;
+        if (EPI == EPI_SUB) v = submod(to_res<TC>(*dst, mp), v, mp);
+        *dst = from_res<TC>(v);
+    }
 }
 
 // C = epi(C, sum of S slice results mod p); slice s holds m x n residues at
@@ -171,6 +236,38 @@ int launch_f64(modp_ctx *ctx, const GemmArgs &g, int R, int tile, const Slices &
                      g.ka, g.kb, g.kc, g.epi);
 }
 
+// Blocks of 16 x 16 times K, what k_gemm_f64_small reads (every block its own
+// rows and columns), if it takes the product at all: at most 1024 blocks (four
+// workgroups per CU; 1024^2 x 32, 4096 blocks: 21 us against 7.8 in 64 x 64
+// tiles) and K up to 1024; else -1.
+int64_t small_work(int64_t m, int64_t n, int64_t k)
+{
+    const int64_t blocks = ((m + 15) / 16) * ((n + 15) / 16);
+    return blocks <= 1024 && k <= 1024 && k > 0 ? blocks * k : -1;
+}
+// against 64 x 64 tiles it pays up to 512 x 512 x 256 (11.9 us, 23 in tiles)
+bool f64_small(const GemmArgs &g)
+{
+    const int64_t w = small_work(g.m, g.n, g.k);
+    return w >= 0 && w <= 262144 && g.ka == g.kb && g.ka == g.kc &&
+           (g.epi == EPI_STORE || (g.epi == EPI_SUB && g.kc == EK_I32));
+}
+int launch_f64_small(modp_ctx *ctx, const GemmArgs &g, int R)
+{
+    TimedLaunch tl(ctx, "gemm_f64");
+    const unsigned grid = (unsigned)(((g.m + 15) / 16) * ((g.n + 15) / 16));
+#define SMALL(T_, EPI_)                                                                                             \
+    k_gemm_f64_small<T_, T_, EPI_><<<grid, 256, 0, ctx->stream>>>(g.m, g.n, g.k, (const T_ *)g.A, g.lda,             \
+                                                                  (const T_ *)g.B, g.ldb, (T_ *)g.C, g.ldc, g.mp, R, \
+                                                                  g.skip)
+    if (g.ka == EK_F64) SMALL(double, EPI_STORE);
+    else if (g.ka == EK_F32) SMALL(float, EPI_STORE);
+    else if (g.epi == EPI_STORE) SMALL(int32_t, EPI_STORE);
+    else SMALL(int32_t, EPI_SUB);
+#undef SMALL
+    return hip_check(ctx, hipGetLastError(), "k_gemm_f64_small launch");
+}
+
 template <typename TC>
 int launch_slice_sum_t(modp_ctx *ctx, const GemmArgs &g, int epi, const int32_t *P, int S)
 {
@@ -199,25 +296,26 @@ int32_t *slice_buffer(modp_ctx *ctx, const GemmArgs &g, int S, int *st)
     return (int32_t *)ws_get(ctx, WS_SLICES, sizeof(int32_t) * (size_t)S * (size_t)g.m * (size_t)g.n, st);
 }
 
-template <typename TA>
-int split_a_t(modp_ctx *ctx, const GemmArgs &g, const void *A, int64_t kbeg, int64_t kc, int8_t *Al,
-              int64_t Mp, int64_t Kp, int L, int32_t top)
+// digit planes of k in [kbeg, kbeg + kc) of both operands (of one type)
+template <typename T>
+int split_t(modp_ctx *ctx, const GemmArgs &g, int64_t kbeg, int64_t kc, int8_t *Al, int64_t Mp, int8_t *Bl, int64_t Np,
+            int64_t Kp, int L)
 {
-    dim3 grid((unsigned)(Kp / 64), (unsigned)(Mp / 64));
-    const TA *Ap = (const TA *)A + kbeg * g.lda;
-    k_split_a<TA><<<grid, 256, 0, ctx->stream>>>(g.m, kc, Ap, g.lda, Al, Mp, Kp, L, top, g.mp, g.skip);
-    return hip_check(ctx, hipGetLastError(), "k_split_a launch");
-}
-
-template <typename TB>
-int split_b_t(modp_ctx *ctx, const GemmArgs &g, const void *B, int64_t kbeg, int64_t kc, int8_t *Bl,
-              int64_t Np, int64_t Kp, int L, int32_t top)
-{
-    int64_t total = Np * (Kp / 4);
-    unsigned grid = (unsigned)((total + 255) / 256);
-    const TB *Bp = (const TB *)B + kbeg;
-    k_split_b<TB><<<grid, 256, 0, ctx->stream>>>(kc, g.n, Bp, g.ldb, Bl, Np, Kp, L, top, g.mp, g.skip);
-    return hip_check(ctx, hipGetLastError(), "k_split_b launch");
+    const unsigned na = (unsigned)((Mp / 64) * (Kp / 64));
+    const unsigned nb = (unsigned)((Np * (Kp / 4) + 1023) / 1024);
+    const T *A = (const T *)g.A + kbeg * g.lda, *B = (const T *)g.B + kbeg;
+    TimedLaunch tl(ctx, "gemm_split");
+#define SPLIT(L_)                                                                                                  \
+    k_split_ab<T, L_><<<na + nb, 256, 0, ctx->stream>>>(g.m, g.n, kc, A, g.lda, B, g.ldb, Al, Mp, Bl, Np, Kp, na, \
+                                                        g.mp, g.skip)
+    switch (L) {
+    case 1: SPLIT(1); break;
+    case 2: SPLIT(2); break;
+    case 3: SPLIT(3); break;
+    default: SPLIT(4); break;
+    }
+#undef SPLIT
+    return hip_check(ctx, hipGetLastError(), "k_split_ab launch");
 }
 
 int launch_limb(modp_ctx *ctx, const GemmArgs &g, int L, int epi, const int8_t *Al, int64_t Mp,
@@ -255,6 +353,7 @@ int gemm_plain_cfg(modp_ctx *ctx, const GemmArgs &g, const GemmConfig &cfg)
     if (g.m <= 0 || g.n <= 0) return MODP_OK;
     const int R = f64_reduce_interval(g.mp.p);
     if (R < 1) return set_error(ctx, MODP_ERR_MODULUS_RANGE, "modulus %lld too large for the FP64 form", (long long)g.mp.p);
+    if (f64_small(g)) return launch_f64_small(ctx, g, R);
     const int tile = cfg.tile_m == 128 ? 128 : 64;
     Slices sl = make_slices(g.k, cfg.ksplit, PBK, 64);
     if (sl.S == 1) {
@@ -271,6 +370,19 @@ int gemm_plain_cfg(modp_ctx *ctx, const GemmArgs &g, const GemmConfig &cfg)
     return launch_slice_sum(ctx, g, g.epi, P, sl.S);
 }
 
+// Output tile that a limb configuration's workgroups take.  With one digit
+// the 128x128 configuration runs 256x256 tiles (twice the MFMA work per LDS
+// byte) on products with at least one for every two CUs and a K that pays for
+// their longer epilogue: float32 mod 127, 3072^3 73.6 us against 80.9, 4096^3
+// 115 against 131, 5000^3 222 against 263, 8192^3 743 against 928; but 2560^3
+// (100 tiles) 63.5 against 49.3, 3000 x 6000 x 500 55.9 against 43.6.
+void limb_tile(const GemmConfig &cfg, int L, int64_t m, int64_t n, int64_t k, bool wide, int *tm, int *tn)
+{
+    *tm = cfg.tile_m >= 128 ? 128 : 64;
+    *tn = (*tm == 128 && cfg.tile_n >= 128 && L <= 2) ? 128 : 64;
+    if (wide && L == 1 && *tn == 128 && k >= 1536 && ((m + 255) / 256) * ((n + 255) / 256) >= 128) *tm = *tn = 256;
+}
+
 // ext: caller-provided workspace for the digit planes (no allocation); the
 // planes of each K chunk must fit in ext->bytes and the launch has one K slice
 int gemm_limb_cfg(modp_ctx *ctx, const GemmArgs &g, const GemmConfig &cfg, const LimbScratch *ext = nullptr)
@@ -283,28 +395,31 @@ int gemm_limb_cfg(modp_ctx *ctx, const GemmArgs &g, const GemmConfig &cfg, const
     // L * K * 2^14 <= 2^31 - 1
     const int64_t pairs = L;
     int64_t kmax = ((int64_t)2147483647 / (pairs * 16384)) / LBK * LBK;
-    // residues above top are represented as r - p (see digit_rep)
-    int64_t S = 0;
-    for (int u = 0; u < L; ++u) S = S * 256 + 1;
-    const int32_t top = (int32_t)(127 * S > 2147483647 ? 2147483647 : 127 * S);
-    const int tm = cfg.tile_m == 128 ? 128 : 64;
-    const int tn = (cfg.tile_m == 128 && cfg.tile_n == 128 && L <= 2) ? 128 : 64;
+    int tm, tn;
+    limb_tile(cfg, L, g.m, g.n, g.k, !ext, &tm, &tn);
     const int64_t Mp = round_up(g.m, tm), Np = round_up(g.n, tn);
     LimbW lw;
     {
         double w = 1.0;
         for (int u = 0; u < 7; ++u) {
-            lw.w[u] = w;
+            lw.w[u] = w > (double)g.mp.half ? w - g.mp.pd : w;
             w = fmod(w * 256.0, (double)g.mp.p);
         }
     }
-    if (g.k <= 0 && g.epi != EPI_STORE) return MODP_OK;  // C unchanged
+    lw.lazy = limb_lazy(L, g.k < kmax ? g.k : kmax, g.mp.p);
+    if (g.ka != g.kb)
+        return set_error(ctx, MODP_ERR_DTYPE, "digit form: operands of different types (%d, %d)", g.ka, g.kb);
+    if (g.k <= 0)  // C unchanged, or zero
+        return g.epi != EPI_STORE ? MODP_OK
+                                  : hip_check(ctx, hipMemset2DAsync(g.C, (size_t)g.ldc * (g.kc == EK_F64 ? 8 : 4), 0,
+                                                                    (size_t)g.m * (g.kc == EK_F64 ? 8 : 4),
+                                                                    (size_t)g.n, ctx->stream), "hipMemset2DAsync");
     int64_t kdone = 0;
     bool first = true;
     do {
         int64_t kc = g.k - kdone;
         if (kc > kmax) kc = kmax;
-        const int64_t Kp = round_up(kc > 0 ? kc : 1, LBK);
+        const int64_t Kp = round_up(kc, LBK);
         int st = MODP_OK;
         int8_t *Al, *Bl;
         if (ext) {
@@ -320,12 +435,9 @@ int gemm_limb_cfg(modp_ctx *ctx, const GemmArgs &g, const GemmConfig &cfg, const
             Bl = (int8_t *)ws_get(ctx, WS_BLIMB, (size_t)L * Np * Kp, &st);
             if (!Bl) return st;
         }
-        if (g.ka == EK_F64) MODP_TRY(split_a_t<double>(ctx, g, g.A, kdone, kc, Al, Mp, Kp, L, top));
-        else if (g.ka == EK_F32) MODP_TRY(split_a_t<float>(ctx, g, g.A, kdone, kc, Al, Mp, Kp, L, top));
-        else MODP_TRY(split_a_t<int32_t>(ctx, g, g.A, kdone, kc, Al, Mp, Kp, L, top));
-        if (g.kb == EK_F64) MODP_TRY(split_b_t<double>(ctx, g, g.B, kdone, kc, Bl, Np, Kp, L, top));
-        else if (g.kb == EK_F32) MODP_TRY(split_b_t<float>(ctx, g, g.B, kdone, kc, Bl, Np, Kp, L, top));
-        else MODP_TRY(split_b_t<int32_t>(ctx, g, g.B, kdone, kc, Bl, Np, Kp, L, top));
+        if (g.ka == EK_F64) MODP_TRY(split_t<double>(ctx, g, kdone, kc, Al, Mp, Bl, Np, Kp, L));
+        else if (g.ka == EK_F32) MODP_TRY(split_t<float>(ctx, g, kdone, kc, Al, Mp, Bl, Np, Kp, L));
+        else MODP_TRY(split_t<int32_t>(ctx, g, kdone, kc, Al, Mp, Bl, Np, Kp, L));
         int epi = g.epi;
         if (!first && epi == EPI_STORE) epi = EPI_ADD;
         Slices sl = make_slices(Kp, cfg.ksplit, LBK, 256);
@@ -359,11 +471,15 @@ int limb_count(int64_t p)
 
 int choose_form(int64_t m, int64_t n, int64_t k, int64_t p)
 {
-    (void)m; (void)n; (void)p;
-    // the limb form pays a split pass over A and B: worth it once the
-    // contraction is deep enough for MFMA time to dominate
-    if (k >= 256) return MODP_FORM_LIMB_I8;
-    return MODP_FORM_PLAIN_F64;
+    // small products: one launch of the plain form's small kernel against the
+    // digit form's two, up to 512 x 512 x 128 (7.4 us against 10.0 to 12.7)
+    const int64_t w = small_work(m, n, k);
+    if (w >= 0 && w <= 131072) return MODP_FORM_PLAIN_F64;
+    // shallow ones: the digit form's split passes and its epilogue against the
+    // plain form's k-steps.  2048^2: at k = 32 13.3, 15.2 and 26 us with one,
+    // two and four digits against 15.8, at k = 64 13.4, 15.4 and 26 against 22,
+    // at k = 128 13.8, 16.5 and 28 against 34
+    return k >= (limb_count(p) <= 3 ? 48 : 96) ? MODP_FORM_LIMB_I8 : MODP_FORM_PLAIN_F64;
 }
 
 bool gemm_config_valid(const GemmArgs &g, const GemmConfig &cfg)
@@ -386,27 +502,26 @@ bool gemm_config_valid(const GemmArgs &g, const GemmConfig &cfg)
     return false;
 }
 
-// the RNS form's r moduli against the limb form's L^2 digit products: it
-// pays when it issues at most three quarters of the limb form's MFMA work,
-// and with one plane (p <= 255) against one digit product, whose core runs
-// at a lower fraction of the MFMA rate
-static bool rns_pays(const GemmArgs &g)
+// The RNS form's r moduli against the limb form's L^2 digit products: it pays
+// when it issues at most three quarters of the limb form's MFMA work and the
+// product is large enough for its two more launches and its residue planes of
+// C.  Four digits: 2501 x 1203 x 1777 121 us against 111, 2048^3 126 against
+// 159.  One plane (p <= 255) issues what one digit does and is the slower one
+// (float64 mod 127: 6000^3 499 us against 436, 8192^3 942 against 862); from
+// four 256 x 256 output tiles per CU it remains the documented choice.
+static bool rns_pays(const modp_ctx *ctx, const GemmArgs &g)
 {
     const int L = limb_count(g.mp.p);
     const int r = rns_planes(g.mp.p, g.k < RNS_KCHUNK ? g.k : RNS_KCHUNK);
-    return r > 0 && (r == 1 || 4 * r <= 3 * L * L);
+    if (r == 1) return tiles_of(g, 256, 256) >= 4 * ctx->num_cus;
+    return r > 0 && 4 * r <= 3 * L * L && (double)g.m * (double)g.n * (double)g.k >= 6.5e9;
 }
 
 GemmConfig gemm_default_config(const modp_ctx *ctx, const GemmArgs &g, int form)
 {
     GemmConfig c;
     c.form = form == MODP_FORM_AUTO ? choose_form(g.m, g.n, g.k, g.mp.p) : form;
-    // (one plane only with at least two 256 x 256 output tiles per CU:
-    // measured at p = 127, the one-digit form is faster at 4096^2 -- 646
-    // against 592 TOPS -- and the one plane at 8192^2, 1060 against 967)
-    if (form == MODP_FORM_AUTO && c.form == MODP_FORM_LIMB_I8 && rns_pays(g) &&
-        (rns_planes(g.mp.p, g.k < RNS_KCHUNK ? g.k : RNS_KCHUNK) > 1 || tiles_of(g, 256, 256) >= 2 * ctx->num_cus))
-        c.form = MODP_FORM_RNS_I8;
+    if (form == MODP_FORM_AUTO && c.form == MODP_FORM_LIMB_I8 && rns_pays(ctx, g)) c.form = MODP_FORM_RNS_I8;
     c.ksplit = 1;
     if (c.form == MODP_FORM_RNS_I8) {
         // 256x256 tiles while the grid (tiles x moduli) still holds two
@@ -416,28 +531,38 @@ GemmConfig gemm_default_config(const modp_ctx *ctx, const GemmArgs &g, int form)
         return c;
     }
     c.tile_m = c.tile_n = 64;
-    // larger tiles while the grid still fills the chip: measured best at
-    // n = 8192 are 128x128 (plain; limb with one digit) and 128x64 (limb with
-    // two digits); three and four digits gain nothing over 64x64
-    if (tiles_of(g, 128, 128) >= 2 * ctx->num_cus) {
-        const int L = limb_count(g.mp.p);
-        if (c.form == MODP_FORM_PLAIN_F64 || L == 1) {
-            c.tile_m = c.tile_n = 128;
-        } else if (L == 2) {
-            c.tile_m = 128;
+    const int64_t t128 = tiles_of(g, 128, 128);
+    if (c.form == MODP_FORM_PLAIN_F64) {
+        // 128x128 tiles measured best at n = 8192; a grid of at most one
+        // workgroup per CU is cut into concurrent K slices, up to about four
+        // workgroups per CU, each at least 256 deep (1024^2: 0.238 ms unsplit,
+        // 0.142 / 0.100 / 0.106 ms with 2 / 4 / 8 slices of 64x64 tiles)
+        if (t128 >= 2 * ctx->num_cus) c.tile_m = c.tile_n = 128;
+        const int64_t t = tiles_of(g, c.tile_m, c.tile_n);
+        if (t <= ctx->num_cus && g.k >= 1024) {
+            int64_t S = 4 * ctx->num_cus / (t > 0 ? t : 1);
+            if (S > 8) S = 8;
+            while (S > 1 && g.k / S < 256) --S;
+            c.ksplit = (int)S;
         }
+        return c;
     }
-    // a grid of at most one workgroup per CU: cut K into concurrent slices,
-    // up to about four workgroups per CU, each slice at least 256 deep
-    // (1024^2 plain: 0.238 ms unsplit, 0.142 / 0.100 / 0.106 ms with 2 / 4 /
-    // 8 slices of 64x64 tiles)
+    // digit form.  One and two digits take 128x128 tiles once there are about
+    // three for every four CUs (two digits: 2048^3 52.7 us against 64 with 64x64,
+    // 2501 x 1203 x 1777 44.0 against 47.4, but 1024^3, 64 tiles, 26 against
+    // 18.9) and K is deep enough for the core to outweigh the epilogue, of which
+    // 64x64 keeps four workgroups on a CU (4000 x 4000 x 128, two digits: 34.2
+    // us against 41.3 with 128x128); three and four digits gain nothing over 64x64
+    const int L = limb_count(g.mp.p);
+    if (L <= 2 && g.k > 256 && 4 * t128 >= 3 * ctx->num_cus) c.tile_m = c.tile_n = 128;
+    // K slices where the tiles leave CUs idle and a slice keeps at least 512 of
+    // a long K: the slices' sum costs a launch, about what 1024 of K cost
+    // (512 x 512 x 4096, two digits: 45 us unsplit, 24.9 / 26.8 with 4 / 8 slices;
+    // 1024^3 18.9 unsplit, 24.6 / 28.0 with 2 / 4)
     const int64_t t = tiles_of(g, c.tile_m, c.tile_n);
-    c.ksplit = 1;
-    if (t <= ctx->num_cus && g.k >= 1024) {
-        int64_t S = 4 * ctx->num_cus / (t > 0 ? t : 1);
-        if (S > 8) S = 8;
-        while (S > 1 && g.k / S < 256) --S;
-        c.ksplit = (int)S;
+    if (g.k >= 2048 && 2 * t <= ctx->num_cus) {
+        int64_t S = std::min<int64_t>(ctx->num_cus / (t > 0 ? t : 1), g.k / 512);
+        c.ksplit = (int)std::min<int64_t>(S, 8);
     }
     return c;
 }
@@ -468,8 +593,8 @@ size_t gemm_limb_scratch_bytes(const modp_ctx *ctx, const GemmArgs &g)
 {
     GemmConfig cfg = gemm_default_config(ctx, g, MODP_FORM_LIMB_I8);
     const int L = limb_count(g.mp.p);
-    const int tm = cfg.tile_m == 128 ? 128 : 64;
-    const int tn = (cfg.tile_m == 128 && cfg.tile_n == 128 && L <= 2) ? 128 : 64;
+    int tm, tn;
+    limb_tile(cfg, L, g.m, g.n, g.k, false, &tm, &tn);
     const int64_t kmax = ((int64_t)2147483647 / ((int64_t)L * 16384)) / LBK * LBK;
     const int64_t kc = g.k < kmax ? g.k : kmax;
     const int64_t Kp = round_up(kc > 0 ? kc : 1, LBK);

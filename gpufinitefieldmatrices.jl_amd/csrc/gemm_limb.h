@@ -26,8 +26,23 @@ struct Slices {
 };
 
 struct LimbW {
-    double w[7];  // 256^u mod p
+    double w[7];  // 256^u mod p, balanced (magnitude at most p/2)
+    int lazy;     // the recombination of this K chunk is exact without reducing
+                  // the digit sums first (limb_lazy)
 };
+
+// Recombination of the digit sums, sum_u acc_u w_u.  Shift u collects
+// min(u + 1, 2L - 1 - u) digit products of magnitude 2^14 per k, so for k up
+// to `kc` the sum is below kc 2^14 (1 + (p/2) sum_{u > 0} pairs(u)); under 2^51
+// it is exact in FP64 as it stands (two digits: always; three: k < 4096 at
+// 2^23).  Otherwise every digit sum is reduced to a balanced residue first:
+// 7 products of at most (2^25 + 1)^2 stay below 2^53.
+static inline int limb_lazy(int L, int64_t kc, int64_t p)
+{
+    double pairs = 0.0;
+    for (int u = 1; u < 2 * L - 1; ++u) pairs += u + 1 < 2 * L - 1 - u ? u + 1 : 2 * L - 1 - u;
+    return (double)kc * 16384.0 * (1.0 + pairs * (double)(p / 2 + 1)) < 2251799813685248.0;
+}
 
 // Launch the limb core for L digits on planes Al (Mp x Kp per digit) and Bl
 // (Np x Kp per digit) with a tile_m x tile_n output tile; defined for
@@ -55,92 +70,85 @@ __device__ __forceinline__ int32_t next_digit(int32_t &x)
     return d;
 }
 
-// A (m x k col-major) -> Al[s][row][kk] (row-major per digit, k contiguous),
-// zero-padded to Mp x Kp.  64x64 tiles transposed through LDS.
-template <typename TA>
-__global__ __launch_bounds__(256) void k_split_a(int64_t m, int64_t k, const TA *__restrict__ A, int64_t lda,
-                                                 int8_t *__restrict__ Al, int64_t Mp, int64_t Kp, int L,
-                                                 int32_t top, ModP mp, const int *__restrict__ skip)
+// The digit planes of both operands in one launch: workgroups [0, na) split A
+// (m x k col-major -> Al[s][row][kk], row-major per digit, k contiguous,
+// zero-padded to Mp x Kp) by 64 x 64 tiles transposed through LDS, the others
+// B (k x n col-major -> Bl[s][col][kk], zero-padded to Np x Kp; k is
+// contiguous in memory already), 1024 groups of four k each.  Bound by
+// memory: every thread has its sixteen loads in flight before it uses one
+// (at indices clamped into the operand, masked afterwards, so that edge
+// tiles wait no more than inner ones).  One launch instead of two:
+// 5.9 + 4.2 us -> 6.1 us at 1024^2 float64 with two digits, 16.6 + 7.0 -> 12 us at
+// 2501 x 1777 and 1777 x 1203 with three.
+template <typename T, int L>
+__global__ __launch_bounds__(256) void k_split_ab(int64_t m, int64_t n, int64_t k, const T *__restrict__ A, int64_t lda,
+                                                  const T *__restrict__ B, int64_t ldb, int8_t *__restrict__ Al,
+                                                  int64_t Mp, int8_t *__restrict__ Bl, int64_t Np, int64_t Kp,
+                                                  unsigned na, ModP mp, const int *__restrict__ skip)
 {
     if (skip && *skip) return;
-    __shared__ int32_t tile[64][65];
+    constexpr int32_t TOP = (int32_t)(127 * ((((int64_t)1) << (8 * L)) - 1) / 255);
     const int tid = threadIdx.x;
-    const int64_t r0 = (int64_t)blockIdx.y * 64, k0 = (int64_t)blockIdx.x * 64;
-    if (r0 + 64 <= m && k0 + 64 <= k) {
-        // a tile wholly inside A (the same for the whole workgroup): the 16
-        // loads of a thread go out together
-        const int row = tid & 63;
-        TA x[16];
+    T x[16];
+    if (blockIdx.x < na) {
+        __shared__ int32_t tile[64][65];
+        const unsigned kt = (unsigned)(Kp / 64);
+        const int64_t r0 = (int64_t)(blockIdx.x / kt) * 64, k0 = (int64_t)(blockIdx.x % kt) * 64;
+        const int row = tid & 63, kq = tid >> 6;
+        const T *src = A + min(r0 + row, m - 1);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) x[i] = A[r0 + row + (k0 + (tid >> 6) + 4 * i) * lda];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) tile[row][(tid >> 6) + 4 * i] = digit_rep(to_res<TA>(x[i], mp), top, mp);
-    } else {
+        for (int i = 0; i < 16; ++i) x[i] = src[min(k0 + kq + 4 * i, k - 1) * lda];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            int row = tid & 63, kk = (tid >> 6) + 4 * i;
-            int64_t gr = r0 + row, gk = k0 + kk;
-            int32_t v = 0;
-            if (gr < m && gk < k) v = digit_rep(to_res<TA>(A[gr + gk * lda], mp), top, mp);
-            tile[row][kk] = v;
+            const bool in = r0 + row < m && k0 + kq + 4 * i < k;
+            tile[row][kq + 4 * i] = in ? digit_rep(to_res<T>(x[i], mp), TOP, mp) : 0;
         }
-    }
-    __syncthreads();
-    const int row = tid >> 2, ch = tid & 3;
-    const size_t plane = (size_t)Mp * Kp;
-    int8_t *dst = Al + (size_t)(r0 + row) * Kp + k0 + ch * 16;
-    union { int8_t b[16]; v4i v; } u[4];
+        __syncthreads();
+        const int orow = tid >> 2, ch = tid & 3;
+        const size_t plane = (size_t)Mp * Kp;
+        int8_t *dst = Al + (size_t)(r0 + orow) * Kp + k0 + ch * 16;
+        union { int8_t b[16]; v4i v; } u[L];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        int32_t x = tile[row][ch * 16 + e];
+        for (int e = 0; e < 16; ++e) {
+            int32_t y = tile[orow][ch * 16 + e];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) u[s].b[e] = (int8_t)next_digit(x);
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-        if (s < L) *reinterpret_cast<v4i *>(dst + s * plane) = u[s].v;
-}
-
-// B (k x n col-major) -> Bl[s][col][kk], zero-padded to Np x Kp.  Same
-// orientation (k contiguous), so each thread maps 4 consecutive k of one
-// column: consecutive threads read consecutive 32-byte runs.
-template <typename TB>
-__global__ __launch_bounds__(256) void k_split_b(int64_t k, int64_t n, const TB *__restrict__ B, int64_t ldb,
-                                                 int8_t *__restrict__ Bl, int64_t Np, int64_t Kp, int L,
-                                                 int32_t top, ModP mp, const int *__restrict__ skip)
-{
-    if (skip && *skip) return;
-    const int64_t quads = Kp / 4;
-    const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (e >= Np * quads) return;
-    const int64_t col = e / quads, k0 = (e % quads) * 4;
-    uint32_t word[4] = {0u, 0u, 0u, 0u};
-    int32_t xs[4];
-    if (col < n && k0 + 4 <= k) {
-        // all four in range: the loads go out together
-        TB v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = B[k0 + i + col * ldb];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) xs[i] = digit_rep(to_res<TB>(v[i], mp), top, mp);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int64_t gk = k0 + i;
-            xs[i] = (col < n && gk < k) ? digit_rep(to_res<TB>(B[gk + col * ldb], mp), top, mp) : 0;
+            for (int s = 0; s < L; ++s) u[s].b[e] = (int8_t)next_digit(y);
         }
+#pragma unroll
+        for (int s = 0; s < L; ++s) *reinterpret_cast<v4i *>(dst + s * plane) = u[s].v;
+        return;
     }
+    const int64_t quads = Kp / 4, total = Np * quads;
+    const int64_t e0 = (int64_t)(blockIdx.x - na) * 1024 + tid;
+    int64_t col[4], kk[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        int32_t x = xs[i];
+    for (int g = 0; g < 4; ++g) {
+        const int64_t e = min(e0 + 256 * g, total - 1);
+        col[g] = e / quads;
+        kk[g] = (e % quads) * 4;
+        const T *src = B + min(col[g], n - 1) * ldb;
 #pragma unroll
-        for (int s = 0; s < 4; ++s) word[s] |= ((uint32_t)next_digit(x) & 255u) << (8 * i);
+        for (int i = 0; i < 4; ++i) x[4 * g + i] = src[min(kk[g] + i, k - 1)];
     }
     const size_t plane = (size_t)Np * Kp;
-    int8_t *dst = Bl + (size_t)col * Kp + k0;
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-        if (s < L) *reinterpret_cast<uint32_t *>(dst + s * plane) = word[s];
+    for (int g = 0; g < 4; ++g) {
+        uint32_t word[L];
+#pragma unroll
+        for (int s = 0; s < L; ++s) word[s] = 0u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool in = col[g] < n && kk[g] + i < k;
+            int32_t y = in ? digit_rep(to_res<T>(x[4 * g + i], mp), TOP, mp) : 0;
+#pragma unroll
+            for (int s = 0; s < L; ++s) word[s] |= ((uint32_t)next_digit(y) & 255u) << (8 * i);
+        }
+        if (e0 + 256 * g < total) {
+            int8_t *dst = Bl + (size_t)col[g] * Kp + kk[g];
+#pragma unroll
+            for (int s = 0; s < L; ++s) *reinterpret_cast<uint32_t *>(dst + s * plane) = word[s];
+        }
+    }
 }
 
 // Limb-form tile shapes: a BM x BN output tile per workgroup of WGM x WGN
@@ -293,10 +301,10 @@ __global__ __launch_bounds__(SH::NT, SH::OCC) void k_gemm_limb(int64_t m, int64_
 #pragma unroll
                         for (int t = 0; t < L; ++t) {
                             if constexpr (MF == 32)
-                                acc[i][j][s + t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[i][ks][s], b[j][ks][t],
+                                acc[i][j][s + t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b[j][ks][t], a[i][ks][s],
                                                                                          acc[i][j][s + t], 0, 0, 0);
                             else
-                                acc[i][j][s + t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][ks][s], b[j][ks][t],
+                                acc[i][j][s + t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b[j][ks][t], a[i][ks][s],
                                                                                          acc[i][j][s + t], 0, 0, 0);
                         }
     };
@@ -351,39 +359,57 @@ __global__ __launch_bounds__(SH::NT, SH::OCC) void k_gemm_limb(int64_t m, int64_
         }
     }
 
-    // accumulator layouts: 16x16 blocks hold column lane % 16, rows
-    // 4 (lane / 16) + e; 32x32 blocks hold column lane % 32, rows
-    // 8 (e / 4) + 4 (lane / 32) + e % 4
+    // The blocks are computed transposed (B digits as the first operand), so
+    // lane l holds row l % MF of C and a store instruction covers runs of MF
+    // rows of a column: element e is column 8 (e / 4) + 4 (l / 32) + e % 4 of a
+    // 32x32 block, 4 (l / 16) + e of a 16x16 one.  The old values of C, where
+    // the epilogue needs them, are loaded together before the arithmetic (at
+    // indices clamped into C).  4000 x 4000 -= K = 128, two digits, int32: 67
+    // -> 34 us (one column run of 4 rows a lane, each digit sum reduced in
+    // turn, loads between the stores); the memory traffic alone takes 26.
+    const bool inside = r0 + BM <= m && c0 + BN <= n;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-            int64_t gc = c0 + wn * WN + j * MF + (lane & (MF - 1));
-            if (gc >= n) continue;
+            const int64_t gr = r0 + wm * WM + i * MF + (lane & (MF - 1));
+            const int64_t gc = c0 + wn * WN + j * MF + 4 * (lane / MF);
+            const bool row_ok = inside || gr < m;
+            TC *const dst = C + (row_ok ? gr : 0);
+            TC old[AE];
+            if (EPI != EPI_STORE) {
+#pragma unroll
+                for (int e = 0; e < AE; ++e) {
+                    const int64_t col = gc + (MF == 32 ? 8 * (e >> 2) + (e & 3) : e);
+                    old[e] = dst[(inside ? col : min(col, n - 1)) * ldc];
+                }
+            }
 #pragma unroll
             for (int e = 0; e < AE; ++e) {
-                const int rr = MF == 32 ? 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3) : 4 * (lane >> 4) + e;
-                int64_t gr = r0 + wm * WM + i * MF + rr;
-                if (gr >= m) continue;
-                double tot = dmod((double)acc[i][j][0][e], mp);
+                double tot;
+                if (lw.lazy) {
+                    tot = (double)acc[i][j][0][e];
 #pragma unroll
-                for (int u = 1; u < NS; ++u) {
-                    double d = dmod((double)acc[i][j][u][e], mp);
-                    tot = dmod(fma(d, lw.w[u], tot), mp);
+                    for (int u = 1; u < NS; ++u) tot = fma((double)acc[i][j][u][e], lw.w[u], tot);
+                } else {
+                    const double d0 = (double)acc[i][j][0][e];
+                    tot = fma(-rint(d0 * mp.pinv), mp.pd, d0);
+#pragma unroll
+                    for (int u = 1; u < NS; ++u) {
+                        const double d = (double)acc[i][j][u][e];
+                        tot = fma(fma(-rint(d * mp.pinv), mp.pd, d), lw.w[u], tot);
+                    }
                 }
-                uint32_t r = (uint32_t)tot;
-                TC *dst = C + gr + gc * ldc;
-                if (EPI == EPI_SUB) r = submod(to_res<TC>(*dst, mp), r, mp);
-                else if (EPI == EPI_ADD) r = addmod(to_res<TC>(*dst, mp), r, mp);
-                *dst = from_res<TC>(r);
+                // |tot| < 2^53: the rounded quotient leaves a balanced residue
+                tot = fma(-rint(tot * mp.pinv), mp.pd, tot);
+                uint32_t r = (uint32_t)(tot < 0.0 ? tot + mp.pd : tot);
+                if (EPI == EPI_SUB) r = submod(to_res<TC>(old[e], mp), r, mp);
+                else if (EPI == EPI_ADD) r = addmod(to_res<TC>(old[e], mp), r, mp);
+                const int64_t col = gc + (MF == 32 ? 8 * (e >> 2) + (e & 3) : e);
+                if (inside || (row_ok && col < n)) dst[col * ldc] = from_res<TC>(r);
             }
         }
 }
-
-
-// MFMA block size and LDS layout used by the library's limb kernels
-constexpr int LIMB_MF = 16;
-constexpr int LIMB_SWZ = 1;
 
 template <int L, typename SH, typename TC>
 int limb_core(modp_ctx *ctx, const GemmArgs &g, int epi, const int8_t *Al, int64_t Mp, const int8_t *Bl, int64_t Np,
@@ -404,18 +430,33 @@ int limb_core(modp_ctx *ctx, const GemmArgs &g, int epi, const int8_t *Al, int64
     return hip_check(ctx, hipGetLastError(), "k_gemm_limb launch");
 }
 
-// tile_m x tile_n -> workgroup shape: 64x64 and 128x64 use 32x32 waves;
-// 128x128 (L <= 2 only; the caller pads to the tile it asks for) uses 2x2
-// waves of 64x64
+// tile_m x tile_n -> workgroup shape, all on 32x32 MFMA blocks with two
+// register sets ahead of two LDS stages (measured on the planes alone).  Four
+// digits on 64x64 hold seven weight planes of accumulators, which leave room
+// for two waves on a SIMD only with one register set: 1500^3 64 us, with two
+// sets and one wave 80; the trailing update 4000 x 4000 x 128 63 against 99.
+//   64x64    2x2 waves; 1024^3, two digits 12.7 us (16x16 blocks, one stage:
+//            14.6), 2501 x 1203 x 1777, three digits 58 (62.9), 5000^3 919 (1002)
+//   128x64   two digits 2x2 waves, else 4x2; 3000^3, two digits 133 us (140;
+//            64x64 136)
+//   128x128  (one or two digits) one digit 2x2 waves, two 4x2
+//   256x256  (one digit) 4x2 waves; 5000^3 177 us (128x128 tiles 219)
 template <int L, typename TC>
 int limb_by_shape(modp_ctx *ctx, const GemmArgs &g, int epi, const int8_t *Al, int64_t Mp, const int8_t *Bl,
                   int64_t Np, int64_t Kp, const LimbW &lw, int tile_m, int tile_n, const Slices &sl)
 {
-    if (L <= 2 && tile_m == 128 && tile_n == 128)
-        return limb_core<L, LimbShape<128, 128, 2, 2, LIMB_MF, LIMB_SWZ>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp, lw, sl);
+    if constexpr (L == 1)
+        if (tile_m == 256)
+            return limb_core<L, LimbShape<256, 256, 4, 2, 32, 1, 2>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp, lw, sl);
+    if constexpr (L <= 2)
+        if (tile_m == 128 && tile_n == 128)
+            return limb_core<L, LimbShape<128, 128, L == 1 ? 2 : 4, 2, 32, 1, 2>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp,
+                                                                                     lw, sl);
     if (tile_m == 128 && tile_n == 64)
-        return limb_core<L, LimbShape<128, 64, 4, 2, LIMB_MF, LIMB_SWZ>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp, lw, sl);
-    return limb_core<L, LimbShape<64, 64, 2, 2, LIMB_MF, LIMB_SWZ>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp, lw, sl);
+        return limb_core<L, LimbShape<128, 64, L == 2 ? 2 : 4, 2, 32, 1, L == 4 ? 1 : 2>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp, lw,
+                                                                                sl);
+    return limb_core<L, LimbShape<64, 64, 2, 2, 32, 1, L == 4 ? 1 : 2, L == 4 ? 2 : 1>, TC>(ctx, g, epi, Al, Mp, Bl,
+                                                                                           Np, Kp, lw, sl);
 }
 
 }  // namespace
