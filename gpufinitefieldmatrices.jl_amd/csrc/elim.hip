@@ -21,9 +21,10 @@
 //                columns are staged.  Above 16,384 rows k_panel_g does the
 //                same with the panel left in W (any row count).
 //     k_update   the block's other columns: the row map, and right of the
-//                panel the triangular solve with L11 (rows of U) and the
-//                rank-w update of every row below the pivots.
-//   after the outer block: k_block_finish applies the block's row maps and
+//                panel the rows of U (a product with the inverse triangle
+//                that the panel leaves) and the rank-w update of every row
+//                below the pivots.
+//   after the outer block: k_block_finish applies the block's row moves and
 //   the solve with the block's L11 to the far columns, then one GEMM with
 //   K = NBO (limb or plain form) updates the far trailing block.
 #include <stdlib.h>
@@ -58,7 +59,7 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
                                                  int32_t *__restrict__ map_src, PanelCtl *__restrict__ ctl,
                                                  int *__restrict__ abort, int KC, int FAR, int32_t *__restrict__ stage,
                                                  int *__restrict__ cursor, int32_t *__restrict__ gpos,
-                                                 int32_t *__restrict__ grow)
+                                                 int32_t *__restrict__ grow, PanelSolve *__restrict__ solve)
 {
     constexpr int NW = GPT / 64;
     if (abort && *abort) {
@@ -79,8 +80,8 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
     __shared__ uint32_t s_U[NBW][NBW];
     __shared__ int s_ip[NBW], s_pv[NBW], s_pi[NBW], s_pcol[NBW];
     __shared__ int s_msrc[2 * NBW], s_mdst[2 * NBW];
-    __shared__ uint32_t s_mv[2 * NBW][NBW];
-    __shared__ int s_cnt;
+    __shared__ uint32_t s_mv[2 * NBW][NBW], s_T[NBW][NBW];
+    __shared__ int s_cnt, s_num[PNW];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int rows = m - kr0;
@@ -230,6 +231,22 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
         pivval[kr0 + tid] = s_pv[tid];
         pivinv[kr0 + tid] = s_pi[tid];
         pivcol[kr0 + tid] = c0 + s_pcol[tid];
+        // column tid of T by substitution, the multipliers from the pivot rows
+        for (int t = 0; t < pc; ++t) {
+            uint32_t x = t == tid ? 1u : 0u;
+            for (int k = tid; k < t; ++k) x = submod(x, mulmod(s_mv[t][s_pcol[k]], s_T[k][tid], mp), mp);
+            s_T[t][tid] = t < tid ? 0u : mulmod(x, (uint32_t)s_pi[t], mp);
+        }
+    }
+    if (tid < PNW) s_num[tid] = -1;
+    __syncthreads();
+    if (tid < pc) s_num[s_pcol[tid]] = tid;
+    __syncthreads();
+    if (tid < PNW) solve->num[tid] = s_num[tid];
+    for (int idx = tid; idx < PNW * PNW; idx += GPT) {
+        const int j = idx / PNW, q = idx % PNW, t = s_num[j];
+        const uint32_t x = t >= 0 && q < pc ? s_T[t][q] : 0u;
+        solve->t[j][q] = x > mp.half ? (int32_t)x - (int32_t)mp.p : (int32_t)x;
     }
     if (tid == 0) {
         ctl->npiv = pc;
@@ -242,283 +259,363 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
     }
 }
 
-// After panel (kr0, c0, w) of the outer block [KC, FAR), in one launch:
-// the panel's row moves for every other column of the block, and for the
-// columns right of the panel the triangular solve with L11 (their rows of U)
-// and the rank-npiv update of every row below the pivots.  The old values
-// of moved rows come from the stage the panel kernel filled before anything
-// moved, so no block reads a row that another block writes.  Grid: x =
-// 64-row tiles from kr0 down, y = 8-column groups, the groups left of the
-// panel first (moves only, done by the blocks of the first row tile).
-// LAZY (p < 2^16): at most 32 products below 2^32 are summed exactly in FP64
-// before one reduction; otherwise every product is reduced.
-constexpr int UT_R = 64, UT_C = 8;
-template <int WMAX, bool LAZY>
-__global__ __launch_bounds__(256) void k_update(int32_t *__restrict__ W, int64_t ldw, int m, int KC, int FAR,
-                                                int c0, int w, const PanelCtl *__restrict__ ctl,
-                                                const int32_t *__restrict__ pivinv,
-                                                const int32_t *__restrict__ pivcol,
-                                                const int32_t *__restrict__ map_dst,
-                                                const int32_t *__restrict__ stage, ModP mp,
-                                                const int *__restrict__ skip)
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ v4d mfma_f64(double a, double b, v4d c)
 {
-    // the skip flag and the panel's counts are read together
-    const int skipped = skip ? *skip : 0;
-    const int npiv = ctl->npiv, nmap = ctl->nmap, kr0 = ctl->kr0;
-    if (skipped || nmap == 0) return;
-    constexpr int CPT = UT_C / 4;            // columns per thread
-    __shared__ uint32_t Lf[WMAX][WMAX + 1];  // the panel's top w x w block
-    __shared__ uint32_t Ls[WMAX][WMAX + 1];  // L11 (row i, pivot j < i)
-    __shared__ uint32_t invs[WMAX];
-    __shared__ int s_pj[WMAX];              // panel column of pivot i
-    __shared__ int s_dst[64];               // row-map destinations
-    __shared__ double Ut[UT_C][WMAX];        // U by column, then panel column (0: no pivot)
-    __shared__ int s_e[UT_R];               // tile row -> row-map entry, or -1
-    const int tid = threadIdx.x, cl = tid >> 6;
-    const int nl = c0 - KC, nr = FAR - (c0 + w);
-    const int gl = (nl + UT_C - 1) / UT_C;
-    const int g = blockIdx.y;
-    if (g < gl) {
-        // left of the panel: the row moves only
-        if (blockIdx.x != 0) return;
-        const int cb = g * UT_C, nc = min(UT_C, nl - cb);
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+// a residue in [0,p) as its balanced representative
+__device__ __forceinline__ double balanced(int32_t x, const ModP &mp)
+{
+    return (double)(x > mp.half ? x - (int32_t)mp.p : x);
+}
+// EVERY (p > 2^24): four products below 2^50 and a reduced sum stay below
+// 2^53, so the sum is reduced after every step; below, up to 128 products
+// below 2^46 are summed exactly and reduced once.
+template <bool EVERY> __device__ __forceinline__ v4d after_step(v4d c, const ModP &mp)
+{
+    if (EVERY)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c[e] = near_mod(c[e], mp);
+    return c;
+}
+
+// The composed row moves of an outer block's panels so far, kept by the updates
+// for k_block_finish: the row that is now at position KR + k comes from top[k],
+// the one at any other moved position dst[i] from src[i].
+struct BlockMoves {
+    int32_t n, pad[3];
+    int32_t top[NBO], dst[NBO], src[NBO];
+};
+
+// After panel t at (kr0, c0, w) of the outer block [KC, FAR), in one launch:
+// the panel's row moves for every other column of the block, and for the
+// columns right of the panel the rows of U and the rank-npiv update of every
+// row below the pivots.  The old values of moved rows come from the stage the
+// panel kernel filled before anything moved, so no block reads a row that
+// another block writes.
+//
+// The launch is bound by the latency of its loads, launch and end; the
+// arithmetic is two short chains of FP64 MFMAs.  The panel supplies T, the
+// inverse of its scaled triangle, so the rows of U are T times the old pivot
+// rows instead of a substitution.  A wave takes 32 rows by 16 columns and
+// works out its 32 x 16 of U itself: the accumulators of v_mfma_f64_16x16x4
+// hold row 4 e + lane / 16 of column lane % 16, which is just the operand of
+// the next product's step e, so nothing passes through LDS and no wave waits
+// for another; in that product the rows of W run along the lanes (64-byte
+// pieces).  Block 0 composes the row moves, the next ones move rows left of
+// the panel.  Mean over the panels of a 4096^2 PLUQ mod 65521 8.3 us, of a
+// 1500^2 inverse mod 2^26 - 5 7.9 us; with a substitution by one lane per column
+// and, above 2^16, a reduction per product 12.7 and 30 us.
+constexpr int UT_R = 64, UT_C = 32, UT_L = 8;  // rows, columns of a tile; columns of a block left of the panel
+template <bool EVERY>
+__global__ __launch_bounds__(256) void k_update(int32_t *__restrict__ W, int64_t ldw, int m, int KR, int KC, int FAR,
+                                                int c0, int w, int kr0_in, int first,
+                                                const PanelCtl *__restrict__ ctl,
+                                                const PanelSolve *__restrict__ solve,
+                                                const int32_t *__restrict__ map_dst,
+                                                const int32_t *__restrict__ map_src,
+                                                const int32_t *__restrict__ stage, BlockMoves *__restrict__ moves,
+                                                ModP mp, const int *__restrict__ skip)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nl = c0 - KC, nr = FAR - (c0 + w), gl = (nl + UT_L - 1) / UT_L;
+    if (blockIdx.x == 0) {
+        // new moves after the old ones: a thread holds the position KR + tid, or
+        // one of the others
+        __shared__ int s_dst[64], s_src[64], s_from[64];
+        __shared__ int s_n;
+        const int skipped = skip ? *skip : 0, nmap = ctl->nmap;
+        const bool top = tid < NBO;
+        const int i = top ? tid : tid - NBO, nold = first ? 0 : moves->n;
+        bool keep = top || i < nold;
+        const int dst = top ? KR + i : keep ? moves->dst[i] : -1;
+        int src = top ? (first ? dst : moves->top[i]) : keep ? moves->src[i] : -1;
+        if (tid < 64) {
+            s_dst[tid] = map_dst[tid];
+            s_src[tid] = s_from[tid] = map_src[tid];
+        }
+        if (tid == 0) s_n = 0;
+        __syncthreads();
+        if (skipped) return;
+        int at = -1;
+        for (int e = 0; e < nmap; ++e) {
+            if (keep && s_src[e] == dst) s_from[e] = src;
+            if (keep && s_dst[e] == dst) at = e;
+        }
+        __syncthreads();
+        if (top) {
+            moves->top[i] = at >= 0 ? s_from[at] : src;
+        } else if (keep && at < 0) {
+            const int k = atomicAdd(&s_n, 1);
+            moves->dst[k] = dst;
+            moves->src[k] = src;
+        }
+        if (tid < nmap && (s_dst[tid] < KR || s_dst[tid] >= KR + NBO)) {
+            const int k = atomicAdd(&s_n, 1);
+            moves->dst[k] = s_dst[tid];
+            moves->src[k] = s_from[tid];
+        }
+        __syncthreads();
+        if (tid == 0) moves->n = s_n;
+        return;
+    }
+    if ((int)blockIdx.x <= gl) {
+        const int skipped = skip ? *skip : 0, nmap = ctl->nmap;
+        if (skipped) return;
+        const int cb = ((int)blockIdx.x - 1) * UT_L, nc = min(UT_L, nl - cb);
         for (int idx = tid; idx < nmap * nc; idx += 256) {
             const int e = idx % nmap, ci = cb + idx / nmap;
             W[(int64_t)map_dst[e] + (int64_t)(KC + ci) * ldw] = stage[e + 64 * ci];
         }
         return;
     }
-    const int cb = (g - gl) * UT_C, nc = min(UT_C, nr - cb);
-    const int ci0 = nl + cb;        // stage column of the group's first column
-    const int cfirst = c0 + w + cb;  // its column in W
-    const int64_t r0 = (int64_t)kr0 + (int64_t)blockIdx.x * UT_R;
-    if (r0 >= m) return;  // the grid covers the most rows the panel can have
-    const int64_t r = r0 + (tid & 63);
-    const bool row_ok = r < m;
-
-    // every global load is issued before anything waits for one: the
-    // panel's top block, pivot columns and inverses, the row map, the
-    // solve's inputs (thread k < nc: column k of the pivot rows' old
-    // values), this thread's row of L and its old values.  Indices are
-    // clamped into range so that the loads are unconditional; values that
-    // are not needed are masked when they are used.
-    constexpr int FPT = (WMAX * WMAX + 255) / 256;
-    const int wl = w - 1;
-    const int64_t rr = row_ok ? r : (int64_t)kr0;
-    int32_t lf[FPT];
+    // Every load that does not depend on another is issued first, at indices
+    // clamped into range; values that are not needed meet a zero of T.
+    const int tile = (int)blockIdx.x - 1 - gl, ncg = (nr + UT_C - 1) / UT_C;
+    const int cl = lane & 15, g = lane >> 4;
+    const int cw = (tile % ncg) * UT_C + (wave >> 1) * 16;  // column right of the panel
+    if (cw >= nr) return;
+    const int skipped = skip ? *skip : 0;
+    const int npiv = ctl->npiv, nmap = ctl->nmap;
+    const int kr0 = kr0_in >= 0 ? kr0_in : ctl->kr0;
+    const int mdst = map_dst[lane];
+    int4 t4[2][2], x4[2];
+    const int32_t *xs = stage + 64 * (int64_t)(nl + min(cw + cl, nr - 1)) + 8 * g;
 #pragma unroll
-    for (int k = 0; k < FPT; ++k) {
-        const int idx = tid + 256 * k, i = min(idx / WMAX, wl), jj = min(idx % WMAX, wl);
-        lf[k] = W[(int64_t)(kr0 + i) + (int64_t)(c0 + jj) * ldw];
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int ti = 0; ti < 2; ++ti) t4[ti][h] = *(const int4 *)&solve->t[16 * ti + cl][8 * g + 4 * h];
+        x4[h] = *(const int4 *)(xs + 4 * h);
     }
-    const int tw = min(tid, WMAX - 1);
-    const int32_t iv = pivinv[kr0 + tw];
-    const int32_t pjv = pivcol[kr0 + tw];
-    const int32_t mdv = map_dst[min(tid, 63)];
-    int32_t xs0[WMAX];
-    const int64_t xcol = 64 * (int64_t)(ci0 + min(tid, nc - 1));
+    const int rel0 = (tile / ncg) * UT_R + (wave & 1) * 32;  // the wave's first row under kr0
+    if (skipped || nmap == 0 || kr0 + rel0 >= m) return;
+    const int32_t *Lp = W + (int64_t)c0 * ldw;
+    int32_t *Cp = W + (int64_t)(c0 + w + cw) * ldw;
+    int32_t lv[2][8], cv[2][4];
 #pragma unroll
-    for (int i = 0; i < WMAX; ++i) xs0[i] = stage[min(i, wl) + xcol];
-    int32_t lr0[WMAX];
+    for (int a = 0; a < 2; ++a) {
+        const int r = min(kr0 + rel0 + 16 * a + cl, m - 1);
 #pragma unroll
-    for (int jj = 0; jj < WMAX; ++jj) lr0[jj] = W[rr + (int64_t)(c0 + min(jj, wl)) * ldw];
-    int32_t cv[CPT];
+        for (int s = 0; s < 8; ++s) lv[a][s] = Lp[r + (int64_t)min(4 * s + g, w - 1) * ldw];
 #pragma unroll
-    for (int k = 0; k < CPT; ++k) cv[k] = W[rr + (int64_t)(cfirst + min(cl + 4 * k, nc - 1)) * ldw];
-    for (int idx = tid; idx < WMAX * UT_C; idx += 256) Ut[idx / WMAX][idx % WMAX] = 0.0;
-    if (tid < UT_R) s_e[tid] = -1;
-#pragma unroll
-    for (int k = 0; k < FPT; ++k) {
-        const int idx = tid + 256 * k;
-        if (idx < WMAX * WMAX) Lf[idx / WMAX][idx % WMAX] = (idx / WMAX < w && idx % WMAX < w) ? (uint32_t)lf[k] : 0u;
+        for (int e = 0; e < 4; ++e) cv[a][e] = Cp[r + (int64_t)min(4 * e + g, nr - 1 - cw) * ldw];
     }
-    if (tid < WMAX) {
-        invs[tid] = (uint32_t)iv;
-        s_pj[tid] = pjv - c0;
+    // the rows of the tile that moved here from elsewhere
+    __shared__ int s_e[4][32];
+    if (lane < 32) s_e[wave][lane] = -1;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const int d = mdst - kr0 - rel0;
+    if (lane >= npiv && lane < nmap && d >= 0 && d < 32) s_e[wave][d] = lane;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    int ent[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) ent[a] = s_e[wave][16 * a + cl];
+    if (__any(ent[0] >= 0 || ent[1] >= 0)) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (ent[a] >= 0) cv[a][e] = stage[ent[a] + 64 * (int64_t)(nl + min(cw + 4 * e + g, nr - 1))];
     }
-    if (tid < 64) s_dst[tid] = mdv;
-    uint32_t xs[WMAX];
+    // U, rows by panel column
+    v4d u[2] = {v4d{0, 0, 0, 0}, v4d{0, 0, 0, 0}};
 #pragma unroll
-    for (int i = 0; i < WMAX; ++i) xs[i] = i < w ? (uint32_t)xs0[i] : 0u;
-    double Lr[WMAX];
+    for (int s = 0; s < 8; ++s) {
+        const int4 xq = x4[s >> 2];
+        const double x = balanced((s & 3) == 0 ? xq.x : (s & 3) == 1 ? xq.y : (s & 3) == 2 ? xq.z : xq.w, mp);
 #pragma unroll
-    for (int jj = 0; jj < WMAX; ++jj) Lr[jj] = jj < w ? (double)lr0[jj] : 0.0;
-    __syncthreads();
-    if (tid >= npiv && tid < nmap) {
-        const int64_t d = (int64_t)s_dst[tid] - r0;
-        if (d >= 0 && d < UT_R) s_e[d] = tid;
+        for (int ti = 0; ti < 2; ++ti) {
+            const int4 tq = t4[ti][s >> 2];
+            const double t = (double)((s & 3) == 0 ? tq.x : (s & 3) == 1 ? tq.y : (s & 3) == 2 ? tq.z : tq.w);
+            u[ti] = after_step<EVERY>(mfma_f64(t, x, u[ti]), mp);
+        }
     }
-    for (int idx = tid; idx < WMAX * WMAX; idx += 256) {
-        const int i = idx / WMAX, j = idx % WMAX;
-        Ls[i][j] = (j < i && i < npiv) ? Lf[i][s_pj[j]] : 0u;
-    }
-    __syncthreads();
-    // rows of U for the group's columns: thread k solves column k, right
-    // looking (each solved value is subtracted from the rows below at once,
-    // so the dependent chain per row is one normalisation and one FMA)
-    if (tid < nc) {
-        double a[WMAX];
+    if (!EVERY)
 #pragma unroll
-        for (int i = 0; i < WMAX; ++i) a[i] = (double)xs[i];
+        for (int ti = 0; ti < 2; ++ti) u[ti] = after_step<true>(u[ti], mp);
+    if (rel0 == 0 && cw + cl < nr) {
+        // the pivot rows
+        int32_t *dst = Cp + (int64_t)cl * ldw + kr0;
 #pragma unroll
-        for (int j = 0; j < WMAX; ++j) {
-            if (j < npiv) {
-                // x_j = a_j / pivot_j mod p; for small p in FP64 throughout
-                // (the reduced a_j times the inverse is below 2^32)
-                const double x = LAZY ? dmod_near(dmod_near(a[j], mp) * (double)invs[j], mp)
-                                      : (double)mulmod((uint32_t)a[j], invs[j], mp);
-                Ut[tid][s_pj[j]] = x;
+        for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
-                for (int i = j + 1; i < WMAX; ++i) {
-                    a[i] = fma(-(double)Ls[i][j], x, a[i]);
-                    if (!LAZY) a[i] = dmod(a[i], mp);
-                }
+            for (int e = 0; e < 4; ++e) {
+                const int t = solve->num[16 * ti + 4 * e + g];
+                if (t >= 0) dst[t] = (int32_t)from_near(u[ti][e], mp);
             }
-        }
     }
-    __syncthreads();
-    if (!row_ok) return;
-    const int rel = (int)(r - kr0);
-    if (rel < npiv) {
-        // pivot row: its row of U
-        const int pj = s_pj[rel];
+    if (rel0 + 32 <= npiv) return;
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-            const int col = cl + 4 * k;
-            if (col < nc) W[r + (int64_t)(cfirst + col) * ldw] = (int32_t)(uint32_t)Ut[col][pj];
-        }
-        return;
-    }
-    const int e = s_e[tid & 63];
-    if (e >= 0) {
-        // a row that moved here: its old values are in the stage
+    for (int a = 0; a < 2; ++a) {
+        v4d c = v4d{0, 0, 0, 0};
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-            const int col = cl + 4 * k;
-            if (col < nc) cv[k] = stage[e + 64 * (ci0 + col)];
-        }
-    }
+        for (int s = 0; s < 8; ++s) c = after_step<EVERY>(mfma_f64(u[s >> 2][s & 3], balanced(lv[a][s], mp), c), mp);
+        const int rel = rel0 + 16 * a + cl;
+        if (rel >= npiv && kr0 + rel < m) {
 #pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-        const int col = cl + 4 * k;
-        if (col < nc) {
-            double acc = (double)cv[k];
-#pragma unroll
-            for (int jj = 0; jj < WMAX; ++jj) {
-                acc = fma(-Lr[jj], Ut[col][jj], acc);
-                if (!LAZY) acc = dmod(acc, mp);
-            }
-            W[r + (int64_t)(cfirst + col) * ldw] = (int32_t)(uint32_t)(LAZY ? dmod_near(acc, mp) : acc);
+            for (int e = 0; e < 4; ++e)
+                if (cw + 4 * e + g < nr)
+                    Cp[kr0 + rel + (int64_t)(4 * e + g) * ldw] =
+                        (int32_t)from_near(near_mod((double)cv[a][e] - c[e], mp), mp);
         }
     }
 }
 
 constexpr int MAXPAN = 64;  // inner panels per outer block (NBO / smallest panel width, 2)
 
-// End of an outer block with P pivots (rows [KR, KR+P)), whose inner panels
-// left their row gather maps in bmap_*: one wave per column outside the block
-// [KC, FAR).  Columns left of the block get the swaps; far columns get the
-// swaps, then the solve with the block's L11 (P x P, in LDS; lanes hold rows
-// i and i+64), and their U rows go to Ubig (rows 0..consumed-1 indexed by
-// block column, zero for block columns without a pivot).
-template <bool LAZY>
-__global__ __launch_bounds__(1024) void k_block_finish(int32_t *__restrict__ W, int64_t ldw, int64_t n, int KR,
-                                                       int KC, int FAR, int P, int consumed, int npanels,
-                                                       const int32_t *__restrict__ bmap_dst,
-                                                       const int32_t *__restrict__ bmap_src,
-                                                       const PanelCtl *__restrict__ bctl,
-                                                       const int32_t *__restrict__ pivinv,
-                                                       const int32_t *__restrict__ pivcol,
-                                                       int32_t *__restrict__ Ubig, int64_t ldub, ModP mp,
-                                                       const int *__restrict__ skip)
+// T of the diagonal 32 x 32 triangles of a block's L11 by pivot number, for
+// blocks whose panels are not 32 pivots in 32 columns each: one thread a column.
+// It replaces the panels' own, and runs only when no update needs them again.
+__global__ __launch_bounds__(NBO) void k_block_solve(const int32_t *__restrict__ W, int64_t ldw, int KR, int P,
+                                                     const int32_t *__restrict__ pivinv,
+                                                     const int32_t *__restrict__ pivcol, ModP mp,
+                                                     PanelSolve *__restrict__ solve, const int *__restrict__ skip)
 {
     if (skip && *skip) return;
-    __shared__ uint32_t Ls[128][129];
-    __shared__ uint32_t invs[128];
-    __shared__ int ucolmap[128];
-    __shared__ int s_pc[128];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid < 128) {
-        const int t = min(tid, P - 1);
-        s_pc[tid] = pivcol[KR + t];
-        invs[tid] = (uint32_t)pivinv[KR + t];
-        ucolmap[tid] = -1;
+    __shared__ uint32_t s_x[NBO][PNW + 1];
+    const int tid = threadIdx.x, b0 = tid / PNW * PNW, q = tid % PNW;
+    for (int t = 0; t < PNW; ++t) {
+        uint32_t x = 0;
+        if (b0 + t < P && t >= q) {
+            x = t == q ? 1u : 0u;
+            for (int k = q; k < t; ++k)
+                x = submod(x, mulmod((uint32_t)W[KR + b0 + t + (int64_t)pivcol[KR + b0 + k] * ldw], s_x[tid][k], mp), mp);
+            x = mulmod(x, (uint32_t)pivinv[KR + b0 + t], mp);
+        }
+        s_x[tid][t] = x;
+        solve[tid / PNW].t[t][q] = (int)x > mp.half ? (int32_t)x - (int32_t)mp.p : (int32_t)x;
     }
-    __syncthreads();
-    // L11 into LDS: lanes take consecutive rows of one pivot column, and
-    // every load is issued before the first LDS store
-    {
-        constexpr int LPT = 128 * 128 / 1024;
-        uint32_t lv[LPT];
+}
+
+// End of an outer block with P pivots (rows [KR, KR+P)): the columns outside
+// the block [KC, FAR) get its row moves, those right of it also the solve with
+// the block's L11, and their U rows go to Ubig (rows 0..consumed-1 by block
+// column, zero for block columns without a pivot).
+//
+// A wave takes 16 columns.  The moved rows are single elements of W far apart
+// in a column (up to 2 x 128 lines of 64 bytes a column, read and written),
+// which bounds the launch from below; the solve goes 32 pivots at a time, X_i
+// = A_i - sum_j<i L_ij U_j and U_i = T_i X_i with T from the panels, in FP64
+// MFMAs whose accumulators are the next product's operands as they are.
+// DENSE: the pivots are the block's first P columns.  Mean over the blocks of a
+// 4096^2 PLUQ mod 65521 21.5 us, of a 1500^2 inverse mod 2^26 - 5 25 us; with the
+// panels' moves one after another and a 128-step substitution by lanes 46 and 53.
+template <bool EVERY, bool DENSE>
+__global__ __launch_bounds__(64) void k_block_finish(int32_t *__restrict__ W, int64_t ldw, int m, int64_t n, int KR,
+                                                     int KC, int FAR, int P, int consumed, int gleft,
+                                                     const BlockMoves *__restrict__ moves,
+                                                     const PanelSolve *__restrict__ solve,
+                                                     const int32_t *__restrict__ pivcol,
+                                                     int32_t *__restrict__ Ubig, int64_t ldub, ModP mp,
+                                                     const int *__restrict__ skip)
+{
+    if (skip && *skip) return;
+    const int lane = threadIdx.x, cl = lane & 15, g = lane >> 4;
+    const bool left = (int)blockIdx.x < gleft;
+    const int64_t cb = left ? (int64_t)blockIdx.x * 16 : FAR + (int64_t)((int)blockIdx.x - gleft) * 16;
+    const int nc = (int)min((int64_t)16, (left ? KC : n) - cb);
+    int32_t *const col = W + (cb + min(cl, nc - 1)) * ldw;
+    constexpr int NT = NBO / 16;
+    // position 16 b + 4 e + g of the block's rows, and the other moved rows
+    int32_t x[NT][4], y[2][16];
 #pragma unroll
-        for (int k = 0; k < LPT; ++k) {
-            const int idx = tid + 1024 * k, i = min(idx % 128, P - 1), j = min(idx / 128, P - 1);
-            lv[k] = (uint32_t)W[(int64_t)(KR + i) + (int64_t)s_pc[j] * ldw];
-        }
-        // rows scaled by their pivot's inverse: the system becomes unit
-        // lower triangular, so the substitution needs no multiply per step
+    for (int b = 0; b < NT; ++b)
 #pragma unroll
-        for (int k = 0; k < LPT; ++k) {
-            const int idx = tid + 1024 * k, i = idx % 128, j = idx / 128;
-            Ls[i][j] = (j < i && i < P) ? mulmod(lv[k], invs[i], mp) : 0u;
+        for (int e = 0; e < 4; ++e) x[b][e] = moves->top[16 * b + 4 * e + g];
+    const int nrest = moves->n;
+    int rs[2], rd[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        rs[h] = moves->src[lane + 64 * h];
+        rd[h] = moves->dst[lane + 64 * h];
+    }
+#pragma unroll
+    for (int b = 0; b < NT; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[b][e] = col[min(x[b][e], m - 1)];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        if (lane + 64 * h < nrest)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) y[h][q] = W[rs[h] + (cb + min(q, nc - 1)) * ldw];
+    auto store_moved = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            if (lane + 64 * h < nrest)
+#pragma unroll
+                for (int q = 0; q < 16; ++q)
+                    if (q < nc) W[rd[h] + (cb + q) * ldw] = y[h][q];
+        if (cl >= nc) return;
+#pragma unroll
+        for (int b = 0; b < NT; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int k = 16 * b + 4 * e + g;
+                if ((left || k >= P) && KR + k < m) col[KR + k] = x[b][e];
+            }
+    };
+    if (left) {
+        store_moved();
+        return;
+    }
+    int64_t lc[NT - 2][4];  // columns of the pivots
+#pragma unroll
+    for (int b = 0; b < NT - 2; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int k = min(16 * b + 4 * e + g, P - 1);
+            lc[b][e] = (DENSE ? KC + k : pivcol[KR + k]) * ldw;
+        }
+    v4d u[NT];
+#pragma unroll
+    for (int i = 0; i < NT / 2; ++i) {
+        if (32 * i >= P) {
+            u[2 * i] = u[2 * i + 1] = v4d{0, 0, 0, 0};
+            continue;
+        }
+        v4d s[2], r[2] = {v4d{0, 0, 0, 0}, v4d{0, 0, 0, 0}};
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            s[a] = v4d{0, 0, 0, 0};
+            const int32_t *Lp = W + min(KR + 32 * i + 16 * a + cl, m - 1);
+#pragma unroll
+            for (int b = 0; b < 2 * i; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    s[a] = after_step<EVERY>(mfma_f64(balanced(Lp[lc[b][e]], mp), u[b][e], s[a]), mp);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[a][e] = near_mod(balanced(x[2 * i + a][e], mp) - s[a][e], mp);
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+#pragma unroll
+            for (int b = 0; b <= a; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    r[a] = after_step<EVERY>(mfma_f64((double)solve[i].t[16 * a + cl][16 * b + 4 * e + g], s[b][e], r[a]), mp);
+            u[2 * i + a] = after_step<true>(r[a], mp);
         }
     }
-    if (tid < P) ucolmap[s_pc[tid] - KC] = tid;
-    __syncthreads();
-    const int64_t nout = n - (FAR - KC);
-    const int um0 = lane < consumed ? ucolmap[lane] : -1;
-    const int um1 = lane + 64 < consumed ? ucolmap[lane + 64] : -1;
-    for (int64_t ci = (int64_t)blockIdx.x * 16 + wave; ci < nout; ci += (int64_t)gridDim.x * 16) {
-        int64_t c = ci < KC ? ci : ci + (FAR - KC);
-        int32_t *col = W + c * ldw;
-        for (int t = 0; t < npanels; ++t) {
-            const int nm = bctl[t].nmap;
-            const int32_t *md = bmap_dst + t * 64, *ms = bmap_src + t * 64;
-            uint32_t v = 0;
-            int d = 0;
-            if (lane < nm) { v = (uint32_t)col[ms[lane]]; d = md[lane]; }
-            if (lane < nm) col[d] = (int32_t)v;
-            __threadfence_block();
-        }
-        if (c < KC) continue;
-        // forward substitution with the unit triangular system (rows and
-        // right-hand side scaled by the pivots' inverses), lanes hold rows
-        // lane and lane + 64: at step j every lane reduces its own sum (only
-        // lane j's is used), readlane broadcasts it, and the rows below
-        // subtract L[i][j] x_j.  LAZY (p < 2^16): the sums of at most 127
-        // products below 2^32 stay exact in FP64 and are reduced once.
-        double a0 = lane < P ? (double)mulmod((uint32_t)col[KR + lane], invs[lane], mp) : 0.0;
-        double a1 = lane + 64 < P ? (double)mulmod((uint32_t)col[KR + lane + 64], invs[lane + 64], mp) : 0.0;
-        for (int j = 0; j < P; ++j) {
-            const double aj = j < 64 ? a0 : a1;
-            const uint32_t xl = (uint32_t)(LAZY ? dmod_near(aj, mp) : aj);
-            const uint32_t xj = (uint32_t)__builtin_amdgcn_readlane((int)xl, j & 63);
-            const double xd = (double)xj;
-            if (j < 64) {
-                a0 = lane == j ? xd : a0;
-                if (lane > j) {
-                    a0 = fma(-(double)Ls[lane][j], xd, a0);
-                    if (!LAZY) a0 = dmod(a0, mp);
-                }
-            } else if (lane == j - 64) {
-                a1 = xd;
-            }
-            if (lane + 64 > j) {
-                a1 = fma(-(double)Ls[lane + 64][j], xd, a1);
-                if (!LAZY) a1 = dmod(a1, mp);
-            }
-        }
-        const uint32_t x0 = (uint32_t)a0, x1 = (uint32_t)a1;
-        if (lane < P) col[KR + lane] = (int32_t)x0;
-        if (lane + 64 < P) col[KR + lane + 64] = (int32_t)x1;
-        // Ubig rows 0..consumed-1 of this column: pivot i's value or zero
-        int32_t *ucol = Ubig + (c - KC) * ldub;
-        const int a0i = um0 < 0 ? 0 : um0, a1i = um1 < 0 ? 0 : um1;
-        const uint32_t y00 = (uint32_t)__shfl((int)x0, a0i & 63), y01 = (uint32_t)__shfl((int)x1, a0i & 63);
-        const uint32_t y10 = (uint32_t)__shfl((int)x0, a1i & 63), y11 = (uint32_t)__shfl((int)x1, a1i & 63);
-        if (lane < consumed) ucol[lane] = um0 < 0 ? 0 : (int32_t)(a0i < 64 ? y00 : y01);
-        if (lane + 64 < consumed) ucol[lane + 64] = um1 < 0 ? 0 : (int32_t)(a1i < 64 ? y10 : y11);
+    store_moved();
+    if (cl >= nc) return;
+    int32_t *ucol = Ubig + (cb + cl - KC) * ldub;
+    if (!DENSE) {
+        for (int j = g; j < consumed; j += 4) ucol[j] = 0;
+        __threadfence_block();
     }
+#pragma unroll
+    for (int b = 0; b < NT; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int k = 16 * b + 4 * e + g;
+            if (k < P) {
+                const int32_t v = (int32_t)from_near(u[b][e], mp);
+                col[KR + k] = v;
+                ucol[DENSE ? k : pivcol[KR + k] - KC] = v;
+            }
+        }
 }
 
 // any nonzero in W[r0:m, c0:n] -> *flag = 1
@@ -698,7 +795,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     // pivot arrays, per-panel control blocks and row gather maps of one outer block
     const size_t npv = (size_t)mn + 64;
     const size_t piv_bytes = sizeof(int32_t) * (4 * npv + 2 * MAXPAN * 64) + sizeof(PanelCtl) * MAXPAN + 512 +
-                             sizeof(int32_t) * 64 * NBO;
+                             sizeof(int32_t) * 64 * NBO + sizeof(PanelSolve) * MAXPAN + sizeof(BlockMoves);
     int32_t *piv = (int32_t *)ws_get(ctx, WS_PIV, piv_bytes, &st);
     if (!piv) return st;
     int32_t *ipiv = piv, *pivval = piv + npv, *pivinv = piv + 2 * npv, *pivcol = piv + 3 * npv;
@@ -709,6 +806,8 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     int *cursor = flag + 2;                         // first row of the next panel (lu, rref)
     uint32_t *arrive = (uint32_t *)(flag + 4);      // one word per panel of the block
     int32_t *stage = (int32_t *)(arrive + MAXPAN);  // moved rows' old values, 64 x NBO
+    PanelSolve *solve = (PanelSolve *)(stage + 64 * NBO);  // one per panel of the block
+    BlockMoves *moves = (BlockMoves *)(solve + MAXPAN);
     int32_t *Ubig = (int32_t *)ws_get(ctx, WS_UBUF, sizeof(int32_t) * (size_t)NBO * (size_t)(n + 1), &st);
     if (!Ubig) return st;
     // row positions of the W-resident panel (position of each row, row at
@@ -770,14 +869,14 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         if (width == GNBW) {
             k_panel_g<GNBW><<<1, GPT, 0, ctx->stream>>>(W, ldw, (int)m, (int)rj, (int)cj, (int)w, mp, ple, ipiv,
                                                         pivval, pivinv, pivcol, mdst, msrc, pctl, abort,
-                                                        (int)KC, (int)FAR, stage, cursor, gpos, grow);
+                                                        (int)KC, (int)FAR, stage, cursor, gpos, grow, solve + t);
             return hip_check(ctx, hipGetLastError(), "k_panel_g launch");
         }
         PanelArgs a = {};
         a.W = W; a.ldw = ldw; a.m = (int)m; a.kr0 = (int)rj; a.c0 = (int)cj; a.w = (int)w; a.ple = ple;
         a.KC = (int)KC; a.FAR = (int)FAR; a.mp = mp; a.invs = invs;
         a.ipiv = ipiv; a.pivval = pivval; a.pivinv = pivinv; a.pivcol = pivcol;
-        a.map_dst = mdst; a.map_src = msrc; a.stage = stage; a.ctl = pctl; a.abort = abort; a.cursor = cursor;
+        a.map_dst = mdst; a.map_src = msrc; a.stage = stage; a.ctl = pctl; a.solve = solve + t; a.abort = abort; a.cursor = cursor;
         const int mode = mp.small ? 0 : mp.p <= ((int64_t)1 << 24) ? 1 : 2;
         if (m - rj <= PSINGLE) {
             if (mode == 0) k_panel<false, 0><<<1, PSINGLE, 0, ctx->stream>>>(a);
@@ -801,48 +900,47 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         return hip_check(ctx, hipMemsetAsync(abort_flag, 0, (size_t)((char *)(arrive + MAXPAN) - (char *)abort_flag),
                                              ctx->stream), "block flags");
     };
-    // the rest of the outer block after panel t: its row moves, and right
-    // of the panel the rows of U and the rank-npiv update below the pivots
-    auto update_t = [&](int t, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w, const int *skip) -> int {
+    // the rest of the outer block [KC, FAR) from row KR after panel t: its row
+    // moves, and right of the panel the rows of U and the rank-npiv update below
+    // the pivots.  rj is the panel's first row, or a lower bound with the row on
+    // the device (ple)
+    auto update_t = [&](int t, int64_t KR, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w,
+                        const int *skip) -> int {
         const int64_t nl = cj - KC, nr = FAR - (cj + w);
-        const unsigned gy = (unsigned)((nl + UT_C - 1) / UT_C + (nr + UT_C - 1) / UT_C);
-        if (gy == 0) return MODP_OK;
-        const dim3 grid((unsigned)((m - rj + UT_R - 1) / UT_R), gy);
+        if (nl + nr + (n - (FAR - KC)) == 0) return MODP_OK;
+        const int64_t tiles = ((m - rj + UT_R - 1) / UT_R) * ((nr + UT_C - 1) / UT_C);
+        const unsigned grid = (unsigned)(1 + (nl + UT_L - 1) / UT_L + tiles);
+        const int kr0 = ple ? -1 : (int)rj;
         TimedLaunch tl(ctx, "elim_update");
-#define LAUNCH_UPDATE(WM_) \
-    if (mp.small) \
-        k_update<WM_, true><<<grid, 256, 0, ctx->stream>>>(W, ldw, (int)m, (int)KC, (int)FAR, (int)cj, (int)w, \
-                                                           bctl + t, pivinv, pivcol, bmap_dst + t * 64, stage, mp, skip); \
-    else \
-        k_update<WM_, false><<<grid, 256, 0, ctx->stream>>>(W, ldw, (int)m, (int)KC, (int)FAR, (int)cj, (int)w, \
-                                                            bctl + t, pivinv, pivcol, bmap_dst + t * 64, stage, mp, skip);
-        if (w <= 8) {
-            LAUNCH_UPDATE(8)
-        } else if (w <= 16) {
-            LAUNCH_UPDATE(16)
-        } else {
-            LAUNCH_UPDATE(32)
-        }
-#undef LAUNCH_UPDATE
+        if (mp.p <= ((int64_t)1 << 24))
+            k_update<false><<<grid, 256, 0, ctx->stream>>>(W, ldw, (int)m, (int)KR, (int)KC, (int)FAR, (int)cj, (int)w,
+                                                           kr0, t == 0, bctl + t, solve + t, bmap_dst + t * 64,
+                                                           bmap_src + t * 64, stage, moves, mp, skip);
+        else
+            k_update<true><<<grid, 256, 0, ctx->stream>>>(W, ldw, (int)m, (int)KR, (int)KC, (int)FAR, (int)cj, (int)w,
+                                                          kr0, t == 0, bctl + t, solve + t, bmap_dst + t * 64,
+                                                          bmap_src + t * 64, stage, moves, mp, skip);
         return hip_check(ctx, hipGetLastError(), "k_update launch");
     };
-    // end of an outer block with P pivots over `consumed` columns
-    auto block_end = [&](int64_t KR, int64_t KC, int64_t FAR, int64_t P, int64_t consumed, int npanels,
+    // end of an outer block with P pivots over `consumed` columns, found in
+    // panels of `width` columns; the multipliers left of it follow the row moves
+    // only where somebody reads them (L)
+    auto block_end = [&](int64_t KR, int64_t KC, int64_t FAR, int64_t P, int64_t consumed, int width,
                          const int *skip) -> int {
         if (P <= 0) return MODP_OK;
-        const int64_t nout = n - (FAR - KC);
-        if (nout > 0) {
+        const int64_t gleft = L ? (KC + 15) / 16 : 0, grid = gleft + (n - FAR + 15) / 16;
+        if (grid > 0) {
+            const bool dense = width == PNW && P == consumed, every = mp.p > ((int64_t)1 << 24);
+            if (!dense && n > FAR) {
+                k_block_solve<<<1, NBO, 0, ctx->stream>>>(W, ldw, (int)KR, (int)P, pivinv, pivcol, mp, solve, skip);
+                HIP_TRY(ctx, hipGetLastError());
+            }
             TimedLaunch tl(ctx, "elim_block_finish");
-            int64_t g = (nout + 15) / 16;
-            if (g > 2048) g = 2048;
-            if (mp.small)
-                k_block_finish<true><<<(unsigned)g, 1024, 0, ctx->stream>>>(
-                    W, ldw, n, (int)KR, (int)KC, (int)FAR, (int)P, (int)consumed, npanels, bmap_dst, bmap_src, bctl,
-                    pivinv, pivcol, Ubig, NBO, mp, skip);
-            else
-                k_block_finish<false><<<(unsigned)g, 1024, 0, ctx->stream>>>(
-                    W, ldw, n, (int)KR, (int)KC, (int)FAR, (int)P, (int)consumed, npanels, bmap_dst, bmap_src, bctl,
-                    pivinv, pivcol, Ubig, NBO, mp, skip);
+            auto *k = dense ? (every ? k_block_finish<true, true> : k_block_finish<false, true>)
+                            : (every ? k_block_finish<true, false> : k_block_finish<false, false>);
+            k<<<(unsigned)grid, 64, 0, ctx->stream>>>(W, ldw, (int)m, n, (int)KR, (int)KC, (int)FAR, (int)P,
+                                                      (int)consumed, (int)gleft, moves, solve, pivcol, Ubig, NBO, mp,
+                                                      skip);
             HIP_TRY(ctx, hipGetLastError());
         }
         const int64_t rbeg = KR + P;
@@ -883,10 +981,10 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             int64_t Pfull = 0;
             for (int t = 0; t < np; ++t) {
                 MODP_TRY(launch_panel_t(NBW, t, KC, FAR, pr[t], pcj[t], pw[t], abort_flag, nullptr));
-                MODP_TRY(update_t(t, KC, FAR, pr[t], pcj[t], pw[t], abort_flag));
+                MODP_TRY(update_t(t, KR, KC, FAR, pr[t], pcj[t], pw[t], abort_flag));
                 Pfull += pw[t];
             }
-            MODP_TRY(block_end(KR, KC, FAR, Pfull, Pfull, np, abort_flag));
+            MODP_TRY(block_end(KR, KC, FAR, Pfull, Pfull, NBW, abort_flag));
             // the control blocks and, right after them, the flags: one copy
             HIP_TRY(ctx, hipMemcpyAsync(hctl, bctl, sizeof(PanelCtl) * MAXPAN + 2 * sizeof(int), hipMemcpyDeviceToHost,
                                         ctx->stream));
@@ -909,9 +1007,9 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 const int64_t npiv = hctl[ts].npiv;
                 int64_t P = 0;
                 for (int t = 0; t < ts; ++t) P += pw[t];
-                if (npiv > 0) MODP_TRY(update_t(ts, KC, FAR, pr[ts], pcj[ts], pw[ts], nullptr));
+                if (npiv > 0) MODP_TRY(update_t(ts, KR, KC, FAR, pr[ts], pcj[ts], pw[ts], nullptr));
                 P += npiv;
-                MODP_TRY(block_end(KR, KC, FAR, P, P, ts + 1, nullptr));
+                MODP_TRY(block_end(KR, KC, FAR, P, P, NBW, nullptr));
                 kr += P;
                 kc += P;
                 stop_zero = hctl[ts].status == 1;
@@ -936,16 +1034,14 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             const int np = (int)pcj.size();
             for (int t = 0; t < np; ++t) {
                 MODP_TRY(launch_panel_t(NBW, t, KC, FAR, KR, pcj[t], pw[t], abort_flag, cursor));
-                MODP_TRY(update_t(t, KC, FAR, KR, pcj[t], pw[t], abort_flag));
+                MODP_TRY(update_t(t, KR, KC, FAR, KR, pcj[t], pw[t], abort_flag));
             }
             HIP_TRY(ctx, hipMemcpyAsync(hctl, bctl, sizeof(PanelCtl) * np, hipMemcpyDeviceToHost, ctx->stream));
             HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
             int64_t P = 0, consumed = 0;
-            int npanels = 0;
             for (int t = 0; t < np; ++t) {
                 const PanelCtl &pc = hctl[t];
                 if (pc.status == 4) break;
-                ++npanels;
                 if (pc.status == 3)
                     return set_error(ctx, MODP_ERR_NOT_INVERTIBLE,
                                      "pivot has no inverse modulo %lld (modulus not prime)", (long long)p);
@@ -956,13 +1052,13 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 consumed += pc.ncols;
                 if (pc.status != 0) {
                     // the update after this panel was skipped by its own flag
-                    if (pc.npiv > 0) MODP_TRY(update_t(t, KC, FAR, KR, pcj[t], pw[t], nullptr));
+                    if (pc.npiv > 0) MODP_TRY(update_t(t, KR, KC, FAR, KR, pcj[t], pw[t], nullptr));
                     break;
                 }
             }
             kr += P;
             kc += consumed;
-            MODP_TRY(block_end(KR, KC, FAR, P, consumed, npanels, nullptr));
+            MODP_TRY(block_end(KR, KC, FAR, P, consumed, NBW, nullptr));
             if (P < consumed && kr < m && kc < n) {
                 // the block met zero columns: if nothing nonzero is left
                 // below row kr, no later column has a pivot and the

@@ -40,6 +40,9 @@
 // cycles with loads that bypass L1 (non-temporal) and plain stores inside one
 // XCD, 2050 with agent-scope loads and stores, 2700 to 3100 across XCDs.
 //
+// The panel also leaves the inverse of its pivot triangle (PanelSolve), from the
+// upper half of the waves that rebuild rows, at no step of the chain.
+//
 // A 32-column panel mod 65521 takes 49 us at 4096 rows (one 512-thread
 // workgroup with eight rows a thread, unrolled, and the rows published by
 // one-lane LDS writes: 94 us, as four panels of 8 columns) and 36 us at 256
@@ -89,7 +92,14 @@ struct PanelCtl {
 // the context; every launch uses tags of its own)
 struct PanelExchange {
     unsigned long long key[2][PXS];       // residue 26, 32767 - position 15, lane 6, tag 17 bits
-    unsigned long long row[2][PXS][PNW];  // entry (signed), tag
+    unsigned long long row[2][PXS][2 * PNW];  // entry (signed), tag
+};
+
+// What a panel leaves for the solves with its pivot rows: the rows of U of any
+// other columns are T times the pivot rows' old values.
+struct PanelSolve {
+    int32_t t[PNW][PNW];  // balanced; row: panel column (0: no pivot), column: pivot
+    int32_t num[PNW];     // pivot of a panel column, or -1
 };
 
 struct PanelArgs {
@@ -100,6 +110,7 @@ struct PanelArgs {
     const uint32_t *invs;  // inverses of 0..PINV-1 (0: none)
     int32_t *ipiv, *pivval, *pivinv, *pivcol, *map_dst, *map_src, *stage;
     PanelCtl *ctl;
+    PanelSolve *solve;
     int *abort, *cursor;
     PanelExchange *x;
     uint32_t *arrive;
@@ -390,7 +401,7 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     // original and reduced columns by local row, a wave's rows of 64 (the odd
     // pitch spreads a row of the panel over the banks)
     __shared__ int32_t s_A[PWAVES][PNW][65], s_L[PWAVES][PNW][65];
-    __shared__ double s_U[PNW][PNW];  // scaled rows (negated) by column
+    __shared__ double s_U[PNW][2 * PNW];  // scaled rows (negated) by column, and the rows of T
     __shared__ uint32_t s_T[PINV];
     __shared__ __attribute__((aligned(16))) double s_key[2][PWAVES];
     __shared__ int s_go;
@@ -449,6 +460,7 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     // that moved it last
     int pos = exists ? i : -1, dk = 0;
     int pc = 0, status = 0, consumed = w, spins = 0;
+    uint32_t pivcols = 0;  // columns that have a pivot
     // lane t: pivot t's old position, value, inverse and column; the position
     // again, or -1 when a later pivot came from there, too
     int ip_l = -1, pv_l = 0, pi_l = 0, pj_l = 0, iq_l = -1;
@@ -456,8 +468,8 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     // the previous pivot: this row's multiplier (negated) and the scaled row,
     // column lane % 16 and 16 + lane % 16 after the pivot's
     double nl = 0.0, u0 = 0.0, u1 = 0.0;
-    // the negated scaled rows, lane j (and 32 + j) column j, zero where a column
-    // has no pivot: column jc of the running chunk in h[3 - jc % 4], older ones
+    // the negated scaled rows, lane j column j, lane 32 + j column j of T, zero
+    // where a column has no pivot: column jc of the running chunk in h[3 - jc % 4], older ones
     // from h[4] on
     constexpr int NH = PNW + 4;
     double h[NH];
@@ -506,9 +518,11 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
                 // local row lr of wave lw as it is now, lane j column j, from its
                 // original entries and multipliers (h is zero where there are
                 // none); below 2^16 the sum stays below 2^37 and the
-                // multipliers need not be balanced
+                // multipliers need not be balanced.  Lanes 32 + j hold the same
+                // for the columns of an identity beside the panel, which turn
+                // into the rows of T: the upper half of the wave is free
                 auto row_now = [&](int lw, int lr) __attribute__((always_inline)) {
-                    double x = (double)s_A[lw][col][lr];
+                    double x = lane < PNW ? (double)s_A[lw][col][lr] : (col == jc ? 1.0 : 0.0);
                     double l0 = (double)s_L[lw][max(jc - 1 - back, 0)][lr], l1 = 0.0;
                     if (HW > 16) l1 = (double)s_L[lw][max(jc - 17 - back, 0)][lr];
                     if (MODE != 0) {
@@ -529,7 +543,7 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
                     // C
                     if (mine >> 15) {
                         const int32_t x = (int32_t)near_mod(row_now(wave, cl), mp);
-                        exchange_store(&a.x->row[par][gw][col], ((u64)(uint32_t)x << 32) | tag);
+                        exchange_store(&a.x->row[par][gw][lane], ((u64)(uint32_t)x << 32) | tag);
                     }
                     // D
                     u64 kt = 0;
@@ -564,7 +578,7 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
                 double x;
                 uint32_t inv;
                 if (MULTI) {
-                    u64 *rp = &a.x->row[par][at][col];
+                    u64 *rp = &a.x->row[par][at][lane];
                     u64 t = exchange_load(rp, 0);
                     inv = wave_inverse<MODE>(V != 0 ? V : 1u, s_T, mp, lane);
                     while (V != 0 && !__all((uint32_t)t == tag)) {
@@ -589,7 +603,8 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
                 nu = near_mod(-xi, mp);
                 nu = piv ? nu : 0.0;
                 un = -readlane_f64(nu, (jc + 1) & 31);
-                s_U[jc][col] = nu;
+                s_U[jc][lane] = nu;
+                pivcols |= piv ? 1u << jc : 0u;
                 // the winner moves to pc, the row at pc to Ip
                 const int Ip = piv ? 0x7fff - (int)(best & 0x7fffu) : -2, at_pc = piv ? pc : -2;
                 const bool out = pos == at_pc;
@@ -632,14 +647,18 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     for (int c = 4; c < chunks; ++c)
         chunk(c, std::integral_constant<int, 32>{}, std::integral_constant<int, 4>{});
 
-    // the pivots' scaled rows at their final places and the pivots' records, by
-    // the first workgroup (every wave has written all of s_U)
+    // the pivots' scaled rows at their final places, T and the pivots' records,
+    // by the first workgroup (every wave has written all of s_U)
     if (rank == 0) {
         int32_t *const dst = Wp + (int64_t)col * ldw + kr0;
-        for (int t = wave; t < pc; t += PWAVES) {
-            const int jc = __builtin_amdgcn_readlane(pj_l, t);
-            if (lane > jc && lane < w) dst[t] = (int32_t)(uint32_t)from_near(-s_U[jc][col], mp);
+        for (int jc = wave; jc < PNW; jc += PWAVES) {
+            const bool piv = (pivcols >> jc) & 1u;
+            const int t = __popc(pivcols & ((1u << jc) - 1u));
+            if (piv && lane > jc && lane < w) dst[t] = (int32_t)(uint32_t)from_near(-s_U[jc][col], mp);
+            if (lane < PNW) a.solve->t[jc][lane] = piv && lane < pc ? -(int32_t)s_U[jc][PNW + pj_l] : 0;
         }
+        if (wave == 0 && lane < PNW)
+            a.solve->num[lane] = ((pivcols >> lane) & 1u) ? (int)__popc(pivcols & ((1u << lane) - 1u)) : -1;
         if (wave == 0 && lane < pc) {
             a.ipiv[kr0 + lane] = kr0 + ip_l;
             a.pivval[kr0 + lane] = pv_l;
