@@ -733,11 +733,12 @@ __global__ void k_set_int(int *p, int v) { *p = v; }
 __global__ void k_inv_table(uint32_t *__restrict__ t, int n, ModP mp)
 {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a < n) t[a] = a > 0 && a < mp.p ? modinv((uint32_t)a, mp) : 0u;
+    if (a < n) t[a] = a > 0 && a < mp.p ? modinv_fast((uint32_t)a, mp) : 0u;
 }
 
-// Inverses of the residues below PINV, from which the panels make every other
-// inverse; built once per modulus and kept in the context.
+// Inverses of the residues below PINV (1 MiB at most, 8 us to build), from which
+// the panels make every other inverse; built once per modulus and kept in the
+// context.
 const uint32_t *inverse_table(modp_ctx *ctx, const ModP &mp, int *st)
 {
     if (ctx->invtab && ctx->invtab_p == mp.p) return ctx->invtab;
@@ -745,7 +746,8 @@ const uint32_t *inverse_table(modp_ctx *ctx, const ModP &mp, int *st)
         hipError_t e = hipMalloc(&ctx->invtab, sizeof(uint32_t) * PINV);
         if (e != hipSuccess) { *st = hip_check(ctx, e, "inverse table"); return nullptr; }
     }
-    k_inv_table<<<PINV / 256, 256, 0, ctx->stream>>>(ctx->invtab, PINV, mp);
+    const int n = mp.p < PINV ? (int)mp.p : PINV;
+    k_inv_table<<<(n + 255) / 256, 256, 0, ctx->stream>>>(ctx->invtab, n, mp);
     if (hipGetLastError() != hipSuccess) { *st = MODP_ERR_DEVICE; return nullptr; }
     ctx->invtab_p = mp.p;
     return ctx->invtab;
@@ -772,7 +774,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     // Panels of an outer block starting at row KR by the rows left: the register
     // panel of one workgroup (256 rows: one wave per SIMD) or of one XCD, the
     // W-resident panel beyond 16,384 rows.  Mod 65521 a 32-column panel takes
-    // 37 us on one workgroup and 49 us on an XCD, whatever its rows (one
+    // 37 us on one workgroup and 45 us on an XCD, whatever its rows (one
     // workgroup with 512 rows, two waves per SIMD: 58 us).
     // MODP_PANEL_GLOBAL=1 sends every panel to the W-resident kernel (used
     // to compare the two panel kernels at sizes both handle)
@@ -826,7 +828,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     if (st != MODP_OK) return st;
     // exchange area of the panels on one XCD: its words are recognised by
     // tags that count the context's panels, so old ones are cleared only when
-    // the 17 bits of a key's tag (the 32 of a residue's) have been through
+    // the 17 bits of a key's tag (the 31 of a row's) have been through
     PanelExchange *xch = nullptr;
     if (!force_global && m > PSINGLE) {
         const bool fresh = !ctx->ws[WS_PANEL];
@@ -836,8 +838,8 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     }
     auto next_tag = [&](uint32_t *t) -> int {
         if ((ctx->panel_tag & 0x1ffffu) == 0)
-            HIP_TRY(ctx, hipMemsetAsync(xch, 0, ctx->panel_tag == 0 ? sizeof(PanelExchange) : sizeof(xch->key),
-                                        ctx->stream));
+            HIP_TRY(ctx, hipMemsetAsync(xch, 0, (ctx->panel_tag & 0x7fffffffu) == 0 ? sizeof(PanelExchange)
+                                                                                     : sizeof(xch->key), ctx->stream));
         *t = ctx->panel_tag;
         ctx->panel_tag += 64;
         return MODP_OK;

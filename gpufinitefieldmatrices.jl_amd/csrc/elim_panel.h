@@ -10,11 +10,13 @@
 //
 //   A  reduce the column, find the wave's best (residue, lowest position) by
 //      DPP and publish it;
-//   B  apply the previous pivot to the columns after this one;
-//   C  (over several workgroups) publish the candidate's row;
+//   C  (over several workgroups) rebuild the candidate's row, scale it by its
+//      inverse and publish it;
+//   B  apply the previous pivot to the columns after this one and write its
+//      record down;
 //   D  find the winner among the waves' candidates;
-//   E  invert its pivot and take its row;
-//   F  scale the row, apply it to the next column, go on.
+//   E  take its row (one workgroup: rebuild and scale it now);
+//   F  apply the row to the next column, go on.
 //
 // A row as it is now is rebuilt by left-looking sums, x_j = a_j -
 // sum_k l_k u_kj with lane j column j, because nothing cheap moves one lane's
@@ -43,11 +45,13 @@
 // The panel also leaves the inverse of its pivot triangle (PanelSolve), from the
 // upper half of the waves that rebuild rows, at no step of the chain.
 //
-// A 32-column panel mod 65521 takes 49 us at 4096 rows (one 512-thread
-// workgroup with eight rows a thread, unrolled, and the rows published by
-// one-lane LDS writes: 94 us, as four panels of 8 columns) and 36 us at 256
-// (52 us); 4096^2 PLUQ 17.0 -> 12.4 ms, a 1500^2 inverse mod 2^26-5 12.7 ->
-// 7.6 ms.
+// A 32-column panel mod 65521 takes 45 us at 4096 rows and 37 us at 256,
+// mod 2^26 - 5 51 and 48 (before the rows were published scaled, the
+// inverses looked up and the records moved off the chain: 50, 38, 60 and 53;
+// one 512-thread workgroup with eight rows a thread, unrolled, and the rows
+// published by one-lane LDS writes: 94 and 52 mod 65521, as four panels of 8
+// columns).  Of a step's 2500 cycles over an XCD about 1100 are the key's way
+// there and 400 the row's; on one workgroup it is 1950.
 #pragma once
 #include <type_traits>
 
@@ -58,10 +62,11 @@ namespace {
 constexpr int PNW = 32;       // panel columns
 constexpr int PWAVES = 4;     // waves of a workgroup, one per SIMD
 constexpr int PXS = 256;      // slots of one exchange set (waves of a panel)
-constexpr int PINV = 1024;    // entries of the table of small inverses
+constexpr int PINV = 1 << 18;  // entries of the table of small inverses
 constexpr int PSINGLE = 64 * PWAVES;  // rows of the one-workgroup panel
 constexpr int PMULTI = 64 * PXS;  // rows of the panel on one XCD
 constexpr uint32_t PABORT = 0x80000000u;
+constexpr uint32_t PUNSCALED = 0x80000000u;  // beside a row's tag: not scaled yet
 
 // compile-time loop: f(integral_constant<int, J>) for J = B .. E-1
 template <int B, int E> struct Unroll {
@@ -92,7 +97,7 @@ struct PanelCtl {
 // the context; every launch uses tags of its own)
 struct PanelExchange {
     unsigned long long key[2][PXS];       // residue 26, 32767 - position 15, lane 6, tag 17 bits
-    unsigned long long row[2][PXS][2 * PNW];  // entry (signed), tag
+    unsigned long long row[2][PXS][2 * PNW];  // entry (signed), 31 bits of tag under PUNSCALED
 };
 
 // What a panel leaves for the solves with its pivot rows: the rows of U of any
@@ -200,83 +205,56 @@ template <int L0, int N> __device__ __forceinline__ void fmac_lanes(double *v, d
             : "v"(x), "v"(y));
     }
 }
-// acc += sum over k < 4 of (x of lane L0 + k) * y[k]
-template <int L0> __device__ __forceinline__ void dot_lanes(double &acc, double x, const double *y)
+// acc[k] += (x of lane L0 + k) * y[k] for k < 4
+template <int L0> __device__ __forceinline__ void dot_lanes(double *acc, double x, const double *y)
 {
     asm("s_nop 1\n\t"
-            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f64_dpp %0, %1, %3 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f64_dpp %0, %1, %4 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f64_dpp %0, %1, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
-        : "+v"(acc)
+            "v_fmac_f64_dpp %0, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %4, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %2, %4, %7 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %3, %4, %8 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
+        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])
         : "v"(x), "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "n"(L0), "n"(L0 + 1), "n"(L0 + 2), "n"(L0 + 3));
 }
 
 // a^{-1} mod p for a wave-uniform a in [1, p), 0 if it has none.  Extended
-// Euclid is a chain of about 15 to 25 divisions; this is one round (p < 2^18)
-// or two of Dirichlet's approximation theorem over the lanes: some multiplier
-// t <= 256 brings a t within p/257 of a multiple of p, every lane tries four
-// of them, and the small remainder s is inverted by table (s < 1024) or by
-// one more round, j p = q s + s2 with |s2| <= s/257 <= 2^26/257^2 < 1024, so
-// s^{-1} = -q s2^{-1}.  The identities hold for any modulus; for one that is
-// not prime a remainder without an inverse says nothing about a, and Euclid
-// decides.  F is the type that holds the products exactly: float for p < 2^16
-// (a t and T t stay below 2^24), double for the rest.
-template <typename F> struct Multiplier {
-    F r, t;  // a t = r mod the modulus, |r| <= modulus / 257
-};
-template <typename F>
-__device__ __forceinline__ Multiplier<F> small_multiple(F a, F mod, F modinv, F lane1)
+// Euclid is a chain of about 15 to 25 divisions on the panel's critical path;
+// this looks a up in the table of the inverses below PINV, or p - a, since
+// pivots are the largest of many residues.  Only p > PINV leaves anything else:
+// then, by Dirichlet's approximation theorem, some multiplier t <= 256 brings
+// a t within p/257 < PINV of a multiple of p (every lane tries four), and the
+// remainder is looked up.  For a modulus that is not prime a remainder without
+// an inverse says nothing about a, and Euclid decides.  With a table of 1024 in
+// LDS and one or two such rounds a step spent 540 cycles here mod 65521 and 940
+// mod 2^26 - 5; the lookup goes on beside the rebuilding of the row.
+template <int MODE> __device__ __forceinline__ uint32_t table_place(uint32_t a, const ModP &mp)
 {
-    // lane l tries l + 1 + 64 i and keeps the one that comes nearest
-    F r = 0, t = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const F ti = lane1 + (F)(64 * i), y = a * ti;
-        const F x = fma(-rint(y * modinv), mod, y);
-        const bool nearer = i == 0 || fabs(x) < fabs(r);
-        r = nearer ? x : r;
-        t = nearer ? ti : t;
-    }
-    const int l = (int)__builtin_ctzll(__ballot(fabs(r) * (F)257 <= mod)) & 63;
-    Multiplier<F> m;
-    if constexpr (sizeof(F) == 8) {
-        m.r = readlane_f64(r, l);
-        m.t = readlane_f64(t, l);
-    } else {
-        m.r = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r), l));
-        m.t = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, t), l));
-    }
-    return m;
+    return MODE == 0 || mp.p <= PINV ? a : mp.p32 - a;
 }
-template <int MODE>
-__device__ __forceinline__ uint32_t wave_inverse(uint32_t a, const uint32_t *T, const ModP &mp, int lane)
+// the inverse from the table's entry t at a's place, 0 if that has none
+template <int MODE> __device__ __forceinline__ uint32_t table_inverse(uint32_t a, uint32_t t, const ModP &mp)
 {
-    if (mp.p <= PINV) return (uint32_t)uniform((int)T[a]);
-    uint32_t inv;
-    if (MODE == 0) {
-        const float pf = (float)mp.p32;
-        const Multiplier<float> m = small_multiple<float>((float)a, pf, mp.pinvf, (float)(lane + 1));
-        float y = (float)T[(uint32_t)fabsf(m.r) & (PINV - 1)] * m.t;
-        y = m.r < 0.f ? -y : y;
-        y = fmaf(-rintf(y * mp.pinvf), pf, y);
-        inv = (uint32_t)uniform((int)(uint32_t)(y < 0.f ? y + pf : y));
-    } else {
-        const Multiplier<double> m = small_multiple<double>((double)a, mp.pd, mp.pinv, (double)(lane + 1));
-        const double s = fabs(m.r);
-        double z;
-        if (s < (double)PINV) {
-            z = (double)T[(uint32_t)s & (PINV - 1)];
-        } else {
-            // p t = r mod s with q = (p t - r) / s
-            const double sinv = __builtin_amdgcn_rcp(s);
-            const Multiplier<double> m2 = small_multiple<double>(mp.pd, s, sinv, (double)(lane + 1));
-            const double q = rint((mp.pd * m2.t - m2.r) * sinv);
-            z = near_mod(q * (double)T[(uint32_t)fabs(m2.r) & (PINV - 1)], mp);
-            z = m2.r > 0.0 ? -z : z;
+    if (MODE == 0 || mp.p <= PINV) return t;
+    return mp.p32 - a < (uint32_t)PINV && t != 0 ? mp.p32 - t : 0u;
+}
+__device__ __forceinline__ uint32_t search_inverse(uint32_t a, const uint32_t *__restrict__ T, const ModP &mp, int lane)
+{
+    uint32_t inv = 0;
+    if (mp.p > PINV) {
+        // lane l tries l + 1 + 64 i and keeps the one that comes nearest
+        double r = 0.0, t = 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const double ti = (double)(lane + 1 + 64 * i), x = near_mod((double)a * ti, mp);
+            const bool nearer = i == 0 || fabs(x) < fabs(r);
+            r = nearer ? x : r;
+            t = nearer ? ti : t;
         }
-        z = near_mod(z * (m.r < 0.0 ? -m.t : m.t), mp);
-        inv = (uint32_t)uniform((int)(uint32_t)from_near(z, mp));
+        const int l = (int)__builtin_ctzll(__ballot(fabs(r) * 257.0 <= mp.pd)) & 63;
+        r = readlane_f64(r, l);
+        t = readlane_f64(t, l);
+        const double z = (double)T[(uint32_t)fabs(r) & (PINV - 1)] * (r < 0.0 ? -t : t);
+        inv = (uint32_t)uniform((int)(uint32_t)from_near(near_mod(z, mp), mp));
     }
     if (inv == 0) inv = (uint32_t)uniform((int)modinv_fast(a, mp));
     return inv;
@@ -335,18 +313,17 @@ constexpr int EXCHANGE_SPINS = 1 << 20;
 //   1  p <= 2^24: 31 products below 2^46 stay below 2^51;
 //   2  p <= 2^26: reduced after at most five products (< 2^53).
 
-// wave64 maximum in every lane: DPP within the rows of 16 lanes, then the row
-// and half-wave exchanges
-__device__ __forceinline__ uint32_t wave_max_lanes(uint32_t v)
+// wave64 maximum: DPP within the rows of 16 lanes, then from row to row (each
+// step takes two wait states and one instruction; the last lane has it all)
+__device__ __forceinline__ uint32_t wave_max_dpp(uint32_t v)
 {
     v = kmax(v, dpp32<0xB1>(v));   // quad_perm [1,0,3,2]
     v = kmax(v, dpp32<0x4E>(v));   // quad_perm [2,3,0,1]
     v = kmax(v, dpp32<0x141>(v));  // row_half_mirror
     v = kmax(v, dpp32<0x140>(v));  // row_mirror
-    const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    v = kmax((uint32_t)a[0], (uint32_t)a[1]);
-    const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    return kmax((uint32_t)b[0], (uint32_t)b[1]);
+    v = kmax(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    v = kmax(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
 // The best of the lanes' (residue, 32767 - position): residue << 15 | the
@@ -355,20 +332,19 @@ __device__ __forceinline__ uint32_t wave_max_lanes(uint32_t v)
 template <int MODE> __device__ __forceinline__ uint64_t panel_best(uint32_t v, uint32_t notpos, int *lane_of)
 {
     if (MODE == 0) {
-        const uint32_t k = (v << 15) | notpos, top = wave_max_lanes(k);
+        const uint32_t k = (v << 15) | notpos, top = wave_max_dpp(k);
         *lane_of = (int)__builtin_ctzll(__ballot(k == top));
-        return (uint32_t)__builtin_amdgcn_readfirstlane((int)top);
+        return top;
     }
-    const uint32_t top = wave_max_lanes(v);
+    const uint32_t top = wave_max_dpp(v);
     uint64_t at = __ballot(v == top);
     if (at & (at - 1)) {
-        const uint32_t np = wave_max_lanes(v == top ? notpos : 0u);
+        const uint32_t np = wave_max_dpp(v == top ? notpos : 0u);
         at = __ballot(v == top && notpos == np);
     }
     const int l = (int)__builtin_ctzll(at);
     *lane_of = l;
-    return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)top) << 15) |
-           (uint32_t)__builtin_amdgcn_readlane((int)notpos, l);
+    return ((uint64_t)top << 15) | (uint32_t)__builtin_amdgcn_readlane((int)notpos, l);
 }
 
 template <bool MULTI, int MODE>
@@ -402,7 +378,6 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     // pitch spreads a row of the panel over the banks)
     __shared__ int32_t s_A[PWAVES][PNW][65], s_L[PWAVES][PNW][65];
     __shared__ double s_U[PNW][2 * PNW];  // scaled rows (negated) by column, and the rows of T
-    __shared__ uint32_t s_T[PINV];
     __shared__ __attribute__((aligned(16))) double s_key[2][PWAVES];
     __shared__ int s_go;
 
@@ -417,10 +392,6 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     constexpr int NV = PNW + 4;
     double v[NV];
     {
-        constexpr int TPT = PINV / (64 * PWAVES);
-        uint32_t t[TPT];
-#pragma unroll
-        for (int k = 0; k < TPT; ++k) t[k] = a.invs[tid + 64 * PWAVES * k];
         const uint32_t r = (uint32_t)min(kr0 + i, a.m - 1);
         const int32_t *col = Wp;
         int32_t x[PNW];
@@ -429,8 +400,6 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
             x[j] = col[r];
             col += j + 1 < w ? ldw : 0;
         }
-#pragma unroll
-        for (int k = 0; k < TPT; ++k) s_T[tid + 64 * PWAVES * k] = t[k];
 #pragma unroll
         for (int j = 0; j < PNW; ++j) {
             s_A[wave][j][lane] = x[j];
@@ -465,9 +434,23 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     // again, or -1 when a later pivot came from there, too
     int ip_l = -1, pv_l = 0, pi_l = 0, pj_l = 0, iq_l = -1;
     bool active = true;
-    // the previous pivot: this row's multiplier (negated) and the scaled row,
-    // column lane % 16 and 16 + lane % 16 after the pivot's
-    double nl = 0.0, u0 = 0.0, u1 = 0.0;
+    // the previous pivot: this row's multiplier and the scaled row (both
+    // negated), and what is still to be written down of it
+    double nl = 0.0, nup = 0.0;
+    int Ipp = -2, atp = -2, Vp = 0;
+    auto write_down = [&](int jc) __attribute__((always_inline)) {
+        s_U[jc & (PNW - 1)][lane] = nup;
+        iq_l = iq_l == Ipp ? -1 : iq_l;
+        const bool here = lane == atp;
+        ip_l = here ? Ipp : ip_l;
+        iq_l = here ? Ipp : iq_l;
+        pv_l = here ? Vp : pv_l;
+        // the identity's own column of the scaled row is the pivot's inverse
+        const double iv = -readlane_f64(nup, (PNW + jc) & 63);
+        pi_l = here ? (int)from_near(iv, mp) : pi_l;
+        pj_l = here ? jc : pj_l;
+        atp = Ipp = -2;
+    };
     // the negated scaled rows, lane j column j, lane 32 + j column j of T, zero
     // where a column has no pivot: column jc of the running chunk in h[3 - jc % 4], older ones
     // from h[4] on
@@ -483,9 +466,19 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
         auto step = [&](auto SC) __attribute__((always_inline)) {
             constexpr int s = decltype(SC)::value, par = s & 1;
             const int jc = 4 * c + s;
-            // A: column jc is final
-            const double cn = near_mod(v[s], mp);
-            const uint32_t ci = (uint32_t)from_near(cn, mp);
+            // A: column jc is final.  Below 2^51 the residue comes without a
+            // fix-up: (x + 1/2) / p is at least 1/(2p) away from every integer,
+            // and its rounded product is nearer to it than that
+            double cn;
+            uint32_t ci;
+            if constexpr (MODE == 2) {
+                cn = near_mod(v[s], mp);
+                ci = (uint32_t)from_near(cn, mp);
+            } else {
+                const double r = fma(-floor(fma(v[s], mp.pinv, 0.5 * mp.pinv)), mp.pd, v[s]);
+                ci = (uint32_t)r;
+                cn = MODE == 0 ? r : to_near(r, mp);
+            }
             s_L[wave][jc][lane] = (int32_t)ci;
             active = active && jc < w;
             if (active && pc >= rows) {
@@ -493,68 +486,97 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
                 consumed = jc;
                 active = false;
             }
-            const uint32_t tag = a.tag + 1 + (uint32_t)jc, tag17 = tag & 0x1ffffu;
-            uint64_t mine = 0;
-            int cl = 0;
-            if (active) {
+            const uint32_t tag = (a.tag + 1 + (uint32_t)jc) & 0x7fffffffu, tag17 = tag & 0x1ffffu;
+            // local row lr of wave lw as it is now, lane j column j, from its
+            // original entries and multipliers (h is zero where there are
+            // none); below 2^16 the sums stay below 2^37 and the
+            // multipliers need not be balanced.  Lanes 32 + j hold the same
+            // for the columns of an identity beside the panel, which turn
+            // into the rows of T: the upper half of the wave is free
+            auto row_now = [&](int lw, int lr) __attribute__((always_inline)) {
+                double x[4] = {lane < PNW ? (double)s_A[lw][col][lr] : (col == jc ? 1.0 : 0.0), 0.0, 0.0, 0.0};
+                double l0 = (double)s_L[lw][max(jc - 1 - back, 0)][lr], l1 = 0.0;
+                if (HW > 16) l1 = (double)s_L[lw][max(jc - 17 - back, 0)][lr];
+                if (MODE != 0) {
+                    l0 = to_near(l0, mp);
+                    l1 = to_near(l1, mp);
+                }
+                auto dot = [&](auto KC) __attribute__((always_inline)) {
+                    constexpr int k = 4 * decltype(KC)::value;
+                    dot_lanes<k & 15>(x, k < 16 ? l0 : l1, h + 4 - s + k);
+                    if constexpr (MODE == 2 && (k & 15) == 12)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) x[q] = near_mod(x[q], mp);
+                };
+                Unroll<0, HW / 4>::run(dot);
+                return (x[0] + x[1]) + (x[2] + x[3]);
+            };
+            // a row as the pivot's: scaled by its inverse, negated, balanced
+            auto scaled = [&](double x, uint32_t inv) __attribute__((always_inline)) {
+                const double xi = MODE == 0 ? x * (double)inv : near_mod(x, mp) * to_near((double)inv, mp);
+                return near_mod(-xi, mp);
+            };
+            // B: the previous pivot on the columns after this one (register k is
+            // k - s + 1 columns after it), its row by the distance from this one
+            double u0 = 0.0, u1 = 0.0;
+            auto fetch_row = [&]() __attribute__((always_inline)) {
+                const uint64_t b = __builtin_bit_cast(uint64_t, -nup);
+                auto column = [&](int j) {
+                    const int src = 4 * (jc - 1 + j);
+                    const uint32_t lo = __builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)b);
+                    const uint32_t hi = __builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)(b >> 32));
+                    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+                };
+                u0 = column(back);
+                u1 = column(16 + back);
+            };
+            auto apply_row = [&]() __attribute__((always_inline)) {
+                fmac_lanes<2, 14>(v + s + 1, u0, nl);
+                fmac_lanes<0, CW>(v + s + 15, u1, nl);
+                if constexpr (MODE == 2 && s == 3) {
+#pragma unroll
+                    for (int k = s + 1; k < (CW == 16 ? PNW : 19); ++k) v[k] = near_mod(v[k], mp);
+                }
+                write_down(jc - 1);
+            };
+            double nu = 0.0, un = 0.0;  // the scaled row (negated); its next column
+            if (!active) {
+                fetch_row();
+                apply_row();
+            } else {
                 const bool alive = pos >= pc;
-                mine = panel_best<MODE>(alive ? ci : 0u, alive ? 0x7fffu - (uint32_t)pos : 0u, &cl);
+                int cl;
+                const uint64_t mine = panel_best<MODE>(alive ? ci : 0u, alive ? 0x7fffu - (uint32_t)pos : 0u, &cl);
                 if (MULTI) {
                     if (lane == 0) exchange_store(&a.x->key[par][gw], (mine << 23) | ((uint32_t)cl << 17) | tag17);
                 } else {
                     if (lane == 0) s_key[par][wave] = __builtin_bit_cast(double, (mine << 8) | (uint32_t)(wave * 64 + cl));
                 }
-            }
-            // B: the previous pivot on the columns after this one (register k is
-            // k - s + 1 columns after it)
-            fmac_lanes<2, 14>(v + s + 1, u0, nl);
-            fmac_lanes<0, CW>(v + s + 15, u1, nl);
-            if constexpr (MODE == 2 && s == 3) {
-#pragma unroll
-                for (int k = s + 1; k < (CW == 16 ? PNW : 19); ++k) v[k] = near_mod(v[k], mp);
-            }
-            double nu = 0.0, un = 0.0;  // the scaled row (negated); its next column
-            if (active) {
-                // local row lr of wave lw as it is now, lane j column j, from its
-                // original entries and multipliers (h is zero where there are
-                // none); below 2^16 the sum stays below 2^37 and the
-                // multipliers need not be balanced.  Lanes 32 + j hold the same
-                // for the columns of an identity beside the panel, which turn
-                // into the rows of T: the upper half of the wave is free
-                auto row_now = [&](int lw, int lr) __attribute__((always_inline)) {
-                    double x = lane < PNW ? (double)s_A[lw][col][lr] : (col == jc ? 1.0 : 0.0);
-                    double l0 = (double)s_L[lw][max(jc - 1 - back, 0)][lr], l1 = 0.0;
-                    if (HW > 16) l1 = (double)s_L[lw][max(jc - 17 - back, 0)][lr];
-                    if (MODE != 0) {
-                        l0 = to_near(l0, mp);
-                        l1 = to_near(l1, mp);
-                    }
-                    auto dot = [&](auto KC) __attribute__((always_inline)) {
-                        constexpr int k = 4 * decltype(KC)::value;
-                        dot_lanes<k & 15>(x, k < 16 ? l0 : l1, h + 4 - s + k);
-                        if constexpr (MODE == 2) x = near_mod(x, mp);
-                    };
-                    Unroll<0, HW / 4>::run(dot);
-                    return x;
-                };
+                // the table's entry for this wave's candidate, in case it wins
+                const uint32_t early = a.invs[min(table_place<MODE>((uint32_t)(mine >> 15), mp), (uint32_t)PINV - 1)];
+                fetch_row();
                 uint64_t best;
                 int at;  // MULTI: winner's slot, else its local row
                 if (MULTI) {
-                    // C
-                    if (mine >> 15) {
-                        const int32_t x = (int32_t)near_mod(row_now(wave, cl), mp);
-                        exchange_store(&a.x->row[par][gw][lane], ((u64)(uint32_t)x << 32) | tag);
-                    }
+                    // C: the first look at the keys goes out before the row, or it
+                    // would wait for that store to end
+                    const double x = row_now(wave, cl);
+                    const uint32_t inv = table_inverse<MODE>((uint32_t)(mine >> 15), early, mp);
+                    const int32_t xi = (int32_t)(inv != 0 ? scaled(x, inv) : near_mod(x, mp));
+                    u64 t = exchange_load(&a.x->key[par][min(lane, nw - 1)], 0);
+                    asm volatile("" ::: "memory");
+                    exchange_store(&a.x->row[par][gw][lane],
+                                   ((u64)(uint32_t)xi << 32) | tag | (inv != 0 ? 0u : PUNSCALED));
+                    apply_row();
                     // D
                     u64 kt = 0;
                     int slot = 0;
                     for (int b = 0; b < nw; b += 64) {
                         const int idx = min(b + lane, nw - 1);
-                        u64 t;
-                        for (;;) {
-                            t = exchange_load(&a.x->key[par][idx], spins);
-                            if (__all((uint32_t)(t & 0x1ffffu) == tag17)) break;
+                        if (b != 0) t = exchange_load(&a.x->key[par][idx], spins);
+                        while (!__all((uint32_t)(t & 0x1ffffu) == tag17)) {
                             if (++spins > EXCHANGE_SPINS) break;
+                            t = exchange_load(&a.x->key[par][idx], spins);
                         }
                         if (t > kt || b == 0) {
                             kt = t;
@@ -565,6 +587,7 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
                     best = panel_best<MODE>((uint32_t)(kt >> 38), (uint32_t)(kt >> 23) & 0x7fffu, &l);
                     at = __builtin_amdgcn_readlane(slot, l);
                 } else {
+                    apply_row();
                     __syncthreads();
                     // words below 2^49 compare as the (denormal) doubles they spell
                     const uint64_t k = __builtin_bit_cast(uint64_t, fmax(fmax(s_key[par][0], s_key[par][1]),
@@ -573,66 +596,60 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
                     best = (((u64)hi << 32) | lo) >> 8;
                     at = (int)(lo & 0xffu);
                 }
+                // E: the scaled row
                 const uint32_t V = (uint32_t)(best >> 15);
-                // E (the inverse of 1 where the column is zero)
-                double x;
-                uint32_t inv;
+                bool piv = V != 0;
                 if (MULTI) {
                     u64 *rp = &a.x->row[par][at][lane];
                     u64 t = exchange_load(rp, 0);
-                    inv = wave_inverse<MODE>(V != 0 ? V : 1u, s_T, mp, lane);
-                    while (V != 0 && !__all((uint32_t)t == tag)) {
+                    while (piv && !__all((((uint32_t)t ^ tag) & ~PUNSCALED) == 0)) {
                         if (++spins > EXCHANGE_SPINS) break;
                         t = exchange_load(rp, spins);
                     }
-                    x = (double)(int32_t)(t >> 32);
+                    nu = (double)(int32_t)(t >> 32);
+                    const bool unscaled = __any((uint32_t)t & PUNSCALED);
+                    if (__builtin_expect(!piv || unscaled || spins > EXCHANGE_SPINS, 0)) {
+                        const uint32_t inv = piv && spins <= EXCHANGE_SPINS ? search_inverse(V, a.invs, mp, lane) : 0u;
+                        nu = scaled(nu, inv);
+                        piv = inv != 0;
+                    }
                 } else {
-                    inv = wave_inverse<MODE>(V != 0 ? V : 1u, s_T, mp, lane);
-                    x = row_now(at >> 6, at & 63);
+                    asm volatile("" ::"v"(early));
+                    const uint32_t entry = a.invs[min(table_place<MODE>(V, mp), (uint32_t)PINV - 1)];
+                    const double x = row_now(at >> 6, at & 63);
+                    uint32_t inv = (uint32_t)uniform((int)table_inverse<MODE>(V, entry, mp));
+                    if (__builtin_expect(inv == 0 || !piv, 0)) {
+                        inv = piv ? search_inverse(V, a.invs, mp, lane) : 0u;
+                        piv = inv != 0;
+                    }
+                    nu = scaled(x, inv);
                 }
-                const bool lost = spins > EXCHANGE_SPINS, piv = V != 0 && inv != 0 && !lost;
-                if (!piv && (V != 0 || !a.ple || lost)) {
-                    // a zero column (lu and rref skip it, pluq stops), or no inverse
-                    status = lost ? 6 : V == 0 ? 1 : 3;
-                    consumed = jc;
-                    active = false;
+                if (__builtin_expect(!piv, 0)) {
+                    const bool lost = spins > EXCHANGE_SPINS;
+                    if (V != 0 || !a.ple || lost) {
+                        // a zero column (lu and rref skip it, pluq stops), or no inverse
+                        status = lost ? 6 : V == 0 ? 1 : 3;
+                        consumed = jc;
+                        active = false;
+                    }
                 }
                 spins = 0;
                 // F: without a pivot the row is zero and no position matches
-                const double xi = MODE == 0 ? x * (double)inv : near_mod(x, mp) * to_near((double)inv, mp);
-                nu = near_mod(-xi, mp);
                 nu = piv ? nu : 0.0;
                 un = -readlane_f64(nu, (jc + 1) & 31);
-                s_U[jc][lane] = nu;
-                pivcols |= piv ? 1u << jc : 0u;
                 // the winner moves to pc, the row at pc to Ip
-                const int Ip = piv ? 0x7fff - (int)(best & 0x7fffu) : -2, at_pc = piv ? pc : -2;
-                const bool out = pos == at_pc;
+                Ipp = piv ? 0x7fff - (int)(best & 0x7fffu) : -2;
+                atp = piv ? pc : -2;
+                const bool out = pos == atp;
                 dk = out ? pc : dk;
-                pos = pos == Ip ? pc : (out ? Ip : pos);
-                iq_l = iq_l == Ip ? -1 : iq_l;
-                const bool here = lane == at_pc;
-                ip_l = here ? Ip : ip_l;
-                iq_l = here ? Ip : iq_l;
-                pv_l = here ? (int)V : pv_l;
-                pi_l = here ? (int)inv : pi_l;
-                pj_l = here ? jc : pj_l;
+                pos = pos == Ipp ? pc : (out ? Ipp : pos);
+                Vp = (int)V;
+                pivcols |= piv ? 1u << jc : 0u;
                 pc += piv ? 1 : 0;
                 nl = pos >= pc ? -cn : 0.0;
             }
             v[s + 1] = fma(nl, un, v[s + 1]);
-            // the scaled row for B, by its distance from column jc
-            {
-                const uint64_t b = __builtin_bit_cast(uint64_t, -nu);
-                auto column = [&](int j) {
-                    const int src = 4 * (jc + j);
-                    const uint32_t lo = __builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)b);
-                    const uint32_t hi = __builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)(b >> 32));
-                    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-                };
-                u0 = column(back);
-                u1 = column(16 + back);
-            }
+            nup = nu;
             h[3 - s] = nu;
         };
         Unroll<0, 4>::run(step);
@@ -646,16 +663,23 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
         chunk(c, std::integral_constant<int, 16>{}, std::integral_constant<int, 16>{});
     for (int c = 4; c < chunks; ++c)
         chunk(c, std::integral_constant<int, 32>{}, std::integral_constant<int, 4>{});
+    write_down(4 * chunks - 1);
 
+    const int pj_q = __shfl(pj_l, col);  // lanes t and 32 + t: column of pivot t
     // the pivots' scaled rows at their final places, T and the pivots' records,
     // by the first workgroup (every wave has written all of s_U)
     if (rank == 0) {
         int32_t *const dst = Wp + (int64_t)col * ldw + kr0;
-        for (int jc = wave; jc < PNW; jc += PWAVES) {
+        constexpr int RPW = PNW / PWAVES;
+        double y[RPW];
+#pragma unroll
+        for (int q = 0; q < RPW; ++q) y[q] = s_U[wave + PWAVES * q][lane < PNW ? lane : PNW + pj_q];
+#pragma unroll
+        for (int q = 0; q < RPW; ++q) {
+            const int jc = wave + PWAVES * q, t = __popc(pivcols & ((1u << jc) - 1u));
             const bool piv = (pivcols >> jc) & 1u;
-            const int t = __popc(pivcols & ((1u << jc) - 1u));
-            if (piv && lane > jc && lane < w) dst[t] = (int32_t)(uint32_t)from_near(-s_U[jc][col], mp);
-            if (lane < PNW) a.solve->t[jc][lane] = piv && lane < pc ? -(int32_t)s_U[jc][PNW + pj_l] : 0;
+            if (lane >= PNW) a.solve->t[jc][col] = piv && col < pc ? -(int32_t)y[q] : 0;
+            else if (piv && lane > jc && lane < w) dst[t] = (int32_t)(uint32_t)from_near(-y[q], mp);
         }
         if (wave == 0 && lane < PNW)
             a.solve->num[lane] = ((pivcols >> lane) & 1u) ? (int)__popc(pivcols & ((1u << lane) - 1u)) : -1;

@@ -2,7 +2,7 @@
 triangles, composed row moves) where tiles, panels and blocks are ragged, bit-exact
 against the oracle: one to sixteen columns beside a block, blocks of fewer than
 128 pivots, pivots that skip columns, 16-column panels, and moduli on both sides
-of the one-reduction bound."""
+of the one-reduction bound and of the table of inverses."""
 import numpy as np
 import pytest
 
@@ -25,7 +25,7 @@ CASES = [
 
 
 @pytest.mark.parametrize("wide", [False, True], ids=["panel32", "panel16"])
-@pytest.mark.parametrize("p", [2, 65521, 2 ** 24 - 3, 2 ** 26 - 5])
+@pytest.mark.parametrize("p", [2, 65521, 131071, 262147, 2 ** 24 - 3, 2 ** 26 - 5])
 @pytest.mark.parametrize("m,n,rank,zero", CASES)
 def test_block_ends_vs_oracle(gffm, monkeypatch, m, n, rank, zero, p, wide):
     if wide:
