@@ -127,52 +127,135 @@ __global__ __launch_bounds__(256) void k_slice_sum(int64_t m, int64_t n, const i
     *dst = from_res<TC>(r);
 }
 
-// y = A x mod p (A m x k column-major, x and y contiguous): one thread per
-// row, blockIdx.y a K slice.  Balanced residues; the FP64 accumulator is
-// reduced every R1 products, |a x| <= floor(p/2)^2, so it stays exact.
-// A slice writes its residues to P + y*m when S > 1, else straight to y.
-template <typename T>
+// y = A x mod p (A m x k column-major, x and y contiguous), bound by reading A
+// once.  A wave reads 16 bytes a lane, 1 KiB of a column, and keeps sixteen such
+// loads in flight; the four waves of a workgroup take quarters of its K slice
+// (blockIdx.y) and meet in LDS.  Elements are balanced by one rounded quotient
+// (at most h = (p + 1) / 2 + 2 in magnitude) and the FP64 sum is reduced every
+// `cadence` columns, so that it stays exact.  Several slices leave their residues in P
+// and the last one of a row block to arrive sums them (stores and loads at
+// agent scope, since the slices run on all XCDs); it also resets the count.
+// 6001 x 7003 in FP64: 64 us, 5.3 TB/s (one row a lane and the slices' sum in
+// a launch of its own: 89); 1000 x 1000 9 us (44).
+constexpr int GV_U = 8;  // columns of a batch
+template <typename T, int V> struct __attribute__((packed, aligned(sizeof(T)))) RowsOf {
+    T v[V];
+};
+template <typename T, int V>
 __global__ __launch_bounds__(256) void k_gemv(int64_t m, int64_t k, const T *__restrict__ A, int64_t lda,
                                               const T *__restrict__ x, T *__restrict__ y, int32_t *__restrict__ P,
-                                              int64_t kslice, int R1, ModP mp)
+                                              int *__restrict__ arrived, int64_t kslice, int cadence, ModP mp)
 {
-    __shared__ double xs[256];
-    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t kb = (int64_t)blockIdx.y * kslice;
-    const int64_t ke = k - kb < kslice ? k : kb + kslice;
-    const double hp = (double)mp.half;
-    double acc = 0.0;
-    int cnt = 0;
-    for (int64_t k0 = kb; k0 < ke; k0 += 256) {
-        const int64_t kk = k0 + threadIdx.x;
-        double xv = 0.0;
-        if (kk < ke) {
-            xv = (double)to_res<T>(x[kk], mp);
-            xv = xv > hp ? xv - mp.pd : xv;
-        }
-        __syncthreads();
-        xs[threadIdx.x] = xv;
-        __syncthreads();
-        const int kn = ke - k0 < 256 ? (int)(ke - k0) : 256;
-        if (r < m) {
-            const T *a = A + r + k0 * lda;
-#pragma unroll 8
-            for (int q = 0; q < kn; ++q) {
-                double av = (double)to_res<T>(a[q * lda], mp);
-                av = av > hp ? av - mp.pd : av;
-                acc = fma(av, xs[q], acc);
-                if (++cnt == R1) {
-                    cnt = 0;
-                    acc = fma(-rint(acc * mp.pinv), mp.pd, acc);
-                }
+    __shared__ double s_acc[4][64 * V];
+    __shared__ int s_last;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t r = (int64_t)blockIdx.x * (64 * V) + lane * V;
+    const int64_t rb = min(r, m - V);  // (m >= V) the last lanes read again what they share
+    const int64_t c0 = (int64_t)blockIdx.y * kslice + wave * (kslice / 4);
+    const int64_t c1 = min(k, c0 + kslice / 4);
+    double acc[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc[e] = 0.0;
+    auto reduce = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc[e] = fma(-rint(acc[e] * mp.pinv), mp.pd, acc[e]);
+    };
+    if (c0 < c1) {
+        const int nb = (int)((c1 - c0 + GV_U - 1) / GV_U);
+        RowsOf<T, V> a[2][GV_U];
+        auto load = [&](int i, RowsOf<T, V> *d) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < GV_U; ++q)
+                d[q] = *(const RowsOf<T, V> *)(A + rb + min(c0 + (int64_t)i * GV_U + q, c1 - 1) * lda);
+        };
+        // 64 elements of x, one a lane; zero past the end
+        auto load_x = [&](int64_t c) __attribute__((always_inline)) {
+            const T v = x[min(c + lane, c1 - 1)];
+            return c + lane < c1 ? bal_of<T>(v, mp) : 0.0;
+        };
+        load(0, a[0]);
+        double xv = load_x(c0);
+        int since = 0;
+        auto batch = [&](int i, const RowsOf<T, V> *d) __attribute__((always_inline)) {
+            const int at = (i * GV_U) & 63;
+#pragma unroll
+            for (int q = 0; q < GV_U; ++q) {
+                const uint64_t b = __builtin_bit_cast(uint64_t, xv);
+                const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, at + q);
+                const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(b >> 32), at + q);
+                const double xq = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+#pragma unroll
+                for (int e = 0; e < V; ++e) acc[e] = fma(bal_of<T>(d[q].v[e], mp), xq, acc[e]);
+                if (q == 3 && cadence == 4) reduce();
+            }
+            since += GV_U;
+            if (since >= cadence) {
+                reduce();
+                since = 0;
+            }
+        };
+        for (int i = 0; i < nb; i += 2) {
+            load(i + 1, a[1]);
+            if (i != 0 && ((i * GV_U) & 63) == 0) xv = load_x(c0 + (int64_t)i * GV_U);
+            batch(i, a[0]);
+            if (i + 1 < nb) {
+                load(i + 2, a[0]);
+                batch(i + 1, a[1]);
             }
         }
+        reduce();
     }
-    if (r < m) {
-        const uint32_t v = (uint32_t)dmod(acc, mp);
-        if (P) P[(int64_t)blockIdx.y * m + r] = (int32_t)v;
-        else y[r] = from_res<T>(v);
+#pragma unroll
+    for (int e = 0; e < V; ++e)
+        if (rb + e >= r) s_acc[wave][(int)(rb - (r - lane * V)) + e] = acc[e];
+    __syncthreads();
+    const int64_t row = (int64_t)blockIdx.x * (64 * V) + tid;
+    const bool mine = tid < 64 * V && row < m;
+    uint32_t v = 0;
+    if (mine) v = (uint32_t)dmod((s_acc[0][tid] + s_acc[1][tid]) + (s_acc[2][tid] + s_acc[3][tid]), mp);
+    if (!P) {
+        if (mine) y[row] = from_res<T>(v);
+        return;
     }
+    if (mine)
+        __hip_atomic_store(P + (int64_t)blockIdx.y * m + row, (int32_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!arrived) return;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (tid == 0) {
+        const int S = (int)gridDim.y;
+        s_last = atomicAdd(arrived + blockIdx.x, 1) == S - 1;
+        if (s_last) __hip_atomic_store(arrived + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!s_last) return;
+    // the threads of a row take every G-th slice each
+    constexpr int R = 64 * V, G = 256 / R, U = 16;
+    const int S = (int)gridDim.y;
+    const int64_t row2 = (int64_t)blockIdx.x * R + tid % R;
+    double sum = 0.0;  // fewer than 2^26 slices
+    for (int t = tid / R; t < S; t += G * U) {
+        int32_t w[U];
+#pragma unroll
+        for (int q = 0; q < U; ++q)
+            w[q] = __hip_atomic_load(P + (int64_t)min(t + G * q, S - 1) * m + min(row2, m - 1), __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int q = 0; q < U; ++q) sum += t + G * q < S ? (double)w[q] : 0.0;
+    }
+    s_acc[tid / R][tid % R] = sum;
+    __syncthreads();
+    if (!mine) return;
+    sum = 0.0;
+#pragma unroll
+    for (int q = 0; q < G; ++q) sum += s_acc[q][tid];
+    y[row] = from_res<T>((uint32_t)dmod(sum, mp));
+}
+
+__global__ void k_zero_ints(int *p, int n)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0;
 }
 
 int64_t round_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
@@ -608,44 +691,71 @@ int gemm_limb_i8_in(modp_ctx *ctx, const GemmArgs &g, const LimbScratch &ws)
     return gemm_limb_cfg(ctx, g, cfg, &ws);
 }
 
+namespace {
+
+template <typename T, int V>
+int gemv_t(modp_ctx *ctx, int64_t m, int64_t k, const T *A, int64_t lda, const T *x, T *y, const ModP &mp)
+{
+    const double h = (double)((mp.p + 1) / 2 + 2);
+    const double r1 = floor((9007199254740992.0 - (double)mp.p) / (h * h));  // at least 7
+    const int cadence = r1 >= 1e6 ? 1000000 / GV_U * GV_U : r1 >= GV_U ? (int)r1 / GV_U * GV_U : 4;
+    const int64_t rb = (m + 64 * V - 1) / (64 * V);
+    // K slices until the grid holds two workgroups per CU, each wave at least two
+    // batches; more than 128 slices cost more to sum than they save (6001 x
+    // 7003: 64 us with two to eight workgroups per CU, 300 x 20000 16 us with
+    // 64 or 128 slices and 19 with 256, 64 x 70000 26 / 18 / 18 us)
+    int64_t S = 2 * (int64_t)ctx->num_cus / rb;
+    if (S > k / (4 * 2 * GV_U)) S = k / (4 * 2 * GV_U);
+    if (S > 128) S = 128;
+    if (S < 1) S = 1;
+    const int64_t kslice = round_up(((k > 0 ? k : 1) + S - 1) / S, 4 * GV_U);
+    S = k > 0 ? (k + kslice - 1) / kslice : 1;
+    // y over x: nothing of y is written before all of x is read
+    const bool over = (const char *)y < (const char *)(x + k) && (const char *)x < (const char *)(y + m);
+    int32_t *P = nullptr;
+    int *arrived = nullptr;
+    if (S > 1 || over) {
+        int st = MODP_OK;
+        P = (int32_t *)ws_get(ctx, WS_SLICES, sizeof(int32_t) * (size_t)S * (size_t)m, &st);
+        if (!P) return st;
+    }
+    if (S > 1 && !over) {
+        int st = MODP_OK;
+        const size_t had = ctx->ws_size[WS_GEMV];
+        arrived = (int *)ws_get(ctx, WS_GEMV, sizeof(int) * (size_t)rb, &st);
+        if (!arrived) return st;
+        if (ctx->ws_size[WS_GEMV] != had) {
+            const int n = (int)(ctx->ws_size[WS_GEMV] / sizeof(int));
+            k_zero_ints<<<(n + 255) / 256, 256, 0, ctx->stream>>>(arrived, n);
+            HIP_TRY(ctx, hipGetLastError());
+        }
+    }
+    {
+        TimedLaunch tl(ctx, "gemv");
+        k_gemv<T, V><<<dim3((unsigned)rb, (unsigned)S), 256, 0, ctx->stream>>>(m, k, A, lda, x, y, P, arrived, kslice,
+                                                                               cadence, mp);
+        HIP_TRY(ctx, hipGetLastError());
+    }
+    if (!over) return MODP_OK;
+    GemmArgs g;
+    g.m = m; g.n = 1; g.k = k;
+    g.C = y; g.ldc = m; g.kc = sizeof(T) == 8 ? EK_F64 : EK_F32;
+    g.epi = EPI_STORE;
+    g.mp = mp;
+    return launch_slice_sum(ctx, g, EPI_STORE, P, (int)S);
+}
+
+}  // namespace
+
 int gemv_run(modp_ctx *ctx, int kind, int64_t m, int64_t k, const void *A, int64_t lda, const void *x, void *y,
              int64_t p)
 {
     if (m <= 0) return MODP_OK;
     const ModP mp = make_modp(p);
-    const double h = (double)(p / 2);
-    const double r1 = h > 0 ? floor((9007199254740992.0 - (double)p) / (h * h)) : 1e9;
-    const int R1 = r1 > 1e6 ? 1000000 : (int)r1;
-    if (R1 < 1) return set_error(ctx, MODP_ERR_MODULUS_RANGE, "modulus %lld too large for the FP64 form", (long long)p);
-    const int64_t rb = (m + 255) / 256;
-    // K slices until the grid holds about two workgroups per CU
-    int64_t S = (2 * (int64_t)ctx->num_cus + rb - 1) / rb;
-    if (S > (k + 511) / 512) S = (k + 511) / 512;
-    if (S < 1) S = 1;
-    const int64_t kslice = round_up((k + S - 1) / S > 0 ? (k + S - 1) / S : 1, 256);
-    S = k > 0 ? (k + kslice - 1) / kslice : 1;
-    int st = MODP_OK;
-    int32_t *P = nullptr;
-    if (S > 1) {
-        P = (int32_t *)ws_get(ctx, WS_SLICES, sizeof(int32_t) * (size_t)S * (size_t)m, &st);
-        if (!P) return st;
+    if (kind == EK_F64) {
+        if (m < 2) return gemv_t<double, 1>(ctx, m, k, (const double *)A, lda, (const double *)x, (double *)y, mp);
+        return gemv_t<double, 2>(ctx, m, k, (const double *)A, lda, (const double *)x, (double *)y, mp);
     }
-    const dim3 grid((unsigned)rb, (unsigned)S);
-    {
-        TimedLaunch tl(ctx, "gemv");
-        if (kind == EK_F64)
-            k_gemv<double><<<grid, 256, 0, ctx->stream>>>(m, k, (const double *)A, lda, (const double *)x, (double *)y,
-                                                          P, kslice, R1, mp);
-        else
-            k_gemv<float><<<grid, 256, 0, ctx->stream>>>(m, k, (const float *)A, lda, (const float *)x, (float *)y, P,
-                                                         kslice, R1, mp);
-        HIP_TRY(ctx, hipGetLastError());
-    }
-    if (S == 1) return MODP_OK;
-    GemmArgs g;
-    g.m = m; g.n = 1; g.k = k;
-    g.C = y; g.ldc = m; g.kc = kind;
-    g.epi = EPI_STORE;
-    g.mp = mp;
-    return launch_slice_sum(ctx, g, EPI_STORE, P, (int)S);
+    if (m < 4) return gemv_t<float, 1>(ctx, m, k, (const float *)A, lda, (const float *)x, (float *)y, mp);
+    return gemv_t<float, 4>(ctx, m, k, (const float *)A, lda, (const float *)x, (float *)y, mp);
 }
