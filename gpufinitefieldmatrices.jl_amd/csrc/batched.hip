@@ -125,57 +125,68 @@ constexpr int BL_TILE = 64, BL_BK = 32, BL_KMAX = 16384;
 typedef int bl_v2i __attribute__((ext_vector_type(2)));
 typedef int bl_v16i __attribute__((ext_vector_type(16)));
 
-// Residue of a stored element in the digit representation (top as in
-// digit_rep): a compare when it is already in [0, p) (the usual case), the
-// FP64 reduction otherwise.
-template <typename T>
-__device__ __forceinline__ int32_t bl_residue(T v, const ModP &mp, int32_t top)
+// Stored elements as words whose byte u is digit u of the residue (top as in
+// digit_rep).  An element that is a residue already (the usual case) only
+// needs the conversion; otherwise the wave takes the FP64 reductions.  The
+// signed base-256 digits d_u of x, x = sum d_u 256^u, are the bytes of
+// (x + 0x80808080) ^ 0x80808080: the addition carries where a byte is 128 or more.
+template <int N, typename T>
+__device__ __forceinline__ void bl_digits(const T *v, uint32_t *w, const ModP &mp, int32_t top)
 {
-    const double x = (double)v;
-    uint32_t r = (uint32_t)x;
-    if (!(x >= 0.0 && x < mp.pd)) r = (uint32_t)dmod(x, mp);
-    return digit_rep(r, top, mp);
+    uint32_t far = 0;
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+        w[e] = (uint32_t)(int32_t)v[e];
+        far = max(far, w[e]);
+    }
+    if (__builtin_expect(__any(far >= mp.p32), 0)) {
+#pragma unroll
+        for (int e = 0; e < N; ++e) w[e] = (uint32_t)dmod((double)v[e], mp);
+    }
+#pragma unroll
+    for (int e = 0; e < N; ++e) w[e] = ((uint32_t)digit_rep(w[e], top, mp) + 0x80808080u) ^ 0x80808080u;
 }
 
-// Digits: the stored byte of digit u of x is the low byte of x_u, with
-// x_0 = x and x_{u+1} = (x_u + 128) >> 8 (arithmetic), the signed base-256
-// digits of the limb form.  Eight consecutive k of one A row: digit u goes to
-// dst(u) as one 8-byte word.
-template <int L, class Dst> __device__ __forceinline__ void bl_store_a8(int32_t (&x)[8], Dst dst)
+// digit planes of four words: plane u holds byte u of each
+template <int L> __device__ __forceinline__ void bl_planes(const uint32_t *w, uint32_t *plane)
 {
-#pragma unroll
-    for (int u = 0; u < L; ++u) {
-        bl_v2i w;
-#pragma unroll
-        for (int d = 0; d < 2; ++d)
-            w[d] = (int)(((uint32_t)x[4 * d] & 255u) | (((uint32_t)x[4 * d + 1] & 255u) << 8) |
-                         (((uint32_t)x[4 * d + 2] & 255u) << 16) | ((uint32_t)x[4 * d + 3] << 24));
-        *reinterpret_cast<bl_v2i *>(dst(u)) = w;
-        if (u + 1 < L) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = (x[e] + 128) >> 8;
-        }
+    const uint32_t a = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u), b = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
+    plane[0] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+    if constexpr (L > 1) plane[1] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    if constexpr (L > 2) {
+        const uint32_t c = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);
+        const uint32_t d = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
+        plane[2] = __builtin_amdgcn_perm(d, c, 0x05040100u);
+        if constexpr (L > 3) plane[3] = __builtin_amdgcn_perm(d, c, 0x07060302u);
     }
 }
 
-// B stage of 32 k into the digit planes Bs[u] (64 columns of 32 bytes, chunk
-// c of column r at slot c ^ ((r >> 3) & 1)): element 2 i + t of vb is k pair
-// bk2 + t of column 16 wave + 4 i + bq.
-template <typename T, int L>
-__device__ __forceinline__ void bl_store_b(const T (&vb)[8], int8_t (*Bs)[BL_TILE * BL_BK], int wave, int bq,
-                                           int bk2, const ModP &mp, int32_t top)
+// Eight elements of one A row: digit u goes to dst(u) as one 8-byte word.
+template <int L, class Dst> __device__ __forceinline__ void bl_store_a8(const uint32_t (&w)[8], Dst dst)
 {
+    uint32_t lo[L], hi[L];
+    bl_planes<L>(w, lo);
+    bl_planes<L>(w + 4, hi);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int c = 16 * wave + 4 * i + bq;
-        const int off = c * BL_BK + 16 * ((bk2 >> 4) ^ ((c >> 3) & 1)) + (bk2 & 15);
-        int32_t x0 = bl_residue(vb[2 * i], mp, top), x1 = bl_residue(vb[2 * i + 1], mp, top);
+    for (int u = 0; u < L; ++u) *reinterpret_cast<bl_v2i *>(dst(u)) = bl_v2i{(int)lo[u], (int)hi[u]};
+}
+
+// B stage of 32 k into the digit planes Bs[u] (64 columns of 32 bytes, chunk
+// c of column r at slot c ^ ((r >> 3) & 1)): words 4 i .. 4 i + 3 of w go to
+// place 4 (lane % 8) of column 16 wave + 8 i + lane / 8, so that a wave writes
+// eight columns whole, every bank once.
+template <int L>
+__device__ __forceinline__ void bl_store_b(const uint32_t (&w)[8], int8_t (*Bs)[BL_TILE * BL_BK], int wave, int lane)
+{
+    const int kq = lane & 7;
 #pragma unroll
-        for (int u = 0; u < L; ++u) {
-            *reinterpret_cast<uint16_t *>(&Bs[u][off]) = (uint16_t)(((uint32_t)x0 & 255u) | (((uint32_t)x1 & 255u) << 8));
-            x0 = (x0 + 128) >> 8;
-            x1 = (x1 + 128) >> 8;
-        }
+    for (int i = 0; i < 2; ++i) {
+        const int c = 16 * wave + 8 * i + (lane >> 3);
+        const int off = c * BL_BK + 16 * ((kq >> 2) ^ ((c >> 3) & 1)) + 4 * (kq & 3);
+        uint32_t plane[L];
+        bl_planes<L>(w + 4 * i, plane);
+#pragma unroll
+        for (int u = 0; u < L; ++u) *reinterpret_cast<uint32_t *>(&Bs[u][off]) = plane[u];
     }
 }
 
@@ -186,24 +197,44 @@ template <typename T, int NA>
 __device__ __forceinline__ void bl_store_block(const bl_v16i (&acc)[NA], const BJob &j, int64_t i, int64_t j0, int h)
 {
     const ModP mp = j.mp;
-    T *C = (T *)j.C;
+    T *C = (T *)j.C + i + (j0 + 4 * h) * j.ldc;
+    const int64_t ldc = j.ldc;
+    const int left = (int)min((int64_t)32, j.n - j0) - 4 * h;  // columns from this lane's first
+    const bool row_ok = i < j.m;
+    // exact integers in [0, p), four at a time
+    auto store4 = [&](int g, const double (&S)[4]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const int64_t jj = j0 + 8 * (e >> 2) + 4 * h + (e & 3);
-        double S = 0.0;
-        if (j.lazy) {
-            // |S| < 2^51: the rounded quotient is within one of the exact
-            // one, so one fix-up gives S mod p
+        for (int e = 0; e < 4; ++e)
+            if (row_ok && 8 * g + e < left) C[(8 * g + e) * ldc] = (T)S[e];
+    };
+    if (j.lazy) {
+        // |S| < 2^51: the rounded quotient is within one of the exact
+        // one, so one fix-up gives S mod p
 #pragma unroll
-            for (int t = 0; t < NA; ++t) S = fma((double)acc[t][e], j.w[t], S);
-            S = fma(-rint(S * mp.pinv), mp.pd, S);
-            S = S < 0.0 ? S + mp.pd : S;
-        } else {
+        for (int g = 0; g < 4; ++g) {
+            double S[4];
 #pragma unroll
-            for (int t = 0; t < NA; ++t) S = dmod(fma(dmod((double)acc[t][e], mp), j.w[t], S), mp);
+            for (int e = 0; e < 4; ++e) {
+                S[e] = (double)acc[0][4 * g + e];
+#pragma unroll
+                for (int t = 1; t < NA; ++t) S[e] = fma((double)acc[t][4 * g + e], j.w[t], S[e]);
+                S[e] = fma(-rint(S[e] * mp.pinv), mp.pd, S[e]);
+                S[e] = S[e] < 0.0 ? S[e] + mp.pd : S[e];
+            }
+            store4(g, S);
         }
-        // S is an exact integer in [0, p)
-        if (i < j.m && jj < j.n) C[i + jj * j.ldc] = (T)S;
+    } else {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            double S[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                S[e] = 0.0;
+#pragma unroll
+                for (int t = 0; t < NA; ++t) S[e] = dmod(fma(dmod((double)acc[t][4 * g + e], mp), j.w[t], S[e]), mp);
+            }
+            store4(g, S);
+        }
     }
 }
 
@@ -221,11 +252,9 @@ __global__ __launch_bounds__(256, 2) void k_batched_limb(const BJob *__restrict_
     __shared__ int s_item;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wr = wave & 1, wc = wave >> 1;
-    // A staging: row sr, k quarter sc (8 k); B staging: column 16 wave +
-    // 4 i + lane / 16 (i < 4), k pair 2 (lane % 16)
+    // A staging: row sr, k quarter sc (8 k); B staging as bl_store_b has it
     const int sr = tid & 63, sc = tid >> 6;
     const int aslot = sr * BK + 16 * ((sc >> 1) ^ ((sr >> 3) & 1)) + 8 * (sc & 1);
-    const int bk2 = 2 * (lane & 15), bq = lane >> 4;
     const int fr = lane & 31, h = lane >> 5, fsw = (fr >> 3) & 1;
     const int home = blockIdx.x % NXCD;
     for (int qq = 0; qq < NXCD; ++qq) {
@@ -256,21 +285,22 @@ __global__ __launch_bounds__(256, 2) void k_batched_limb(const BJob *__restrict_
                     va[e] = (arow_ok && kk < K) ? A[arow + kk * j.lda] : (T)0;
                 }
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int64_t col = c0 + 16 * wave + 4 * i + bq;
+                for (int i = 0; i < 2; ++i) {
+                    const int64_t col = c0 + 16 * wave + 8 * i + (lane >> 3);
 #pragma unroll
-                    for (int t = 0; t < 2; ++t) {
-                        const int64_t kk = kb + bk2 + t;
-                        vb[2 * i + t] = (col < j.n && kk < K) ? B[kk + col * j.ldb] : (T)0;
+                    for (int t = 0; t < 4; ++t) {
+                        const int64_t kk = kb + 4 * (lane & 7) + t;
+                        vb[4 * i + t] = (col < j.n && kk < K) ? B[kk + col * j.ldb] : (T)0;
                     }
                 }
             };
             auto lstore = [&](int buf) {
-                int32_t xa[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) xa[e] = bl_residue(va[e], mp, TOP);
+                uint32_t xa[8];
+                bl_digits<8>(va, xa, mp, TOP);
                 bl_store_a8<L>(xa, [&](int u) { return &As[buf][u][aslot]; });
-                bl_store_b<T, L>(vb, Bs[buf], wave, bq, bk2, mp, TOP);
+                uint32_t xb[8];
+                bl_digits<8>(vb, xb, mp, TOP);
+                bl_store_b<L>(xb, Bs[buf], wave, lane);
             };
             v16i acc[NA];
 #pragma unroll
@@ -310,7 +340,20 @@ __global__ __launch_bounds__(256, 2) void k_batched_limb(const BJob *__restrict_
 // (rows of 256 + 16 bytes: 16 consecutive rows read at one offset fall in
 // distinct bank groups).  The A digits of a product are computed once per row
 // panel instead of once per tile.
+//
+// Two workgroups on a CU cannot hide a load behind each other, so the stages
+// of all column tiles form one sequence with two stages of loads in flight
+// (also during an epilogue).  The next item is asked for three stages before
+// the end: earlier, and the panels of a product would drift apart and read its B
+// from memory each.  Loads are clamped into the operands instead of
+// predicated: past K the A digits are zero, and nothing reads other rows or
+// columns.  10,000 products of 16 to 256 rows, columns and k, three digits:
+// 1.23 ms, about 4.8 TB/s with the repeated B reads (one stage in flight,
+// predicated loads, digits by shifts and masks: 1.74 ms).
 constexpr int RP_KMAX = 256;
+template <typename T> struct __attribute__((packed, aligned(sizeof(T)))) BlPair {
+    T v[2];
+};
 template <typename T, int L>
 __global__ __launch_bounds__(256, L == 4 ? 1 : 2) void k_batched_limb_rp(const BJob *__restrict__ jobs,
                                                             const BItem *__restrict__ items, XcdRanges xr,
@@ -326,87 +369,140 @@ __global__ __launch_bounds__(256, L == 4 ? 1 : 2) void k_batched_limb_rp(const B
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wr = wave & 1, wc = wave >> 1;
     const int sr = tid & 63, sc = tid >> 6;
-    const int bk2 = 2 * (lane & 15), bq = lane >> 4;
+    const int kq = lane & 7, bc = 16 * wave + (lane >> 3);
     const int fr = lane & 31, h = lane >> 5, fsw = (fr >> 3) & 1;
     const int home = blockIdx.x % NXCD;
     for (int qq = 0; qq < NXCD; ++qq) {
         const int q = (home + qq) % NXCD;
         const int64_t base = xr.off[q], cnt = xr.off[q + 1] - base;
         if (cnt <= 0) continue;
+        int next = 0;  // thread 0: the item after this one
+        if (tid == 0) next = atomicAdd(counter + 16 * q, 1);
         for (;;) {
-            if (threadIdx.x == 0) s_item = atomicAdd(counter + 16 * q, 1);
+            if (tid == 0) s_item = next;
             __syncthreads();
-            const int it = s_item;
-            __syncthreads();
-            if (it >= cnt) break;
+            const int it = __builtin_amdgcn_readfirstlane(s_item);
+            if (it >= cnt) {
+                __syncthreads();  // s_item is written again for the next queue
+                break;
+            }
             const BItem item = items[base + it];
             const BJob &j = jobs[item.job];
             const int64_t r0 = (int64_t)item.tile * TL;
-            const T *A = (const T *)j.A, *B = (const T *)j.B;
             const ModP mp = j.mp;
-            const int K = j.k, ns = (K + BK - 1) / BK;
-            const int64_t arow = r0 + sr;
-            const bool arow_ok = arow < j.m;
-            for (int tj = 0; tj < j.tiles_n; ++tj) {
-                const int64_t c0 = (int64_t)tj * TL;
-                // the first column tile also stages the A panel: thread (row
-                // sr, quarter sc) splits k = 32 st + 8 sc .. + 7 of each stage
-                const bool first = tj == 0;
-                T va[8], vb[8];
-                auto gload = [&](int st) {
-                    const int64_t kb = (int64_t)st * BK;
-                    if (first) {
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            const int64_t kk = kb + 8 * sc + e;
-                            va[e] = (arow_ok && kk < K) ? A[arow + kk * j.lda] : (T)0;
-                        }
-                    }
-#pragma unroll
-                    for (int ii = 0; ii < 4; ++ii) {
-                        const int64_t col = c0 + 16 * wave + 4 * ii + bq;
-#pragma unroll
-                        for (int t = 0; t < 2; ++t) {
-                            const int64_t kk = kb + bk2 + t;
-                            vb[2 * ii + t] = (col < j.n && kk < K) ? B[kk + col * j.ldb] : (T)0;
-                        }
-                    }
-                };
-                auto lstore = [&](int buf, int st) {
-                    if (first) {
-                        int32_t xa[8];
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) xa[e] = bl_residue(va[e], mp, TOP);
-                        bl_store_a8<L>(xa, [&](int u) { return &As[u][sr * AP + st * BK + 8 * sc]; });
-                    }
-                    bl_store_b<T, L>(vb, Bs[buf], wave, bq, bk2, mp, TOP);
-                };
-                v16i acc[NA];
-#pragma unroll
-                for (int t = 0; t < NA; ++t) acc[t] = v16i{0};
-                if (ns > 0) {
-                    gload(0);
-                    lstore(0, 0);
-                }
+            const int K = j.k, n = j.n, ns = (K + BK - 1) / BK, total = ns * j.tiles_n;
+            const int64_t lda = j.lda, ldb = j.ldb;
+            const T *const A = (const T *)j.A + min(r0 + sr, (int64_t)j.m - 1), *const B = (const T *)j.B;
+            if (total == 0) {
+                const v16i none[NA] = {};
+                for (int t = 0; t < j.tiles_n; ++t)
+                    bl_store_block<T, NA>(none, j, r0 + wr * 32 + fr, (int64_t)t * TL + wc * 32, h);
                 __syncthreads();
-                for (int st = 0; st < ns; ++st) {
-                    const int buf = st & 1;
-                    if (st + 1 < ns) gload(st + 1);
-                    v4i fa[L], fb[L];
+                if (tid == 0) next = atomicAdd(counter + 16 * q, 1);
+                continue;
+            }
+            T va[2][8], vb[2][8];
+            // Stage x of the sequence: tile x / ns, k = 32 (x % ns) ...  Word w of
+            // a digit row holds k = 2 w, 2 w + 1, 16 + 2 w and 17 + 2 w of the
+            // stage (in A and B alike), so that a lane reads B in pairs and
+            // eight lanes 128 bytes of a column: thread (row sr, quarter sc)
+            // has A's words 2 sc and 2 sc + 1, its lane B's word kq of columns
+            // bc and bc + 8.  K >= 2: the last pair is moved back into the
+            // column, and forth when it is stored.  No branch goes round a
+            // load, or its registers would be waited for where the paths
+            // meet; past the end the last stage is read again.
+            int ltj = 0, lk = 0;  // the next stage to load
+            auto a_k = [&](int e) { return 4 * sc + (e >> 2) * 2 + (e & 1) + 8 * (e & 2); };
+            auto gload = [&](T *a, T *b, auto WITH_A) __attribute__((always_inline)) {
+                if constexpr (decltype(WITH_A)::value) {
 #pragma unroll
-                    for (int u = 0; u < L; ++u) {
-                        fa[u] = *reinterpret_cast<const v4i *>(&As[u][(wr * 32 + fr) * AP + st * BK + 16 * h]);
-                        fb[u] = *reinterpret_cast<const v4i *>(&Bs[buf][u][(wc * 32 + fr) * BK + 16 * (h ^ fsw)]);
-                    }
-#pragma unroll
-                    for (int u = 0; u < L; ++u)
-#pragma unroll
-                        for (int v = 0; v < L; ++v)
-                            acc[u + v] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[v], fa[u], acc[u + v], 0, 0, 0);
-                    if (st + 1 < ns) lstore(buf ^ 1, st + 1);
-                    __syncthreads();
+                    for (int e = 0; e < 8; ++e) a[e] = A[min(lk + a_k(e), K - 1) * lda];
                 }
-                bl_store_block<T, NA>(acc, j, r0 + wr * 32 + fr, c0 + wc * 32, h);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const T *src = B + min(ltj * TL + bc + 8 * i, n - 1) * ldb;
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        const BlPair<T> x = *reinterpret_cast<const BlPair<T> *>(src + min(lk + 16 * t + 2 * kq, K - 2));
+                        b[4 * i + 2 * t] = x.v[0];
+                        b[4 * i + 2 * t + 1] = x.v[1];
+                    }
+                }
+                lk += BK;
+                const bool wrap = lk >= K;
+                lk = wrap ? 0 : lk;
+                ltj += wrap ? 1 : 0;
+            };
+            // B's pairs of the stage at k0 into the planes Bs[buf]
+            auto bstore = [&](int buf, int k0, const T (&b)[8]) __attribute__((always_inline)) {
+                uint32_t w[8];
+                bl_digits<8>(b, w, mp, TOP);
+                if (k0 + BK > K) {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+                        if (k0 + 16 * t + 2 * kq == K - 1) {
+                            w[2 * t] = w[2 * t + 1];
+                            w[4 + 2 * t] = w[5 + 2 * t];
+                        }
+                }
+                bl_store_b<L>(w, Bs[buf], wave, lane);
+            };
+            auto astore = [&](int k0, const T *a) __attribute__((always_inline)) {
+                uint32_t w[8];
+                bl_digits<8>(a, w, mp, TOP);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) w[e] = k0 + a_k(e) < K ? w[e] : 0u;
+                bl_store_a8<L>(w, [&](int u) { return &As[u][sr * AP + k0 + 8 * sc]; });
+            };
+            v16i acc[NA];
+#pragma unroll
+            for (int t = 0; t < NA; ++t) acc[t] = v16i{0};
+            int x = 0, st = 0, tj = 0;  // the stage at hand, and where it is
+            const int ask = max(total - 3, 0);
+            auto stage = [&](auto PAR, auto WITH_A) __attribute__((always_inline)) {
+                constexpr int par = decltype(PAR)::value;
+                if (x == ask && tid == 0) next = atomicAdd(counter + 16 * q, 1);
+                gload(va[par], vb[par], WITH_A);  // stage x + 2
+                v4i fa[L], fb[L];
+#pragma unroll
+                for (int u = 0; u < L; ++u) {
+                    fa[u] = *reinterpret_cast<const v4i *>(&As[u][(wr * 32 + fr) * AP + st * BK + 16 * h]);
+                    fb[u] = *reinterpret_cast<const v4i *>(&Bs[par][u][(wc * 32 + fr) * BK + 16 * (h ^ fsw)]);
+                }
+#pragma unroll
+                for (int u = 0; u < L; ++u)
+#pragma unroll
+                    for (int v = 0; v < L; ++v)
+                        acc[u + v] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[v], fa[u], acc[u + v], 0, 0, 0);
+                const int k1 = st + 1 == ns ? 0 : (st + 1) * BK;
+                if constexpr (decltype(WITH_A)::value) {
+                    if (x + 1 < ns) astore(k1, va[par ^ 1]);
+                }
+                if (x + 1 < total) bstore(par ^ 1, k1, vb[par ^ 1]);
+                __syncthreads();
+                ++x;
+                if (++st == ns) {
+                    bl_store_block<T, NA>(acc, j, r0 + wr * 32 + fr, (int64_t)tj * TL + wc * 32, h);
+#pragma unroll
+                    for (int t = 0; t < NA; ++t) acc[t] = v16i{0};
+                    st = 0;
+                    ++tj;
+                }
+            };
+            gload(va[0], vb[0], std::true_type{});
+            gload(va[1], vb[1], std::true_type{});
+            astore(0, va[0]);
+            bstore(0, 0, vb[0]);
+            __syncthreads();
+            while (x < ns) {
+                stage(std::integral_constant<int, 0>{}, std::true_type{});
+                if (x == total) break;
+                stage(std::integral_constant<int, 1>{}, std::true_type{});
+            }
+            while (x < total) {
+                stage(std::integral_constant<int, 0>{}, std::false_type{});
+                if (x == total) break;
+                stage(std::integral_constant<int, 1>{}, std::false_type{});
             }
         }
     }
@@ -599,7 +695,8 @@ int plan_build(modp_ctx *ctx, int kind, const modp_gemm_job *jobs, int64_t count
     auto cost = [&](int64_t i) { return (int64_t)hj[i].tile * hj[i].tile * hj[i].k; };
     std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return cost(a) > cost(b); });
     auto cls_of = [&](const BJob &d) {
-        if (d.L > 0) return (d.k <= RP_KMAX && !tile_items ? 7 : 3) + d.L;
+        // the row panels read B by pairs
+        if (d.L > 0) return (d.k <= RP_KMAX && d.k != 1 && !tile_items ? 7 : 3) + d.L;
         const bool exact = (int64_t)d.R >= ((int64_t)d.k + 3) / 4;
         return (d.tile == 64 ? 0 : 2) + (exact ? 0 : 1);
     };
