@@ -59,7 +59,7 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
                                                  int32_t *__restrict__ map_src, PanelCtl *__restrict__ ctl,
                                                  int *__restrict__ abort, int KC, int FAR, int32_t *__restrict__ stage,
                                                  int *__restrict__ cursor, int32_t *__restrict__ gpos,
-                                                 int32_t *__restrict__ grow, PanelSolve *__restrict__ solve)
+                                                 int32_t *__restrict__ grow, PanelSolve *__restrict__ solve, int strict)
 {
     constexpr int NW = GPT / 64;
     if (abort && *abort) {
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
         ctl->nmap = nmap_all;
         ctl->kr0 = kr0;
         if (cursor) *cursor = kr0 + pc;
-        if (abort && status != 0) *abort = 1;
+        if (abort && (status != 0 || (strict && pc < w))) *abort = 1;
     }
 }
 
@@ -464,6 +464,7 @@ __global__ __launch_bounds__(256) void k_update(int32_t *__restrict__ W, int64_t
 }
 
 constexpr int MAXPAN = 64;  // inner panels per outer block (NBO / smallest panel width, 2)
+constexpr int NBATCH = 8;   // outer blocks enqueued without waiting for the host
 
 // T of the diagonal 32 x 32 triangles of a block's L11 by pivot number, for
 // blocks whose panels are not 32 pivots in 32 columns each: one thread a column.
@@ -727,7 +728,16 @@ unsigned grid_for(int64_t total, int64_t cap = 16384)
 
 int64_t rup(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 
-__global__ void k_set_int(int *p, int v) { *p = v; }
+// before a batch of blocks: no abort, the first row, nobody arrived
+__global__ void k_blocks_begin(int *abort, int *cursor, int row, uint32_t *arrive, int n)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) {
+        *abort = 0;
+        *cursor = row;
+    }
+    if (i < n) arrive[i] = 0;
+}
 
 // t[a] = a^{-1} mod p for a < n, 0 where there is none
 __global__ void k_inv_table(uint32_t *__restrict__ t, int n, ModP mp)
@@ -796,18 +806,19 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     if (!W) return st;
     // pivot arrays, per-panel control blocks and row gather maps of one outer block
     const size_t npv = (size_t)mn + 64;
-    const size_t piv_bytes = sizeof(int32_t) * (4 * npv + 2 * MAXPAN * 64) + sizeof(PanelCtl) * MAXPAN + 512 +
+    const size_t piv_bytes = sizeof(int32_t) * (4 * npv + 2 * MAXPAN * 64) + sizeof(PanelCtl) * NBATCH * MAXPAN + 64 +
+                             sizeof(uint32_t) * NBATCH * MAXPAN +
                              sizeof(int32_t) * 64 * NBO + sizeof(PanelSolve) * MAXPAN + sizeof(BlockMoves);
     int32_t *piv = (int32_t *)ws_get(ctx, WS_PIV, piv_bytes, &st);
     if (!piv) return st;
     int32_t *ipiv = piv, *pivval = piv + npv, *pivinv = piv + 2 * npv, *pivcol = piv + 3 * npv;
     int32_t *bmap_dst = piv + 4 * npv, *bmap_src = bmap_dst + MAXPAN * 64;
-    PanelCtl *bctl = (PanelCtl *)(bmap_src + MAXPAN * 64);
-    int *flag = (int *)(bctl + MAXPAN);
+    PanelCtl *bctl = (PanelCtl *)(bmap_src + MAXPAN * 64);  // by block of the batch
+    int *flag = (int *)(bctl + NBATCH * MAXPAN);
     int *abort_flag = flag + 1;
     int *cursor = flag + 2;                         // first row of the next panel (lu, rref)
-    uint32_t *arrive = (uint32_t *)(flag + 4);      // one word per panel of the block
-    int32_t *stage = (int32_t *)(arrive + MAXPAN);  // moved rows' old values, 64 x NBO
+    uint32_t *arrive = (uint32_t *)(flag + 4);      // one word per panel of the batch
+    int32_t *stage = (int32_t *)(arrive + NBATCH * MAXPAN);  // moved rows' old values, 64 x NBO
     PanelSolve *solve = (PanelSolve *)(stage + 64 * NBO);  // one per panel of the block
     BlockMoves *moves = (BlockMoves *)(solve + MAXPAN);
     int32_t *Ubig = (int32_t *)ws_get(ctx, WS_UBUF, sizeof(int32_t) * (size_t)NBO * (size_t)(n + 1), &st);
@@ -820,7 +831,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         if (!gpos) return st;
         grow = gpos + m;
     }
-    PanelCtl *hctl = (PanelCtl *)pinned_get(ctx, sizeof(PanelCtl) * (MAXPAN + 1) + 64, &st);
+    PanelCtl *hctl = (PanelCtl *)pinned_get(ctx, sizeof(PanelCtl) * NBATCH * MAXPAN + 64, &st);
     if (!hctl) return st;
 
     MODP_TRY(util_convert(ctx, kind, m, n, A, lda, EK_I32, W, ldw, mp));
@@ -860,18 +871,18 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         if (use_form == MODP_FORM_LIMB_I8) return gemm_limb_i8(ctx, g);
         return gemm_plain_f64(ctx, g);
     };
-    // panel t of the current outer block at (rj, cj), width w; it has at most
+    // panel t of block blk of the batch at (rj, cj), width w; it has at most
     // m - rj rows
-    auto launch_panel_t = [&](int width, int t, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w, int *abort,
-                              int *cursor) -> int {
+    auto launch_panel_t = [&](int width, int blk, int t, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w,
+                              int *abort, int *cursor, bool strict) -> int {
         if (t >= MAXPAN) return set_error(ctx, MODP_ERR_DEVICE, "more than %d panels in an outer block", MAXPAN);
         int32_t *mdst = bmap_dst + t * 64, *msrc = bmap_src + t * 64;
-        PanelCtl *pctl = bctl + t;
+        PanelCtl *pctl = bctl + blk * MAXPAN + t;
         TimedLaunch tl(ctx, "elim_panel");
         if (width == GNBW) {
             k_panel_g<GNBW><<<1, GPT, 0, ctx->stream>>>(W, ldw, (int)m, (int)rj, (int)cj, (int)w, mp, ple, ipiv,
                                                         pivval, pivinv, pivcol, mdst, msrc, pctl, abort,
-                                                        (int)KC, (int)FAR, stage, cursor, gpos, grow, solve + t);
+                                                        (int)KC, (int)FAR, stage, cursor, gpos, grow, solve + t, strict);
             return hip_check(ctx, hipGetLastError(), "k_panel_g launch");
         }
         PanelArgs a = {};
@@ -879,6 +890,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         a.KC = (int)KC; a.FAR = (int)FAR; a.mp = mp; a.invs = invs;
         a.ipiv = ipiv; a.pivval = pivval; a.pivinv = pivinv; a.pivcol = pivcol;
         a.map_dst = mdst; a.map_src = msrc; a.stage = stage; a.ctl = pctl; a.solve = solve + t; a.abort = abort; a.cursor = cursor;
+        a.strict = strict;
         const int mode = mp.small ? 0 : mp.p <= ((int64_t)1 << 24) ? 1 : 2;
         if (m - rj <= PSINGLE) {
             if (mode == 0) k_panel<false, 0><<<1, PSINGLE, 0, ctx->stream>>>(a);
@@ -887,7 +899,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             return hip_check(ctx, hipGetLastError(), "k_panel launch");
         }
         a.x = xch;
-        a.arrive = arrive + t;
+        a.arrive = arrive + blk * MAXPAN + t;
         a.G = (int)((m - rj + 255) / 256);
         a.patience = patience;
         MODP_TRY(next_tag(&a.tag));
@@ -897,30 +909,36 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         else k_panel<true, 2><<<grid, 256, 0, ctx->stream>>>(a);
         return hip_check(ctx, hipGetLastError(), "k_panel launch");
     };
-    // abort flag, cursor and arrival words of a block
-    auto block_begin = [&]() -> int {
-        return hip_check(ctx, hipMemsetAsync(abort_flag, 0, (size_t)((char *)(arrive + MAXPAN) - (char *)abort_flag),
-                                             ctx->stream), "block flags");
+    auto blocks_begin = [&](int64_t row, int blocks) -> int {
+        k_blocks_begin<<<(unsigned)((blocks * MAXPAN + 255) / 256), 256, 0, ctx->stream>>>(
+            abort_flag, cursor, (int)row, arrive, blocks * MAXPAN);
+        return hip_check(ctx, hipGetLastError(), "k_blocks_begin launch");
+    };
+    // the control blocks of the batch and the flags after them
+    auto read_back = [&]() -> int {
+        HIP_TRY(ctx, hipMemcpyAsync(hctl, bctl, sizeof(PanelCtl) * NBATCH * MAXPAN + 2 * sizeof(int),
+                                    hipMemcpyDeviceToHost, ctx->stream));
+        return hip_check(ctx, hipStreamSynchronize(ctx->stream), "elimination blocks");
     };
     // the rest of the outer block [KC, FAR) from row KR after panel t: its row
     // moves, and right of the panel the rows of U and the rank-npiv update below
-    // the pivots.  rj is the panel's first row, or a lower bound with the row on
-    // the device (ple)
-    auto update_t = [&](int t, int64_t KR, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w,
+    // the pivots.  rj is the panel's first row, or (known false) a lower bound with
+    // the row on the device
+    auto update_t = [&](int blk, int t, bool known, int64_t KR, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w,
                         const int *skip) -> int {
         const int64_t nl = cj - KC, nr = FAR - (cj + w);
         if (nl + nr + (n - (FAR - KC)) == 0) return MODP_OK;
         const int64_t tiles = ((m - rj + UT_R - 1) / UT_R) * ((nr + UT_C - 1) / UT_C);
         const unsigned grid = (unsigned)(1 + (nl + UT_L - 1) / UT_L + tiles);
-        const int kr0 = ple ? -1 : (int)rj;
+        const int kr0 = known ? (int)rj : -1;
         TimedLaunch tl(ctx, "elim_update");
         if (mp.p <= ((int64_t)1 << 24))
             k_update<false><<<grid, 256, 0, ctx->stream>>>(W, ldw, (int)m, (int)KR, (int)KC, (int)FAR, (int)cj, (int)w,
-                                                           kr0, t == 0, bctl + t, solve + t, bmap_dst + t * 64,
+                                                           kr0, t == 0, bctl + blk * MAXPAN + t, solve + t, bmap_dst + t * 64,
                                                            bmap_src + t * 64, stage, moves, mp, skip);
         else
             k_update<true><<<grid, 256, 0, ctx->stream>>>(W, ldw, (int)m, (int)KR, (int)KC, (int)FAR, (int)cj, (int)w,
-                                                          kr0, t == 0, bctl + t, solve + t, bmap_dst + t * 64,
+                                                          kr0, t == 0, bctl + blk * MAXPAN + t, solve + t, bmap_dst + t * 64,
                                                           bmap_src + t * 64, stage, moves, mp, skip);
         return hip_check(ctx, hipGetLastError(), "k_update launch");
     };
@@ -951,73 +969,119 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
 
     std::vector<int64_t> col_stack;
     int64_t kr = 0, kc = 0, last = n - 1;
-    bool done = false;
+    bool done = false, careful = false;
+    // ple: the block met zero columns; if nothing nonzero is left below row
+    // kr, no later column has a pivot and the factorisation is complete (rank = kr)
+    auto rest_is_zero = [&]() -> int {
+        if (kr >= m || kc >= n) return MODP_OK;
+        HIP_TRY(ctx, hipMemsetAsync(flag, 0, sizeof(int), ctx->stream));
+        k_any_nonzero<<<grid_for((m - kr) * (n - kc), 4096), 256, 0, ctx->stream>>>(W, ldw, kr, m, kc, n, flag);
+        HIP_TRY(ctx, hipGetLastError());
+        int *hflag = (int *)hctl;
+        HIP_TRY(ctx, hipMemcpyAsync(hflag, flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+        if (!*hflag) done = true;
+        return MODP_OK;
+    };
+    auto panel_error = [&](const PanelCtl &c) -> int {
+        if (c.status == 3)
+            return set_error(ctx, MODP_ERR_NOT_INVERTIBLE, "pivot has no inverse modulo %lld (modulus not prime)",
+                             (long long)p);
+        if (c.status == 6) return set_error(ctx, MODP_ERR_DEVICE, "an elimination panel's exchange did not end");
+        return MODP_OK;
+    };
+    // A batch of blocks is enqueued as if every panel of it found a pivot in
+    // each of its columns, so that each block's place is known beforehand.  A panel
+    // that does not raises the abort flag, which turns the rest of the batch
+    // into no-ops, and its block is completed from the host after one
+    // synchronization.  One a block cost 50 us of an idle GPU each (PLUQ of
+    // 4096^2 10.3 ms, in batches of eight 9.8).  After an abort the batches
+    // start again from one block, since the next one may be near.
+    struct Block {
+        int64_t KR, KC, FAR, P;
+        int width;
+        std::vector<int64_t> rj, cj, w;
+    };
+    int batch = NBATCH;
     while (!done && kr < m && kc < n) {
-        // ---- one outer block of columns [KC, FAR) ----
-        const int64_t KR = kr, KC = kc;
-        const int64_t colend = ple ? n : last + 1;  // columns usable as pivot columns
-        int64_t nbo = colend - KC;
-        if (nbo > NBO) nbo = NBO;
-        if (nbo < 0) nbo = 0;  // pluq: only moved zero columns remain
-        const int64_t FAR = KC + nbo;
-        const int NBW = panel_width(KR);
-        gave_up = false;
+        std::vector<Block> blocks;
+        {
+            int64_t r = kr, c = kc;
+            while ((int)blocks.size() < batch && !careful && r < m) {
+                const int64_t colend = ple ? n : last + 1;  // columns usable as pivot columns
+                const int64_t nbo = std::min<int64_t>(colend - c, NBO);
+                if (nbo <= 0 || (ple && r + nbo > m)) break;
+                Block b;
+                b.KR = r; b.KC = c; b.FAR = c + nbo; b.P = 0;
+                b.width = panel_width(r);
+                for (int64_t cj = c; cj < b.FAR && r + b.P < m;) {
+                    const int64_t w = std::min(std::min<int64_t>(b.width, b.FAR - cj), m - (r + b.P));
+                    b.rj.push_back(r + b.P); b.cj.push_back(cj); b.w.push_back(w);
+                    b.P += w;
+                    cj += w;
+                }
+                r += b.P;
+                c += b.P;
+                blocks.push_back(b);
+                if (gave_up) break;
+            }
+        }
         bool stop_zero = false;
-        if (!ple && nbo > 0) {
-            // pluq: every panel of the block is enqueued assuming it finds a
-            // pivot in each column; a panel that meets a zero column raises
-            // the abort flag, which turns the rest of the block into no-ops,
-            // and the block is completed from the host after one sync
-            MODP_TRY(block_begin());
-            std::vector<int64_t> pr, pcj, pw;
-            for (int64_t cj = KC; cj < FAR;) {
-                const int64_t rj = KR + (cj - KC);
-                if (rj >= m) break;
-                int64_t w = FAR - cj;
-                if (w > NBW) w = NBW;
-                if (w > m - rj) w = m - rj;
-                pr.push_back(rj); pcj.push_back(cj); pw.push_back(w);
-                cj += w;
+        int64_t nbo = 0;
+        if (!blocks.empty()) {
+            MODP_TRY(blocks_begin(kr, (int)blocks.size()));
+            for (int i = 0; i < (int)blocks.size(); ++i) {
+                const Block &b = blocks[i];
+                for (int t = 0; t < (int)b.w.size(); ++t) {
+                    MODP_TRY(launch_panel_t(b.width, i, t, b.KC, b.FAR, b.rj[t], b.cj[t], b.w[t], abort_flag, nullptr,
+                                            true));
+                    MODP_TRY(update_t(i, t, true, b.KR, b.KC, b.FAR, b.rj[t], b.cj[t], b.w[t], abort_flag));
+                }
+                MODP_TRY(block_end(b.KR, b.KC, b.FAR, b.P, b.P, b.width, abort_flag));
             }
-            const int np = (int)pr.size();
-            int64_t Pfull = 0;
-            for (int t = 0; t < np; ++t) {
-                MODP_TRY(launch_panel_t(NBW, t, KC, FAR, pr[t], pcj[t], pw[t], abort_flag, nullptr));
-                MODP_TRY(update_t(t, KR, KC, FAR, pr[t], pcj[t], pw[t], abort_flag));
-                Pfull += pw[t];
-            }
-            MODP_TRY(block_end(KR, KC, FAR, Pfull, Pfull, NBW, abort_flag));
-            // the control blocks and, right after them, the flags: one copy
-            HIP_TRY(ctx, hipMemcpyAsync(hctl, bctl, sizeof(PanelCtl) * MAXPAN + 2 * sizeof(int), hipMemcpyDeviceToHost,
-                                        ctx->stream));
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            const int aborted = reinterpret_cast<const int *>(hctl + MAXPAN)[1];
-            if (!aborted) {
-                kr += Pfull;
-                kc += Pfull;
+            MODP_TRY(read_back());
+            gave_up = false;
+            nbo = blocks[0].FAR - blocks[0].KC;
+            if (!reinterpret_cast<const int *>(hctl + NBATCH * MAXPAN)[1]) {
+                kr = blocks.back().KR + blocks.back().P;
+                kc = blocks.back().KC + blocks.back().P;
+                batch = std::min(2 * batch, NBATCH);
             } else {
-                int ts = 0;
-                while (ts < np && hctl[ts].status == 0) ++ts;
-                if (ts >= np)
+                int i = 0, t = 0;
+                auto full = [&]() {
+                    const PanelCtl &c = hctl[i * MAXPAN + t];
+                    return c.status == 0 && c.npiv == blocks[i].w[t];
+                };
+                while (i < (int)blocks.size() && full())
+                    if (++t == (int)blocks[i].w.size()) {
+                        t = 0;
+                        ++i;
+                    }
+                if (i == (int)blocks.size())
                     return set_error(ctx, MODP_ERR_DEVICE, "elimination pipeline aborted without a stopping panel");
-                if (hctl[ts].status == 3)
-                    return set_error(ctx, MODP_ERR_NOT_INVERTIBLE,
-                                     "pivot has no inverse modulo %lld (modulus not prime)", (long long)p);
-                if (hctl[ts].status == 6)
-                    return set_error(ctx, MODP_ERR_DEVICE, "an elimination panel's exchange did not end");
-                gave_up = hctl[ts].status == 5;
-                const int64_t npiv = hctl[ts].npiv;
+                const Block &b = blocks[i];
+                const PanelCtl pc = hctl[i * MAXPAN + t];
+                MODP_TRY(panel_error(pc));
+                gave_up = pc.status == 5;
                 int64_t P = 0;
-                for (int t = 0; t < ts; ++t) P += pw[t];
-                if (npiv > 0) MODP_TRY(update_t(ts, KR, KC, FAR, pr[ts], pcj[ts], pw[ts], nullptr));
-                P += npiv;
-                MODP_TRY(block_end(KR, KC, FAR, P, P, NBW, nullptr));
-                kr += P;
-                kc += P;
-                stop_zero = hctl[ts].status == 1;
+                for (int q = 0; q < t; ++q) P += b.w[q];
+                const int64_t consumed = P + pc.ncols;
+                // the update after this panel was skipped by its own flag
+                if (pc.npiv > 0) MODP_TRY(update_t(i, t, true, b.KR, b.KC, b.FAR, b.rj[t], b.cj[t], b.w[t], nullptr));
+                P += pc.npiv;
+                MODP_TRY(block_end(b.KR, b.KC, b.FAR, P, consumed, b.width, nullptr));
+                kr = b.KR + P;
+                kc = b.KC + consumed;
+                nbo = b.FAR - b.KC;
+                stop_zero = pc.status == 1;
+                batch = 1;
+                if (P < consumed) {
+                    careful = true;
+                    MODP_TRY(rest_is_zero());
+                }
             }
-        } else if (nbo > 0) {
-            // ple: panels skip zero columns, so a panel's first row depends
+        } else if (ple) {
+            // Panels skip zero columns here, so a panel's first row depends
             // on the pivots found before it.  The panels of the block are
             // enqueued at their fixed columns and each takes its first row
             // from a device cursor that the previous one advanced; the
@@ -1025,9 +1089,11 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             // runs out of rows (or meets a pivot without inverse) raises the
             // abort flag, which turns the rest of the block into no-ops, and
             // the host reads the outcome once per block.
-            MODP_TRY(block_begin());
-            k_set_int<<<1, 1, 0, ctx->stream>>>(cursor, (int)KR);
-            HIP_TRY(ctx, hipGetLastError());
+            const int64_t KR = kr, KC = kc, FAR = KC + std::min<int64_t>(n - KC, NBO);
+            const int NBW = panel_width(KR);
+            gave_up = false;
+            nbo = FAR - KC;
+            MODP_TRY(blocks_begin(KR, 1));
             std::vector<int64_t> pcj, pw;
             for (int64_t cj = KC; cj < FAR; cj += NBW) {
                 pcj.push_back(cj);
@@ -1035,44 +1101,29 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             }
             const int np = (int)pcj.size();
             for (int t = 0; t < np; ++t) {
-                MODP_TRY(launch_panel_t(NBW, t, KC, FAR, KR, pcj[t], pw[t], abort_flag, cursor));
-                MODP_TRY(update_t(t, KR, KC, FAR, KR, pcj[t], pw[t], abort_flag));
+                MODP_TRY(launch_panel_t(NBW, 0, t, KC, FAR, KR, pcj[t], pw[t], abort_flag, cursor, false));
+                MODP_TRY(update_t(0, t, false, KR, KC, FAR, KR, pcj[t], pw[t], abort_flag));
             }
-            HIP_TRY(ctx, hipMemcpyAsync(hctl, bctl, sizeof(PanelCtl) * np, hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+            MODP_TRY(read_back());
             int64_t P = 0, consumed = 0;
             for (int t = 0; t < np; ++t) {
                 const PanelCtl &pc = hctl[t];
                 if (pc.status == 4) break;
-                if (pc.status == 3)
-                    return set_error(ctx, MODP_ERR_NOT_INVERTIBLE,
-                                     "pivot has no inverse modulo %lld (modulus not prime)", (long long)p);
-                if (pc.status == 6)
-                    return set_error(ctx, MODP_ERR_DEVICE, "an elimination panel's exchange did not end");
+                MODP_TRY(panel_error(pc));
                 gave_up = pc.status == 5;
                 P += pc.npiv;
                 consumed += pc.ncols;
                 if (pc.status != 0) {
                     // the update after this panel was skipped by its own flag
-                    if (pc.npiv > 0) MODP_TRY(update_t(t, KR, KC, FAR, KR, pcj[t], pw[t], nullptr));
+                    if (pc.npiv > 0) MODP_TRY(update_t(0, t, false, KR, KC, FAR, KR, pcj[t], pw[t], nullptr));
                     break;
                 }
             }
             kr += P;
             kc += consumed;
             MODP_TRY(block_end(KR, KC, FAR, P, consumed, NBW, nullptr));
-            if (P < consumed && kr < m && kc < n) {
-                // the block met zero columns: if nothing nonzero is left
-                // below row kr, no later column has a pivot and the
-                // factorisation is complete (rank = kr)
-                HIP_TRY(ctx, hipMemsetAsync(flag, 0, sizeof(int), ctx->stream));
-                k_any_nonzero<<<grid_for((m - kr) * (n - kc), 4096), 256, 0, ctx->stream>>>(W, ldw, kr, m, kc, n, flag);
-                HIP_TRY(ctx, hipGetLastError());
-                int *hflag = (int *)hctl;
-                HIP_TRY(ctx, hipMemcpyAsync(hflag, flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-                HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-                if (!*hflag) done = true;
-            }
+            careful = P < nbo;
+            if (P < consumed) MODP_TRY(rest_is_zero());
         }
         if (!ple && kr < m && kc < n && (stop_zero || nbo == 0 || kc > last)) {
             // pluq zero column at kc (rows >= kr zero): whole block zero -> tail,

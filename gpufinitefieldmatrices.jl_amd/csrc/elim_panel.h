@@ -117,6 +117,7 @@ struct PanelArgs {
     PanelCtl *ctl;
     PanelSolve *solve;
     int *abort, *cursor;
+    int strict;          // a column without a pivot raises the abort flag, too
     PanelExchange *x;
     uint32_t *arrive;
     int G;               // workgroups that take part
@@ -764,7 +765,7 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     if (gw == 0 && lane == 0) {
         *a.ctl = PanelCtl{pc, status, consumed, pc + (int)__popc(mask), kr0};
         if (a.cursor) *a.cursor = kr0 + pc;
-        if (a.abort && status != 0) *a.abort = 1;
+        if (a.abort && (status != 0 || (a.strict && pc < w))) *a.abort = 1;
     }
 }
 
