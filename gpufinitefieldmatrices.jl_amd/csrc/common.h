@@ -242,7 +242,7 @@ struct TuneEntry {
     double ms = 0.0;    // measured time of the winner
 };
 
-constexpr int WS_COUNT = 23;
+constexpr int WS_COUNT = 24;
 
 struct modp_ctx {
     int device = 0;
@@ -305,7 +305,8 @@ enum {
     WS_PERM = 19,      // lines moved by a permutation
     WS_GPOS = 20,      // row positions of the W-resident elimination panel
     WS_PANEL = 21,     // exchange area of the elimination panels on one XCD
-    WS_GEMV = 22       // K slices of a matrix-vector product that have arrived, by row block
+    WS_GEMV = 22,      // K slices of a matrix-vector product that have arrived, by row block
+    WS_RNS = 23        // multi-modular form: rows' sums and whether one modulus fewer does
 };
 
 // error plumbing: every internal function returns a modp_status

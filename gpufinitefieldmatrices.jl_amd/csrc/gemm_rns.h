@@ -7,15 +7,23 @@
 // moduli q_0..q_{r-1} <= 256 with M = prod q_j > 2 |C_int|:
 //
 //   * split: every operand entry is reduced mod each q_j into a residue
-//     held in int8 (one plane per modulus, |residue| <= 128); the B side is
-//     multiplied by y_j = (M/q_j)^{-1} mod q_j on the way;
+//     held in int8 (one plane per modulus, |residue| <= 128);
 //   * core: one int8 GEMM per modulus on v_mfma_i32_32x32x32_i8 with int32
 //     accumulation (|partial sums| <= k 2^14 < 2^31 for k <= 131071), whose
-//     epilogue writes e_j = D_j mod q_j = (y_j C_int) mod q_j as one byte;
-//   * combine: C_int = sum_j e_j M/q_j - t M with t = round(sum_j e_j / q_j)
-//     (exact: |C_int| / M < 1/2 leaves a margin far above the FP64 error of
-//     the sum), so C mod p = (sum_j e_j (M/q_j mod p) - t (M mod p)) mod p,
-//     every term an exact integer below 2^40 in FP64.
+//     epilogue writes e_j = C_int mod q_j as one byte;
+//   * combine: with y_j = (M/q_j)^{-1} mod q_j, C_int = sum_j e_j y_j M/q_j -
+//     t M and t = round(sum_j e_j y_j / q_j) (exact: |C_int| / M < 0.498
+//     leaves a margin far above the FP64 error of the sum, below 2^-33), so
+//     C mod p = (sum_j e_j (y_j M/q_j mod p) - t (M mod p)) mod p, every term an
+//     exact integer below 2^47 in FP64.
+//
+// The residues do not depend on M, so the same planes serve r and r - 1 moduli.
+// |C_int| <= max_i sum_k |a_ik| floor(p/2), about half of k floor(p/2)^2 for
+// entries that are spread over their range: where that may be enough for
+// r - 1, the A split sums the rows, and a small launch compares the largest
+// with the bound; the last plane's core then has nothing to do, and combine leaves
+// it out.  Entries that do not meet the bound take all r.  8192^3 mod 2^26 - 5
+// (eight of nine): 4.91 -> 4.44 ms.
 //
 // This is the Chinese-remainder reconstruction (Garner 1959; Knuth TAOCP
 // vol. 2 4.3.2) applied to an integer matrix product, as in the Ozaki
@@ -40,9 +48,8 @@ struct Moduli {
     int r;
     int single;               // one plane with q_0 = p (2 <= p <= 255): C mod p directly
     int q[NMOD_MAX];
-    int y[NMOD_MAX];          // (M/q_j)^{-1} mod q_j
-    double w[NMOD_MAX];       // (M/q_j) mod p
-    double invq[NMOD_MAX];    // 1/q_j
+    double w[NMOD_MAX];       // y_j (M/q_j) mod p, y_j = (M/q_j)^{-1} mod q_j
+    double yq[NMOD_MAX];      // y_j / q_j
     double wm;                // M mod p
 };
 
@@ -60,22 +67,18 @@ template <int Q> __device__ __forceinline__ int res8(float t)
 }
 
 // the 16 residue bytes of x[0..15] mod Q, packed little-endian, with
-// x = xh 4096 + xl (|xh| <= 2^13, 0 <= xl < 4096):
-//   A side  t = xh (4096 mod Q) + xl,          |t| < 2^21;
-//   B side  t = xh (4096 y mod Q) + xl y,      |t| < 255 (2^13 + 4096),
-// i.e. x y mod Q in one reduction (y < Q is the CRT weight of the plane).
-template <int Q, bool mulY> __device__ __forceinline__ v4i pack16q(const float *xh, const float *xl, int y)
+// x = xh 4096 + xl (|xh| <= 2^13, 0 <= xl < 4096): t = xh (4096 mod Q) + xl,
+// |t| < 2^21
+template <int Q> __device__ __forceinline__ v4i pack16q(const float *xh, const float *xl)
 {
-    const float C = mulY ? (float)((4096 * y) % Q) : (float)(4096 % Q);
-    const float yf = (float)y;
+    constexpr float C = (float)(4096 % Q);
     v4i w;
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
         uint32_t u = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float lo = mulY ? xl[4 * d + e] * yf : xl[4 * d + e];
-            const int v = res8<Q>(fmaf(xh[4 * d + e], C, lo));
+            const int v = res8<Q>(fmaf(xh[4 * d + e], C, xl[4 * d + e]));
             u |= ((uint32_t)v & 255u) << (8 * e);
         }
         w[d] = (int)u;
@@ -88,19 +91,16 @@ template <int Q, bool mulY> __device__ __forceinline__ v4i pack16q(const float *
 // 2^-20 of t / q, far closer than a non-tie quotient is to a half-integer
 // (1 / (2q) for odd q, 1 / q for even q): r is the balanced residue, or +-q/2
 // at an exact tie of an even q; |r| <= 127 either way.
-template <bool mulY> __device__ __forceinline__ v4i pack16r(const float *xh, const float *xl, int q, int y)
+__device__ __forceinline__ v4i pack16r(const float *xh, const float *xl, int q)
 {
-    const float qf = (float)q, iq = 1.0f / qf;
-    const float C = mulY ? (float)((4096 * y) % q) : (float)(4096 % q);
-    const float yf = (float)y;
+    const float qf = (float)q, iq = 1.0f / qf, C = (float)(4096 % q);
     v4i w;
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
         uint32_t u = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float lo = mulY ? xl[4 * d + e] * yf : xl[4 * d + e];
-            const float t = fmaf(xh[4 * d + e], C, lo);
+            const float t = fmaf(xh[4 * d + e], C, xl[4 * d + e]);
             const int v = (int)fmaf(-rintf(t * iq), qf, t);
             u |= ((uint32_t)v & 255u) << (8 * e);
         }
@@ -117,22 +117,22 @@ __device__ __forceinline__ void split12(int x, float &xh, float &xl)
 }
 
 // the same for modulus q_j (a wave-uniform j: one branch per plane)
-template <bool mulY> __device__ __forceinline__ v4i pack16(const float *xh, const float *xl, int j, const Moduli &md)
+__device__ __forceinline__ v4i pack16(const float *xh, const float *xl, int j, const Moduli &md)
 {
-    if (md.single) return pack16r<mulY>(xh, xl, md.q[0], md.y[0]);
+    if (md.single) return pack16r(xh, xl, md.q[0]);
     switch (j) {
-    case 0: return pack16q<QLIST[0], mulY>(xh, xl, md.y[0]);
-    case 1: return pack16q<QLIST[1], mulY>(xh, xl, md.y[1]);
-    case 2: return pack16q<QLIST[2], mulY>(xh, xl, md.y[2]);
-    case 3: return pack16q<QLIST[3], mulY>(xh, xl, md.y[3]);
-    case 4: return pack16q<QLIST[4], mulY>(xh, xl, md.y[4]);
-    case 5: return pack16q<QLIST[5], mulY>(xh, xl, md.y[5]);
-    case 6: return pack16q<QLIST[6], mulY>(xh, xl, md.y[6]);
-    case 7: return pack16q<QLIST[7], mulY>(xh, xl, md.y[7]);
-    case 8: return pack16q<QLIST[8], mulY>(xh, xl, md.y[8]);
-    case 9: return pack16q<QLIST[9], mulY>(xh, xl, md.y[9]);
-    case 10: return pack16q<QLIST[10], mulY>(xh, xl, md.y[10]);
-    default: return pack16q<QLIST[11], mulY>(xh, xl, md.y[11]);
+    case 0: return pack16q<QLIST[0]>(xh, xl);
+    case 1: return pack16q<QLIST[1]>(xh, xl);
+    case 2: return pack16q<QLIST[2]>(xh, xl);
+    case 3: return pack16q<QLIST[3]>(xh, xl);
+    case 4: return pack16q<QLIST[4]>(xh, xl);
+    case 5: return pack16q<QLIST[5]>(xh, xl);
+    case 6: return pack16q<QLIST[6]>(xh, xl);
+    case 7: return pack16q<QLIST[7]>(xh, xl);
+    case 8: return pack16q<QLIST[8]>(xh, xl);
+    case 9: return pack16q<QLIST[9]>(xh, xl);
+    case 10: return pack16q<QLIST[10]>(xh, xl);
+    default: return pack16q<QLIST[11]>(xh, xl);
     }
 }
 
@@ -181,8 +181,10 @@ template <int CPR> __device__ __forceinline__ int slot(int row, int q)
 template <class SH>
 __global__ __launch_bounds__(SH::NT, 1) void k_rns_gemm2(const int8_t *__restrict__ X, const int8_t *__restrict__ Y,
                                                        int64_t Np, int64_t Mp, int64_t Kp,
-                                                       uint8_t *__restrict__ E, Moduli md)
+                                                       uint8_t *__restrict__ E, Moduli md,
+                                                       const int *__restrict__ fewer)
 {
+    if (fewer && (int)blockIdx.y == md.r - 1 && *fewer) return;
     constexpr int TN = SH::TN, TM = SH::TM, BK = SH::BK, NT = SH::NT, CPR = SH::CPR, KK = SH::KK;
     constexpr int FN = SH::FN, FM = SH::FM;
     constexpr int XC = TN * CPR / NT, YC = TM * CPR / NT;
@@ -383,7 +385,8 @@ template <typename T> __device__ __forceinline__ int balanced(T v, const ModP &m
 template <typename TA>
 __global__ __launch_bounds__(256) void k_split_rows(int64_t m, int64_t k, const TA *__restrict__ A, int64_t lda,
                                                    int8_t *__restrict__ Yp, int64_t Mp, int64_t Kp, ModP mp,
-                                                   Moduli md, const int *__restrict__ skip)
+                                                   Moduli md, unsigned long long *__restrict__ rowsum,
+                                                   const int *__restrict__ skip)
 {
     if (skip && *skip) return;
     constexpr int TR = 64, TK = 128, LDT = TK + 1;  // odd pitch: conflict-free column writes
@@ -441,16 +444,27 @@ __global__ __launch_bounds__(256) void k_split_rows(int64_t m, int64_t k, const 
     for (int pass = 0; pass < 2; ++pass) {
         const int row = 32 * pass + (tid >> 3);
         float xh[16], xl[16];
+        uint32_t sum = 0;  // at most 16 2^25
 #pragma unroll
-        for (int e = 0; e < 16; ++e) split12(tile[row * LDT + ch * 16 + e], xh[e], xl[e]);
+        for (int e = 0; e < 16; ++e) {
+            const int x = tile[row * LDT + ch * 16 + e];
+            split12(x, xh[e], xl[e]);
+            sum += (uint32_t)(x < 0 ? -x : x);
+        }
+        if (rowsum) {
+            // |a| over the row's 128 k, in units of eight, rounded up
+            sum = (sum + 7) >> 3;
+#pragma unroll
+            for (int d = 1; d < 8; d <<= 1) sum += (uint32_t)__shfl_xor((int)sum, d);
+            if (ch == 0) atomicAdd(rowsum + r0 + row, (unsigned long long)sum);
+        }
         int8_t *dst = Yp + (size_t)(r0 + row) * Kp + k0 + ch * 16;
 #pragma unroll 1
-        for (int j = 0; j < md.r; ++j) *reinterpret_cast<v4i *>(dst + j * plane) = pack16<false>(xh, xl, j, md);
+        for (int j = 0; j < md.r; ++j) *reinterpret_cast<v4i *>(dst + j * plane) = pack16(xh, xl, j, md);
     }
 }
 
-// B (k x n column-major) -> planes X[j][col][kk] (k contiguous, times y_j),
-// zero-padded to Np x Kp.  Same orientation: each thread maps 16 consecutive
+// B (k x n column-major) -> planes X[j][col][kk] (k contiguous), zero-padded to Np x Kp.  Same orientation: each thread maps 16 consecutive
 // k of one column.
 template <typename TB>
 __global__ __launch_bounds__(256) void k_split_cols(int64_t k, int64_t n, const TB *__restrict__ B, int64_t ldb,
@@ -483,18 +497,49 @@ __global__ __launch_bounds__(256) void k_split_cols(int64_t k, int64_t n, const 
     const size_t plane = (size_t)Np * Kp;
     int8_t *dst = Xp + (size_t)col * Kp + k0;
 #pragma unroll 1
-    for (int j = 0; j < md.r; ++j) *reinterpret_cast<v4i *>(dst + j * plane) = pack16<true>(xh, xl, j, md);
+    for (int j = 0; j < md.r; ++j) *reinterpret_cast<v4i *>(dst + j * plane) = pack16(xh, xl, j, md);
 }
 
 // ---------------------------------------------------------------------------
 // combine: the r residue bytes of each entry -> C = epi(C, C_int mod p)
 // ---------------------------------------------------------------------------
+
+__global__ void k_rns_zero(int *p, int n)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0;
+}
+
+// whether the rows' sums of |a| (units of eight) leave |C_int| far enough below
+// half the product of one modulus fewer; the sums are cleared for the next call
+__global__ __launch_bounds__(1024) void k_rns_bound(unsigned long long *__restrict__ rowsum, int64_t rows, double h,
+                                                    double M, int *__restrict__ fewer)
+{
+    __shared__ double s_max[16];
+    unsigned long long top = 0;
+    for (int64_t r = threadIdx.x; r < rows; r += 1024) {
+        top = max(top, rowsum[r]);
+        rowsum[r] = 0;
+    }
+    double t = (double)top;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) t = fmax(t, __shfl_xor(t, d));
+    if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < 16; ++i) t = fmax(t, s_max[i]);
+        *fewer = 8.0 * t * h < 0.498 * M;
+    }
+}
+
 template <typename TC, int EPI>
 __global__ __launch_bounds__(256) void k_combine(int64_t m, int64_t n, const uint8_t *__restrict__ E, int64_t Mp,
-                                                int64_t plane, Moduli md, TC *__restrict__ C, int64_t ldc,
-                                                ModP mp, const int *__restrict__ skip, bool vec_ok)
+                                                int64_t plane, Moduli all, Moduli less, TC *__restrict__ C, int64_t ldc,
+                                                ModP mp, const int *__restrict__ fewer, const int *__restrict__ skip,
+                                                bool vec_ok)
 {
     if (skip && *skip) return;
+    const bool use_less = fewer && *fewer;
     // four consecutive rows of one column per thread: one 4-byte load per
     // modulus (Mp is a multiple of the output tile, so the load is aligned
     // and stays inside the plane)
@@ -503,30 +548,39 @@ __global__ __launch_bounds__(256) void k_combine(int64_t m, int64_t n, const uin
     if (idx >= mq * n) return;
     const int64_t j0 = 4 * (idx % mq), i = idx / mq;
     const uint8_t *src = E + i * Mp + j0;
-    double S[4] = {0.0, 0.0, 0.0, 0.0}, T[4] = {0.0, 0.0, 0.0, 0.0};
-    // every plane's word loaded before the first is used (planes past the
-    // r-th re-read the last one, so no load waits behind a branch)
-    uint32_t w[NMOD_MAX];
+    double S[4];
+    auto gather = [&](const Moduli &md) __attribute__((always_inline)) {
+        double T[4] = {0.0, 0.0, 0.0, 0.0};
+        // every plane's word loaded before the first is used (planes past the
+        // r-th re-read the last one, so no load waits behind a branch)
+        uint32_t w[NMOD_MAX];
 #pragma unroll
-    for (int jj = 0; jj < NMOD_MAX; ++jj)
-        w[jj] = *reinterpret_cast<const uint32_t *>(src + (size_t)(jj < md.r ? jj : md.r - 1) * plane);
+        for (int e = 0; e < 4; ++e) S[e] = 0.0;
 #pragma unroll
-    for (int jj = 0; jj < NMOD_MAX; ++jj) {
-        if (jj < md.r) {
-            const uint32_t w4 = w[jj];
+        for (int jj = 0; jj < NMOD_MAX; ++jj)
+            w[jj] = *reinterpret_cast<const uint32_t *>(src + (size_t)(jj < md.r ? jj : md.r - 1) * plane);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const double v = (double)((w4 >> (8 * e)) & 255u);
-                S[e] = fma(v, md.w[jj], S[e]);  // < 12 * 2^8 * 2^26: exact
-                T[e] = fma(v, md.invq[jj], T[e]);
+        for (int jj = 0; jj < NMOD_MAX; ++jj) {
+            if (jj < md.r) {
+                const uint32_t w4 = w[jj];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const double v = (double)((w4 >> (8 * e)) & 255u);
+                    S[e] = fma(v, md.w[jj], S[e]);  // < 12 * 2^8 * 2^26: exact
+                    T[e] = fma(v, md.yq[jj], T[e]);
+                }
             }
         }
-    }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[e] = fma(-rint(T[e]), md.wm, S[e]);  // < 2^47: exact
+    };
+    if (use_less) gather(less);
+    else gather(all);
     TC *dst = C + j0 + i * ldc;
     uint32_t r[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        r[e] = (uint32_t)dmod(fma(-rint(T[e]), md.wm, S[e]), mp);
+        r[e] = (uint32_t)dmod(S[e], mp);
         if (EPI != EPI_STORE && j0 + e < m) {
             const uint32_t c = to_res<TC>(dst[e], mp);
             r[e] = EPI == EPI_SUB ? submod(c, r[e], mp) : addmod(c, r[e], mp);

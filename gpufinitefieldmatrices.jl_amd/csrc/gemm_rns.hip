@@ -47,17 +47,15 @@ bool rns_single(int64_t p) { return p >= 2 && p <= 255; }
 
 int rns_planes(int64_t p, int64_t k) { return rns_single(p) ? 1 : rns_count(p, k); }
 
-// the single plane as a one-modulus system with M = q_0 = p: y_0 = 1,
-// w_0 = 1 and M mod p = 0, so the recombination returns the plane's residue
+// the single plane as a one-modulus system with M = q_0 = p: y_0 = w_0 = 1 and M mod p = 0, so the recombination returns the plane's residue
 static Moduli single_modulus(int64_t p)
 {
     Moduli md{};
     md.r = 1;
     md.single = 1;
     md.q[0] = (int)p;
-    md.y[0] = 1;
     md.w[0] = 1.0;
-    md.invq[0] = 1.0 / (double)p;
+    md.yq[0] = 1.0 / (double)p;
     md.wm = 0.0;
     return md;
 }
@@ -72,9 +70,9 @@ static Moduli make_moduli(int64_t p, int r)
         const int64_t q = QLIST[j];
         const u128 Mj = M / (u128)q;
         md.q[j] = (int)q;
-        md.y[j] = (int)inv_mod_small((int64_t)(Mj % (u128)q), q);
-        md.w[j] = (double)(int64_t)(Mj % (u128)p);
-        md.invq[j] = 1.0 / (double)q;
+        const int64_t y = inv_mod_small((int64_t)(Mj % (u128)q), q);
+        md.w[j] = (double)(int64_t)(Mj % (u128)p * (u128)y % (u128)p);
+        md.yq[j] = (double)y / (double)q;
     }
     md.wm = (double)(int64_t)(M % (u128)p);
     return md;
@@ -84,21 +82,22 @@ namespace {
 
 template <class SH>
 int launch_core(modp_ctx *ctx, const int8_t *X, const int8_t *Y, int64_t Np, int64_t Mp, int64_t Kp, uint8_t *E,
-                const Moduli &md)
+                const Moduli &md, const int *fewer)
 {
     const dim3 grid(xcd_grid((Np / SH::TN) * (Mp / SH::TM)), (unsigned)md.r);
     TimedLaunch tl(ctx, "gemm_rns");
-    rns::k_rns_gemm2<SH><<<grid, SH::NT, 0, ctx->stream>>>(X, Y, Np, Mp, Kp, E, md);
+    rns::k_rns_gemm2<SH><<<grid, SH::NT, 0, ctx->stream>>>(X, Y, Np, Mp, Kp, E, md, fewer);
     return hip_check(ctx, hipGetLastError(), "k_rns_gemm launch");
 }
 
 template <typename T>
 int split_rows_t(modp_ctx *ctx, const GemmArgs &g, int64_t kbeg, int64_t kc, int8_t *Yp, int64_t Mp, int64_t Kp,
-                 const Moduli &md)
+                 const Moduli &md, unsigned long long *rowsum)
 {
     const dim3 grid((unsigned)(Kp / 128), (unsigned)(Mp / 64));
     const T *A = (const T *)g.A + kbeg * g.lda;
-    rns::k_split_rows<T><<<grid, 256, 0, ctx->stream>>>(g.m, kc, A, g.lda, Yp, Mp, Kp, g.mp, md, g.skip);
+    rns::k_split_rows<T><<<grid, 256, 0, ctx->stream>>>(g.m, kc, A, g.lda, Yp, Mp, Kp, g.mp, md, rowsum,
+                                                     g.skip);
     return hip_check(ctx, hipGetLastError(), "k_split_rows launch");
 }
 
@@ -115,7 +114,7 @@ int split_cols_t(modp_ctx *ctx, const GemmArgs &g, int64_t kbeg, int64_t kc, int
 
 template <typename TC>
 int combine_t(modp_ctx *ctx, const GemmArgs &g, int epi, const uint8_t *E, int64_t Mp, int64_t plane,
-              const Moduli &md)
+              const Moduli &md, const Moduli &less, const int *fewer)
 {
     TC *C = (TC *)g.C;
     if (md.single) {
@@ -132,15 +131,9 @@ int combine_t(modp_ctx *ctx, const GemmArgs &g, int epi, const uint8_t *E, int64
     const unsigned grid = (unsigned)((((g.m + 3) / 4) * g.n + 255) / 256);
     // 16-byte stores of four rows need every column start 16-byte aligned
     const bool vec = sizeof(TC) == 8 && (g.ldc & 1) == 0 && ((uintptr_t)C & 15) == 0;
-    if (epi == EPI_STORE)
-        rns::k_combine<TC, EPI_STORE><<<grid, 256, 0, ctx->stream>>>(g.m, g.n, E, Mp, plane, md, C, g.ldc, g.mp, g.skip,
-                                                                      vec);
-    else if (epi == EPI_SUB)
-        rns::k_combine<TC, EPI_SUB><<<grid, 256, 0, ctx->stream>>>(g.m, g.n, E, Mp, plane, md, C, g.ldc, g.mp, g.skip,
-                                                                    vec);
-    else
-        rns::k_combine<TC, EPI_ADD><<<grid, 256, 0, ctx->stream>>>(g.m, g.n, E, Mp, plane, md, C, g.ldc, g.mp, g.skip,
-                                                                    vec);
+    auto *k = epi == EPI_STORE ? rns::k_combine<TC, EPI_STORE>
+                               : epi == EPI_SUB ? rns::k_combine<TC, EPI_SUB> : rns::k_combine<TC, EPI_ADD>;
+    k<<<grid, 256, 0, ctx->stream>>>(g.m, g.n, E, Mp, plane, md, less, C, g.ldc, g.mp, fewer, g.skip, vec);
     return hip_check(ctx, hipGetLastError(), "k_combine launch");
 }
 
@@ -149,10 +142,10 @@ int combine_t(modp_ctx *ctx, const GemmArgs &g, int epi, const uint8_t *E, int64
 // against 5.00 ms for 2x2 waves of 128x128 with the accumulators in AGPRs)
 // or 128x128 with 2x2 waves of 64x64
 int core_by_tile(modp_ctx *ctx, int tile, const int8_t *X, const int8_t *Y, int64_t Np, int64_t Mp, int64_t Kp,
-                 uint8_t *E, const Moduli &md)
+                 uint8_t *E, const Moduli &md, const int *fewer)
 {
-    if (tile == 256) return launch_core<rns::Shape<256, 256, 2, 4, 128>>(ctx, X, Y, Np, Mp, Kp, E, md);
-    return launch_core<rns::Shape<128, 128, 2, 2, 128>>(ctx, X, Y, Np, Mp, Kp, E, md);
+    if (tile == 256) return launch_core<rns::Shape<256, 256, 2, 4, 128>>(ctx, X, Y, Np, Mp, Kp, E, md, fewer);
+    return launch_core<rns::Shape<128, 128, 2, 2, 128>>(ctx, X, Y, Np, Mp, Kp, E, md, fewer);
 }
 
 }  // namespace
@@ -183,18 +176,43 @@ int gemm_rns_run(modp_ctx *ctx, const GemmArgs &g, int tile)
         if (!Xp) return st;
         uint8_t *E = (uint8_t *)ws_get(ctx, WS_SLICES, (size_t)r * Np * Mp, &st);
         if (!E) return st;
-        if (g.ka == EK_F64) MODP_TRY(split_rows_t<double>(ctx, g, kdone, kc, Yp, Mp, Kp, md));
-        else if (g.ka == EK_F32) MODP_TRY(split_rows_t<float>(ctx, g, kdone, kc, Yp, Mp, Kp, md));
-        else MODP_TRY(split_rows_t<int32_t>(ctx, g, kdone, kc, Yp, Mp, Kp, md));
+        // one modulus fewer where entries spread over their range would do
+        // with it; the rows' sums start and end at zero
+        const u128 h = (u128)(g.mp.p / 2), kh2 = (u128)(kc > 0 ? kc : 1) * h * h;
+        u128 M = 1;
+        for (int j = 0; j + 1 < r; ++j) M *= (u128)QLIST[j];
+        unsigned long long *rowsum = nullptr;
+        int *fewer = nullptr;
+        Moduli less = md;
+        if (!md.single && r > 1 && M > kh2 + kh2 / 32) {
+            const size_t had = ctx->ws_size[WS_RNS];
+            int *buf = (int *)ws_get(ctx, WS_RNS, 256 + sizeof(unsigned long long) * (size_t)Mp, &st);
+            if (!buf) return st;
+            fewer = buf;
+            rowsum = (unsigned long long *)(buf + 64);
+            if (ctx->ws_size[WS_RNS] != had) {
+                const int words = (int)(ctx->ws_size[WS_RNS] / sizeof(int));
+                rns::k_rns_zero<<<(words + 255) / 256, 256, 0, ctx->stream>>>(buf, words);
+                HIP_TRY(ctx, hipGetLastError());
+            }
+            less = make_moduli(g.mp.p, r - 1);
+        }
+        if (g.ka == EK_F64) MODP_TRY(split_rows_t<double>(ctx, g, kdone, kc, Yp, Mp, Kp, md, rowsum));
+        else if (g.ka == EK_F32) MODP_TRY(split_rows_t<float>(ctx, g, kdone, kc, Yp, Mp, Kp, md, rowsum));
+        else MODP_TRY(split_rows_t<int32_t>(ctx, g, kdone, kc, Yp, Mp, Kp, md, rowsum));
         if (g.kb == EK_F64) MODP_TRY(split_cols_t<double>(ctx, g, kdone, kc, Xp, Np, Kp, md));
         else if (g.kb == EK_F32) MODP_TRY(split_cols_t<float>(ctx, g, kdone, kc, Xp, Np, Kp, md));
         else MODP_TRY(split_cols_t<int32_t>(ctx, g, kdone, kc, Xp, Np, Kp, md));
-        MODP_TRY(core_by_tile(ctx, (int)T, Xp, Yp, Np, Mp, Kp, E, md));
+        if (fewer) {
+            rns::k_rns_bound<<<1, 1024, 0, ctx->stream>>>(rowsum, Mp, (double)(g.mp.p / 2), (double)M, fewer);
+            HIP_TRY(ctx, hipGetLastError());
+        }
+        MODP_TRY(core_by_tile(ctx, (int)T, Xp, Yp, Np, Mp, Kp, E, md, fewer));
         int epi = g.epi;
         if (!first && epi == EPI_STORE) epi = EPI_ADD;
-        if (g.kc == EK_F64) MODP_TRY(combine_t<double>(ctx, g, epi, E, Mp, Np * Mp, md));
-        else if (g.kc == EK_F32) MODP_TRY(combine_t<float>(ctx, g, epi, E, Mp, Np * Mp, md));
-        else MODP_TRY(combine_t<int32_t>(ctx, g, epi, E, Mp, Np * Mp, md));
+        if (g.kc == EK_F64) MODP_TRY(combine_t<double>(ctx, g, epi, E, Mp, Np * Mp, md, less, fewer));
+        else if (g.kc == EK_F32) MODP_TRY(combine_t<float>(ctx, g, epi, E, Mp, Np * Mp, md, less, fewer));
+        else MODP_TRY(combine_t<int32_t>(ctx, g, epi, E, Mp, Np * Mp, md, less, fewer));
         kdone += kc;
         first = false;
     } while (kdone < g.k);
