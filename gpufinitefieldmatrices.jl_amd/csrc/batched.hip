@@ -806,13 +806,21 @@ struct EJob {
 };
 
 // Instances are grouped by the LDS element their modulus needs (8-bit
-// residues below 2^8, 16-bit below 2^16, else 32-bit): each class has its own
-// kernel, queue, LDS slot (sized for its largest instance) and persistent
-// grid, so the small-element classes keep their occupancy.
-constexpr int ECLASS = 3;
-struct ElimClass {
+// residues below 2^8, 16-bit below 2^16, else 32-bit) and, below 2^16, by
+// size: each group has its own kernel, queue, LDS slot (sized for its largest
+// instance) and persistent grid, so small instances and elements keep their
+// occupancy.  Instances of more than EBIG elements run on EWAVES wavefronts:
+// a lone wavefront issues an instruction every eight cycles, and the 128 pivots
+// of a 128 x 128 instance mod 65521 took 440 us, the whole batch's time.  4096
+// instances of 8 to 128 rows and columns, PLUQ: 500 us on one wavefront each,
+// 378 on two from 6144 elements on (391 from 8192, 382 from 4096), 412 to 474
+// on four, whose idle halves cost more than the shorter chains save.
+constexpr int EGROUP = 5;  // class 0 small, large, class 1 small, large, class 2
+constexpr int EWAVES = 2;
+constexpr int64_t EBIG = 6144;
+struct ElimGroup {
     int64_t off = 0, count = 0;  // range of the job table
-    size_t slot = 0;             // LDS bytes per workgroup (one wavefront)
+    size_t slot = 0;             // LDS bytes per workgroup (one instance)
     int bk_off = 0;              // offset of the pivot bookkeeping in the slot
     int grid = 0;
 };
@@ -821,11 +829,11 @@ struct modp_elim_plan {
     int op = 0, kind = EK_F64;
     int64_t count = 0;
     EJob *djobs = nullptr;
-    int *dcounter = nullptr;  // one queue counter per class, 64 bytes apart
-    ElimClass cls[ECLASS];
+    int *dcounter = nullptr;  // one queue counter per group, 64 bytes apart
+    ElimGroup group[EGROUP];
     uint16_t *dtab = nullptr;  // inverse tables of the distinct primes below 2^16
-    hipStream_t side[ECLASS - 1] = {nullptr, nullptr};  // fork streams of the capture
-    hipEvent_t fork = nullptr, join[ECLASS - 1] = {nullptr, nullptr};
+    hipStream_t side[EGROUP - 1] = {};  // fork streams of the capture
+    hipEvent_t fork = nullptr, join[EGROUP - 1] = {};
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
 };
@@ -847,9 +855,16 @@ __device__ __forceinline__ void wave_sync()
     asm volatile("" ::: "memory");
 }
 
+// the same among the NW wavefronts of an instance
+template <int NW> __device__ __forceinline__ void inst_sync()
+{
+    if constexpr (NW == 1) wave_sync();
+    else __syncthreads();
+}
+
 __global__ void k_elim_counter_reset(int *counter)
 {
-    if (threadIdx.x < ECLASS && blockIdx.x == 0) counter[16 * threadIdx.x] = 0;
+    if (threadIdx.x < EGROUP && blockIdx.x == 0) counter[16 * threadIdx.x] = 0;
 }
 
 // argmax keys: larger key = larger residue, then lower row (rows < 256)
@@ -991,12 +1006,13 @@ typedef int ev16i __attribute__((ext_vector_type(16)));
 // D mod p: q = rint(fl(D) fl(1/p)) is within 0.01 of D/p (|D|/p < 2^16), so
 // r = D - q p lies in (-0.51 p, 0.51 p) and one fix-up, min(r, r + p) in
 // unsigned arithmetic, finishes it.
-template <int KB>
+template <int KB, int NW>
 __device__ __forceinline__ void flush_rows_mfma8(uint8_t *M, int pitch, int a, int b, int pe, int n, int prow,
                                                  int np, const int *pc, const ModP &mp)
 {
-    if (a >= b) return;
-    const int lane = threadIdx.x, l32 = lane & 31, hi = lane >> 5;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (a + 32 * wave >= b) return;
+    const int l32 = lane & 31, hi = lane >> 5;
     const int p = (int)mp.p32, half = p >> 1;
     const int ntc = (n - pe + 31) >> 5;  // column tiles, at most 4
     ev4i bop[4];
@@ -1016,7 +1032,7 @@ __device__ __forceinline__ void flush_rows_mfma8(uint8_t *M, int pitch, int a, i
         }
         bop[ct] = hi ? ev4i{0, 0, 0, 0} : ev4i{(int)w[0], (int)w[1], 0, 0};
     }
-    for (int r0 = a; r0 < b; r0 += 32) {
+    for (int r0 = a + 32 * wave; r0 < b; r0 += 32 * NW) {
         uint32_t w[2] = {0u, 0u};
         const int rr = min(r0 + l32, b - 1);
 #pragma unroll
@@ -1060,20 +1076,21 @@ __device__ __forceinline__ void flush_rows_mfma8(uint8_t *M, int pitch, int a, i
 // with K index l >> 4; accumulator column l & 15, rows (l >> 4) + 4 e.  Rows
 // and columns past the range repeat the last one.  V comes from the pivot
 // rows' trailing columns, written by the flush's first step.
-template <int KB>
+template <int KB, int NW>
 __device__ __forceinline__ void flush_rows_mfma16(uint16_t *M, int pitch, int a, int b, int pe, int n, int prow,
                                                   int np, const int16_t *pivcol, const ModP &mp)
 {
     static_assert(KB == 8, "two K=4 steps per tile");
-    if (a >= b) return;
-    const int lane = threadIdx.x, l16 = lane & 15, kq = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (a + 16 * wave >= b) return;
+    const int l16 = lane & 15, kq = lane >> 4;
     const int ntc = (n - pe + 15) >> 4;  // column tiles, at most 8
     // this lane's pivots kq and kq + 4 (their columns from the bookkeeping)
     const bool ka = kq < np, kb = kq + 4 < np;
     const int pca = ka ? (int)pivcol[prow + kq] : 0;
     const int pcb = kb ? (int)pivcol[prow + kq + 4] : 0;
     const int va = (prow + (ka ? kq : 0)) * pitch, vb = (prow + (kb ? kq + 4 : 0)) * pitch;
-    for (int r0 = a; r0 < b; r0 += 16) {
+    for (int r0 = a + 16 * wave; r0 < b; r0 += 16 * NW) {
         const int rr = min(r0 + l16, b - 1);
         const double a0 = ka ? (double)M[rr * pitch + pca] : 0.0;
         const double a1 = kb ? (double)M[rr * pitch + pcb] : 0.0;
@@ -1102,7 +1119,12 @@ __device__ __forceinline__ void flush_rows_mfma16(uint16_t *M, int pitch, int a,
 #pragma unroll
             for (int g = 0; g < NG; ++g)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) M[ro[e] + cc[g]] = (uint16_t)dmod(acc[g][e], mp);
+                for (int e = 0; e < 4; ++e) {
+                    // (x + 1/2) / p is at least 1/(2p) away from every integer
+                    // and far below 2^51 / p, so the floor is the quotient
+                    const double x = acc[g][e];
+                    M[ro[e] + cc[g]] = (uint16_t)fma(-floor(fma(x, mp.pinv, 0.5 * mp.pinv)), mp.pd, x);
+                }
         };
         int ct = 0;
         for (; ct + 4 <= ntc; ct += 4) tiles(ct, std::integral_constant<int, 4>());
@@ -1112,22 +1134,26 @@ __device__ __forceinline__ void flush_rows_mfma16(uint16_t *M, int pitch, int a,
 
 // Trailing columns pe..n-1 of the pending pivots (rows prow..prow+np-1) on
 // lanes over columns: lane q owns columns pe+q and (WIDE) pe+64+q; lanes
-// past the last column repeat it, computing and storing the same value.
-template <typename S, int KB, int ACC, bool WIDE>
+// past the last column repeat it, computing and storing the same value.  With
+// several wavefronts wave w owns pe+64w+q instead (not WIDE; none past the
+// last column), and the rows of the trailing update are dealt out by tiles.
+template <typename S, int KB, int ACC, bool WIDE, int NW>
 __device__ __forceinline__ void flush_cols(S *M, int pitch, int m, int n, int op, int prow, int np, int pe,
                                            const int *pc, const int16_t *pivcol, const uint32_t *inv,
                                            const uint32_t *lq0, const uint32_t *lq1, const ModP &mp)
 {
     typedef Acc<ACC> A;
     constexpr bool SMALL = sizeof(S) < 4;
-    const int lane = threadIdx.x;
-    const int c0 = min(pe + lane, n - 1), c1 = min(pe + 64 + lane, n - 1);
+    static_assert(NW == 1 || (!WIDE && SMALL), "rows by matrix instructions");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool mine = NW == 1 || pe + 64 * wave < n;
+    const int c0 = min(pe + (NW == 1 ? 0 : 64 * wave) + lane, n - 1), c1 = min(pe + 64 + lane, n - 1);
     typename A::V v0[KB], v1[KB];
     // pivot rows, in order: V_j = (x_j - sum_{i<j} L_{r_j,i} V_i) inv_j
 #pragma unroll
     for (int jj = 0; jj < KB; ++jj) {
         v0[jj] = v1[jj] = typename A::V(0);
-        if (jj < np) {
+        if (jj < np && mine) {
             const int r = prow + jj;
             typename A::S a0 = A::init(M[r * pitch + c0]), a1 = A::init(WIDE ? (uint32_t)M[r * pitch + c1] : 0u);
 #pragma unroll
@@ -1146,7 +1172,7 @@ __device__ __forceinline__ void flush_cols(S *M, int pitch, int m, int n, int op
             }
         }
     }
-    wave_sync();
+    inst_sync<NW>();
     // every other row
     constexpr int RB = 4;
     auto rows = [&](int a, int b) {
@@ -1155,21 +1181,22 @@ __device__ __forceinline__ void flush_cols(S *M, int pitch, int m, int n, int op
     };
     if (sizeof(S) == 1) {
         uint8_t *M8 = reinterpret_cast<uint8_t *>(M);
-        flush_rows_mfma8<KB>(M8, pitch, prow + np, m, pe, n, prow, np, pc, mp);
-        if (op == MODP_ELIM_RREF) flush_rows_mfma8<KB>(M8, pitch, 0, prow, pe, n, prow, np, pc, mp);
+        flush_rows_mfma8<KB, NW>(M8, pitch, prow + np, m, pe, n, prow, np, pc, mp);
+        if (op == MODP_ELIM_RREF) flush_rows_mfma8<KB, NW>(M8, pitch, 0, prow, pe, n, prow, np, pc, mp);
     } else if (sizeof(S) == 2 && KB == 8) {
         uint16_t *M16 = reinterpret_cast<uint16_t *>(M);
-        flush_rows_mfma16<8>(M16, pitch, prow + np, m, pe, n, prow, np, pivcol, mp);
-        if (op == MODP_ELIM_RREF) flush_rows_mfma16<8>(M16, pitch, 0, prow, pe, n, prow, np, pivcol, mp);
+        flush_rows_mfma16<8, NW>(M16, pitch, prow + np, m, pe, n, prow, np, pivcol, mp);
+        if (op == MODP_ELIM_RREF) flush_rows_mfma16<8, NW>(M16, pitch, 0, prow, pe, n, prow, np, pivcol, mp);
     } else {
         rows(prow + np, m);
         if (op == MODP_ELIM_RREF) rows(0, prow);
     }
     if (op == MODP_ELIM_RREF) {
         // the panel's pivot rows take the later pivots of the panel
+        if (NW > 1) inst_sync<NW>();  // every wave has read them
 #pragma unroll
         for (int own = 0; own + 1 < KB; ++own) {
-            if (own + 1 < np) {
+            if (own + 1 < np && mine) {
                 const int r = prow + own;
                 typename A::S a0 = A::init(M[r * pitch + c0]), a1 = A::init(WIDE ? (uint32_t)M[r * pitch + c1] : 0u);
 #pragma unroll
@@ -1183,15 +1210,15 @@ __device__ __forceinline__ void flush_cols(S *M, int pitch, int m, int n, int op
             }
         }
     }
-    wave_sync();
+    inst_sync<NW>();
 }
 
-template <typename S, int KB, int ACC>
+template <typename S, int KB, int ACC, int NW>
 __device__ __forceinline__ void flush(S *M, int pitch, int m, int n, int op, int prow, int np, int pe,
                                       const int16_t *pivcol, const uint32_t *pivinv, const ModP &mp)
 {
     if (np <= 0) return;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
     int pc[KB];
     uint32_t inv[KB], lq0[KB], lq1[KB];
 #pragma unroll
@@ -1206,19 +1233,21 @@ __device__ __forceinline__ void flush(S *M, int pitch, int m, int n, int op, int
         }
     }
     if (pe < n) {
-        if (n - pe > 64)
-            flush_cols<S, KB, ACC, true>(M, pitch, m, n, op, prow, np, pe, pc, pivcol, inv, lq0, lq1, mp);
+        if (NW == 1 && n - pe > 64)
+            flush_cols<S, KB, ACC, NW == 1, NW>(M, pitch, m, n, op, prow, np, pe, pc, pivcol, inv, lq0, lq1, mp);
         else
-            flush_cols<S, KB, ACC, false>(M, pitch, m, n, op, prow, np, pe, pc, pivcol, inv, lq0, lq1, mp);
+            flush_cols<S, KB, ACC, false, NW>(M, pitch, m, n, op, prow, np, pe, pc, pivcol, inv, lq0, lq1, mp);
     }
     if (op == MODP_ELIM_RREF) {
-        // the multipliers have been applied: clear the pivot columns but the pivots
+        // the multipliers have been applied (and, without trailing columns,
+        // read by every wave): clear the pivot columns but the pivots
+        if (NW > 1) inst_sync<NW>();
 #pragma unroll
         for (int jj = 0; jj < KB; ++jj)
             if (jj < np)
-                for (int r = lane; r < m; r += 64)
+                for (int r = threadIdx.x; r < m; r += 64 * NW)
                     if (r != prow + jj) M[r * pitch + pc[jj]] = S(0);
-        wave_sync();
+        inst_sync<NW>();
     }
 }
 
@@ -1228,8 +1257,14 @@ __device__ __forceinline__ void flush(S *M, int pitch, int m, int n, int op, int
 // with the lanes over rows and the flushes with the lanes over columns.
 // S is the LDS element; every control value (m, n, row, col, the pivot) is
 // wave-uniform, so the branches are scalar.
-template <typename T, typename S, int KB, int ACC>
-__device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned char *esm, int bk_off)
+//
+// NW > 1: the columns of the panel's immediate updates, the swaps, the row
+// tiles of the flushes, input and output are dealt out to the wavefronts; the
+// first owns the next pivot column, finds its largest residue and leaves the key
+// in `found`.  Two barriers a pivot.
+template <typename T, typename S, int KB, int ACC, int NW>
+__device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned char *esm, int bk_off,
+                                              typename EKey<S>::T *found)
 {
     typedef EKey<S> K;
     typedef typename K::T key_t;
@@ -1241,7 +1276,7 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
     int16_t *ipiv = pivcol + EMAX;
     int16_t *perm = ipiv + EMAX;
     uint8_t *itab8 = reinterpret_cast<uint8_t *>(perm + EMAX);
-    const int lane = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m = j.m, n = j.n, pitch = j.pitch;
     const ModP &mp = j.mp;
     const T *A = (const T *)j.A;
@@ -1263,7 +1298,7 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
     {
         const int r0 = min(lane, m - 1), r1 = min(lane + 64, m - 1);
         const bool two = m > 64;
-        for (int c0 = 0; c0 < n; c0 += 16) {
+        for (int c0 = 16 * wave; c0 < n; c0 += 16 * NW) {
             T x0[16], x1[16];
 #pragma unroll
             for (int t = 0; t < 16; ++t) {
@@ -1279,7 +1314,7 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
             }
         }
     }
-    wave_sync();
+    inst_sync<NW>();
     int row = 0, col = 0, last = n - 1, nr = 0, nc = 0;
     int prow = 0;               // first pivot row whose trailing update is pending
     int pe = KB < n ? KB : n;   // end of the current panel's columns
@@ -1290,8 +1325,9 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
     while (row < m && col < n) {
         // largest residue of column col in rows row..m-1, lowest row on ties
         key_t mine = 0;
+        const bool known = NW > 1 && have_pre;
         if (have_pre) {
-            mine = pre;
+            if (NW == 1) mine = pre;
             have_pre = false;
         } else {
             if (lane >= row && lane < m) mine = K::make(M[lane * pitch + col], lane);
@@ -1300,20 +1336,21 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
                 mine = k > mine ? k : mine;
             }
         }
-        const key_t best = wave_max(mine);
-        const uint32_t bv = K::val(best);
+        const key_t best = known ? *found : wave_max(mine);
+        const uint32_t bv = (uint32_t)__builtin_amdgcn_readfirstlane((int)K::val(best));
         if (bv == 0 && op == MODP_ELIM_PLUQ) {
-            flush<S, KB, ACC>(M, pitch, m, n, op, prow, row - prow, pe, pivcol, pivinv, mp);
+            flush<S, KB, ACC, NW>(M, pitch, m, n, op, prow, row - prow, pe, pivcol, pivinv, mp);
             prow = row;
             // is the whole block rows row.., columns col.. zero?
             int nz = 0;
             for (int c = col + lane; c < n; c += 64)
                 for (int r = row; r < m; ++r) nz |= M[r * pitch + c] != 0;
+            if (NW > 1) inst_sync<NW>();  // every wave has looked
             if (!__any(nz)) {
                 // the reference's tail: (c, n) for c = col..n-1 in order,
                 // which rotates columns col..n-1 right by one
                 const int ca = col + 1 + lane, cb = col + 65 + lane;
-                for (int r = 0; r < m; ++r) {
+                for (int r = wave; r < m; r += NW) {
                     const S first = M[r * pitch + n - 1];
                     const S va = ca < n ? M[r * pitch + ca - 1] : S(0);
                     const S vb = cb < n ? M[r * pitch + cb - 1] : S(0);
@@ -1323,28 +1360,29 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
                     if (lane == 0) M[r * pitch + col] = first;
                     wave_sync();
                 }
-                if (lane == 0)
+                if (tid == 0)
                     for (int c = col, k = nc; c < n; ++c, ++k) {
                         j.col_info[2 * k] = c + 1;
                         j.col_info[2 * k + 1] = n;
                     }
                 nc += n - col;
                 ended = true;
+                inst_sync<NW>();
                 break;
             }
             // swap with the last column not yet swapped; retry this column
-            for (int r = lane; r < m; r += 64) {
+            for (int r = tid; r < m; r += 64 * NW) {
                 const S t = M[r * pitch + col];
                 M[r * pitch + col] = M[r * pitch + last];
                 M[r * pitch + last] = t;
             }
-            if (lane == 0) {
+            if (tid == 0) {
                 j.col_info[2 * nc] = col + 1;
                 j.col_info[2 * nc + 1] = last + 1;
             }
             ++nc;
             --last;
-            wave_sync();
+            inst_sync<NW>();
             continue;
         }
         if (bv == 0) {
@@ -1353,10 +1391,18 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
             const uint32_t inv = tab8 ? (uint32_t)itab8[bv]
                                       : (sizeof(S) == 2 && j.itab ? (uint32_t)j.itab[bv] : modinv_fast(bv, mp));
             if (inv == 0) { bad = true; break; }
-            const int I = K::row(best);
+            const int I = __builtin_amdgcn_readfirstlane(K::row(best));
             // swap rows row <-> I (every column) and normalise the pivot row
             // over the panel (the flush normalises the trailing columns)
-            {
+            if constexpr (NW > 1) {
+                static_assert(64 * NW >= EMAX, "a thread per column");
+                inst_sync<NW>();  // every wave has read the column's keys
+                if (tid < n) {
+                    const uint32_t a0 = M[row * pitch + tid], b0 = M[I * pitch + tid];
+                    M[I * pitch + tid] = (S)a0;
+                    M[row * pitch + tid] = (S)((tid >= col && tid < pe) ? mulmod_c<SMALL>(b0, inv, mp) : b0);
+                }
+            } else {
                 const int ca = min(lane, n - 1), cb = min(lane + 64, n - 1);
                 const uint32_t a0 = M[row * pitch + ca], b0 = M[I * pitch + ca];
                 const uint32_t a1 = M[row * pitch + cb], b1 = M[I * pitch + cb];
@@ -1368,7 +1414,7 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
                     M[row * pitch + cb] = (S)((cb >= col && cb < pe) ? mulmod_c<SMALL>(b1, inv, mp) : b1);
                 }
             }
-            if (lane == 0) {
+            if (tid == 0) {
                 pivval[row] = bv;
                 pivinv[row] = inv;
                 pivcol[row] = (int16_t)col;
@@ -1379,7 +1425,7 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
                 }
             }
             if (op == MODP_ELIM_PLUQ && I != row) ++nr;
-            wave_sync();
+            inst_sync<NW>();
             // the panel's columns col+1..pe-1, lanes over rows: rows below the
             // pivot (pluq, lu) or every other row (rref)
             if (col + 1 < pe) {
@@ -1391,47 +1437,52 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
                 const int i0 = op == MODP_ELIM_RREF ? 0 : row + 1;
                 const int ra = min(lane, m - 1), rb = min(lane + 64, m - 1);
                 const bool two = m > 64;
-                uint32_t kp[KB], xa[KB], xb[KB];
+                // Wave w takes columns col + 1 + w, + NW, ...
+                constexpr int KT = (KB + NW - 2) / NW > 0 ? (KB + NW - 2) / NW : 1;
+                uint32_t kp[KT], xa[KT], xb[KT];
 #pragma unroll
-                for (int t = 0; t + 1 < KB; ++t) {
-                    const uint32_t v = M[row * pitch + col + 1 + t];
+                for (int t = 0; t < KT; ++t) {
+                    const int c = col + 1 + wave + NW * t;
+                    const uint32_t v = M[row * pitch + c];
                     kp[t] = SMALL ? (v ? mp.p32 - v : 0u) : v;
-                    xa[t] = M[ra * pitch + col + 1 + t];
-                    xb[t] = two ? (uint32_t)M[rb * pitch + col + 1 + t] : 0u;
+                    xa[t] = M[ra * pitch + c];
+                    xb[t] = two ? (uint32_t)M[rb * pitch + c] : 0u;
                 }
                 const uint32_t la = (ra >= i0 && ra != row) ? (uint32_t)M[ra * pitch + col] : 0u;
                 const uint32_t lb = (two && rb >= i0 && rb != row) ? (uint32_t)M[rb * pitch + col] : 0u;
                 wave_sync();
 #pragma unroll
-                for (int t = 0; t + 1 < KB; ++t) {
-                    if (col + 1 + t < pe) {
+                for (int t = 0; t < KT; ++t) {
+                    const int c = col + 1 + wave + NW * t;
+                    if (c < pe) {
                         const uint32_t ya = row_update<SMALL>(xa[t], la, kp[t], mp);
                         const uint32_t yb = two ? row_update<SMALL>(xb[t], lb, kp[t], mp) : 0u;
-                        M[ra * pitch + col + 1 + t] = (S)ya;
-                        if (two) M[rb * pitch + col + 1 + t] = (S)yb;
-                        if (t == 0) {
+                        M[ra * pitch + c] = (S)ya;
+                        if (two) M[rb * pitch + c] = (S)yb;
+                        if (t == 0 && wave == 0) {
                             // keys of column col+1 over rows row+1.. for the next argmax
                             pre = ra > row ? K::make(ya, ra) : key_t(0);
                             if (two && rb > row) {
                                 const key_t kb = K::make(yb, rb);
                                 pre = kb > pre ? kb : pre;
                             }
-                            have_pre = true;
+                            if (NW > 1) *found = wave_max(pre);
                         }
                     }
                 }
-                wave_sync();
+                have_pre = true;
+                inst_sync<NW>();
             }
             ++row;
             ++col;
         }
         if (col >= pe || row >= m) {
-            flush<S, KB, ACC>(M, pitch, m, n, op, prow, row - prow, pe, pivcol, pivinv, mp);
+            flush<S, KB, ACC, NW>(M, pitch, m, n, op, prow, row - prow, pe, pivcol, pivinv, mp);
             prow = row;
             pe = col + KB < n ? col + KB : n;
         }
     }
-    if (!bad && !ended && prow < row) flush<S, KB, ACC>(M, pitch, m, n, op, prow, row - prow, pe, pivcol, pivinv, mp);
+    if (!bad && !ended && prow < row) flush<S, KB, ACC, NW>(M, pitch, m, n, op, prow, row - prow, pe, pivcol, pivinv, mp);
     const int rank = row;
     // outputs, column-major: lanes over rows write consecutive elements,
     // 16 columns of LDS reads before their stores; lanes past the last row
@@ -1443,7 +1494,7 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
         // first column of row r's U part (n: none)
         const int f0 = r0 < rank ? (op == MODP_ELIM_RREF ? 0 : (int)pivcol[r0]) : n;
         const int f1 = r1 < rank ? (op == MODP_ELIM_RREF ? 0 : (int)pivcol[r1]) : n;
-        for (int c0 = 0; c0 < n; c0 += 16) {
+        for (int c0 = 16 * wave; c0 < n; c0 += 16 * NW) {
             uint32_t x0[16], x1[16];
 #pragma unroll
             for (int t = 0; t < 16; ++t) {
@@ -1463,7 +1514,7 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
         // L: column k < rank holds the pivot value on the diagonal and the
         // multipliers (pivot column k) below it
         T *L = (T *)j.L;
-        for (int k0 = 0; k0 < m; k0 += 16) {
+        for (int k0 = 16 * wave; k0 < m; k0 += 16 * NW) {
             int pc[16];
             uint32_t pv[16], x0[16], x1[16];
 #pragma unroll
@@ -1492,7 +1543,7 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
     if (op == MODP_ELIM_LU) {
         // row permutation: the identity with the pivot swaps applied in order
         // (built in LDS, written by all lanes)
-        if (lane == 0) {
+        if (tid == 0) {
             for (int q = 0; q < m; ++q) perm[q] = (int16_t)q;
             for (int q = 0; q < rank; ++q) {
                 const int16_t t = perm[q];
@@ -1500,18 +1551,18 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
                 perm[ipiv[q]] = t;
             }
         }
-        wave_sync();
-        for (int q = lane; q < m; q += 64) j.row_info[q] = perm[q] + 1;
-        for (int q = lane; q < rank; q += 64) j.col_info[q] = pivcol[q] + 1;
+        inst_sync<NW>();
+        for (int q = tid; q < m; q += 64 * NW) j.row_info[q] = perm[q] + 1;
+        for (int q = tid; q < rank; q += 64 * NW) j.col_info[q] = pivcol[q] + 1;
     } else if (op == MODP_ELIM_RREF) {
-        for (int q = lane; q < rank; q += 64) j.row_info[q] = pivcol[q] + 1;
+        for (int q = tid; q < rank; q += 64 * NW) j.row_info[q] = pivcol[q] + 1;
     }
-    if (lane == 0) {
+    if (tid == 0) {
         j.counts[0] = op == MODP_ELIM_PLUQ ? nr : 0;
         j.counts[1] = op == MODP_ELIM_PLUQ ? nc : 0;
         j.counts[2] = bad ? -1 : rank;
     }
-    wave_sync();
+    inst_sync<NW>();
 }
 
 // Persistent kernel of one class: workgroup w (one wavefront) starts with
@@ -1520,44 +1571,58 @@ __device__ __forceinline__ void elim_instance(const EJob &j, int op, unsigned ch
 // class's queue as it finishes.  Taking the next index only after an
 // instance is done keeps a workgroup that starts early from claiming two
 // large instances while later workgroups are still being dispatched.
-template <typename T, int CLS>
-__global__ __launch_bounds__(64) void k_elim_wave(const EJob *__restrict__ jobs, int64_t njobs, int op,
-                                                  int *__restrict__ counter, int bk_off)
+template <typename T, int CLS, int NW>
+__global__ __launch_bounds__(64 * NW, CLS == 0 ? 4 : 3) void k_elim_wave(const EJob *__restrict__ jobs, int64_t njobs, int op,
+                                                       int *__restrict__ counter, int bk_off)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char esm[];
+    __shared__ uint64_t s_found;
+    __shared__ int s_next;
     int64_t it = blockIdx.x;
     while (it < njobs) {
         const EJob j = jobs[it];
-        if (CLS == 0) elim_instance<T, uint8_t, 8, 0>(j, op, esm, bk_off);
-        else if (CLS == 1) elim_instance<T, uint16_t, 8, 1>(j, op, esm, bk_off);
-        else elim_instance<T, uint32_t, 1, 1>(j, op, esm, bk_off);
+        if constexpr (CLS == 0) elim_instance<T, uint8_t, 8, 0, NW>(j, op, esm, bk_off, (uint32_t *)&s_found);
+        else if constexpr (CLS == 1) elim_instance<T, uint16_t, 8, 1, NW>(j, op, esm, bk_off, (uint32_t *)&s_found);
+        else elim_instance<T, uint32_t, 1, 1, NW>(j, op, esm, bk_off, &s_found);
         int next = 0;
         if (threadIdx.x == 0) next = atomicAdd(counter, 1);
+        if constexpr (NW > 1) {
+            if (threadIdx.x == 0) s_next = next;
+            __syncthreads();
+            next = s_next;  // (written again only after the next instance's barriers)
+        }
         it = (int64_t)gridDim.x + __builtin_amdgcn_readfirstlane(next);
     }
 }
 
-template <typename T, int CLS> hipError_t class_kernel(const modp_elim_plan *pl, hipStream_t st, bool allow)
+template <typename T, int CLS, int NW> hipError_t group_kernel(const modp_elim_plan *pl, int g, hipStream_t st, bool allow)
 {
-    const ElimClass &ec = pl->cls[CLS];
+    const ElimGroup &eg = pl->group[g];
     // the dynamic LDS can exceed the default 64 KiB (32-bit residues of
     // 128 x 128 instances)
     if (allow)
-        return hipFuncSetAttribute((const void *)k_elim_wave<T, CLS>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)ec.slot);
-    k_elim_wave<T, CLS><<<(unsigned)ec.grid, 64, ec.slot, st>>>(pl->djobs + ec.off, ec.count, pl->op,
-                                                                 pl->dcounter + 16 * CLS, ec.bk_off);
+        return hipFuncSetAttribute((const void *)k_elim_wave<T, CLS, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)eg.slot);
+    k_elim_wave<T, CLS, NW><<<(unsigned)eg.grid, 64 * NW, eg.slot, st>>>(pl->djobs + eg.off, eg.count, pl->op,
+                                                                         pl->dcounter + 16 * g, eg.bk_off);
     return hipGetLastError();
 }
 
-template <typename T> hipError_t class_launch(const modp_elim_plan *pl, int c, hipStream_t st, bool allow)
+template <typename T> hipError_t group_launch(const modp_elim_plan *pl, int g, hipStream_t st, bool allow)
 {
-    if (c == 0) return class_kernel<T, 0>(pl, st, allow);
-    if (c == 1) return class_kernel<T, 1>(pl, st, allow);
-    return class_kernel<T, 2>(pl, st, allow);
+    switch (g) {
+    case 0: return group_kernel<T, 0, 1>(pl, g, st, allow);
+    case 1: return group_kernel<T, 0, EWAVES>(pl, g, st, allow);
+    case 2: return group_kernel<T, 1, 1>(pl, g, st, allow);
+    case 3: return group_kernel<T, 1, EWAVES>(pl, g, st, allow);
+    default: return group_kernel<T, 2, 1>(pl, g, st, allow);
+    }
 }
 
-int elim_class(int64_t p) { return p < 256 ? 0 : (p < 65536 ? 1 : 2); }
+int elim_group(int64_t m, int64_t n, int64_t p)
+{
+    return p >= 65536 ? 4 : (p < 256 ? 0 : 2) + (m * n > EBIG ? 1 : 0);
+}
 
 // a row pitch of an odd number of 32-bit words, so the lanes of a column
 // walk hit distinct banks
@@ -1576,7 +1641,7 @@ int batched_elim_destroy(modp_ctx *ctx, modp_elim_plan *pl)
     (void)hipStreamSynchronize(ctx->stream);
     if (pl->exec) (void)hipGraphExecDestroy(pl->exec);
     if (pl->graph) (void)hipGraphDestroy(pl->graph);
-    for (int i = 0; i < ECLASS - 1; ++i) {
+    for (int i = 0; i < EGROUP - 1; ++i) {
         if (pl->join[i]) (void)hipEventDestroy(pl->join[i]);
         if (pl->side[i]) (void)hipStreamDestroy(pl->side[i]);
     }
@@ -1633,15 +1698,15 @@ int batched_elim_plan(modp_ctx *ctx, int op, int kind, const modp_elim_job *jobs
             e = hipMemcpyAsync(pl->dtab, htab.data(), htab.size() * sizeof(uint16_t), hipMemcpyHostToDevice,
                                ctx->stream);
     }
-    for (int c = 0; c < ECLASS; ++c) {
+    for (int g = 0; g < EGROUP; ++g) {
         std::vector<int64_t> order;
         for (int64_t i = 0; i < count; ++i)
-            if (elim_class(jobs[i].p) == c) order.push_back(i);
+            if (elim_group(jobs[i].m, jobs[i].n, jobs[i].p) == g) order.push_back(i);
         std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return cost(a) > cost(b); });
-        ElimClass &ec = pl->cls[c];
-        ec.off = (int64_t)hj.size();
-        ec.count = (int64_t)order.size();
-        const int eb = c == 0 ? 1 : (c == 1 ? 2 : 4);
+        ElimGroup &eg = pl->group[g];
+        eg.off = (int64_t)hj.size();
+        eg.count = (int64_t)order.size();
+        const int c = g / 2, eb = c == 0 ? 1 : (c == 1 ? 2 : 4);
         size_t mat_bytes = 16;
         for (int64_t oi : order) {
             const modp_elim_job &s = jobs[oi];
@@ -1657,36 +1722,36 @@ int batched_elim_plan(modp_ctx *ctx, int op, int kind, const modp_elim_job *jobs
             mat_bytes = std::max(mat_bytes, (size_t)d.m * (size_t)d.pitch * (size_t)eb);
             hj.push_back(d);
         }
-        ec.bk_off = (int)((mat_bytes + 15) & ~(size_t)15);
-        ec.slot = (size_t)ec.bk_off + EBOOK;
-        // persistent grid: as many single-wavefront workgroups as the LDS holds
+        eg.bk_off = (int)((mat_bytes + 15) & ~(size_t)15);
+        eg.slot = (size_t)eg.bk_off + EBOOK;
+        // persistent grid: as many workgroups as the LDS holds
         const size_t lds_cu = 160 * 1024;
-        int64_t per_cu = (int64_t)(lds_cu / ec.slot);
+        int64_t per_cu = (int64_t)(lds_cu / (eg.slot + 16));
         if (per_cu > 16) per_cu = 16;
         if (per_cu < 1) per_cu = 1;
-        const int64_t g = per_cu * ctx->num_cus;
-        ec.grid = (int)(g < ec.count ? g : ec.count);
+        const int64_t w = per_cu * ctx->num_cus;
+        eg.grid = (int)(w < eg.count ? w : eg.count);
     }
     if (e == hipSuccess) e = hipMalloc(&pl->djobs, sizeof(EJob) * (count > 0 ? count : 1));
-    if (e == hipSuccess) e = hipMalloc(&pl->dcounter, 256);
+    if (e == hipSuccess) e = hipMalloc(&pl->dcounter, 64 * EGROUP);
     if (e == hipSuccess && count > 0)
         e = hipMemcpyAsync(pl->djobs, hj.data(), sizeof(EJob) * count, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // hj is released on return
-    // classes with work, the one with the costliest instance (the longest
-    // single-wavefront latency) first: its workgroups are dispatched before
-    // the other classes fill the CUs' LDS
-    int act[ECLASS], na = 0;
-    int64_t top[ECLASS] = {0, 0, 0};
-    for (int c = 0; c < ECLASS; ++c) {
-        if (pl->cls[c].count == 0) continue;
-        const EJob &f = hj[(size_t)pl->cls[c].off];
-        top[c] = (int64_t)f.m * f.n * (f.m < f.n ? f.m : f.n) * (c == 2 ? 3 : (c == 1 ? 5 : 4));
-        act[na++] = c;
+    // groups with work, the one with the costliest instance (the longest
+    // latency) first: its workgroups are dispatched before the others fill
+    // the CUs' LDS
+    int act[EGROUP], na = 0;
+    int64_t top[EGROUP] = {};
+    for (int g = 0; g < EGROUP; ++g) {
+        if (pl->group[g].count == 0) continue;
+        const EJob &f = hj[(size_t)pl->group[g].off];
+        top[g] = (int64_t)f.m * f.n * (f.m < f.n ? f.m : f.n) * (g == 4 ? 3 : (g >= 2 ? 5 : 4));
+        act[na++] = g;
     }
     std::sort(act, act + na, [&](int x, int y) { return top[x] > top[y]; });
     for (int i = 0; i < na && e == hipSuccess; ++i)
-        e = kind == EK_F64 ? class_launch<double>(pl, act[i], ctx->stream, true)
-                           : class_launch<float>(pl, act[i], ctx->stream, true);
+        e = kind == EK_F64 ? group_launch<double>(pl, act[i], ctx->stream, true)
+                           : group_launch<float>(pl, act[i], ctx->stream, true);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&pl->fork, hipEventDisableTiming);
     for (int i = 0; i + 1 < na && e == hipSuccess; ++i) {
         e = hipStreamCreateWithFlags(&pl->side[i], hipStreamNonBlocking);
@@ -1699,14 +1764,14 @@ int batched_elim_plan(modp_ctx *ctx, int op, int kind, const modp_elim_job *jobs
         le = hipGetLastError();
         if (le == hipSuccess && na > 1) le = hipEventRecord(pl->fork, ctx->stream);
         if (le == hipSuccess && na > 0)
-            le = kind == EK_F64 ? class_launch<double>(pl, act[0], ctx->stream, false)
-                                : class_launch<float>(pl, act[0], ctx->stream, false);
+            le = kind == EK_F64 ? group_launch<double>(pl, act[0], ctx->stream, false)
+                                : group_launch<float>(pl, act[0], ctx->stream, false);
         for (int i = 1; i < na && le == hipSuccess; ++i) {
             hipStream_t st = pl->side[i - 1];
             le = hipStreamWaitEvent(st, pl->fork, 0);
             if (le == hipSuccess)
-                le = kind == EK_F64 ? class_launch<double>(pl, act[i], st, false)
-                                    : class_launch<float>(pl, act[i], st, false);
+                le = kind == EK_F64 ? group_launch<double>(pl, act[i], st, false)
+                                    : group_launch<float>(pl, act[i], st, false);
             if (le == hipSuccess) le = hipEventRecord(pl->join[i - 1], st);
         }
         for (int i = 1; i < na && le == hipSuccess; ++i) le = hipStreamWaitEvent(ctx->stream, pl->join[i - 1], 0);
