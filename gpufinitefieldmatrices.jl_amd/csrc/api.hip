@@ -245,11 +245,6 @@ int modp_ctx_destroy(modp_ctx *ctx)
     for (auto e : ctx->event_pool) (void)hipEventDestroy(e);
     for (auto e : ctx->slots)
         if (e) (void)hipEventDestroy(e);
-    for (int i = 0; i < modp_ctx::NSIDE; ++i) {
-        if (ctx->side[i]) (void)hipStreamDestroy(ctx->side[i]);
-        if (ctx->join_ev[i]) (void)hipEventDestroy(ctx->join_ev[i]);
-    }
-    if (ctx->fork_ev) (void)hipEventDestroy(ctx->fork_ev);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return MODP_OK;

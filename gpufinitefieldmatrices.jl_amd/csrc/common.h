@@ -268,12 +268,6 @@ struct modp_ctx {
     // autotuner: MODP_TUNE_OFF / _CACHED / _ON_MISS and its cache
     int tune_mode = 0;
     std::map<TuneKey, TuneEntry> tune_cache;
-    // side streams (default priority) and fork/join events for independent
-    // small launches; created on first use
-    static constexpr int NSIDE = 8;
-    hipStream_t side[NSIDE] = {nullptr};
-    hipEvent_t fork_ev = nullptr;
-    hipEvent_t join_ev[NSIDE] = {nullptr};
     // device address of the library's static scratch array on this
     // context's device (modp_gemm_noalloc), and a flag set while such a call
     // runs (no timing events are taken then)
@@ -360,6 +354,13 @@ struct GemmArgs {
 // heuristic configurations (gemm.hip)
 int gemm_plain_f64(modp_ctx *ctx, const GemmArgs &g);
 int gemm_limb_i8(modp_ctx *ctx, const GemmArgs &g);
+// `count` small products (blocks of 16 x 16, int32 operands) of g's size in one
+// launch, product i at A + i sa, B + i sb, C + i sc; the last may be smaller
+struct GemmSize {
+    int64_t m, n, k;
+};
+int gemm_small_strided(modp_ctx *ctx, const GemmArgs &g, int64_t count, int64_t sa, int64_t sb, int64_t sc,
+                       const GemmSize &last);
 int gemm_rns_i8(modp_ctx *ctx, const GemmArgs &g);
 // the limb form with its digit planes in a caller's workspace (no allocation,
 // one K slice); gemm_limb_scratch_bytes is the workspace that product needs

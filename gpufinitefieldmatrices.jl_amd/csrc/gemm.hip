@@ -51,18 +51,29 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64(int64_t m, int64_t n, int64
 // straight from the operands (16 runs of 16 rows of A, 16 columns of B), all
 // before it uses one.  The block is computed transposed, so a lane holds one
 // row.  48 x 40 x 56 mod 11: 8.6 -> 3.5 us (64 x 64 tiles in stages of 16 k).
+// blockIdx.y: products at the strides sa, sb and sc, the last of its own size.
 template <typename T, typename TC, int EPI>
 __global__ __launch_bounds__(256) void k_gemm_f64_small(int64_t m, int64_t n, int64_t k, const T *__restrict__ A,
                                                         int64_t lda, const T *__restrict__ B, int64_t ldb,
                                                         TC *__restrict__ C, int64_t ldc, ModP mp, int R,
+                                                        int64_t sa, int64_t sb, int64_t sc, GemmSize last,
                                                         const int *__restrict__ skip)
 {
     if (skip && *skip) return;
+    A += blockIdx.y * sa;
+    B += blockIdx.y * sb;
+    C += blockIdx.y * sc;
+    if (blockIdx.y + 1 == gridDim.y) {
+        m = last.m;
+        n = last.n;
+        k = last.k;
+    }
     constexpr int U = 8;
     __shared__ double part[4][16][17];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t mt = (m + 15) / 16;
     const int64_t r0 = (blockIdx.x % mt) * 16, c0 = (blockIdx.x / mt) * 16;
+    if (c0 >= n) return;
     const int64_t kq = (k + 15) / 16 * 4;  // a wave's share of K, in whole k4-steps
     const int64_t kbeg = wave * kq, kend = min(k, kbeg + kq);
     const int64_t row = r0 + (lane & 15), col = c0 + (lane & 15);
@@ -335,14 +346,15 @@ bool f64_small(const GemmArgs &g)
     return w >= 0 && w <= 262144 && g.ka == g.kb && g.ka == g.kc &&
            (g.epi == EPI_STORE || (g.epi == EPI_SUB && g.kc == EK_I32));
 }
-int launch_f64_small(modp_ctx *ctx, const GemmArgs &g, int R)
+int launch_f64_small(modp_ctx *ctx, const GemmArgs &g, int R, int64_t count, int64_t sa, int64_t sb, int64_t sc,
+                     const GemmSize &last)
 {
     TimedLaunch tl(ctx, "gemm_f64");
     const unsigned grid = (unsigned)(((g.m + 15) / 16) * ((g.n + 15) / 16));
 #define SMALL(T_, EPI_)                                                                                             \
-    k_gemm_f64_small<T_, T_, EPI_><<<grid, 256, 0, ctx->stream>>>(g.m, g.n, g.k, (const T_ *)g.A, g.lda,             \
+    k_gemm_f64_small<T_, T_, EPI_><<<dim3(grid, (unsigned)count), 256, 0, ctx->stream>>>(g.m, g.n, g.k, (const T_ *)g.A, g.lda,             \
                                                                   (const T_ *)g.B, g.ldb, (T_ *)g.C, g.ldc, g.mp, R, \
-                                                                  g.skip)
+                                                                  sa, sb, sc, last, g.skip)
     if (g.ka == EK_F64) SMALL(double, EPI_STORE);
     else if (g.ka == EK_F32) SMALL(float, EPI_STORE);
     else if (g.epi == EPI_STORE) SMALL(int32_t, EPI_STORE);
@@ -436,7 +448,7 @@ int gemm_plain_cfg(modp_ctx *ctx, const GemmArgs &g, const GemmConfig &cfg)
     if (g.m <= 0 || g.n <= 0) return MODP_OK;
     const int R = f64_reduce_interval(g.mp.p);
     if (R < 1) return set_error(ctx, MODP_ERR_MODULUS_RANGE, "modulus %lld too large for the FP64 form", (long long)g.mp.p);
-    if (f64_small(g)) return launch_f64_small(ctx, g, R);
+    if (f64_small(g)) return launch_f64_small(ctx, g, R, 1, 0, 0, 0, GemmSize{g.m, g.n, g.k});
     const int tile = cfg.tile_m == 128 ? 128 : 64;
     Slices sl = make_slices(g.k, cfg.ksplit, PBK, 64);
     if (sl.S == 1) {
@@ -660,6 +672,12 @@ int gemm_run(modp_ctx *ctx, const GemmArgs &g, const GemmConfig &cfg)
 int gemm_plain_f64(modp_ctx *ctx, const GemmArgs &g)
 {
     return gemm_plain_cfg(ctx, g, gemm_default_config(ctx, g, MODP_FORM_PLAIN_F64));
+}
+
+int gemm_small_strided(modp_ctx *ctx, const GemmArgs &g, int64_t count, int64_t sa, int64_t sb, int64_t sc,
+                       const GemmSize &last)
+{
+    return launch_f64_small(ctx, g, f64_reduce_interval(g.mp.p), count, sa, sb, sc, last);
 }
 
 int gemm_limb_i8(modp_ctx *ctx, const GemmArgs &g)
