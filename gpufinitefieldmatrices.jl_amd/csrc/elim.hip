@@ -475,18 +475,23 @@ __global__ __launch_bounds__(NBO) void k_block_solve(const int32_t *__restrict__
                                                      PanelSolve *__restrict__ solve, const int *__restrict__ skip)
 {
     if (skip && *skip) return;
-    __shared__ uint32_t s_x[NBO][PNW + 1];
+    __shared__ double s_l[NBO][PNW + 1], s_x[NBO][PNW + 1], s_inv[NBO];
     const int tid = threadIdx.x, b0 = tid / PNW * PNW, q = tid % PNW;
+    // the rows of the triangles (row b0 + t, pivot q), all loads before the first use
+    int32_t l[PNW];
+    const int64_t lc = (int64_t)pivcol[KR + min(b0 + q, P - 1)] * ldw;
+#pragma unroll
+    for (int t = 0; t < PNW; ++t) l[t] = W[KR + min(b0 + t, P - 1) + lc];
+    s_inv[tid] = balanced(pivinv[KR + min(tid, P - 1)], mp);
+#pragma unroll
+    for (int t = 0; t < PNW; ++t) s_l[b0 + t][q] = balanced(l[t], mp);
+    __syncthreads();
     for (int t = 0; t < PNW; ++t) {
-        uint32_t x = 0;
-        if (b0 + t < P && t >= q) {
-            x = t == q ? 1u : 0u;
-            for (int k = q; k < t; ++k)
-                x = submod(x, mulmod((uint32_t)W[KR + b0 + t + (int64_t)pivcol[KR + b0 + k] * ldw], s_x[tid][k], mp), mp);
-            x = mulmod(x, (uint32_t)pivinv[KR + b0 + t], mp);
-        }
+        double x = t == q ? 1.0 : 0.0;
+        for (int k = q; k < t; ++k) x = near_mod(fma(-s_l[b0 + t][k], s_x[tid][k], x), mp);
+        x = b0 + t < P && t >= q ? near_mod(x * s_inv[b0 + t], mp) : 0.0;
         s_x[tid][t] = x;
-        solve[tid / PNW].t[t][q] = (int)x > mp.half ? (int32_t)x - (int32_t)mp.p : (int32_t)x;
+        solve[tid / PNW].t[t][q] = (int32_t)x;
     }
 }
 
@@ -684,12 +689,16 @@ __global__ void k_gather_cols(const int32_t *__restrict__ W, int64_t ldw, int64_
 }
 
 // Back substitution with a unit upper triangular T (nb x nb, gathered into
-// G) on rows [i0, i0+nb) of columns [cs, n): one wave per column.
+// G) on rows [i0, i0+nb) of columns [cs, n): one wave per column, bound by the
+// chain of its 63 steps: the solved row goes to all lanes by readlane, one FMA
+// and a rounded quotient bring every other row up to date, still balanced.
+// Mean over the blocks of a 4096^2 RREF of rank 3000 mod 65521 8.8 us (13.8 with
+// integer residues and their canonical reductions).
 __global__ __launch_bounds__(256) void k_trsm_upper_unit(int32_t *__restrict__ W, int64_t ldw, int64_t n, int i0,
                                                          int nb, int64_t cs, const int32_t *__restrict__ G,
                                                          int64_t ldg, ModP mp)
 {
-    __shared__ uint32_t Ts[64][65];
+    __shared__ double Ts[64][65];  // negated, by column
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     {
         // every load issued before the first LDS store
@@ -703,18 +712,15 @@ __global__ __launch_bounds__(256) void k_trsm_upper_unit(int32_t *__restrict__ W
 #pragma unroll
         for (int k = 0; k < TPT; ++k) {
             const int idx = tid + 256 * k, i = idx % 64, j = idx / 64;
-            Ts[i][j] = (i < nb && j < nb) ? (uint32_t)tv[k] : 0u;
+            Ts[j][i] = i < j && j < nb ? -balanced(tv[k], mp) : 0.0;
         }
     }
     __syncthreads();
     for (int64_t c = cs + (int64_t)blockIdx.x * 4 + wave; c < n; c += (int64_t)gridDim.x * 4) {
         int32_t *col = W + c * ldw + i0;
-        uint32_t x = lane < nb ? (uint32_t)col[lane] : 0u;
-        for (int j = nb - 1; j > 0; --j) {
-            const uint32_t xj = (uint32_t)__builtin_amdgcn_readlane((int)x, j);
-            if (lane < j) x = submod(x, mulmod(Ts[lane][j], xj, mp), mp);
-        }
-        if (lane < nb) col[lane] = (int32_t)x;
+        double x = lane < nb ? balanced(col[lane], mp) : 0.0;
+        for (int j = nb - 1; j > 0; --j) x = near_mod(fma(Ts[j][lane], readlane_f64(x, j), x), mp);
+        if (lane < nb) col[lane] = (int32_t)from_near(x, mp);
     }
 }
 
