@@ -263,6 +263,7 @@ struct modp_ctx {
     // table of small modular inverses for the current elimination modulus
     uint32_t *invtab = nullptr;
     int64_t invtab_p = 0;
+    bool invtab_prime = false;
     // steps of the elimination panels so far (64 a panel): their exchange tags
     uint32_t panel_tag = 0;
     // autotuner: MODP_TUNE_OFF / _CACHED / _ON_MISS and its cache
@@ -412,7 +413,7 @@ int util_crt2(modp_ctx *ctx, int kind, int64_t rows, int64_t cols, const void *X
               const void *X2, int64_t ld2, int64_t p2, void *Y, int64_t ldy);
 
 // elimination driver (elim.hip)
-enum ElimMode { ELIM_PLUQ = 0, ELIM_LU = 1, ELIM_RREF = 2 };
+enum ElimMode { ELIM_PLUQ = 0, ELIM_LU = 1, ELIM_RREF = 2, ELIM_INVERSE = 3 };
 struct ElimResult {
     std::vector<int64_t> row_swaps, col_swaps, perm, pivcols;
     int64_t rank = 0;
@@ -422,9 +423,14 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n,
              int64_t p, ElimResult &res);
 int elim_rref(modp_ctx *ctx, int form, int kind, int64_t m, int64_t n, const void *A, int64_t lda, void *R,
               int64_t ldr, int64_t p, ElimResult &res);
+// *taken = 0: not a prime modulus, nothing done
+int elim_inverse(modp_ctx *ctx, int form, int kind, int64_t n, const void *A, int64_t lda, void *Ainv, int64_t ldai,
+                 int64_t p, int *invertible, int *taken);
 
 // inverses (trinv.hip)
 int tri_inverse(modp_ctx *ctx, int kind, int upper, int64_t m, int64_t n, const void *A, int64_t lda, void *Ainv,
                 int64_t ldai, int64_t p);
+int trinv_i32(modp_ctx *ctx, bool upper, const int32_t *T, int64_t ldt, int32_t *X, int64_t ldx, int64_t k,
+              const ModP &mp);
 int mat_inverse(modp_ctx *ctx, int form, int kind, int64_t n, const void *A, int64_t lda, void *Ainv, int64_t ldai,
                 int64_t p, int *invertible);

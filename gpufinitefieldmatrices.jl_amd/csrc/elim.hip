@@ -597,7 +597,7 @@ __global__ __launch_bounds__(64) void k_block_finish(int32_t *__restrict__ W, in
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
 #pragma unroll
-            for (int b = 0; b <= a; ++b)
+            for (int b = 0; b < 2; ++b)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     r[a] = after_step<EVERY>(mfma_f64((double)solve[i].t[16 * a + cl][16 * b + 4 * e + g], s[b][e], r[a]), mp);
@@ -745,6 +745,14 @@ __global__ void k_blocks_begin(int *abort, int *cursor, int row, uint32_t *arriv
     if (i < n) arrive[i] = 0;
 }
 
+// the identity, with the rows of padding
+__global__ void k_identity(int32_t *__restrict__ W, int64_t ldw, int64_t n)
+{
+    const int64_t total = ldw * n;
+    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x)
+        W[e] = e % ldw == e / ldw;
+}
+
 // t[a] = a^{-1} mod p for a < n, 0 where there is none
 __global__ void k_inv_table(uint32_t *__restrict__ t, int n, ModP mp)
 {
@@ -758,6 +766,8 @@ __global__ void k_inv_table(uint32_t *__restrict__ t, int n, ModP mp)
 const uint32_t *inverse_table(modp_ctx *ctx, const ModP &mp, int *st)
 {
     if (ctx->invtab && ctx->invtab_p == mp.p) return ctx->invtab;
+    ctx->invtab_prime = mp.p >= 2;
+    for (int64_t q = 2; q * q <= mp.p && ctx->invtab_prime; q += q == 2 ? 1 : 2) ctx->invtab_prime = mp.p % q != 0;
     if (!ctx->invtab) {
         hipError_t e = hipMalloc(&ctx->invtab, sizeof(uint32_t) * PINV);
         if (e != hipSuccess) { *st = hip_check(ctx, e, "inverse table"); return nullptr; }
@@ -777,6 +787,8 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     const ModP mp = make_modp(p);
     const bool ple = mode != ELIM_PLUQ;
     const int64_t mn = m < n ? m : n;
+    // ELIM_INVERSE: an identity right of the pivot columns
+    const int64_t nt = mode == ELIM_INVERSE ? n + m : n;
     res = ElimResult();
     if (m <= 0 || n <= 0) {
         if (mode == ELIM_LU)
@@ -808,7 +820,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
 
     int st = MODP_OK;
     const int64_t ldw = rup(m, 64);
-    int32_t *W = (int32_t *)ws_get(ctx, WS_WORK, sizeof(int32_t) * (size_t)ldw * (size_t)n, &st);
+    int32_t *W = (int32_t *)ws_get(ctx, WS_WORK, sizeof(int32_t) * (size_t)ldw * (size_t)nt, &st);
     if (!W) return st;
     // pivot arrays, per-panel control blocks and row gather maps of one outer block
     const size_t npv = (size_t)mn + 64;
@@ -827,7 +839,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     int32_t *stage = (int32_t *)(arrive + NBATCH * MAXPAN);  // moved rows' old values, 64 x NBO
     PanelSolve *solve = (PanelSolve *)(stage + 64 * NBO);  // one per panel of the block
     BlockMoves *moves = (BlockMoves *)(solve + MAXPAN);
-    int32_t *Ubig = (int32_t *)ws_get(ctx, WS_UBUF, sizeof(int32_t) * (size_t)NBO * (size_t)(n + 1), &st);
+    int32_t *Ubig = (int32_t *)ws_get(ctx, WS_UBUF, sizeof(int32_t) * (size_t)NBO * (size_t)(nt + 1), &st);
     if (!Ubig) return st;
     // row positions of the W-resident panel (position of each row, row at
     // each position)
@@ -841,8 +853,18 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     if (!hctl) return st;
 
     MODP_TRY(util_convert(ctx, kind, m, n, A, lda, EK_I32, W, ldw, mp));
+    if (nt > n) {
+        k_identity<<<grid_for(ldw * m, 4096), 256, 0, ctx->stream>>>(W + n * ldw, ldw, m);
+        HIP_TRY(ctx, hipGetLastError());
+    }
     const uint32_t *invs = inverse_table(ctx, mp, &st);
     if (st != MODP_OK) return st;
+    // Where the result does not depend on the pivots, the panels may take any
+    // (k_panel_any): 15 us a panel against 37 to 53.  Not for a composite
+    // modulus, where a pivot without inverse is an error that depends on which
+    // one is taken.
+    const bool any_pivot = (mode == ELIM_RREF || mode == ELIM_INVERSE) && !force_global && ctx->invtab_prime;
+    bool local_moves = true;  // every row moved so far stayed within 64 rows
     // exchange area of the panels on one XCD: its words are recognised by
     // tags that count the context's panels, so old ones are cleared only when
     // the 17 bits of a key's tag (the 31 of a row's) have been through
@@ -862,6 +884,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         return MODP_OK;
     };
 
+    const int64_t pivot_cols = n;
     auto gemm_sub = [&](int64_t r0, int64_t rows, int64_t ca, int64_t cols, int64_t kcol, int64_t K,
                         const int32_t *Ub, const int *skip) -> int {
         if (rows <= 0 || cols <= 0 || K <= 0) return MODP_OK;
@@ -876,6 +899,16 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         const int use_form = form != MODP_FORM_AUTO ? form : choose_form(rows, cols, K, p);
         if (use_form == MODP_FORM_LIMB_I8) return gemm_limb_i8(ctx, g);
         return gemm_plain_f64(ctx, g);
+    };
+    auto launch_panel_any = [&](int blk, int t, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w) -> int {
+        PanelAnyArgs a = {};
+        a.W = W; a.ldw = ldw; a.m = (int)m; a.kr0 = (int)rj; a.c0 = (int)cj; a.w = (int)w;
+        a.KC = (int)KC; a.FAR = (int)FAR; a.mp = mp; a.invs = invs;
+        a.ipiv = ipiv; a.pivcol = pivcol; a.map_dst = bmap_dst + t * 64; a.map_src = bmap_src + t * 64;
+        a.stage = stage; a.ctl = bctl + blk * MAXPAN + t; a.solve = solve + t; a.abort = abort_flag;
+        TimedLaunch tl(ctx, "elim_panel");
+        k_panel_any<<<1, 64 * PWAVES, 0, ctx->stream>>>(a);
+        return hip_check(ctx, hipGetLastError(), "k_panel_any launch");
     };
     // panel t of block blk of the batch at (rj, cj), width w; it has at most
     // m - rj rows
@@ -933,7 +966,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     auto update_t = [&](int blk, int t, bool known, int64_t KR, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w,
                         const int *skip) -> int {
         const int64_t nl = cj - KC, nr = FAR - (cj + w);
-        if (nl + nr + (n - (FAR - KC)) == 0) return MODP_OK;
+        if (nl + nr + (nt - (FAR - KC)) == 0) return MODP_OK;
         const int64_t tiles = ((m - rj + UT_R - 1) / UT_R) * ((nr + UT_C - 1) / UT_C);
         const unsigned grid = (unsigned)(1 + (nl + UT_L - 1) / UT_L + tiles);
         const int kr0 = known ? (int)rj : -1;
@@ -954,6 +987,9 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     auto block_end = [&](int64_t KR, int64_t KC, int64_t FAR, int64_t P, int64_t consumed, int width,
                          const int *skip) -> int {
         if (P <= 0) return MODP_OK;
+        // columns of the identity that have not met a pivot row yet are left
+        // out: while rows move within 64, those from KR + NBO + 64 on
+        const int64_t n = mode == ELIM_INVERSE && local_moves ? pivot_cols + std::min(m, KR + NBO + 64) : nt;
         const int64_t gleft = L ? (KC + 15) / 16 : 0, grid = gleft + (n - FAR + 15) / 16;
         if (grid > 0) {
             const bool dense = width == PNW && P == consumed, every = mp.p > ((int64_t)1 << 24);
@@ -1009,17 +1045,21 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         std::vector<int64_t> rj, cj, w;
     };
     int batch = NBATCH;
+    // after a panel that found no pivot among its 64 rows the general panels
+    // take `hold` blocks, twice as many each time
+    int hold = 0, next_hold = 1;
     while (!done && kr < m && kc < n) {
         std::vector<Block> blocks;
+        const bool any = any_pivot && hold == 0;
         {
             int64_t r = kr, c = kc;
-            while ((int)blocks.size() < batch && !careful && r < m) {
+            while ((int)blocks.size() < (hold > 0 ? std::min(hold, batch) : batch) && !careful && r < m) {
                 const int64_t colend = ple ? n : last + 1;  // columns usable as pivot columns
-                const int64_t nbo = std::min<int64_t>(colend - c, NBO);
+                const int64_t nbo = std::min<int64_t>(std::min<int64_t>(colend - c, NBO), any ? m - r : NBO);
                 if (nbo <= 0 || (ple && r + nbo > m)) break;
                 Block b;
                 b.KR = r; b.KC = c; b.FAR = c + nbo; b.P = 0;
-                b.width = panel_width(r);
+                b.width = any ? PNW : panel_width(r);
                 for (int64_t cj = c; cj < b.FAR && r + b.P < m;) {
                     const int64_t w = std::min(std::min<int64_t>(b.width, b.FAR - cj), m - (r + b.P));
                     b.rj.push_back(r + b.P); b.cj.push_back(cj); b.w.push_back(w);
@@ -1029,18 +1069,23 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 r += b.P;
                 c += b.P;
                 blocks.push_back(b);
-                if (gave_up) break;
+                if (gave_up && !any) break;
             }
         }
         bool stop_zero = false;
         int64_t nbo = 0;
         if (!blocks.empty()) {
             MODP_TRY(blocks_begin(kr, (int)blocks.size()));
+            if (!any) {
+                local_moves = false;
+                hold -= std::min(hold, (int)blocks.size());
+            }
             for (int i = 0; i < (int)blocks.size(); ++i) {
                 const Block &b = blocks[i];
                 for (int t = 0; t < (int)b.w.size(); ++t) {
-                    MODP_TRY(launch_panel_t(b.width, i, t, b.KC, b.FAR, b.rj[t], b.cj[t], b.w[t], abort_flag, nullptr,
-                                            true));
+                    if (any) MODP_TRY(launch_panel_any(i, t, b.KC, b.FAR, b.rj[t], b.cj[t], b.w[t]));
+                    else MODP_TRY(launch_panel_t(b.width, i, t, b.KC, b.FAR, b.rj[t], b.cj[t], b.w[t], abort_flag,
+                                                 nullptr, true));
                     MODP_TRY(update_t(i, t, true, b.KR, b.KC, b.FAR, b.rj[t], b.cj[t], b.w[t], abort_flag));
                 }
                 MODP_TRY(block_end(b.KR, b.KC, b.FAR, b.P, b.P, b.width, abort_flag));
@@ -1081,6 +1126,10 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 nbo = b.FAR - b.KC;
                 stop_zero = pc.status == 1;
                 batch = 1;
+                if (pc.status == 7) {
+                    hold = next_hold;
+                    next_hold = std::min(2 * next_hold, 64);
+                }
                 if (P < consumed) {
                     careful = true;
                     MODP_TRY(rest_is_zero());
@@ -1098,6 +1147,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             const int64_t KR = kr, KC = kc, FAR = KC + std::min<int64_t>(n - KC, NBO);
             const int NBW = panel_width(KR);
             gave_up = false;
+            local_moves = false;
             nbo = FAR - KC;
             MODP_TRY(blocks_begin(KR, 1));
             std::vector<int64_t> pcj, pw;
@@ -1159,6 +1209,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             }
         }
         if (ple && kr >= m) break;
+        if (mode == ELIM_INVERSE && kr < kc) break;  // singular
     }
     const int64_t rank = kr;
 
@@ -1196,6 +1247,36 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         for (int64_t i = 0; i < rank; ++i) std::swap(res.perm[i], res.perm[hp[i]]);
     }
     return MODP_OK;
+}
+
+// Inverse under a prime modulus: [A | I] to [U | Y] with any pivots, then
+// A^{-1} = U^{-1} Y.  U is unit upper triangular, and no row order has to be undone.
+int elim_inverse(modp_ctx *ctx, int form, int kind, int64_t n, const void *A, int64_t lda, void *Ainv, int64_t ldai,
+                 int64_t p, int *invertible, int *taken)
+{
+    const ModP mp = make_modp(p);
+    int st = MODP_OK;
+    inverse_table(ctx, mp, &st);
+    if (st != MODP_OK || !ctx->invtab_prime) return st;
+    *taken = 1;
+    ElimResult r;
+    MODP_TRY(elim_run(ctx, ELIM_INVERSE, form, kind, n, n, A, lda, nullptr, 0, nullptr, 0, p, r));
+    if (r.rank < n) return MODP_OK;
+    *invertible = 1;
+    const int64_t ld = rup(n, 64);
+    int32_t *W = (int32_t *)ws_get(ctx, WS_WORK, sizeof(int32_t) * (size_t)ld * (size_t)(2 * n), &st);
+    if (!W) return st;
+    int32_t *X = (int32_t *)ws_get(ctx, WS_TRI_X, sizeof(int32_t) * (size_t)ld * (size_t)n, &st);
+    if (!X) return st;
+    MODP_TRY(trinv_i32(ctx, true, W, ld, X, ld, n, mp));
+    GemmArgs g;
+    g.m = n; g.n = n; g.k = n;
+    g.A = X; g.lda = ld; g.ka = EK_I32;
+    g.B = W + n * ld; g.ldb = ld; g.kb = EK_I32;
+    g.C = Ainv; g.ldc = ldai; g.kc = kind;
+    g.epi = EPI_STORE;
+    g.mp = mp;
+    return gemm_run(ctx, g, gemm_default_config(ctx, g, form));
 }
 
 // Back-elimination of a PLE-reduced working array into RREF: row blocks of

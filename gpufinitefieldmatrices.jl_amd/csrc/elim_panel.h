@@ -87,7 +87,8 @@ struct PanelCtl {
     int status;  // 0 all columns consumed, 1 zero column (pluq stop),
                  // 2 rows exhausted, 3 pivot not invertible, 4 not run (an
                  // earlier panel stopped), 5 not run (its workgroups did not
-                 // meet on one XCD), 6 an exchange did not end
+                 // meet on one XCD), 6 an exchange did not end, 7 not run
+                 // (no pivot among the first rows, k_panel_any)
     int ncols;   // panel columns consumed
     int nmap;    // entries of the row gather map
     int kr0;     // first row of the panel
@@ -766,6 +767,167 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
         *a.ctl = PanelCtl{pc, status, consumed, pc + (int)__popc(mask), kr0};
         if (a.cursor) *a.cursor = kr0 + pc;
         if (a.abort && (status != 0 || (a.strict && pc < w))) *a.abort = 1;
+    }
+}
+
+// Panel of a reduction whose result does not depend on the pivots (reduced
+// echelon form and inverse, prime modulus): any nonzero entry will do, so the
+// first 64 rows are enough and no other row is looked at.  One workgroup, a
+// row per lane, eight columns per wave, Gauss-Jordan in place without
+// divisions: every row but the pivot's becomes V row - m (pivot row), and the
+// column is replaced by the identity's, so what is left is A11^{-1} of the
+// pivot rows up to a factor per row, whose inverses are taken at the end, all
+// at once.  A11^{-1} serves as T and the panel's columns stay as they are: the
+// updates subtract A21 (A11^{-1} A12) instead of L21 U12 with L21 = A21 U11^{-1},
+// so rows below are never touched here.  The panel's part of U is the identity.
+//
+// It is bound by its chain: per column one LDS word a row, a barrier, and 40
+// FP64 instructions; the next column is updated and passed on before the
+// others.  A 32-column panel takes 15 us mod 65521 and 16 us mod
+// 2^26 - 5, whatever its rows, against 44 and 53 of the general panel over an XCD:
+// RREF of 4096^2 and rank 3000 8.2 -> 5.1 ms, and with the identity beside the
+// matrix in place of L^{-1}, inverse of 1500^2 mod 2^26 - 5 4.0 -> 1.94 ms.
+// A column without a nonzero entry among the 64 rows says nothing about the rows
+// below: status 7, nothing written, and the general panel takes the block.
+struct PanelAnyArgs {
+    int32_t *W;
+    int64_t ldw;
+    int m, kr0, c0, w, KC, FAR;
+    ModP mp;
+    const uint32_t *invs;
+    int32_t *ipiv, *pivcol, *map_dst, *map_src, *stage;
+    PanelCtl *ctl;
+    PanelSolve *solve;
+    int *abort;
+};
+constexpr int PAC = PNW / PWAVES;               // panel columns of a wave
+constexpr int PAO = (128 - PNW) / PWAVES;       // other columns of the block, at most
+
+__global__ __launch_bounds__(64 * PWAVES) void k_panel_any(PanelAnyArgs a)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
+    if (*a.abort) {
+        if (tid == 0) *a.ctl = PanelCtl{0, 4, 0, 0, a.kr0};
+        return;
+    }
+    __shared__ double s_col[2][64];
+    __shared__ int s_vac[64];
+    const ModP mp = a.mp;
+    const int w = a.w, kr0 = a.kr0;
+    const bool exists = kr0 + lane < a.m;
+    const int64_t ldw = a.ldw;
+    const uint32_t r = (uint32_t)min(kr0 + lane, a.m - 1);
+    const int nleft = a.c0 - a.KC, nother = (a.FAR - a.KC) - w;
+    int32_t x[PAC], o[PAO];
+#pragma unroll
+    for (int k = 0; k < PAC; ++k) x[k] = a.W[r + (int64_t)(a.c0 + min(PAC * wave + k, w - 1)) * ldw];
+    // the old values of the other columns, for the stage
+    if (nother > 0)
+#pragma unroll
+        for (int k = 0; k < PAO; ++k) {
+            const int c = min(PAO * wave + k, nother - 1);
+            o[k] = a.W[r + (int64_t)(c < nleft ? a.KC + c : a.KC + c + w) * ldw];
+        }
+    double v[PAC];
+#pragma unroll
+    for (int k = 0; k < PAC; ++k) v[k] = (double)(x[k] > mp.half ? x[k] - (int32_t)mp.p : x[k]);
+    uint64_t cand = __ballot(exists);  // rows that are not pivots
+    int pk = -1;                       // pivot that this row is
+    double d = 1.0, S = 1.0;           // the factor of this row; of the rows that are no pivots yet
+    if (wave == 0) s_col[0][lane] = v[0];
+    __syncthreads();
+    int done = 0;
+    for (int ow = 0; ow < PWAVES; ++ow) {
+        auto step = [&](auto SC) __attribute__((always_inline)) {
+            constexpr int s = decltype(SC)::value, nx = (s + 1) % PAC;
+            const int jc = PAC * ow + s;
+            if (done != jc || jc >= w) return;  // uniform over the workgroup
+            const double mult = s_col[s & 1][lane];
+            const uint64_t at = __ballot(mult != 0.0) & cand;
+            if (at == 0) return;
+            const int l = (int)__builtin_ctzll(at);
+            cand &= ~(1ull << l);
+            const bool pivot = lane == l;
+            const double V = readlane_f64(mult, l);
+            if (wave == ow) v[s] = pivot ? S : 0.0;
+            // products of balanced residues below 2^50 + 2^30, their difference below 2^52
+            const double f = pivot ? 1.0 : V, g = pivot ? 0.0 : -mult;
+            auto one = [&](int k) __attribute__((always_inline)) {
+                v[k] = near_mod(fma(g, readlane_f64(v[k], l), f * v[k]), mp);
+            };
+            one(nx);
+            if (wave == (s + 1 == PAC ? ow + 1 : ow)) s_col[(s + 1) & 1][lane] = v[nx];
+#pragma unroll
+            for (int k = 0; k < PAC; ++k)
+                if (k != nx) one(k);
+            d = pivot ? V : near_mod(d * V, mp);
+            S = near_mod(S * V, mp);
+            pk = pivot ? jc : pk;
+            done = jc + 1;
+            __syncthreads();
+        };
+        Unroll<0, PAC>::run(step);
+    }
+    if (done < w) {
+        if (tid == 0) {
+            *a.ctl = PanelCtl{0, 7, 0, 0, kr0};
+            *a.abort = 1;
+        }
+        return;
+    }
+    // 1/d: from the table, or d^(p-2)
+    double inv;
+    {
+        const uint32_t dr = (uint32_t)from_near(pk >= 0 ? d : 1.0, mp);
+        if (mp.p <= PINV) {
+            inv = (double)a.invs[dr];
+        } else {
+            double b = pk >= 0 ? d : 1.0;
+            inv = 1.0;
+            for (uint32_t e = mp.p32 - 2; e != 0; e >>= 1) {
+                if (e & 1) inv = near_mod(inv * b, mp);
+                b = near_mod(b * b, mp);
+            }
+        }
+        inv = to_near(from_near(inv, mp), mp);
+    }
+    for (int i = tid; i < PNW * PNW; i += 64 * PWAVES)
+        if (i / PNW >= w) a.solve->t[i / PNW][i % PNW] = 0;
+    if (pk >= 0)
+#pragma unroll
+        for (int k = 0; k < PAC; ++k)
+            a.solve->t[pk][PAC * wave + k] = PAC * wave + k < w ? (int32_t)near_mod(v[k] * inv, mp) : 0;
+    // the pivots go to the first w rows, the rows there that are none to the
+    // pivots' places
+    const bool vacated = pk >= 0 && lane >= w, moves = pk < 0 && lane < w;
+    const uint64_t below = (1ull << lane) - 1, mask = __ballot(moves);
+    const int rank_v = (int)__popcll(__ballot(vacated) & below), rank_m = (int)__popcll(mask & below);
+    if (wave == 0 && vacated) s_vac[rank_v] = lane;
+    __syncthreads();
+    const int pos = pk >= 0 ? pk : moves ? s_vac[rank_m] : lane;
+    const int e = pk >= 0 ? pk : w + rank_m;
+    const bool moved = pk >= 0 || moves;
+    if (moved) {
+#pragma unroll
+        for (int k = 0; k < PAC; ++k) {
+            const int j = PAC * wave + k;
+            if (j < w) a.W[kr0 + pos + (int64_t)(a.c0 + j) * ldw] = pk >= 0 ? (j == pk ? 1 : 0) : x[k];
+        }
+#pragma unroll
+        for (int k = 0; k < PAO; ++k)
+            if (PAO * wave + k < nother) a.stage[e + 64 * (PAO * wave + k)] = o[k];
+        if (wave == 0) {
+            a.map_dst[e] = kr0 + pos;
+            a.map_src[e] = kr0 + lane;
+        }
+    }
+    if (wave == 0) {
+        if (lane < PNW) a.solve->num[lane] = lane < w ? lane : -1;
+        if (lane < w) {  // (nobody reads the pivots' values here, and no swaps)
+            a.ipiv[kr0 + lane] = kr0 + lane;
+            a.pivcol[kr0 + lane] = a.c0 + lane;
+        }
+        if (lane == 0) *a.ctl = PanelCtl{w, 0, w, w + (int)__popcll(mask), kr0};
     }
 }
 

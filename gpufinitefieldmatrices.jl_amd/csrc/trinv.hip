@@ -213,8 +213,8 @@ size_t elem_size(int kind) { return kind == EK_F64 ? 8 : 4; }
 
 // X (k x k int32 in a workspace of k columns of ldx) = inverse of the triangular k x k
 // int32 matrix T; entries of T outside the triangle are ignored.
-static int trinv_i32(modp_ctx *ctx, bool upper, const int32_t *T, int64_t ldt, int32_t *X, int64_t ldx, int64_t k,
-                     const ModP &mp)
+int trinv_i32(modp_ctx *ctx, bool upper, const int32_t *T, int64_t ldt, int32_t *X, int64_t ldx, int64_t k,
+              const ModP &mp)
 {
     int st = MODP_OK;
     int *bad = (int *)ws_get(ctx, WS_TRI_FLAG, 64, &st);
@@ -267,6 +267,9 @@ int mat_inverse(modp_ctx *ctx, int form, int kind, int64_t n, const void *A, int
         *invertible = 1;
         return MODP_OK;
     }
+    int taken = 0;
+    MODP_TRY(elim_inverse(ctx, form, kind, n, A, lda, Ainv, ldai, p, invertible, &taken));
+    if (taken) return MODP_OK;
     const ModP mp = make_modp(p);
     const int64_t ld = rup64(n);
     const size_t es = elem_size(kind);
