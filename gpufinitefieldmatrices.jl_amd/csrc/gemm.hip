@@ -7,7 +7,7 @@
 // applied per MFMA step instead of per cuBLAS stripe).
 //
 // Limb form (kernels in gemm_limb.h): residues as signed base-256 digits in
-// int8 on v_mfma_i32_16x16x64_i8; this file splits the operands into digit
+// int8 on v_mfma_i32_32x32x32_i8; this file splits the operands into digit
 // planes, cuts K into int32-safe chunks and picks the launch.
 //
 // Both forms can cut K into slices that run concurrently (blockIdx.y) and are

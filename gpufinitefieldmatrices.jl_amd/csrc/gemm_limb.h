@@ -3,7 +3,7 @@
 // Each residue r in [0,p) is written in balanced base 256,
 // r == sum_u d_u 256^u (mod p), with signed digits d_u in [-128,127] held in
 // int8; L = ceil(log256 p) digits (p <= 256^L) cover every residue class.
-// The L*L digit products run on v_mfma_i32_16x16x64_i8 with int32
+// The L*L digit products run on v_mfma_i32_32x32x32_i8 with int32
 // accumulation, products of equal shift s+t sharing one accumulator; K is cut
 // into chunks so that no int32 partial sum can overflow; the 2L-1 shift sums
 // are reduced mod p and recombined with weights 256^u mod p in FP64.

@@ -706,8 +706,8 @@ def _inverse(A: CuModArray, form: int):
 
 
 def inverse(A: CuModArray, form: int = FORM_AUTO) -> CuModArray:
-    """inverse(A) (CuModMatrix.jl:480-502): A^{-1} mod N from PLUQ and the two
-    triangular inverses; raises MatrixNotInvertibleException when the mod-N
+    """inverse(A) (CuModMatrix.jl:480-502): A^{-1} mod N from the elimination
+    of [A | I] (for composite N from PLUQ and the two triangular inverses); raises MatrixNotInvertibleException when the mod-N
     rank is deficient."""
     ok, Ainv = _inverse(A, form)
     if not ok:
