@@ -36,6 +36,26 @@ int hip_check(modp_ctx *ctx, hipError_t e, const char *what)
     return set_error(ctx, MODP_ERR_DEVICE, "%s: %s", what, hipGetErrorString(e));
 }
 
+static void release_freed(FreedMemory &f)
+{
+    for (auto &b : f.freed) (void)hipFree(b.first);
+    f.freed.clear();
+    f.bytes = 0;
+}
+
+hipError_t device_alloc(modp_ctx *ctx, void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        std::lock_guard<std::mutex> lk(ctx->memory.mu);
+        if (ctx->memory.freed.empty()) return e;
+        (void)hipGetLastError();
+        release_freed(ctx->memory);
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 void *ws_get(modp_ctx *ctx, int slot, size_t bytes, int *status)
 {
     if (bytes == 0) bytes = 256;
@@ -49,7 +69,7 @@ void *ws_get(modp_ctx *ctx, int slot, size_t bytes, int *status)
     }
     size_t sz = (bytes + 4095) & ~(size_t)4095;
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, sz);
+    hipError_t e = device_alloc(ctx, &p, sz);
     if (e != hipSuccess) {
         *status = hip_check(ctx, e, "workspace allocation");
         return nullptr;
@@ -239,6 +259,7 @@ int modp_ctx_destroy(modp_ctx *ctx)
     (void)hipStreamSynchronize(ctx->stream);
     for (int i = 0; i < WS_COUNT; ++i)
         if (ctx->ws[i]) (void)hipFree(ctx->ws[i]);
+    release_freed(ctx->memory);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->invtab) (void)hipFree(ctx->invtab);
     for (auto &t : ctx->timings) { (void)hipEventDestroy(t.a); (void)hipEventDestroy(t.b); }
@@ -266,15 +287,61 @@ int modp_malloc(modp_ctx *ctx, size_t bytes, void **dptr)
     if (!dptr) return set_error(ctx, MODP_ERR_ARG, "null output pointer");
     *dptr = nullptr;
     if (bytes == 0) bytes = 1;
-    return hip_check(ctx, hipMalloc(dptr, bytes), "hipMalloc");
+    FreedMemory &f = ctx->memory;
+    int current = -1;
+    if (hipGetDevice(&current) != hipSuccess || current != ctx->device)
+        return hip_check(ctx, hipMalloc(dptr, bytes), "hipMalloc");
+    {
+        std::lock_guard<std::mutex> lk(f.mu);
+        // the latest block that is not more than an eighth too large
+        for (size_t i = f.freed.size(); i-- > 0;) {
+            const auto b = f.freed[i];
+            if (b.second < bytes || b.second - bytes > bytes / 8) continue;
+            f.live[b.first] = b.second;
+            f.freed.erase(f.freed.begin() + (ptrdiff_t)i);
+            f.bytes -= b.second;
+            *dptr = b.first;
+            return MODP_OK;
+        }
+    }
+    MODP_TRY(hip_check(ctx, device_alloc(ctx, dptr, bytes), "hipMalloc"));
+    std::lock_guard<std::mutex> lk(f.mu);
+    f.live[*dptr] = bytes;
+    return MODP_OK;
 }
 
 int modp_free(modp_ctx *ctx, void *dptr)
 {
     CTX_CHECK(ctx);
     if (!dptr) return MODP_OK;
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    return hip_check(ctx, hipFree(dptr), "hipFree");
+    FreedMemory &f = ctx->memory;
+    size_t bytes = 0;
+    {
+        std::lock_guard<std::mutex> lk(f.mu);
+        for (auto &b : f.freed)
+            if (b.first == dptr) return hip_check(ctx, hipErrorInvalidValue, "modp_free of freed memory");
+        auto it = f.live.find(dptr);
+        if (it != f.live.end()) {
+            bytes = it->second;
+            f.live.erase(it);
+        }
+    }
+    // Every stream of the device may still use the memory, not this context's alone:
+    // hipFree waits for all of them, and so does this
+    int current = -1;
+    hipError_t e = hipGetDevice(&current);
+    if (e == hipSuccess && current != ctx->device) e = hipErrorInvalidDevice;
+    if (e == hipSuccess && bytes != 0) e = hipDeviceSynchronize();
+    if (e != hipSuccess || bytes == 0 || bytes > FREED_BYTES) return hip_check(ctx, hipFree(dptr), "hipFree");
+    std::lock_guard<std::mutex> lk(f.mu);
+    while (f.bytes + bytes > FREED_BYTES) {
+        (void)hipFree(f.freed[0].first);
+        f.bytes -= f.freed[0].second;
+        f.freed.erase(f.freed.begin());
+    }
+    f.freed.emplace_back(dptr, bytes);
+    f.bytes += bytes;
+    return MODP_OK;
 }
 
 int modp_memcpy_h2d(modp_ctx *ctx, void *dst, const void *src, size_t bytes)

@@ -730,9 +730,9 @@ int plan_build(modp_ctx *ctx, int kind, const modp_gemm_job *jobs, int64_t count
     }
     pl->cls_off[NCLASS] = (int64_t)items.size();
     pl->items = (int64_t)items.size();
-    hipError_t e = hipMalloc(&pl->djobs, sizeof(BJob) * (count > 0 ? count : 1));
-    if (e == hipSuccess) e = hipMalloc(&pl->ditems, sizeof(BItem) * (items.empty() ? 1 : items.size()));
-    if (e == hipSuccess) e = hipMalloc(&pl->dcounter, sizeof(int) * 16 * NCLASS * NXCD);
+    hipError_t e = device_alloc(ctx, (void **)&pl->djobs, sizeof(BJob) * (count > 0 ? count : 1));
+    if (e == hipSuccess) e = device_alloc(ctx, (void **)&pl->ditems, sizeof(BItem) * (items.empty() ? 1 : items.size()));
+    if (e == hipSuccess) e = device_alloc(ctx, (void **)&pl->dcounter, sizeof(int) * 16 * NCLASS * NXCD);
     if (e == hipSuccess && count > 0)
         e = hipMemcpyAsync(pl->djobs, hj.data(), sizeof(BJob) * count, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess && !items.empty())
@@ -1693,7 +1693,7 @@ int batched_elim_plan(modp_ctx *ctx, int op, int kind, const modp_elim_job *jobs
     }
     hipError_t e = hipSuccess;
     if (!htab.empty()) {
-        e = hipMalloc(&pl->dtab, htab.size() * sizeof(uint16_t));
+        e = device_alloc(ctx, (void **)&pl->dtab, htab.size() * sizeof(uint16_t));
         if (e == hipSuccess)
             e = hipMemcpyAsync(pl->dtab, htab.data(), htab.size() * sizeof(uint16_t), hipMemcpyHostToDevice,
                                ctx->stream);
@@ -1732,8 +1732,8 @@ int batched_elim_plan(modp_ctx *ctx, int op, int kind, const modp_elim_job *jobs
         const int64_t w = per_cu * ctx->num_cus;
         eg.grid = (int)(w < eg.count ? w : eg.count);
     }
-    if (e == hipSuccess) e = hipMalloc(&pl->djobs, sizeof(EJob) * (count > 0 ? count : 1));
-    if (e == hipSuccess) e = hipMalloc(&pl->dcounter, 64 * EGROUP);
+    if (e == hipSuccess) e = device_alloc(ctx, (void **)&pl->djobs, sizeof(EJob) * (count > 0 ? count : 1));
+    if (e == hipSuccess) e = device_alloc(ctx, (void **)&pl->dcounter, 64 * EGROUP);
     if (e == hipSuccess && count > 0)
         e = hipMemcpyAsync(pl->djobs, hj.data(), sizeof(EJob) * count, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // hj is released on return

@@ -755,7 +755,7 @@ const uint32_t *inverse_table(modp_ctx *ctx, const ModP &mp, int *st)
     ctx->invtab_prime = mp.p >= 2;
     for (int64_t q = 2; q * q <= mp.p && ctx->invtab_prime; q += q == 2 ? 1 : 2) ctx->invtab_prime = mp.p % q != 0;
     if (!ctx->invtab) {
-        hipError_t e = hipMalloc(&ctx->invtab, sizeof(uint32_t) * PINV);
+        hipError_t e = device_alloc(ctx, (void **)&ctx->invtab, sizeof(uint32_t) * PINV);
         if (e != hipSuccess) { *st = hip_check(ctx, e, "inverse table"); return nullptr; }
     }
     const int n = mp.p < PINV ? (int)mp.p : PINV;
