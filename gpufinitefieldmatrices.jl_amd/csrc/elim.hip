@@ -846,7 +846,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     const uint32_t *invs = inverse_table(ctx, mp, &st);
     if (st != MODP_OK) return st;
     // Where the result does not depend on the pivots, the panels may take any
-    // (k_panel_any): 15 us a panel against 37 to 53.  Not for a composite
+    // (k_panel_any): 15 us a panel at most, against 37 to 53.  Not for a composite
     // modulus, where a pivot without inverse is an error that depends on which
     // one is taken.
     const bool any_pivot = (mode == ELIM_RREF || mode == ELIM_INVERSE) && !force_global && ctx->invtab_prime;

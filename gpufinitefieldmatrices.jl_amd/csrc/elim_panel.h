@@ -783,8 +783,9 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
 //
 // It is bound by its chain: per column one LDS word a row, a barrier, and 40
 // FP64 instructions; the next column is updated and passed on before the
-// others.  A 32-column panel takes 15 us mod 65521 and 16 us mod
-// 2^26 - 5, whatever its rows, against 44 and 53 of the general panel over an XCD:
+// others, some of which wait until the next barrier is behind.  A 32-column
+// panel takes 14.3 us mod 65521 and 15.2 us mod 2^26 - 5 (15.0 and 16.0 with all
+// of them before the barrier; two thirds of it is the chain), whatever its rows, against 44 and 53 of the general panel over an XCD:
 // RREF of 4096^2 and rank 3000 8.2 -> 5.1 ms, and with the identity beside the
 // matrix in place of L^{-1}, inverse of 1500^2 mod 2^26 - 5 4.0 -> 1.94 ms.
 // A column without a nonzero entry among the 64 rows says nothing about the rows
@@ -801,6 +802,7 @@ struct PanelAnyArgs {
     int *abort;
 };
 constexpr int PAC = PNW / PWAVES;               // panel columns of a wave
+constexpr int PAB = 3;                          // columns updated before a step's barrier, the rest after it
 constexpr int PAO = (128 - PNW) / PWAVES;       // other columns of the block, at most
 
 __global__ __launch_bounds__(64 * PWAVES) void k_panel_any(PanelAnyArgs a)
@@ -837,12 +839,12 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel_any(PanelAnyArgs a)
     if (wave == 0) s_col[0][lane] = v[0];
     __syncthreads();
     int done = 0;
+    double mult = s_col[0][lane];
     for (int ow = 0; ow < PWAVES; ++ow) {
         auto step = [&](auto SC) __attribute__((always_inline)) {
             constexpr int s = decltype(SC)::value, nx = (s + 1) % PAC;
             const int jc = PAC * ow + s;
             if (done != jc || jc >= w) return;  // uniform over the workgroup
-            const double mult = s_col[s & 1][lane];
             const uint64_t at = __ballot(mult != 0.0) & cand;
             if (at == 0) return;
             const int l = (int)__builtin_ctzll(at);
@@ -857,14 +859,18 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel_any(PanelAnyArgs a)
             };
             one(nx);
             if (wave == (s + 1 == PAC ? ow + 1 : ow)) s_col[(s + 1) & 1][lane] = v[nx];
+            // the other columns while the next one is on its way
 #pragma unroll
-            for (int k = 0; k < PAC; ++k)
-                if (k != nx) one(k);
+            for (int k = 1; k <= PAB; ++k) one((nx + k) % PAC);
+            __syncthreads();
+            mult = s_col[(s + 1) & 1][lane];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = PAB + 1; k < PAC; ++k) one((nx + k) % PAC);
             d = pivot ? V : near_mod(d * V, mp);
             S = near_mod(S * V, mp);
             pk = pivot ? jc : pk;
             done = jc + 1;
-            __syncthreads();
         };
         Unroll<0, PAC>::run(step);
     }
