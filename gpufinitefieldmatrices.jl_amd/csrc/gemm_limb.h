@@ -152,10 +152,9 @@ __global__ __launch_bounds__(256) void k_split_ab(int64_t m, int64_t n, int64_t 
 }
 
 // Limb-form tile shapes: a BM x BN output tile per workgroup of WGM x WGN
-// waves, each wave a (BM/WGM) x (BN/WGN) block of MF x MF MFMA blocks: MF = 32
-// uses v_mfma_i32_32x32x32_i8 (two k-steps per 64-deep stage), MF = 16 uses
-// v_mfma_i32_16x16x64_i8.  On gfx950 the 32x32 form sustains about 1.4x the
-// int8 rate of the 16x16 form (3.96 vs 2.8 POP/s measured).
+// waves, each wave a (BM/WGM) x (BN/WGN) block of 32 x 32 blocks of
+// v_mfma_i32_32x32x32_i8 (two k-steps per 64-deep stage), which sustains 1.4x
+// or more of the int8 rate of the 16x16x64 form (4.36 vs 2.76 POP/s measured).
 // LDS rows hold the 64 digits of one row (A) or column (B) for one K stage
 // as four 16-byte chunks.  SWZ = 0: rows padded to 80 bytes.  SWZ = 1: rows of
 // 64 bytes with chunk q of row r stored at slot q ^ ((r >> 2) & 3), so both
@@ -163,9 +162,9 @@ __global__ __launch_bounds__(256) void k_split_ab(int64_t m, int64_t n, int64_t 
 // every bank group once.  DB = 1: two LDS stages; stage k+1 is stored while
 // stage k feeds the MFMAs, with one barrier per stage.  DB = 2: in addition
 // two register staging sets, so each global load has two stages to land.
-template <int BM_, int BN_, int WGM_, int WGN_, int MF_ = 16, int SWZ_ = 1, int DB_ = 0, int OCC_ = 1>
+template <int BM_, int BN_, int WGM_, int WGN_, int SWZ_ = 1, int DB_ = 0, int OCC_ = 1>
 struct LimbShape {
-    static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, MF = MF_, SWZ = SWZ_, DB = DB_;
+    static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, MF = 32, SWZ = SWZ_, DB = DB_;
     static constexpr int OCC = OCC_;  // waves per SIMD the register budget must allow
     static constexpr int NT = 64 * WGM * WGN;
     static constexpr int PITCH = SWZ ? 64 : 80;
@@ -192,9 +191,9 @@ __global__ __launch_bounds__(SH::NT, SH::OCC) void k_gemm_limb(int64_t m, int64_
     constexpr int MF = SH::MF;
     constexpr int WM = BM / SH::WGM, WN = BN / SH::WGN;
     constexpr int FM = WM / MF, FN = WN / MF;
-    constexpr int KS = MF == 32 ? 2 : 1;     // MFMA k-steps per 64-deep stage
-    constexpr int AE = MF == 32 ? 16 : 4;    // accumulator elements per lane
-    typedef std::conditional_t<MF == 32, v16i, v4i> acc_t;
+    constexpr int KS = 2;     // MFMA k-steps per 64-deep stage
+    constexpr int AE = 16;    // accumulator elements per lane
+    typedef v16i acc_t;
     constexpr int ACH = L * BM * (LBK / 16);  // 16-byte chunks of A per stage
     constexpr int BCH = L * BN * (LBK / 16);
     constexpr int NBUF = SH::DB ? 2 : 1;
@@ -267,12 +266,12 @@ __global__ __launch_bounds__(SH::NT, SH::OCC) void k_gemm_limb(int64_t m, int64_
         }
     };
     // fragments: lane holds row (lane % MF) of the block and 16 digits of
-    // k-chunk q (16x16x64: q = lane / 16; 32x32x32: q = 2 ks + lane / 32)
+    // k-chunk q = 2 ks + lane / 32
     v4i a[FM][KS][L], b[FN][KS][L];
     auto fragments = [&](int buf) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            const int q = MF == 32 ? ks * 2 + (lane >> 5) : (lane >> 4);
+            const int q = ks * 2 + (lane >> 5);
 #pragma unroll
             for (int i = 0; i < FM; ++i) {
                 const int row = wm * WM + i * MF + (lane & (MF - 1));
@@ -299,14 +298,9 @@ __global__ __launch_bounds__(SH::NT, SH::OCC) void k_gemm_limb(int64_t m, int64_
 #pragma unroll
                     for (int s = 0; s < L; ++s)
 #pragma unroll
-                        for (int t = 0; t < L; ++t) {
-                            if constexpr (MF == 32)
-                                acc[i][j][s + t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b[j][ks][t], a[i][ks][s],
-                                                                                         acc[i][j][s + t], 0, 0, 0);
-                            else
-                                acc[i][j][s + t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b[j][ks][t], a[i][ks][s],
-                                                                                         acc[i][j][s + t], 0, 0, 0);
-                        }
+                        for (int t = 0; t < L; ++t)
+                            acc[i][j][s + t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b[j][ks][t], a[i][ks][s],
+                                                                                     acc[i][j][s + t], 0, 0, 0);
     };
 
     const int64_t nk = (kend - kbeg) / LBK;
@@ -380,7 +374,7 @@ __global__ __launch_bounds__(SH::NT, SH::OCC) void k_gemm_limb(int64_t m, int64_
             if (EPI != EPI_STORE) {
 #pragma unroll
                 for (int e = 0; e < AE; ++e) {
-                    const int64_t col = gc + (MF == 32 ? 8 * (e >> 2) + (e & 3) : e);
+                    const int64_t col = gc + 8 * (e >> 2) + (e & 3);
                     old[e] = dst[(inside ? col : min(col, n - 1)) * ldc];
                 }
             }
@@ -405,7 +399,7 @@ __global__ __launch_bounds__(SH::NT, SH::OCC) void k_gemm_limb(int64_t m, int64_
                 uint32_t r = (uint32_t)(tot < 0.0 ? tot + mp.pd : tot);
                 if (EPI == EPI_SUB) r = submod(to_res<TC>(old[e], mp), r, mp);
                 else if (EPI == EPI_ADD) r = addmod(to_res<TC>(old[e], mp), r, mp);
-                const int64_t col = gc + (MF == 32 ? 8 * (e >> 2) + (e & 3) : e);
+                const int64_t col = gc + 8 * (e >> 2) + (e & 3);
                 if (inside || (row_ok && col < n)) dst[col * ldc] = from_res<TC>(r);
             }
         }
@@ -447,15 +441,15 @@ int limb_by_shape(modp_ctx *ctx, const GemmArgs &g, int epi, const int8_t *Al, i
 {
     if constexpr (L == 1)
         if (tile_m == 256)
-            return limb_core<L, LimbShape<256, 256, 4, 2, 32, 1, 2>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp, lw, sl);
+            return limb_core<L, LimbShape<256, 256, 4, 2, 1, 2>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp, lw, sl);
     if constexpr (L <= 2)
         if (tile_m == 128 && tile_n == 128)
-            return limb_core<L, LimbShape<128, 128, L == 1 ? 2 : 4, 2, 32, 1, 2>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp,
+            return limb_core<L, LimbShape<128, 128, L == 1 ? 2 : 4, 2, 1, 2>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp,
                                                                                      lw, sl);
     if (tile_m == 128 && tile_n == 64)
-        return limb_core<L, LimbShape<128, 64, L == 2 ? 2 : 4, 2, 32, 1, L == 4 ? 1 : 2>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp, lw,
+        return limb_core<L, LimbShape<128, 64, L == 2 ? 2 : 4, 2, 1, L == 4 ? 1 : 2>, TC>(ctx, g, epi, Al, Mp, Bl, Np, Kp, lw,
                                                                                 sl);
-    return limb_core<L, LimbShape<64, 64, 2, 2, 32, 1, L == 4 ? 1 : 2, L == 4 ? 2 : 1>, TC>(ctx, g, epi, Al, Mp, Bl,
+    return limb_core<L, LimbShape<64, 64, 2, 2, 1, L == 4 ? 1 : 2, L == 4 ? 2 : 1>, TC>(ctx, g, epi, Al, Mp, Bl,
                                                                                            Np, Kp, lw, sl);
 }
 
