@@ -784,10 +784,11 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
 // It is bound by its chain: per column one LDS word a row, a barrier, and 40
 // FP64 instructions; the next column is updated and passed on before the
 // others, some of which wait until the next barrier is behind.  A 32-column
-// panel takes 14.3 us mod 65521 and 15.2 us mod 2^26 - 5 (15.0 and 16.0 with all
-// of them before the barrier; two thirds of it is the chain), whatever its rows, against 44 and 53 of the general panel over an XCD:
-// RREF of 4096^2 and rank 3000 8.2 -> 5.1 ms, and with the identity beside the
-// matrix in place of L^{-1}, inverse of 1500^2 mod 2^26 - 5 4.0 -> 1.94 ms.
+// panel takes 14.3 us mod 65521 and 15.2 us mod 2^26 - 5, whatever its rows (15.0
+// and 16.0 with all of them before the barrier; two thirds of it is the chain),
+// against 44 and 53 of the general panel over an XCD.  When it came in, RREF of
+// 4096^2 and rank 3000 went from 8.2 to 5.1 ms, and with the identity beside the
+// matrix in place of L^{-1}, the inverse of 1500^2 mod 2^26 - 5 from 4.0 to 1.94 ms.
 // A column without a nonzero entry among the 64 rows says nothing about the rows
 // below: status 7, nothing written, and the general panel takes the block.
 struct PanelAnyArgs {
