@@ -711,6 +711,12 @@ int gemm_limb_i8_in(modp_ctx *ctx, const GemmArgs &g, const LimbScratch &ws)
 
 namespace {
 
+// whether the address ranges [a0, a1) and [b0, b1) have a byte in common
+bool meet(const void *a0, const void *a1, const void *b0, const void *b1)
+{
+    return (const char *)a0 < (const char *)b1 && (const char *)b0 < (const char *)a1;
+}
+
 template <typename T, int V>
 int gemv_t(modp_ctx *ctx, int64_t m, int64_t k, const T *A, int64_t lda, const T *x, T *y, const ModP &mp)
 {
@@ -728,8 +734,8 @@ int gemv_t(modp_ctx *ctx, int64_t m, int64_t k, const T *A, int64_t lda, const T
     if (S < 1) S = 1;
     const int64_t kslice = round_up(((k > 0 ? k : 1) + S - 1) / S, 4 * GV_U);
     S = k > 0 ? (k + kslice - 1) / kslice : 1;
-    // y over x: nothing of y is written before all of x is read
-    const bool over = (const char *)y < (const char *)(x + k) && (const char *)x < (const char *)(y + m);
+    // y over x or within A: nothing of y is written before all of both is read
+    const bool over = k > 0 && m > 0 && (meet(y, y + m, x, x + k) || meet(y, y + m, A, A + (k - 1) * lda + m));
     int32_t *P = nullptr;
     int *arrived = nullptr;
     if (S > 1 || over) {
