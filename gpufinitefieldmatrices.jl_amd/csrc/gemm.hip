@@ -271,6 +271,24 @@ __global__ void k_zero_ints(int *p, int n)
 
 int64_t round_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 
+// whether the address ranges [a0, a1) and [b0, b1) have a byte in common
+bool meet(const void *a0, const void *a1, const void *b0, const void *b1)
+{
+    return (const char *)a0 < (const char *)b1 && (const char *)b0 < (const char *)a1;
+}
+
+// whether C lies (partly) in the memory of A or B
+bool over_operand(const GemmArgs &g)
+{
+    auto bytes = [](int kind) -> int64_t { return kind == EK_F64 ? 8 : 4; };
+    auto end = [&](const void *X, int64_t rows, int64_t cols, int64_t ld, int kind) {
+        return (const char *)X + ((cols - 1) * ld + rows) * bytes(kind);
+    };
+    if (g.m <= 0 || g.n <= 0 || g.k <= 0) return false;
+    const char *const c1 = end(g.C, g.m, g.n, g.ldc, g.kc);
+    return meet(g.C, c1, g.A, end(g.A, g.m, g.k, g.lda, g.ka)) || meet(g.C, c1, g.B, end(g.B, g.k, g.n, g.ldb, g.kb));
+}
+
 // ---- dispatch helpers -----------------------------------------------------
 
 template <typename TA, typename TB, typename TC, int BM, int BN, int EPI>
@@ -448,12 +466,15 @@ int gemm_plain_cfg(modp_ctx *ctx, const GemmArgs &g, const GemmConfig &cfg)
     if (g.m <= 0 || g.n <= 0) return MODP_OK;
     const int R = f64_reduce_interval(g.mp.p);
     if (R < 1) return set_error(ctx, MODP_ERR_MODULUS_RANGE, "modulus %lld too large for the FP64 form", (long long)g.mp.p);
-    if (f64_small(g)) return launch_f64_small(ctx, g, R, 1, 0, 0, 0, GemmSize{g.m, g.n, g.k});
+    // a C over an operand is written only after all workgroups have read it:
+    // through the residues of the slices, also where there is one slice
+    const bool over = over_operand(g);
+    if (!over && f64_small(g)) return launch_f64_small(ctx, g, R, 1, 0, 0, 0, GemmSize{g.m, g.n, g.k});
     const int tile = cfg.tile_m == 128 ? 128 : 64;
     Slices sl = make_slices(g.k, cfg.ksplit, PBK, 64);
     if (sl.S == 1) {
         sl.kslice = g.k > 0 ? g.k : 1;
-        return launch_f64(ctx, g, R, tile, sl);
+        if (!over) return launch_f64(ctx, g, R, tile, sl);
     }
     int st = MODP_OK;
     int32_t *P = slice_buffer(ctx, g, sl.S, &st);
@@ -710,12 +731,6 @@ int gemm_limb_i8_in(modp_ctx *ctx, const GemmArgs &g, const LimbScratch &ws)
 }
 
 namespace {
-
-// whether the address ranges [a0, a1) and [b0, b1) have a byte in common
-bool meet(const void *a0, const void *a1, const void *b0, const void *b1)
-{
-    return (const char *)a0 < (const char *)b1 && (const char *)b0 < (const char *)a1;
-}
 
 template <typename T, int V>
 int gemv_t(modp_ctx *ctx, int64_t m, int64_t k, const T *A, int64_t lda, const T *x, T *y, const ModP &mp)
