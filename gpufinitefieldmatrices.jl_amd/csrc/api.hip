@@ -467,7 +467,7 @@ int modp_gemm_noalloc(modp_ctx *ctx, int dtype, int64_t m, int64_t n, int64_t k,
     MODP_TRY(gemm_prepare(ctx, dtype, m, n, k, A, lda, B, ldb, C, ldc, p, g));
     if (m == 0 || n == 0) return MODP_OK;
     if (k == 0) return gemm_zero(ctx, g);
-    const size_t need = gemm_limb_scratch_bytes(ctx, g);
+    const size_t need = gemm_limb_scratch_bytes(g);
     if (need > NOALLOC_SCRATCH_BYTES)
         return set_error(ctx, MODP_ERR_ARG,
                          "%lld x %lld x %lld needs %zu bytes of digit planes, above the %zu-byte no-allocation scratch",

@@ -389,7 +389,7 @@ struct LimbScratch {
     int8_t *base;
     size_t bytes;
 };
-size_t gemm_limb_scratch_bytes(const modp_ctx *ctx, const GemmArgs &g);
+size_t gemm_limb_scratch_bytes(const GemmArgs &g);
 // the multi-modular (RNS) int8 form (gemm_rns.hip): moduli needed for an
 // exact k-deep product mod p (0: none suffice), and the product with a
 // tile x tile output tile

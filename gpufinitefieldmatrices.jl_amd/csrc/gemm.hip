@@ -711,9 +711,9 @@ int gemm_rns_i8(modp_ctx *ctx, const GemmArgs &g)
     return gemm_run(ctx, g, gemm_default_config(ctx, g, MODP_FORM_RNS_I8));
 }
 
-size_t gemm_limb_scratch_bytes(const modp_ctx *ctx, const GemmArgs &g)
+// bytes of the digit planes of a product without K slices
+static size_t limb_plane_bytes(const GemmArgs &g, const GemmConfig &cfg)
 {
-    GemmConfig cfg = gemm_default_config(ctx, g, MODP_FORM_LIMB_I8);
     const int L = limb_count(g.mp.p);
     int tm, tn;
     limb_tile(cfg, L, g.m, g.n, g.k, false, &tm, &tn);
@@ -723,10 +723,20 @@ size_t gemm_limb_scratch_bytes(const modp_ctx *ctx, const GemmArgs &g)
     return (size_t)L * (size_t)(round_up(g.m, tm) + round_up(g.n, tn)) * (size_t)Kp;
 }
 
+// the least that the product needs, in 64 x 64 tiles
+size_t gemm_limb_scratch_bytes(const GemmArgs &g)
+{
+    GemmConfig cfg;
+    cfg.tile_m = cfg.tile_n = 64;
+    return limb_plane_bytes(g, cfg);
+}
+
 int gemm_limb_i8_in(modp_ctx *ctx, const GemmArgs &g, const LimbScratch &ws)
 {
     GemmConfig cfg = gemm_default_config(ctx, g, MODP_FORM_LIMB_I8);
     cfg.ksplit = 1;
+    // planes rounded up to larger tiles may not fit where those of 64 x 64 do
+    if (limb_plane_bytes(g, cfg) > ws.bytes) cfg.tile_m = cfg.tile_n = 64;
     return gemm_limb_cfg(ctx, g, cfg, &ws);
 }
 

@@ -123,8 +123,8 @@ int modp_gemm(modp_ctx *ctx, int form, int dtype, int64_t m, int64_t n, int64_t 
  * the reference: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid allocation).  The
  * planes take L * (m' + n') * k' bytes (L digits of p, m' and n' rounded up to
- * the output tile, k' = min(k, 32704) rounded up to 64); larger products
- * return MODP_ERR_ARG.  Every call on a device shares that device's array:
+ * 64, k' the smaller of k rounded up to 64 and 131008, 65472, 43648 or 32704
+ * for one to four digits); larger products return MODP_ERR_ARG.  Every call on a device shares that device's array:
  * calls that overlap on one device (two streams, two contexts, two threads)
  * race and must be serialised by the caller.  Kernel timing hooks are not
  * recorded for these calls. */
