@@ -36,6 +36,16 @@ int hip_check(modp_ctx *ctx, hipError_t e, const char *what)
     return set_error(ctx, MODP_ERR_DEVICE, "%s: %s", what, hipGetErrorString(e));
 }
 
+// the device's; never destroyed, since finalizers may free as the process ends
+static FreedMemory *freed_memory(int device)
+{
+    static std::mutex mu;
+    static auto *devices = new std::map<int, FreedMemory>();
+    std::lock_guard<std::mutex> lk(mu);
+    return &(*devices)[device];
+}
+
+// (with f.mu held)
 static void release_freed(FreedMemory &f)
 {
     for (auto &b : f.freed) (void)hipFree(b.first);
@@ -47,10 +57,10 @@ hipError_t device_alloc(modp_ctx *ctx, void **p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory) {
-        std::lock_guard<std::mutex> lk(ctx->memory.mu);
-        if (ctx->memory.freed.empty()) return e;
+        std::lock_guard<std::mutex> lk(ctx->memory->mu);
+        if (ctx->memory->freed.empty()) return e;
         (void)hipGetLastError();
-        release_freed(ctx->memory);
+        release_freed(*ctx->memory);
         e = hipMalloc(p, bytes);
     }
     return e;
@@ -241,6 +251,7 @@ int modp_ctx_create(int device, modp_ctx **out)
     if (strncmp(prop.gcnArchName, "gfx950", 6) != 0) return MODP_ERR_NO_DEVICE;
     modp_ctx *c = new modp_ctx();
     c->device = device;
+    c->memory = freed_memory(device);
     c->num_cus = prop.multiProcessorCount;
     // a failure here leaves only modp_gemm_noalloc unavailable on this device
     c->noalloc_scratch = scratch_address(device);
@@ -259,7 +270,10 @@ int modp_ctx_destroy(modp_ctx *ctx)
     (void)hipStreamSynchronize(ctx->stream);
     for (int i = 0; i < WS_COUNT; ++i)
         if (ctx->ws[i]) (void)hipFree(ctx->ws[i]);
-    release_freed(ctx->memory);
+    {
+        std::lock_guard<std::mutex> lk(ctx->memory->mu);
+        release_freed(*ctx->memory);
+    }
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->invtab) (void)hipFree(ctx->invtab);
     for (auto &t : ctx->timings) { (void)hipEventDestroy(t.a); (void)hipEventDestroy(t.b); }
@@ -287,7 +301,7 @@ int modp_malloc(modp_ctx *ctx, size_t bytes, void **dptr)
     if (!dptr) return set_error(ctx, MODP_ERR_ARG, "null output pointer");
     *dptr = nullptr;
     if (bytes == 0) bytes = 1;
-    FreedMemory &f = ctx->memory;
+    FreedMemory &f = *ctx->memory;
     int current = -1;
     if (hipGetDevice(&current) != hipSuccess || current != ctx->device)
         return hip_check(ctx, hipMalloc(dptr, bytes), "hipMalloc");
@@ -314,7 +328,7 @@ int modp_free(modp_ctx *ctx, void *dptr)
 {
     CTX_CHECK(ctx);
     if (!dptr) return MODP_OK;
-    FreedMemory &f = ctx->memory;
+    FreedMemory &f = *ctx->memory;
     size_t bytes = 0;
     {
         std::lock_guard<std::mutex> lk(f.mu);

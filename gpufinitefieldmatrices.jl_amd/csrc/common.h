@@ -250,9 +250,11 @@ constexpr int WS_COUNT = 24;
 // Device memory that modp_free got back, for the next modp_malloc: allocating
 // and releasing the 256 MiB of results of a 4096^2 PLUQ took 0.6 ms of its 9.7,
 // the 23 MiB of a 2501 x 1203 product 25 of its 120 us.  Freeing waits for the
-// device, as hipFree does, so a block has no reader left.  At most FREED_BYTES are kept, the oldest go first, and all of it is released when an
-// allocation fails and with the context.  The finalizers of a program's objects
-// may run in any of its threads.
+// device, as hipFree does, so a block has no reader left.  One per device, for
+// all of its contexts: memory may be freed through another context than the one
+// that allocated it.  At most FREED_BYTES are kept, the oldest go first, and
+// all of it is released when an allocation fails and with any context of the
+// device.  The finalizers of a program's objects may run in any of its threads.
 constexpr size_t FREED_BYTES = (size_t)1 << 30;
 struct FreedMemory {
     std::mutex mu;
@@ -269,7 +271,7 @@ struct modp_ctx {
     // grow-only device workspaces
     void *ws[WS_COUNT] = {nullptr};
     size_t ws_size[WS_COUNT] = {0};
-    FreedMemory memory;
+    FreedMemory *memory = nullptr;  // of the device
     // pinned host staging for small device->host readbacks
     void *pinned = nullptr;
     size_t pinned_size = 0;

@@ -1,0 +1,40 @@
+"""Freed device memory that the contexts of a device share."""
+import ctypes
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def alloc(ctx, nbytes):
+    p = ctypes.c_void_p()
+    assert ctx.lib.modp_malloc(ctx.h, nbytes, ctypes.byref(p)) == 0
+    return p
+
+
+def free(ctx, p):
+    return ctx.lib.modp_free(ctx.h, p)
+
+
+@pytest.mark.parametrize("nbytes", [12345, 33 << 20])
+def test_contexts_share_what_is_freed(gffm, nbytes):
+    one, two = gffm.context(), gffm.Context()
+    p = alloc(one, nbytes)
+    assert free(two, p) == 0
+    assert free(one, p) != 0 and free(two, p) != 0  # freed already
+    q = alloc(two, nbytes)
+    assert q.value == p.value
+    r = alloc(one, nbytes)
+    assert r.value != q.value
+    assert free(one, q) == 0 and free(two, r) == 0
+
+
+def test_reused_at_once(gffm):
+    # the same block again, also for up to an eighth less, not for more or much less
+    ctx, n = gffm.context(), 7777777
+    p = alloc(ctx, n)
+    assert free(ctx, p) == 0
+    for size, same in ((n, True), (n - n // 10, True), (n // 2, False), (n + 4096, False)):
+        q = alloc(ctx, size)
+        assert (q.value == p.value) == same, size
+        assert free(ctx, q) == 0
