@@ -332,12 +332,14 @@ int modp_free(modp_ctx *ctx, void *dptr)
     size_t bytes = 0;
     {
         std::lock_guard<std::mutex> lk(f.mu);
-        for (auto &b : f.freed)
-            if (b.first == dptr) return hip_check(ctx, hipErrorInvalidValue, "modp_free of freed memory");
+        bool freed = f.leaving.count(dptr) != 0;
+        for (auto &b : f.freed) freed = freed || b.first == dptr;
+        if (freed) return hip_check(ctx, hipErrorInvalidValue, "modp_free of freed memory");
         auto it = f.live.find(dptr);
         if (it != f.live.end()) {
             bytes = it->second;
             f.live.erase(it);
+            f.leaving.insert(dptr);
         }
     }
     // Every stream of the device may still use the memory, not this context's alone:
@@ -346,16 +348,21 @@ int modp_free(modp_ctx *ctx, void *dptr)
     hipError_t e = hipGetDevice(&current);
     if (e == hipSuccess && current != ctx->device) e = hipErrorInvalidDevice;
     if (e == hipSuccess && bytes != 0) e = hipDeviceSynchronize();
-    if (e != hipSuccess || bytes == 0 || bytes > FREED_BYTES) return hip_check(ctx, hipFree(dptr), "hipFree");
-    std::lock_guard<std::mutex> lk(f.mu);
-    while (f.bytes + bytes > FREED_BYTES) {
-        (void)hipFree(f.freed[0].first);
-        f.bytes -= f.freed[0].second;
-        f.freed.erase(f.freed.begin());
+    {
+        std::lock_guard<std::mutex> lk(f.mu);
+        f.leaving.erase(dptr);
+        if (e == hipSuccess && bytes != 0 && bytes <= FREED_BYTES) {
+            while (f.bytes + bytes > FREED_BYTES) {
+                (void)hipFree(f.freed[0].first);
+                f.bytes -= f.freed[0].second;
+                f.freed.erase(f.freed.begin());
+            }
+            f.freed.emplace_back(dptr, bytes);
+            f.bytes += bytes;
+            return MODP_OK;
+        }
     }
-    f.freed.emplace_back(dptr, bytes);
-    f.bytes += bytes;
-    return MODP_OK;
+    return hip_check(ctx, hipFree(dptr), "hipFree");
 }
 
 int modp_memcpy_h2d(modp_ctx *ctx, void *dst, const void *src, size_t bytes)

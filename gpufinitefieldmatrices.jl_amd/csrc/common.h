@@ -8,6 +8,7 @@
 #include <mutex>
 #include <string>
 #include <unordered_map>
+#include <unordered_set>
 #include <utility>
 #include <vector>
 
@@ -259,6 +260,7 @@ constexpr size_t FREED_BYTES = (size_t)1 << 30;
 struct FreedMemory {
     std::mutex mu;
     std::unordered_map<void *, size_t> live;       // allocations of modp_malloc
+    std::unordered_set<void *> leaving;            // in a modp_free that waits for the device
     std::vector<std::pair<void *, size_t>> freed;  // oldest first
     size_t bytes = 0;                              // of freed
 };

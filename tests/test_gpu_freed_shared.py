@@ -1,5 +1,7 @@
-"""Freed device memory that the contexts of a device share."""
+"""Freed device memory that the contexts of a device share: one table of what is
+kept, a block that several threads free at once."""
 import ctypes
+import threading
 
 import pytest
 
@@ -38,3 +40,26 @@ def test_reused_at_once(gffm):
         q = alloc(ctx, size)
         assert (q.value == p.value) == same, size
         assert free(ctx, q) == 0
+
+
+def test_freed_by_several_threads_at_once(gffm):
+    # one of them frees it, the others are told so, and it is handed out once
+    contexts = [gffm.Context() for _ in range(4)]
+    n = 1234567
+    for _ in range(50):
+        p, status = alloc(contexts[0], n), []
+        start = threading.Barrier(len(contexts))
+
+        def work(ctx):
+            start.wait()
+            status.append(free(ctx, p))
+
+        threads = [threading.Thread(target=work, args=(c,)) for c in contexts]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert sorted(s == 0 for s in status) == [False, False, False, True]
+        q, r = alloc(contexts[1], n), alloc(contexts[2], n)
+        assert q.value != r.value
+        assert free(contexts[1], q) == 0 and free(contexts[2], r) == 0
