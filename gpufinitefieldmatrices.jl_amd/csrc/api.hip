@@ -45,6 +45,8 @@ static FreedMemory *freed_memory(int device)
     return &(*devices)[device];
 }
 
+static size_t freed_units(size_t bytes) { return (bytes + FREED_UNIT - 1) / FREED_UNIT * FREED_UNIT; }
+
 // (with f.mu held)
 static void release_freed(FreedMemory &f)
 {
@@ -313,7 +315,7 @@ int modp_malloc(modp_ctx *ctx, size_t bytes, void **dptr)
             if (b.second < bytes || b.second - bytes > bytes / 8) continue;
             f.live[b.first] = b.second;
             f.freed.erase(f.freed.begin() + (ptrdiff_t)i);
-            f.bytes -= b.second;
+            f.bytes -= freed_units(b.second);
             *dptr = b.first;
             return MODP_OK;
         }
@@ -351,14 +353,15 @@ int modp_free(modp_ctx *ctx, void *dptr)
     {
         std::lock_guard<std::mutex> lk(f.mu);
         f.leaving.erase(dptr);
-        if (e == hipSuccess && bytes != 0 && bytes <= FREED_BYTES) {
-            while (f.bytes + bytes > FREED_BYTES) {
+        const size_t units = freed_units(bytes);
+        if (e == hipSuccess && bytes != 0 && units <= FREED_BYTES) {
+            while (f.bytes + units > FREED_BYTES) {
                 (void)hipFree(f.freed[0].first);
-                f.bytes -= f.freed[0].second;
+                f.bytes -= freed_units(f.freed[0].second);
                 f.freed.erase(f.freed.begin());
             }
             f.freed.emplace_back(dptr, bytes);
-            f.bytes += bytes;
+            f.bytes += units;
             return MODP_OK;
         }
     }

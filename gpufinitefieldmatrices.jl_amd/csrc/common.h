@@ -253,16 +253,18 @@ constexpr int WS_COUNT = 24;
 // the 23 MiB of a 2501 x 1203 product 25 of its 120 us.  Freeing waits for the
 // device, as hipFree does, so a block has no reader left.  One per device, for
 // all of its contexts: memory may be freed through another context than the one
-// that allocated it.  At most FREED_BYTES are kept, the oldest go first, and
+// that allocated it.  At most FREED_BYTES are kept, counted in units of
+// FREED_UNIT (a large page of the device, which a small block may hold for
+// itself) and so at most 512 blocks to look through; the oldest go first, and
 // all of it is released when an allocation fails and with any context of the
 // device.  The finalizers of a program's objects may run in any of its threads.
-constexpr size_t FREED_BYTES = (size_t)1 << 30;
+constexpr size_t FREED_BYTES = (size_t)1 << 30, FREED_UNIT = (size_t)2 << 20;
 struct FreedMemory {
     std::mutex mu;
     std::unordered_map<void *, size_t> live;       // allocations of modp_malloc
     std::unordered_set<void *> leaving;            // in a modp_free that waits for the device
     std::vector<std::pair<void *, size_t>> freed;  // oldest first
-    size_t bytes = 0;                              // of freed
+    size_t bytes = 0;                              // of freed, in whole units
 };
 
 struct modp_ctx {

@@ -1,5 +1,5 @@
 """Freed device memory that the contexts of a device share: one table of what is
-kept, a block that several threads free at once."""
+kept, a block that several threads free at once, and many small ones."""
 import ctypes
 import threading
 
@@ -16,6 +16,20 @@ def alloc(ctx, nbytes):
 
 def free(ctx, p):
     return ctx.lib.modp_free(ctx.h, p)
+
+
+def hip():
+    with open("/proc/self/maps") as maps:  # the HIP runtime that the library uses
+        return ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+
+
+def allocated(runtime, p):
+    """Bytes of the runtime's allocation at p, 0 if there is none."""
+    base, size = ctypes.c_void_p(), ctypes.c_size_t()
+    if runtime.hipMemGetAddressRange(ctypes.byref(base), ctypes.byref(size), p) != 0:
+        runtime.hipGetLastError()
+        return 0
+    return size.value
 
 
 @pytest.mark.parametrize("nbytes", [12345, 33 << 20])
@@ -63,3 +77,15 @@ def test_freed_by_several_threads_at_once(gffm):
         q, r = alloc(contexts[1], n), alloc(contexts[2], n)
         assert q.value != r.value
         assert free(contexts[1], q) == 0 and free(contexts[2], r) == 0
+
+
+@pytest.mark.parametrize("nbytes", [1, 5000])
+def test_small_blocks_are_bounded(gffm, nbytes):
+    # as many as there are large pages in 1 GiB, the latest ones
+    ctx, runtime = gffm.context(), hip()
+    blocks = [alloc(ctx, nbytes + i) for i in range(1500)]
+    assert all(allocated(runtime, p) for p in blocks)
+    for p in blocks:
+        assert free(ctx, p) == 0
+    left = [p for p in blocks if allocated(runtime, p)]
+    assert len(left) <= 512 and left[-1].value == blocks[-1].value
