@@ -47,6 +47,16 @@ static FreedMemory *freed_memory(int device)
 
 static size_t freed_units(size_t bytes) { return (bytes + FREED_UNIT - 1) / FREED_UNIT * FREED_UNIT; }
 
+// bytes of the runtime's allocation at p, 0 if there is none
+static size_t allocated_at(void *p)
+{
+    hipDeviceptr_t base = nullptr;
+    size_t bytes = 0;
+    if (hipMemGetAddressRange(&base, &bytes, (hipDeviceptr_t)p) == hipSuccess) return base == p ? bytes : 0;
+    (void)hipGetLastError();
+    return 0;
+}
+
 // (with f.mu held)
 static void release_freed(FreedMemory &f)
 {
@@ -321,8 +331,9 @@ int modp_malloc(modp_ctx *ctx, size_t bytes, void **dptr)
         }
     }
     MODP_TRY(hip_check(ctx, device_alloc(ctx, dptr, bytes), "hipMalloc"));
+    const size_t got = allocated_at(*dptr);
     std::lock_guard<std::mutex> lk(f.mu);
-    f.live[*dptr] = bytes;
+    f.live[*dptr] = got;
     return MODP_OK;
 }
 
@@ -332,6 +343,7 @@ int modp_free(modp_ctx *ctx, void *dptr)
     if (!dptr) return MODP_OK;
     FreedMemory &f = *ctx->memory;
     size_t bytes = 0;
+    const size_t now = allocated_at(dptr);
     {
         std::lock_guard<std::mutex> lk(f.mu);
         bool freed = f.leaving.count(dptr) != 0;
@@ -339,9 +351,11 @@ int modp_free(modp_ctx *ctx, void *dptr)
         if (freed) return hip_check(ctx, hipErrorInvalidValue, "modp_free of freed memory");
         auto it = f.live.find(dptr);
         if (it != f.live.end()) {
-            bytes = it->second;
+            // not the block that was allocated, if something else released that
+            // one and the address came back: then it is hipFree's
+            if (it->second == now) bytes = now;
             f.live.erase(it);
-            f.leaving.insert(dptr);
+            if (bytes != 0) f.leaving.insert(dptr);
         }
     }
     // Every stream of the device may still use the memory, not this context's alone:

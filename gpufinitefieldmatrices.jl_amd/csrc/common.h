@@ -261,7 +261,7 @@ constexpr int WS_COUNT = 24;
 constexpr size_t FREED_BYTES = (size_t)1 << 30, FREED_UNIT = (size_t)2 << 20;
 struct FreedMemory {
     std::mutex mu;
-    std::unordered_map<void *, size_t> live;       // allocations of modp_malloc
+    std::unordered_map<void *, size_t> live;       // allocations of modp_malloc, as large as the runtime has them
     std::unordered_set<void *> leaving;            // in a modp_free that waits for the device
     std::vector<std::pair<void *, size_t>> freed;  // oldest first
     size_t bytes = 0;                              // of freed, in whole units

@@ -1,5 +1,6 @@
 """Freed device memory that the contexts of a device share: one table of what is
-kept, a block that several threads free at once, and many small ones."""
+kept, a block that several threads free at once, many small ones, and
+one whose address came back after something else had released it."""
 import ctypes
 import threading
 
@@ -89,3 +90,23 @@ def test_small_blocks_are_bounded(gffm, nbytes):
         assert free(ctx, p) == 0
     left = [p for p in blocks if allocated(runtime, p)]
     assert len(left) <= 512 and left[-1].value == blocks[-1].value
+
+
+@pytest.mark.parametrize("n", [48 << 20, 1 << 20, 100000])
+def test_address_that_came_back(gffm, n):
+    ctx, runtime = gffm.context(), hip()
+    runtime.hipMalloc.argtypes = [ctypes.c_void_p, ctypes.c_size_t]
+    for size in (n - 1, n - 4096, n - 70000):
+        p = alloc(ctx, n)
+        assert allocated(runtime, p) >= n
+        assert runtime.hipFree(p) == 0
+        q = ctypes.c_void_p()
+        assert runtime.hipMalloc(ctypes.byref(q), size) == 0
+        print(n, size, hex(p.value), hex(q.value), flush=True)
+        assert free(ctx, q) == 0
+        r = alloc(ctx, n)
+        assert allocated(runtime, r) >= n
+        assert free(ctx, r) == 0
+        again = alloc(ctx, n)
+        assert again.value == r.value
+        assert runtime.hipFree(again) == 0
