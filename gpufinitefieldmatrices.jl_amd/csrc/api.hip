@@ -382,6 +382,17 @@ int modp_free(modp_ctx *ctx, void *dptr)
     return hip_check(ctx, hipFree(dptr), "hipFree");
 }
 
+int modp_release_freed(modp_ctx *ctx, size_t *bytes)
+{
+    CTX_CHECK(ctx);
+    std::lock_guard<std::mutex> lk(ctx->memory->mu);
+    size_t sum = 0;
+    for (auto &b : ctx->memory->freed) sum += b.second;
+    release_freed(*ctx->memory);
+    if (bytes) *bytes = sum;
+    return MODP_OK;
+}
+
 int modp_memcpy_h2d(modp_ctx *ctx, void *dst, const void *src, size_t bytes)
 {
     CTX_CHECK(ctx);

@@ -131,6 +131,13 @@ class Context:
     def malloc(self, nbytes: int) -> "DeviceBuffer":
         return DeviceBuffer(self, nbytes)
 
+    def release_freed(self) -> int:
+        """Give the device memory that is kept for the next allocations (at
+        most 1 GiB) back to the device; returns its bytes."""
+        n = ctypes.c_size_t()
+        self.check(self.lib.modp_release_freed(self.h, ctypes.byref(n)), "release_freed")
+        return n.value
+
     # timing helpers used by the benchmark
     def kernel_timing(self, enable: bool):
         self.check(self.lib.modp_kernel_timing(self.h, 1 if enable else 0))

@@ -75,6 +75,7 @@ SIGNATURES = [
     ("modp_stream", _vp, [_vp]),
     ("modp_malloc", _int, [_vp, _sz, ctypes.POINTER(_vp)]),
     ("modp_free", _int, [_vp, _vp]),
+    ("modp_release_freed", _int, [_vp, ctypes.POINTER(_sz)]),
     ("modp_memcpy_h2d", _int, [_vp, _vp, _vp, _sz]),
     ("modp_memcpy_d2h", _int, [_vp, _vp, _vp, _sz]),
     ("modp_memcpy_d2d", _int, [_vp, _vp, _vp, _sz]),

@@ -96,6 +96,18 @@ function DeviceBuffer(nbytes::Integer)
     return b
 end
 
+"""
+    release_freed()
+
+Give the device memory that is kept for the next allocations (at most 1 GiB)
+back to the device; returns its bytes.
+"""
+function release_freed()
+    n = Ref{Csize_t}(0)
+    check(ccall((:modp_release_freed, LIB), Cint, (Ptr{Cvoid}, Ref{Csize_t}), context().h, n), "release_freed")
+    return Int(n[])
+end
+
 # ---- the matrix type (CuModArray{T,2}, CuModMatrix.jl:42-122) -----------------
 struct ModMatrix{T} <: AbstractMatrix{T}
     data::DeviceBuffer      # padded (rows+32) x (cols+32), column-major

@@ -80,8 +80,15 @@ void *modp_stream(modp_ctx *ctx);
 
 /* ---- device memory (CuArray allocation / copyto! / Array) ------------- */
 
+/* modp_free waits for the device and may keep the memory for the next
+ * modp_malloc of about its size, at most 1 GiB per device.  Other allocators
+ * and processes do not see that memory as free; it is released when one of the
+ * library's own allocations on the device would fail, when a context of the
+ * device is destroyed, and by modp_release_freed, which returns the bytes in
+ * *bytes (NULL: not wanted). */
 int modp_malloc(modp_ctx *ctx, size_t bytes, void **dptr);
 int modp_free(modp_ctx *ctx, void *dptr);
+int modp_release_freed(modp_ctx *ctx, size_t *bytes);
 int modp_memcpy_h2d(modp_ctx *ctx, void *dst, const void *src, size_t bytes);
 int modp_memcpy_d2h(modp_ctx *ctx, void *dst, const void *src, size_t bytes);
 int modp_memcpy_d2d(modp_ctx *ctx, void *dst, const void *src, size_t bytes);

@@ -1,6 +1,6 @@
 """Freed device memory that the contexts of a device share: one table of what is
-kept, a block that several threads free at once, many small ones, and
-one whose address came back after something else had released it."""
+kept, a block that several threads free at once, many small ones, one whose
+address came back after something else had released it, and giving it all back."""
 import ctypes
 import threading
 
@@ -110,3 +110,16 @@ def test_address_that_came_back(gffm, n):
         again = alloc(ctx, n)
         assert again.value == r.value
         assert runtime.hipFree(again) == 0
+
+
+def test_release(gffm):
+    ctx, other, runtime = gffm.context(), gffm.Context(), hip()
+    ctx.release_freed()
+    assert ctx.release_freed() == 0
+    blocks = [alloc(ctx, n) for n in (1, 100000, 300 << 20)]
+    for p in blocks:
+        assert free(ctx, p) == 0
+    assert other.release_freed() >= (300 << 20) + 100001
+    assert not any(allocated(runtime, p) for p in blocks)
+    assert ctx.release_freed() == 0
+    assert ctx.lib.modp_release_freed(ctx.h, None) == 0
