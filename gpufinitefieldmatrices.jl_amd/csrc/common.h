@@ -290,6 +290,7 @@ struct modp_ctx {
     bool invtab_prime = false;
     // steps of the elimination panels so far (64 a panel): their exchange tags
     uint32_t panel_tag = 0;
+    int64_t panel_rows[3] = {0, 0, 0};  // that a panel on one XCD takes, by its arithmetic (0: not asked yet)
     // autotuner: MODP_TUNE_OFF / _CACHED / _ON_MISS and its cache
     int tune_mode = 0;
     std::map<TuneKey, TuneEntry> tune_cache;

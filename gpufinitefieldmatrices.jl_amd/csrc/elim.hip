@@ -18,8 +18,9 @@
 //                inverse, and the rank-1 update of the remaining panel
 //                columns; rows move only at the end, by a row map, and
 //                the old values of the moved rows in the block's other
-//                columns are staged.  Above 16,384 rows k_panel_g does the
-//                same with the panel left in W (any row count).
+//                columns are staged.  Above what an XCD holds at once
+//                (16,384 rows) k_panel_g does the same with the panel left in
+//                W (any row count).
 //     k_update   the block's other columns: the row map, and right of the
 //                panel the rows of U (a product with the inverse triangle
 //                that the panel leaves) and the rank-w update of every row
@@ -29,6 +30,7 @@
 //   K = NBO (limb or plain form) updates the far trailing block.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "elim_panel.h"
@@ -38,8 +40,8 @@ namespace {
 constexpr int NBO = 128;  // outer block width (K of the trailing GEMM)
 
 // Panel factorisation for any number of rows (the register panel holds at
-// most 16,384 and its keys 2^15 positions): the same outputs as k_panel from one 1024-thread workgroup that keeps the panel in
-// W.  Thread t owns local rows t + 1024 q and is the only thread that reads
+// most 16,384 and its keys 2^15 positions): the same outputs as k_panel from
+// one 1024-thread workgroup that keeps the panel in W.  Thread t owns local rows t + 1024 q and is the only thread that reads
 // or writes them during the column steps; a row's current position (the
 // reference's swap of positions pc and Ip) is kept in gpos[row], the row at
 // each position in grow[pos].  Per column: the owners scan their eligible
@@ -767,6 +769,27 @@ const uint32_t *inverse_table(modp_ctx *ctx, const ModP &mp, int *st)
 
 }  // namespace
 
+// Rows that the panel on one XCD takes: all of its workgroups (of 256 rows) wait
+// for each other, so all have to be on the XCD's CUs at once.  Two fit on a CU
+// (75 KB of LDS, at most 231 registers), 64 workgroups or 16,384 rows.
+static int64_t panel_rows(modp_ctx *ctx, int arith)
+{
+    int64_t &rows = ctx->panel_rows[arith];
+    if (rows == 0) {
+        int n = 0;
+        const void *k = arith == 0   ? (const void *)k_panel<true, 0>
+                        : arith == 1 ? (const void *)k_panel<true, 1>
+                                     : (const void *)k_panel<true, 2>;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, 64 * PWAVES, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            n = 1;
+        }
+        const int64_t waves = (int64_t)n * std::min(XCD_CUS, ctx->num_cus) * PWAVES;
+        rows = std::max<int64_t>(PSINGLE, 64 * std::min<int64_t>(waves, PXS));
+    }
+    return rows;
+}
+
 int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, const void *A, int64_t lda,
              void *U, int64_t ldu, void *L, int64_t ldl, int64_t p, ElimResult &res)
 {
@@ -787,9 +810,11 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
 
     // Panels of an outer block starting at row KR by the rows left: the register
     // panel of one workgroup (256 rows: one wave per SIMD) or of one XCD, the
-    // W-resident panel beyond 16,384 rows.  Mod 65521 a 32-column panel takes
-    // 37 us on one workgroup and 45 us on an XCD, whatever its rows (one
-    // workgroup with 512 rows, two waves per SIMD: 58 us).
+    // W-resident panel beyond what an XCD holds (panel_rows).  Mod 65521 a
+    // 32-column panel takes 37 us on one workgroup, and on an XCD 45 us up to
+    // 4096 rows, 56 at 8192 and 76 at 16,384 (one workgroup with 512 rows, two
+    // waves per SIMD: 58 us).  The W-resident panel takes 17,000 rows at about
+    // 0.7 ms for 16 columns.
     // MODP_PANEL_GLOBAL=1 sends every panel to the W-resident kernel (used
     // to compare the two panel kernels at sizes both handle)
     const char *genv = getenv("MODP_PANEL_GLOBAL");
@@ -800,8 +825,9 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     const char *penv = getenv("MODP_PANEL_PATIENCE");
     const long long patience = penv ? atoll(penv) : 50000000LL;
     bool gave_up = false;  // in the previous outer block
+    const int arith = mp.small ? 0 : mp.p <= ((int64_t)1 << 24) ? 1 : 2;  // of the panels
     auto panel_width = [&](int64_t KR) {
-        return force_global || gave_up || m - KR > PMULTI ? GNBW : PNW;
+        return force_global || gave_up || m - KR > panel_rows(ctx, arith) ? GNBW : PNW;
     };
 
     int st = MODP_OK;
@@ -892,7 +918,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         a.KC = (int)KC; a.FAR = (int)FAR; a.mp = mp; a.invs = invs;
         a.ipiv = ipiv; a.pivcol = pivcol; a.map_dst = bmap_dst + t * 64; a.map_src = bmap_src + t * 64;
         a.stage = stage; a.ctl = bctl + blk * MAXPAN + t; a.solve = solve + t; a.abort = abort_flag;
-        TimedLaunch tl(ctx, "elim_panel");
+        TimedLaunch tl(ctx, "elim_panel_any");
         k_panel_any<<<1, 64 * PWAVES, 0, ctx->stream>>>(a);
         return hip_check(ctx, hipGetLastError(), "k_panel_any launch");
     };
@@ -903,7 +929,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         if (t >= MAXPAN) return set_error(ctx, MODP_ERR_DEVICE, "more than %d panels in an outer block", MAXPAN);
         int32_t *mdst = bmap_dst + t * 64, *msrc = bmap_src + t * 64;
         PanelCtl *pctl = bctl + blk * MAXPAN + t;
-        TimedLaunch tl(ctx, "elim_panel");
+        TimedLaunch tl(ctx, width == GNBW ? "elim_panel_global" : m - rj <= PSINGLE ? "elim_panel_one" : "elim_panel_xcd");
         if (width == GNBW) {
             k_panel_g<GNBW><<<1, GPT, 0, ctx->stream>>>(W, ldw, (int)m, (int)rj, (int)cj, (int)w, mp, ple, ipiv,
                                                         pivval, pivinv, pivcol, mdst, msrc, pctl, abort,
@@ -916,10 +942,9 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         a.ipiv = ipiv; a.pivval = pivval; a.pivinv = pivinv; a.pivcol = pivcol;
         a.map_dst = mdst; a.map_src = msrc; a.stage = stage; a.ctl = pctl; a.solve = solve + t; a.abort = abort; a.cursor = cursor;
         a.strict = strict;
-        const int mode = mp.small ? 0 : mp.p <= ((int64_t)1 << 24) ? 1 : 2;
         if (m - rj <= PSINGLE) {
-            if (mode == 0) k_panel<false, 0><<<1, PSINGLE, 0, ctx->stream>>>(a);
-            else if (mode == 1) k_panel<false, 1><<<1, PSINGLE, 0, ctx->stream>>>(a);
+            if (arith == 0) k_panel<false, 0><<<1, PSINGLE, 0, ctx->stream>>>(a);
+            else if (arith == 1) k_panel<false, 1><<<1, PSINGLE, 0, ctx->stream>>>(a);
             else k_panel<false, 2><<<1, PSINGLE, 0, ctx->stream>>>(a);
             return hip_check(ctx, hipGetLastError(), "k_panel launch");
         }
@@ -929,8 +954,8 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         a.patience = patience;
         MODP_TRY(next_tag(&a.tag));
         const unsigned grid = 8 * (a.G - 1) + 1;
-        if (mode == 0) k_panel<true, 0><<<grid, 256, 0, ctx->stream>>>(a);
-        else if (mode == 1) k_panel<true, 1><<<grid, 256, 0, ctx->stream>>>(a);
+        if (arith == 0) k_panel<true, 0><<<grid, 256, 0, ctx->stream>>>(a);
+        else if (arith == 1) k_panel<true, 1><<<grid, 256, 0, ctx->stream>>>(a);
         else k_panel<true, 2><<<grid, 256, 0, ctx->stream>>>(a);
         return hip_check(ctx, hipGetLastError(), "k_panel launch");
     };

@@ -45,8 +45,14 @@
 // The panel also leaves the inverse of its pivot triangle (PanelSolve), from the
 // upper half of the waves that rebuild rows, at no step of the chain.
 //
+// All workgroups have to be on the XCD at once.  The rows' own LDS is 66.6 KB,
+// and the scaled rows are int32 there rather than FP64, so that two workgroups
+// fit on a CU and 64 (16,384 rows) on an XCD.
+//
 // A 32-column panel mod 65521 takes 45 us at 4096 rows and 37 us at 256,
-// mod 2^26 - 5 51 and 48 (before the rows were published scaled, the
+// mod 2^26 - 5 51 and 48; at 8192 rows, where every CU has one workgroup, 56
+// and 65, with two of them on some or all CUs 66 and 80 at 9000 rows and 76 and
+// 89 at 16,384 (before the rows were published scaled, the
 // inverses looked up and the records moved off the chain: 50, 38, 60 and 53;
 // one 512-thread workgroup with eight rows a thread, unrolled, and the rows
 // published by one-lane LDS writes: 94 and 52 mod 65521, as four panels of 8
@@ -64,7 +70,7 @@ constexpr int PWAVES = 4;     // waves of a workgroup, one per SIMD
 constexpr int PXS = 256;      // slots of one exchange set (waves of a panel)
 constexpr int PINV = 1 << 18;  // entries of the table of small inverses
 constexpr int PSINGLE = 64 * PWAVES;  // rows of the one-workgroup panel
-constexpr int PMULTI = 64 * PXS;  // rows of the panel on one XCD
+constexpr int XCD_CUS = 32;   // CUs of an XCD
 constexpr uint32_t PABORT = 0x80000000u;
 constexpr uint32_t PUNSCALED = 0x80000000u;  // beside a row's tag: not scaled yet
 
@@ -350,7 +356,7 @@ template <int MODE> __device__ __forceinline__ uint64_t panel_best(uint32_t v, u
 }
 
 template <bool MULTI, int MODE>
-__global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
+__global__ __launch_bounds__(64 * PWAVES, MULTI ? 2 : 1) void k_panel(PanelArgs a)
 {
     typedef unsigned long long u64;
     int rank = 0;
@@ -379,7 +385,7 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     // original and reduced columns by local row, a wave's rows of 64 (the odd
     // pitch spreads a row of the panel over the banks)
     __shared__ int32_t s_A[PWAVES][PNW][65], s_L[PWAVES][PNW][65];
-    __shared__ double s_U[PNW][2 * PNW];  // scaled rows (negated) by column, and the rows of T
+    __shared__ int32_t s_U[PNW][2 * PNW];  // scaled rows (negated, balanced) by column, and the rows of T
     __shared__ __attribute__((aligned(16))) double s_key[2][PWAVES];
     __shared__ int s_go;
 
@@ -441,7 +447,7 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     double nl = 0.0, nup = 0.0;
     int Ipp = -2, atp = -2, Vp = 0;
     auto write_down = [&](int jc) __attribute__((always_inline)) {
-        s_U[jc & (PNW - 1)][lane] = nup;
+        s_U[jc & (PNW - 1)][lane] = (int32_t)nup;
         iq_l = iq_l == Ipp ? -1 : iq_l;
         const bool here = lane == atp;
         ip_l = here ? Ipp : ip_l;
@@ -673,15 +679,15 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel(PanelArgs a)
     if (rank == 0) {
         int32_t *const dst = Wp + (int64_t)col * ldw + kr0;
         constexpr int RPW = PNW / PWAVES;
-        double y[RPW];
+        int32_t y[RPW];
 #pragma unroll
         for (int q = 0; q < RPW; ++q) y[q] = s_U[wave + PWAVES * q][lane < PNW ? lane : PNW + pj_q];
 #pragma unroll
         for (int q = 0; q < RPW; ++q) {
             const int jc = wave + PWAVES * q, t = __popc(pivcols & ((1u << jc) - 1u));
             const bool piv = (pivcols >> jc) & 1u;
-            if (lane >= PNW) a.solve->t[jc][col] = piv && col < pc ? -(int32_t)y[q] : 0;
-            else if (piv && lane > jc && lane < w) dst[t] = (int32_t)(uint32_t)from_near(-y[q], mp);
+            if (lane >= PNW) a.solve->t[jc][col] = piv && col < pc ? -y[q] : 0;
+            else if (piv && lane > jc && lane < w) dst[t] = y[q] > 0 ? (int32_t)mp.p32 - y[q] : -y[q];
         }
         if (wave == 0 && lane < PNW)
             a.solve->num[lane] = ((pivcols >> lane) & 1u) ? (int)__popc(pivcols & ((1u << lane) - 1u)) : -1;

@@ -1,0 +1,49 @@
+"""Which kernel factors the panels, by the rows that are left: one workgroup, the
+workgroups of one XCD (all of them resident at once) or the matrix in memory.  The
+launches are counted by the names of the kernel timings."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+KERNELS = ("one", "xcd", "global", "any")
+
+
+def launches(ctx, run):
+    ctx.kernel_timing_reset()
+    ctx.kernel_timing(True)
+    try:
+        out = run()
+    finally:
+        ctx.kernel_timing(False)
+    return {k: ctx.kernel_time("elim_panel_" + k)[1] for k in KERNELS}, out
+
+
+@pytest.mark.parametrize("p", [251, 2 ** 23 - 15, 2 ** 26 - 5])
+@pytest.mark.parametrize("m", [256, 257, 4097, 8192, 8200, 12001, 16384])
+def test_panels_on_one_xcd(gffm, m, p):
+    g = gffm
+    Ah = O.draw_matrix(m, 150, p, seed=61)
+    A = g.CuModMatrix(Ah, p, elem_type=np.float64)
+    n, (U, L, P, Q, rank) = launches(A.ctx, lambda: g.pluq(A))
+    print(m, p, n, flush=True)
+    assert n["global"] == 0 and n["any"] == 0
+    assert n["xcd"] == {256: 0, 257: 1}.get(m, 5) and n["one"] == 5 - n["xcd"]
+    ref = O.pluq(Ah, p, O.PLUQ_OPTC)
+    assert rank == ref["rank"] and P == ref["row_swaps"] and Q == ref["col_swaps"]
+    assert np.array_equal(g.Array(U).astype(np.int64), ref["U"])
+    assert np.array_equal(g.Array(L)[:, :150].astype(np.int64), ref["L"][:, :150])
+
+
+def test_panels_of_more_rows(gffm):
+    g, p, m = gffm, 65521, 16385
+    Ah = O.draw_matrix(m, 40, p, seed=62)
+    A = g.CuModMatrix(Ah, p, elem_type=np.float64)
+    n, (U, L, P, Q, rank) = launches(A.ctx, lambda: g.pluq(A))
+    print(m, n, flush=True)
+    assert n["xcd"] == 0 and n["global"] > 0
+    ref = O.pluq(Ah, p, O.PLUQ_OPTC)
+    assert rank == ref["rank"] and P == ref["row_swaps"]
+    assert np.array_equal(g.Array(U).astype(np.int64), ref["U"])
