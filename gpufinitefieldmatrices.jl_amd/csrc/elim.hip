@@ -813,21 +813,31 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     // W-resident panel beyond what an XCD holds (panel_rows).  Mod 65521 a
     // 32-column panel takes 37 us on one workgroup, and on an XCD 45 us up to
     // 4096 rows, 56 at 8192 and 76 at 16,384 (one workgroup with 512 rows, two
-    // waves per SIMD: 58 us).  The W-resident panel takes 17,000 rows at about
-    // 0.7 ms for 16 columns.
+    // waves per SIMD: 58 us).  The W-resident panel takes 16,384
+    // rows in 0.55 ms for 16 columns.
     // MODP_PANEL_GLOBAL=1 sends every panel to the W-resident kernel (used
     // to compare the two panel kernels at sizes both handle)
     const char *genv = getenv("MODP_PANEL_GLOBAL");
     const bool force_global = genv && atoi(genv) != 0;
     // the cycles that a workgroup of a panel on one XCD waits for the others to
-    // start before the panel is left to the W-resident kernel
-    // (MODP_PANEL_PATIENCE sets it: 0 makes every such panel give up)
+    // start before the panel is left to the W-resident kernel: 2 ms, about what
+    // a block takes there (1.6 ms at 4096 rows, 4.4 at 16,384;
+    // MODP_PANEL_PATIENCE sets it; below 0 every such panel gives up).  They start together unless other work
+    // holds the XCD's CUs, perhaps another context's panel that waits in turn,
+    // so after a panel that gave up the W-resident kernel keeps `away` blocks,
+    // twice as many each time in a row, and the next try is one block.
     const char *penv = getenv("MODP_PANEL_PATIENCE");
-    const long long patience = penv ? atoll(penv) : 50000000LL;
-    bool gave_up = false;  // in the previous outer block
+    const long long patience = penv ? atoll(penv) : 5000000LL;
+    int away = 0, next_away = 1;
     const int arith = mp.small ? 0 : mp.p <= ((int64_t)1 << 24) ? 1 : 2;  // of the panels
-    auto panel_width = [&](int64_t KR) {
-        return force_global || gave_up || m - KR > panel_rows(ctx, arith) ? GNBW : PNW;
+    auto panel_width = [&](int64_t KR, int away) {
+        return force_global || (away > 0 && m - KR > PSINGLE) || m - KR > panel_rows(ctx, arith) ? GNBW : PNW;
+    };
+    // whether a block's panels met, if it had such panels
+    auto met = [&](int64_t KR, int width, bool yes) {
+        if (width != PNW || m - KR <= PSINGLE) return;
+        away = yes ? 0 : next_away;
+        next_away = yes ? 1 : std::min(2 * next_away, 64);
     };
 
     int st = MODP_OK;
@@ -1064,13 +1074,14 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         const bool any = any_pivot && hold == 0;
         {
             int64_t r = kr, c = kc;
+            int left = away;
             while ((int)blocks.size() < (hold > 0 ? std::min(hold, batch) : batch) && !careful && r < m) {
                 const int64_t colend = ple ? n : last + 1;  // columns usable as pivot columns
                 const int64_t nbo = std::min<int64_t>(std::min<int64_t>(colend - c, NBO), any ? m - r : NBO);
                 if (nbo <= 0 || (ple && r + nbo > m)) break;
                 Block b;
                 b.KR = r; b.KC = c; b.FAR = c + nbo; b.P = 0;
-                b.width = any ? PNW : panel_width(r);
+                b.width = any ? PNW : panel_width(r, left);
                 for (int64_t cj = c; cj < b.FAR && r + b.P < m;) {
                     const int64_t w = std::min(std::min<int64_t>(b.width, b.FAR - cj), m - (r + b.P));
                     b.rj.push_back(r + b.P); b.cj.push_back(cj); b.w.push_back(w);
@@ -1080,7 +1091,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 r += b.P;
                 c += b.P;
                 blocks.push_back(b);
-                if (gave_up && !any) break;
+                if (!any && left-- <= 0 && next_away > 1) break;
             }
         }
         bool stop_zero = false;
@@ -1090,6 +1101,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             if (!any) {
                 local_moves = false;
                 hold -= std::min(hold, (int)blocks.size());
+                away -= std::min(away, (int)blocks.size());
             }
             for (int i = 0; i < (int)blocks.size(); ++i) {
                 const Block &b = blocks[i];
@@ -1102,12 +1114,12 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 MODP_TRY(block_end(b.KR, b.KC, b.FAR, b.P, b.P, b.width, abort_flag));
             }
             MODP_TRY(read_back());
-            gave_up = false;
             nbo = blocks[0].FAR - blocks[0].KC;
             if (!reinterpret_cast<const int *>(hctl + NBATCH * MAXPAN)[1]) {
                 kr = blocks.back().KR + blocks.back().P;
                 kc = blocks.back().KC + blocks.back().P;
                 batch = std::min(2 * batch, NBATCH);
+                if (!any) met(blocks.back().KR, blocks.back().width, true);
             } else {
                 int i = 0, t = 0;
                 auto full = [&]() {
@@ -1124,7 +1136,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 const Block &b = blocks[i];
                 const PanelCtl pc = hctl[i * MAXPAN + t];
                 MODP_TRY(panel_error(pc));
-                gave_up = pc.status == 5;
+                if (pc.status == 5) met(b.KR, b.width, false);
                 int64_t P = 0;
                 for (int q = 0; q < t; ++q) P += b.w[q];
                 const int64_t consumed = P + pc.ncols;
@@ -1156,8 +1168,8 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             // abort flag, which turns the rest of the block into no-ops, and
             // the host reads the outcome once per block.
             const int64_t KR = kr, KC = kc, FAR = KC + std::min<int64_t>(n - KC, NBO);
-            const int NBW = panel_width(KR);
-            gave_up = false;
+            const int NBW = panel_width(KR, away);
+            away -= std::min(away, 1);
             local_moves = false;
             nbo = FAR - KC;
             MODP_TRY(blocks_begin(KR, 1));
@@ -1173,6 +1185,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
             }
             MODP_TRY(read_back());
             int64_t P = 0, consumed = 0;
+            bool gave_up = false;
             for (int t = 0; t < np; ++t) {
                 const PanelCtl &pc = hctl[t];
                 if (pc.status == 4) break;
@@ -1186,6 +1199,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                     break;
                 }
             }
+            met(KR, NBW, !gave_up);
             kr += P;
             kc += consumed;
             MODP_TRY(block_end(KR, KC, FAR, P, consumed, NBW, nullptr));

@@ -129,7 +129,7 @@ struct PanelArgs {
     uint32_t *arrive;
     int G;               // workgroups that take part
     uint32_t tag;        // tag of the step before the first
-    long long patience;  // cycles a workgroup waits for the others to start
+    long long patience;  // cycles a workgroup waits for the others to start; below 0 none goes on
 };
 
 // x mod p for exact integers |x| <= 2^51: fl(x * pinv) is within
@@ -292,7 +292,7 @@ __device__ __forceinline__ bool panel_meet(uint32_t *word, uint32_t G, long long
     for (;;) {
         const uint32_t cur = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (cur & PABORT) return false;
-        if ((cur & 0x7fu) == G) return cur == G * (1u + (x << 8) + (x * x << 17));
+        if ((cur & 0x7fu) == G && patience >= 0) return cur == G * (1u + (x << 8) + (x * x << 17));
         if ((long long)__builtin_readcyclecounter() - t0 > patience && atomicCAS(word, cur, cur | PABORT) == cur)
             return false;
         __builtin_amdgcn_s_sleep(1);

@@ -47,3 +47,36 @@ def test_panels_of_more_rows(gffm):
     ref = O.pluq(Ah, p, O.PLUQ_OPTC)
     assert rank == ref["rank"] and P == ref["row_swaps"]
     assert np.array_equal(g.Array(U).astype(np.int64), ref["U"])
+
+
+def test_tries_after_giving_up(gffm, monkeypatch):
+    # 15 blocks, every panel on an XCD gives up: after the first batch of eight
+    # blocks one block is tried at a time, with 1, 2, 4 and 8 blocks in between
+    monkeypatch.setenv("MODP_PANEL_PATIENCE", "-1")
+    g, p, m, blocks = gffm, 65521, 3000, 15
+    Ah = O.draw_matrix(m, 128 * blocks, p, seed=63)
+    A = g.CuModMatrix(Ah, p, elem_type=np.float64)
+    n, (U, L, P, Q, rank) = launches(A.ctx, lambda: g.pluq(A))
+    print(n, flush=True)
+    assert n["one"] == 0 and n["global"] == 8 * blocks
+    assert n["xcd"] == 4 * 8 + 4 * 3
+    ref = O.pluq(Ah, p, O.PLUQ_OPTC)
+    assert rank == ref["rank"] and P == ref["row_swaps"] and Q == ref["col_swaps"]
+    assert np.array_equal(g.Array(U).astype(np.int64), ref["U"])
+    assert np.array_equal(g.Array(L)[:, :rank].astype(np.int64), ref["L"][:, :rank])
+
+
+def test_tries_after_giving_up_lu(gffm, monkeypatch):
+    # blocks with zero columns go one by one
+    monkeypatch.setenv("MODP_PANEL_PATIENCE", "-1")
+    g, p, m = gffm, 65521, 1500
+    Ah = O.draw_matrix(m, 128 * 7, p, seed=64)
+    Ah[:, 5::100] = 0
+    A = g.CuModMatrix(Ah, p, elem_type=np.float64)
+    n, (U, L, perm, piv, rank) = launches(A.ctx, lambda: g.lu_full(A))
+    print(n, flush=True)
+    assert n["xcd"] > 0 and n["global"] > 0
+    ref = O.lu(Ah, p)
+    assert rank == ref["rank"] and perm == ref["perm"].tolist() and piv == ref["pivcols"].tolist()
+    assert np.array_equal(g.Array(U).astype(np.int64), ref["U"])
+    assert np.array_equal(g.Array(L).astype(np.int64), ref["L"])
