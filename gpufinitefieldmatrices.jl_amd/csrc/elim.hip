@@ -722,12 +722,13 @@ unsigned grid_for(int64_t total, int64_t cap = 16384)
 
 int64_t rup(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 
-// before a batch of blocks: no abort, the first row, nobody arrived
-__global__ void k_blocks_begin(int *abort, int *cursor, int row, uint32_t *arrive, int n)
+// before a batch of blocks: no abort, nothing lost, the first row, nobody arrived
+__global__ void k_blocks_begin(int *abort, int *lost, int *cursor, int row, uint32_t *arrive, int n)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) {
         *abort = 0;
+        *lost = 0;
         *cursor = row;
     }
     if (i < n) arrive[i] = 0;
@@ -790,9 +791,12 @@ static int64_t panel_rows(modp_ctx *ctx, int arith)
     return rows;
 }
 
-int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, const void *A, int64_t lda,
-             void *U, int64_t ldu, void *L, int64_t ldl, int64_t p, ElimResult &res)
+// One run from A to the outputs.  meet: panels may go to the workgroups of an
+// XCD; *lost: an exchange of theirs did not end, and nothing has been put out.
+static int elim_attempt(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, const void *A, int64_t lda,
+                        void *U, int64_t ldu, void *L, int64_t ldl, int64_t p, ElimResult &res, bool meet, bool *lost)
 {
+    *lost = false;
     const ModP mp = make_modp(p);
     const bool ple = mode != ELIM_PLUQ;
     const int64_t mn = m < n ? m : n;
@@ -829,9 +833,13 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     const char *penv = getenv("MODP_PANEL_PATIENCE");
     const long long patience = penv ? atoll(penv) : 5000000LL;
     int away = 0, next_away = 1;
+    // MODP_PANEL_SPINS sets how often they look again for a step's words (0: an
+    // exchange is lost when one is late, -1: at the first step)
+    const char *senv = getenv("MODP_PANEL_SPINS");
+    const int spins = senv ? atoi(senv) : EXCHANGE_SPINS;
     const int arith = mp.small ? 0 : mp.p <= ((int64_t)1 << 24) ? 1 : 2;  // of the panels
     auto panel_width = [&](int64_t KR, int away) {
-        return force_global || (away > 0 && m - KR > PSINGLE) || m - KR > panel_rows(ctx, arith) ? GNBW : PNW;
+        return force_global || ((away > 0 || !meet) && m - KR > PSINGLE) || m - KR > panel_rows(ctx, arith) ? GNBW : PNW;
     };
     // whether a block's panels met, if it had such panels
     auto met = [&](int64_t KR, int width, bool yes) {
@@ -856,7 +864,8 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     PanelCtl *bctl = (PanelCtl *)(bmap_src + MAXPAN * 64);  // by block of the batch
     int *flag = (int *)(bctl + NBATCH * MAXPAN);
     int *abort_flag = flag + 1;
-    int *cursor = flag + 2;                         // first row of the next panel (lu, rref)
+    int *lost_flag = flag + 2;
+    int *cursor = flag + 3;                         // first row of the next panel (lu, rref)
     uint32_t *arrive = (uint32_t *)(flag + 4);      // one word per panel of the batch
     int32_t *stage = (int32_t *)(arrive + NBATCH * MAXPAN);  // moved rows' old values, 64 x NBO
     PanelSolve *solve = (PanelSolve *)(stage + 64 * NBO);  // one per panel of the block
@@ -962,6 +971,8 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         a.arrive = arrive + blk * MAXPAN + t;
         a.G = (int)((m - rj + 255) / 256);
         a.patience = patience;
+        a.spins = spins;
+        a.lost = lost_flag;
         MODP_TRY(next_tag(&a.tag));
         const unsigned grid = 8 * (a.G - 1) + 1;
         if (arith == 0) k_panel<true, 0><<<grid, 256, 0, ctx->stream>>>(a);
@@ -971,14 +982,16 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
     };
     auto blocks_begin = [&](int64_t row, int blocks) -> int {
         k_blocks_begin<<<(unsigned)((blocks * MAXPAN + 255) / 256), 256, 0, ctx->stream>>>(
-            abort_flag, cursor, (int)row, arrive, blocks * MAXPAN);
+            abort_flag, lost_flag, cursor, (int)row, arrive, blocks * MAXPAN);
         return hip_check(ctx, hipGetLastError(), "k_blocks_begin launch");
     };
     // the control blocks of the batch and the flags after them
     auto read_back = [&]() -> int {
-        HIP_TRY(ctx, hipMemcpyAsync(hctl, bctl, sizeof(PanelCtl) * NBATCH * MAXPAN + 2 * sizeof(int),
+        HIP_TRY(ctx, hipMemcpyAsync(hctl, bctl, sizeof(PanelCtl) * NBATCH * MAXPAN + 3 * sizeof(int),
                                     hipMemcpyDeviceToHost, ctx->stream));
-        return hip_check(ctx, hipStreamSynchronize(ctx->stream), "elimination blocks");
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+        *lost = reinterpret_cast<const int *>(hctl + NBATCH * MAXPAN)[2] != 0;
+        return MODP_OK;
     };
     // the rest of the outer block [KC, FAR) from row KR after panel t: its row
     // moves, and right of the panel the rows of U and the rank-npiv update below
@@ -1050,7 +1063,6 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         if (c.status == 3)
             return set_error(ctx, MODP_ERR_NOT_INVERTIBLE, "pivot has no inverse modulo %lld (modulus not prime)",
                              (long long)p);
-        if (c.status == 6) return set_error(ctx, MODP_ERR_DEVICE, "an elimination panel's exchange did not end");
         return MODP_OK;
     };
     // A batch of blocks is enqueued as if every panel of it found a pivot in
@@ -1114,6 +1126,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 MODP_TRY(block_end(b.KR, b.KC, b.FAR, b.P, b.P, b.width, abort_flag));
             }
             MODP_TRY(read_back());
+            if (*lost) return MODP_OK;
             nbo = blocks[0].FAR - blocks[0].KC;
             if (!reinterpret_cast<const int *>(hctl + NBATCH * MAXPAN)[1]) {
                 kr = blocks.back().KR + blocks.back().P;
@@ -1184,6 +1197,7 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
                 MODP_TRY(update_t(0, t, false, KR, KC, FAR, KR, pcj[t], pw[t], abort_flag));
             }
             MODP_TRY(read_back());
+            if (*lost) return MODP_OK;
             int64_t P = 0, consumed = 0;
             bool gave_up = false;
             for (int t = 0; t < np; ++t) {
@@ -1272,6 +1286,15 @@ int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, 
         for (int64_t i = 0; i < rank; ++i) std::swap(res.perm[i], res.perm[hp[i]]);
     }
     return MODP_OK;
+}
+
+int elim_run(modp_ctx *ctx, int mode, int form, int kind, int64_t m, int64_t n, const void *A, int64_t lda,
+             void *U, int64_t ldu, void *L, int64_t ldl, int64_t p, ElimResult &res)
+{
+    bool lost = false;
+    MODP_TRY(elim_attempt(ctx, mode, form, kind, m, n, A, lda, U, ldu, L, ldl, p, res, true, &lost));
+    if (!lost) return MODP_OK;
+    return elim_attempt(ctx, mode, form, kind, m, n, A, lda, U, ldu, L, ldl, p, res, false, &lost);
 }
 
 // Inverse under a prime modulus: [A | I] to [U | Y] with any pivots, then

@@ -129,6 +129,8 @@ struct PanelArgs {
     uint32_t *arrive;
     int G;               // workgroups that take part
     uint32_t tag;        // tag of the step before the first
+    int *lost;           // raised by a wave whose exchange did not end
+    int spins;           // EXCHANGE_SPINS
     long long patience;  // cycles a workgroup waits for the others to start; below 0 none goes on
 };
 
@@ -312,7 +314,7 @@ __device__ __forceinline__ void exchange_store(unsigned long long *p, unsigned l
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-constexpr int EXCHANGE_SPINS = 1 << 20;
+constexpr int EXCHANGE_SPINS = 1 << 20;  // looks at a word before its step counts as lost
 
 // Arithmetic of a panel by the modulus.  The columns are exact integers in
 // FP64 and one FMA applies a pivot; multipliers and scaled rows are balanced
@@ -583,7 +585,7 @@ __global__ __launch_bounds__(64 * PWAVES, MULTI ? 2 : 1) void k_panel(PanelArgs 
                         const int idx = min(b + lane, nw - 1);
                         if (b != 0) t = exchange_load(&a.x->key[par][idx], spins);
                         while (!__all((uint32_t)(t & 0x1ffffu) == tag17)) {
-                            if (++spins > EXCHANGE_SPINS) break;
+                            if (++spins > a.spins) break;
                             t = exchange_load(&a.x->key[par][idx], spins);
                         }
                         if (t > kt || b == 0) {
@@ -611,13 +613,13 @@ __global__ __launch_bounds__(64 * PWAVES, MULTI ? 2 : 1) void k_panel(PanelArgs 
                     u64 *rp = &a.x->row[par][at][lane];
                     u64 t = exchange_load(rp, 0);
                     while (piv && !__all((((uint32_t)t ^ tag) & ~PUNSCALED) == 0)) {
-                        if (++spins > EXCHANGE_SPINS) break;
+                        if (++spins > a.spins) break;
                         t = exchange_load(rp, spins);
                     }
                     nu = (double)(int32_t)(t >> 32);
                     const bool unscaled = __any((uint32_t)t & PUNSCALED);
-                    if (__builtin_expect(!piv || unscaled || spins > EXCHANGE_SPINS, 0)) {
-                        const uint32_t inv = piv && spins <= EXCHANGE_SPINS ? search_inverse(V, a.invs, mp, lane) : 0u;
+                    if (__builtin_expect(!piv || unscaled || spins > a.spins, 0)) {
+                        const uint32_t inv = piv && spins <= a.spins ? search_inverse(V, a.invs, mp, lane) : 0u;
                         nu = scaled(nu, inv);
                         piv = inv != 0;
                     }
@@ -633,7 +635,7 @@ __global__ __launch_bounds__(64 * PWAVES, MULTI ? 2 : 1) void k_panel(PanelArgs 
                     nu = scaled(x, inv);
                 }
                 if (__builtin_expect(!piv, 0)) {
-                    const bool lost = spins > EXCHANGE_SPINS;
+                    const bool lost = spins > a.spins;
                     if (V != 0 || !a.ple || lost) {
                         // a zero column (lu and rref skip it, pluq stops), or no inverse
                         status = lost ? 6 : V == 0 ? 1 : 3;
@@ -768,6 +770,13 @@ __global__ __launch_bounds__(64 * PWAVES, MULTI ? 2 : 1) void k_panel(PanelArgs 
             for (int c = 0; c < nother; ++c)
                 dst[64 * c] = a.W[from + (int64_t)(c < nleft ? a.KC + c : a.KC + c + w) * ldw];
         }
+    }
+    // A wave that misses a step publishes nothing more, so the others miss the
+    // next one; but after the last step only the wave itself knows.  Its rows
+    // are wrong then: the whole elimination starts again from its input.
+    if (MULTI && status == 6 && lane == 0) {
+        *a.lost = 1;
+        *a.abort = 1;
     }
     if (gw == 0 && lane == 0) {
         *a.ctl = PanelCtl{pc, status, consumed, pc + (int)__popc(mask), kr0};

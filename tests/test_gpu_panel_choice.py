@@ -80,3 +80,33 @@ def test_tries_after_giving_up_lu(gffm, monkeypatch):
     assert rank == ref["rank"] and perm == ref["perm"].tolist() and piv == ref["pivcols"].tolist()
     assert np.array_equal(g.Array(U).astype(np.int64), ref["U"])
     assert np.array_equal(g.Array(L).astype(np.int64), ref["L"])
+
+
+@pytest.mark.parametrize("spins", [-1, 0, 1])
+@pytest.mark.parametrize("p", [7, 65521, 2 ** 26 - 5])
+@pytest.mark.parametrize("m,n", [(300, 20), (700, 300), (3000, 260)])
+def test_exchange_that_does_not_end(gffm, monkeypatch, m, n, p, spins):
+    # the elimination starts again from its input; from 0 on some wave may lose
+    # some step, below every wave the first one
+    monkeypatch.setenv("MODP_PANEL_SPINS", str(spins))
+    g = gffm
+    Ah = O.draw_matrix(m, n, p, seed=65)
+    A = g.CuModMatrix(Ah, p, elem_type=np.float64)
+    count, (U, L, P, Q, rank) = launches(A.ctx, lambda: g.pluq(A))
+    print(m, n, p, spins, count, flush=True)
+    assert count["xcd"] > 0 and (count["global"] > 0 or spins >= 0)
+    ref = O.pluq(Ah, p, O.PLUQ_OPTC)
+    assert rank == ref["rank"] and P == ref["row_swaps"] and Q == ref["col_swaps"]
+    assert np.array_equal(g.Array(U).astype(np.int64), ref["U"])
+    assert np.array_equal(g.Array(L).astype(np.int64), ref["L"])
+    Ah[:, ::7] = 0
+    A = g.CuModMatrix(Ah, p, elem_type=np.float64)
+    U, L, perm, piv, rank = g.lu_full(A)
+    ref = O.lu(Ah, p)
+    assert rank == ref["rank"] and perm == ref["perm"].tolist() and piv == ref["pivcols"].tolist()
+    assert np.array_equal(g.Array(U).astype(np.int64), ref["U"])
+    assert np.array_equal(g.Array(L).astype(np.int64), ref["L"])
+    # no pivot in the first rows: rref with panels that meet, too
+    Ah[:64] = 0
+    A = g.CuModMatrix(Ah, p, elem_type=np.float64)
+    assert np.array_equal(g.Array(g.rref(A)).astype(np.int64), O.rref(Ah, p)["R"])
