@@ -101,6 +101,12 @@ void *ws_get(modp_ctx *ctx, int slot, size_t bytes, int *status)
     return p;
 }
 
+bool capturing(modp_ctx *ctx)
+{
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+}
+
 void *pinned_get(modp_ctx *ctx, size_t bytes, int *status)
 {
     if (ctx->pinned_size >= bytes) return ctx->pinned;

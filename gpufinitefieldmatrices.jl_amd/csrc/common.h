@@ -344,6 +344,9 @@ int hip_check(modp_ctx *ctx, hipError_t e, const char *what);
 hipError_t device_alloc(modp_ctx *ctx, void **p, size_t bytes);
 void *ws_get(modp_ctx *ctx, int slot, size_t bytes, int *status);
 void *pinned_get(modp_ctx *ctx, size_t bytes, int *status);
+// whether the context's stream is being captured into a graph: no workspace can
+// grow then, and one that does not grow may be gone when the graph runs
+bool capturing(modp_ctx *ctx);
 
 // timing hooks around hot kernel launches
 struct TimedLaunch {

@@ -467,14 +467,15 @@ int gemm_plain_cfg(modp_ctx *ctx, const GemmArgs &g, const GemmConfig &cfg)
     const int R = f64_reduce_interval(g.mp.p);
     if (R < 1) return set_error(ctx, MODP_ERR_MODULUS_RANGE, "modulus %lld too large for the FP64 form", (long long)g.mp.p);
     // a C over an operand is written only after all workgroups have read it:
-    // through the residues of the slices, also where there is one slice
+    // through the residues of the slices, also where there is one slice (a
+    // single tile's workgroup has read everything before it stores)
     const bool over = over_operand(g);
     if (!over && f64_small(g)) return launch_f64_small(ctx, g, R, 1, 0, 0, 0, GemmSize{g.m, g.n, g.k});
     const int tile = cfg.tile_m == 128 ? 128 : 64;
     Slices sl = make_slices(g.k, cfg.ksplit, PBK, 64);
     if (sl.S == 1) {
         sl.kslice = g.k > 0 ? g.k : 1;
-        if (!over) return launch_f64(ctx, g, R, tile, sl);
+        if (!over || (g.m <= 64 && g.n <= 64)) return launch_f64(ctx, g, R, tile, sl);
     }
     int st = MODP_OK;
     int32_t *P = slice_buffer(ctx, g, sl.S, &st);
@@ -756,7 +757,8 @@ int gemv_t(modp_ctx *ctx, int64_t m, int64_t k, const T *A, int64_t lda, const T
     int64_t S = 2 * (int64_t)ctx->num_cus / rb;
     if (S > k / (4 * 2 * GV_U)) S = k / (4 * 2 * GV_U);
     if (S > 128) S = 128;
-    if (S < 1) S = 1;
+    // one slice needs no workspace
+    if (S < 1 || (S > 1 && k <= 512 && capturing(ctx))) S = 1;
     const int64_t kslice = round_up(((k > 0 ? k : 1) + S - 1) / S, 4 * GV_U);
     S = k > 0 ? (k + kslice - 1) / kslice : 1;
     // y over x or within A: nothing of y is written before all of both is read
