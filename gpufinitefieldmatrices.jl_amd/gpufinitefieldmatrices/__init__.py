@@ -104,6 +104,20 @@ _STATUS_EXC = {
 # context and device buffers
 # ---------------------------------------------------------------------------
 
+class _Handle:
+    """The library's context, destroyed after everything that was made from
+    it: the finalizers of buffers and plans hold it, and a cycle of Python
+    objects that is collected at once runs its finalizers in no fixed order."""
+
+    def __init__(self, lib, h):
+        self.h = h
+        self._fin = weakref.finalize(self, lib.modp_ctx_destroy, h)
+
+
+def _release(f, handle: _Handle, what):
+    f(handle.h, what)
+
+
 class Context:
     """One device, one HIP stream, the library's workspaces."""
 
@@ -116,7 +130,7 @@ class Context:
                               "(needs an MI355X / gfx950 GPU)")
         self.h = h
         self.device = device
-        self._fin = weakref.finalize(self, self.lib.modp_ctx_destroy, h)
+        self._handle = _Handle(self.lib, h)
 
     def check(self, st: int, what: str = ""):
         if st == 0:
@@ -222,7 +236,7 @@ class DeviceBuffer:
         p = ctypes.c_void_p()
         ctx.check(ctx.lib.modp_malloc(ctx.h, max(1, self.nbytes), ctypes.byref(p)), "malloc")
         self.ptr = p.value
-        self._fin = weakref.finalize(self, ctx.lib.modp_free, ctx.h, ctypes.c_void_p(self.ptr))
+        self._fin = weakref.finalize(self, _release, ctx.lib.modp_free, ctx._handle, ctypes.c_void_p(self.ptr))
 
     def upload(self, host: np.ndarray):
         host = np.ascontiguousarray(host) if not host.flags.f_contiguous else host
@@ -849,7 +863,7 @@ class GemmBatchPlan:
         self.ctx.check(self.ctx.lib.modp_gemm_batched_plan(self.ctx.h, _dtype_code(elem_type), arr, len(jobs),
                                                            ctypes.byref(h)), "gemm_batched_plan")
         self.h = h
-        self._fin = weakref.finalize(self, self.ctx.lib.modp_gemm_batched_destroy, self.ctx.h, h)
+        self._fin = weakref.finalize(self, _release, self.ctx.lib.modp_gemm_batched_destroy, self.ctx._handle, h)
 
     def run(self):
         self.ctx.check(self.ctx.lib.modp_gemm_batched_run(self.ctx.h, self.h), "gemm_batched_run")
@@ -873,7 +887,7 @@ class ElimBatchPlan:
         self.ctx.check(self.ctx.lib.modp_elim_batched_plan(self.ctx.h, int(op), _dtype_code(elem_type), arr,
                                                            len(jobs_raw), ctypes.byref(h)), "elim_batched_plan")
         self.h = h
-        self._fin = weakref.finalize(self, self.ctx.lib.modp_elim_batched_destroy, self.ctx.h, h)
+        self._fin = weakref.finalize(self, _release, self.ctx.lib.modp_elim_batched_destroy, self.ctx._handle, h)
 
     def run(self):
         self.ctx.check(self.ctx.lib.modp_elim_batched_run(self.ctx.h, self.h), "elim_batched_run")
