@@ -47,6 +47,15 @@ static FreedMemory *freed_memory(int device)
 
 static size_t freed_units(size_t bytes) { return (bytes + FREED_UNIT - 1) / FREED_UNIT * FREED_UNIT; }
 
+// The contexts there are.  Finalizers of another language's objects may free
+// their memory after the context is gone; never destroyed, either.
+static std::mutex g_contexts_mu;
+static std::unordered_set<modp_ctx *> &contexts()
+{
+    static auto *all = new std::unordered_set<modp_ctx *>();
+    return *all;
+}
+
 // bytes of the runtime's allocation at p, 0 if there is none
 static size_t allocated_at(void *p)
 {
@@ -277,6 +286,10 @@ int modp_ctx_create(int device, modp_ctx **out)
         delete c;
         return MODP_ERR_DEVICE;
     }
+    {
+        std::lock_guard<std::mutex> lk(g_contexts_mu);
+        contexts().insert(c);
+    }
     *out = c;
     return MODP_OK;
 }
@@ -284,6 +297,10 @@ int modp_ctx_create(int device, modp_ctx **out)
 int modp_ctx_destroy(modp_ctx *ctx)
 {
     if (!ctx) return MODP_OK;
+    {
+        std::lock_guard<std::mutex> lk(g_contexts_mu);
+        if (contexts().erase(ctx) == 0) return MODP_ERR_ARG;
+    }
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     for (int i = 0; i < WS_COUNT; ++i)
@@ -345,6 +362,11 @@ int modp_malloc(modp_ctx *ctx, size_t bytes, void **dptr)
 
 int modp_free(modp_ctx *ctx, void *dptr)
 {
+    {
+        std::lock_guard<std::mutex> lk(g_contexts_mu);
+        if (ctx && contexts().count(ctx) == 0)
+            return !dptr || hipFree(dptr) == hipSuccess ? MODP_OK : MODP_ERR_DEVICE;
+    }
     CTX_CHECK(ctx);
     if (!dptr) return MODP_OK;
     FreedMemory &f = *ctx->memory;

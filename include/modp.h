@@ -85,7 +85,8 @@ void *modp_stream(modp_ctx *ctx);
  * and processes do not see that memory as free; it is released when one of the
  * library's own allocations on the device would fail, when a context of the
  * device is destroyed, and by modp_release_freed, which returns the bytes in
- * *bytes (NULL: not wanted). */
+ * *bytes (NULL: not wanted).  modp_free may come after the context has been
+ * destroyed (finalizers in no fixed order): then it only releases. */
 int modp_malloc(modp_ctx *ctx, size_t bytes, void **dptr);
 int modp_free(modp_ctx *ctx, void *dptr);
 int modp_release_freed(modp_ctx *ctx, size_t *bytes);

@@ -123,3 +123,15 @@ def test_release(gffm):
     assert not any(allocated(runtime, p) for p in blocks)
     assert ctx.release_freed() == 0
     assert ctx.lib.modp_release_freed(ctx.h, None) == 0
+
+
+def test_freed_after_the_context(gffm):
+    lib, runtime = gffm.context().lib, hip()
+    h, p = ctypes.c_void_p(), ctypes.c_void_p()
+    assert lib.modp_ctx_create(0, ctypes.byref(h)) == 0
+    assert lib.modp_malloc(h, 3 << 20, ctypes.byref(p)) == 0
+    assert lib.modp_ctx_destroy(h) == 0
+    assert allocated(runtime, p) >= 3 << 20
+    assert lib.modp_free(h, p) == 0 and lib.modp_free(h, None) == 0
+    assert allocated(runtime, p) == 0
+    assert lib.modp_ctx_destroy(h) != 0  # once
