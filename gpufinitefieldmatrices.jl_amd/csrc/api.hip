@@ -78,26 +78,31 @@ hipError_t device_alloc(modp_ctx *ctx, void **p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory) {
+        // (the failure stays the runtime's last error until somebody asks)
+        (void)hipGetLastError();
         std::lock_guard<std::mutex> lk(ctx->memory->mu);
         if (ctx->memory->freed.empty()) return e;
-        (void)hipGetLastError();
         release_freed(*ctx->memory);
         e = hipMalloc(p, bytes);
+        if (e != hipSuccess) (void)hipGetLastError();
     }
     return e;
+}
+
+void ws_drop(modp_ctx *ctx, int slot)
+{
+    if (!ctx->ws[slot]) return;
+    (void)hipStreamSynchronize(ctx->stream);
+    (void)hipFree(ctx->ws[slot]);
+    ctx->ws[slot] = nullptr;
+    ctx->ws_size[slot] = 0;
 }
 
 void *ws_get(modp_ctx *ctx, int slot, size_t bytes, int *status)
 {
     if (bytes == 0) bytes = 256;
     if (ctx->ws_size[slot] >= bytes) return ctx->ws[slot];
-    if (ctx->ws[slot]) {
-        // in-flight kernels may still read the old buffer
-        (void)hipStreamSynchronize(ctx->stream);
-        (void)hipFree(ctx->ws[slot]);
-        ctx->ws[slot] = nullptr;
-        ctx->ws_size[slot] = 0;
-    }
+    ws_drop(ctx, slot);  // (waits: in-flight kernels may still read the old buffer)
     size_t sz = (bytes + 4095) & ~(size_t)4095;
     void *p = nullptr;
     hipError_t e = device_alloc(ctx, &p, sz);

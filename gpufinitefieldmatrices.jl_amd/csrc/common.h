@@ -343,6 +343,7 @@ int hip_check(modp_ctx *ctx, hipError_t e, const char *what);
 // hipMalloc, once more without the freed memory if that fails
 hipError_t device_alloc(modp_ctx *ctx, void **p, size_t bytes);
 void *ws_get(modp_ctx *ctx, int slot, size_t bytes, int *status);
+void ws_drop(modp_ctx *ctx, int slot);
 void *pinned_get(modp_ctx *ctx, size_t bytes, int *status);
 // whether the context's stream is being captured into a graph: no workspace can
 // grow then, and one that does not grow may be gone when the graph runs

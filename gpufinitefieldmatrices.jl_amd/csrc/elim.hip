@@ -699,16 +699,30 @@ __global__ void k_column_kinds(const int32_t *__restrict__ pivcol, int rank, int
 }
 
 // the reduced echelon form: unit vectors in the pivots' columns, Z elsewhere
+// (pivots_only: nothing there)
 template <typename T>
-__global__ void k_write_rref(int64_t m, int64_t n, int rank, const int32_t *__restrict__ kinds,
+__global__ void k_write_rref(int64_t m, int64_t n, int rank, const int32_t *__restrict__ kinds, bool pivots_only,
                              const int32_t *__restrict__ Z, int64_t ldz, T *__restrict__ R, int64_t ldr)
 {
     const int64_t total = m * n;
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
         const int64_t r = e % m, c = e / m;
         const int k = kinds[c];
+        if (k < 0 && pivots_only) continue;
         const uint32_t v = k >= 0 ? (uint32_t)(r == k) : r < rank ? (uint32_t)Z[r + (int64_t)(-1 - k) * ldz] : 0u;
         R[r + c * ldr] = from_res<T>(v);
+    }
+}
+
+// nf of the other columns
+template <typename T>
+__global__ void k_write_free(int64_t m, int64_t nf, int rank, const int32_t *__restrict__ free_cols,
+                             const int32_t *__restrict__ Z, int64_t ldz, T *__restrict__ R, int64_t ldr)
+{
+    const int64_t total = m * nf;
+    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t r = e % m, j = e / m;
+        R[r + free_cols[j] * ldr] = from_res<T>(r < rank ? (uint32_t)Z[r + j * ldz] : 0u);
     }
 }
 
@@ -1327,6 +1341,114 @@ int elim_inverse(modp_ctx *ctx, int form, int kind, int64_t n, const void *A, in
     return gemm_run(ctx, g, gemm_default_config(ctx, g, form));
 }
 
+// U of a factored W: unit upper triangular in the pivots' columns
+struct Echelon {
+    const int32_t *W;
+    int64_t ldw, rank, nfree;
+    const int32_t *pivcol, *free_cols;
+    bool first;  // the pivots are in the first columns
+};
+
+static GemmArgs i32_product(int64_t m, int64_t n, int64_t k, const int32_t *A, int64_t lda, const int32_t *B, int64_t ldb,
+                            int32_t *C, int64_t ldc, int epi, const ModP &mp)
+{
+    GemmArgs g;
+    g.m = m; g.n = n; g.k = k;
+    g.A = A; g.lda = lda; g.ka = EK_I32;
+    g.B = B; g.ldb = ldb; g.kb = EK_I32;
+    g.C = C; g.ldc = ldc; g.kc = EK_I32;
+    g.epi = epi;
+    g.mp = mp;
+    return g;
+}
+
+// Z = U_piv^{-1} U_free (leading dimension rank rounded up to 64) by one triangular inverse and one product
+static int rref_free(modp_ctx *ctx, int form, const Echelon &u, const ModP &mp, int32_t **Zout)
+{
+    const int64_t rank = u.rank, nfree = u.nfree, ld = rup(rank, 64);
+    int st = MODP_OK;
+    // pivots in the first columns: U_piv and U_free are where they are
+    const int32_t *T = u.W, *Y = u.W + rank * u.ldw;
+    int64_t ldt = u.ldw, ldy = u.ldw;
+    if (!u.first) {
+        int32_t *Tg = (int32_t *)ws_get(ctx, WS_TRI_T, sizeof(int32_t) * (size_t)ld * (size_t)rank, &st);
+        if (!Tg) return st;
+        int32_t *Yg = (int32_t *)ws_get(ctx, WS_INV_U, sizeof(int32_t) * (size_t)ld * (size_t)nfree, &st);
+        if (!Yg) return st;
+        k_gather_cols<<<grid_for(rank * rank), 256, 0, ctx->stream>>>(u.W, u.ldw, rank, u.pivcol, u.pivcol, rank, Tg, ld);
+        HIP_TRY(ctx, hipGetLastError());
+        k_gather_cols<<<grid_for(rank * nfree), 256, 0, ctx->stream>>>(u.W, u.ldw, rank, u.pivcol, u.free_cols, nfree, Yg, ld);
+        HIP_TRY(ctx, hipGetLastError());
+        T = Tg; Y = Yg;
+        ldt = ldy = ld;
+    }
+    int32_t *X = (int32_t *)ws_get(ctx, WS_TRI_X, sizeof(int32_t) * (size_t)ld * (size_t)rank, &st);
+    if (!X) return st;
+    int32_t *Z = (int32_t *)ws_get(ctx, WS_INV_L, sizeof(int32_t) * (size_t)ld * (size_t)nfree, &st);
+    if (!Z) return st;
+    MODP_TRY(trinv_i32(ctx, true, T, ldt, X, ld, rank, mp));
+    const GemmArgs g = i32_product(rank, nfree, rank, X, ld, Y, ldy, Z, ld, EPI_STORE, mp);
+    MODP_TRY(gemm_run(ctx, g, gemm_default_config(ctx, g, form)));
+    *Zout = Z;
+    return MODP_OK;
+}
+
+// The same by back substitution, RB_ROWS pivots at a time and RB_COLS free
+// columns at a time, written out as they are done: workspaces of about 2 RB_ROWS
+// + RB_COLS columns, where the inverse and the product above take up to 2.5
+// rank + 2 nfree columns and the product's residue planes.  For matrices with
+// no room for those beside them: mod 65521 a whole call of 16,384^2 and rank
+// 12,000 takes 46 ms instead of 44, 4096^2 and rank 3000 4.13 instead of 3.73.
+constexpr int64_t RB_ROWS = 512, RB_COLS = 1024;
+template <typename T>
+static int rref_free_blocks(modp_ctx *ctx, int form, const Echelon &u, const ModP &mp, int64_t m, T *R, int64_t ldr)
+{
+    const int64_t rank = u.rank, ld = rup(rank, 64), nc = std::min(u.nfree, RB_COLS);
+    int st = MODP_OK;
+    int32_t *P = (int32_t *)ws_get(ctx, WS_TRI_T, sizeof(int32_t) * (size_t)ld * (size_t)RB_ROWS, &st);
+    if (!P) return st;
+    int32_t *X = (int32_t *)ws_get(ctx, WS_TRI_X, sizeof(int32_t) * (size_t)RB_ROWS * (size_t)rank, &st);
+    if (!X) return st;
+    int32_t *Y = (int32_t *)ws_get(ctx, WS_INV_U, sizeof(int32_t) * (size_t)ld * (size_t)nc, &st);
+    if (!Y) return st;
+    int32_t *Z = (int32_t *)ws_get(ctx, WS_INV_L, sizeof(int32_t) * (size_t)RB_ROWS * (size_t)nc, &st);
+    if (!Z) return st;
+    auto product = [&](const GemmArgs &g) -> int {
+        const int use = form != MODP_FORM_AUTO ? form : choose_form(g.m, g.n, g.k, mp.p);
+        return use == MODP_FORM_LIMB_I8 ? gemm_limb_i8(ctx, g) : gemm_plain_f64(ctx, g);
+    };
+    // rows [r0, r0 + rows) of the pivots' columns [c0, c0 + cols)
+    auto gather = [&](int64_t r0, int64_t rows, int64_t c0, int64_t cols) -> int {
+        k_gather_cols<<<grid_for(rows * cols), 256, 0, ctx->stream>>>(u.W + r0, u.ldw, rows, u.pivcol + r0,
+                                                                      u.pivcol + c0, cols, P, ld);
+        return hip_check(ctx, hipGetLastError(), "k_gather_cols launch");
+    };
+    const int64_t blocks = (rank + RB_ROWS - 1) / RB_ROWS;
+    for (int64_t b = 0; b < blocks; ++b) {
+        const int64_t r0 = b * RB_ROWS, nb = std::min(RB_ROWS, rank - r0);
+        MODP_TRY(gather(r0, nb, r0, nb));
+        MODP_TRY(trinv_i32(ctx, true, P, ld, X + r0 * RB_ROWS, RB_ROWS, nb, mp));
+    }
+    for (int64_t f0 = 0; f0 < u.nfree; f0 += nc) {
+        const int64_t nf = std::min(nc, u.nfree - f0);
+        k_gather_cols<<<grid_for(rank * nf), 256, 0, ctx->stream>>>(u.W, u.ldw, rank, u.pivcol, u.free_cols + f0, nf, Y, ld);
+        HIP_TRY(ctx, hipGetLastError());
+        for (int64_t b = blocks - 1; b >= 0; --b) {
+            const int64_t r0 = b * RB_ROWS, nb = std::min(RB_ROWS, rank - r0);
+            MODP_TRY(product(i32_product(nb, nf, nb, X + r0 * RB_ROWS, RB_ROWS, Y + r0, ld, Z, RB_ROWS, EPI_STORE, mp)));
+            HIP_TRY(ctx, hipMemcpy2DAsync(Y + r0, sizeof(int32_t) * (size_t)ld, Z, sizeof(int32_t) * (size_t)RB_ROWS,
+                                          sizeof(int32_t) * (size_t)nb, (size_t)nf, hipMemcpyDeviceToDevice, ctx->stream));
+            if (r0 == 0) break;
+            if (!u.first) MODP_TRY(gather(0, r0, r0, nb));
+            MODP_TRY(product(i32_product(r0, nf, nb, u.first ? u.W + r0 * u.ldw : P, u.first ? u.ldw : ld, Z, RB_ROWS, Y,
+                                         ld, EPI_SUB, mp)));
+        }
+        k_write_free<T><<<grid_for(m * nf), 256, 0, ctx->stream>>>(m, nf, (int)rank, u.free_cols + f0, Y, ld, R, ldr);
+        HIP_TRY(ctx, hipGetLastError());
+    }
+    return MODP_OK;
+}
+
 // Reduced echelon form: PLE to U, unit upper triangular in the pivots' columns,
 // then U_piv^{-1} U_free for the others alone (nothing at all for a matrix of
 // full column rank).  Back substitution in blocks of 64 rows over every column,
@@ -1355,43 +1477,32 @@ int elim_rref(modp_ctx *ctx, int form, int kind, int64_t m, int64_t n, const voi
     k_column_kinds<<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(pivcol, (int)rank, (int)n, kinds, free_cols);
     HIP_TRY(ctx, hipGetLastError());
     int32_t *Z = nullptr;
-    const int64_t ld = rup(rank, 64);
+    bool blocks = false;  // where U_piv^{-1} U_free has no room (MODP_RREF_BLOCKS=1: always)
     if (rank > 0 && nfree > 0) {
-        // pivots in the first columns: U_piv and U_free are where they are
-        const bool first = res.pivcols[(size_t)rank - 1] == rank;
-        const int32_t *T = W, *Y = W + rank * ldw;
-        int64_t ldt = ldw, ldy = ldw;
-        if (!first) {
-            int32_t *Tg = (int32_t *)ws_get(ctx, WS_TRI_T, sizeof(int32_t) * (size_t)ld * (size_t)rank, &st);
-            if (!Tg) return st;
-            int32_t *Yg = (int32_t *)ws_get(ctx, WS_INV_U, sizeof(int32_t) * (size_t)ld * (size_t)nfree, &st);
-            if (!Yg) return st;
-            k_gather_cols<<<grid_for(rank * rank), 256, 0, ctx->stream>>>(W, ldw, rank, pivcol, pivcol, rank, Tg, ld);
-            HIP_TRY(ctx, hipGetLastError());
-            k_gather_cols<<<grid_for(rank * nfree), 256, 0, ctx->stream>>>(W, ldw, rank, pivcol, free_cols, nfree, Yg, ld);
-            HIP_TRY(ctx, hipGetLastError());
-            T = Tg; Y = Yg;
-            ldt = ldy = ld;
+        const Echelon u{W, ldw, rank, nfree, pivcol, free_cols, res.pivcols[(size_t)rank - 1] == rank};
+        const char *benv = getenv("MODP_RREF_BLOCKS");
+        blocks = benv && atoi(benv) != 0;
+        if (!blocks) {
+            st = rref_free(ctx, form, u, mp, &Z);
+            if (st == MODP_ERR_OOM) {
+                blocks = true;
+                ctx->last_error.clear();
+                for (int slot : {WS_TRI_T, WS_TRI_X, WS_TRI_TMP, WS_INV_U, WS_INV_L, WS_ALIMB, WS_BLIMB, WS_SLICES})
+                    ws_drop(ctx, slot);
+            } else {
+                MODP_TRY(st);
+            }
         }
-        int32_t *X = (int32_t *)ws_get(ctx, WS_TRI_X, sizeof(int32_t) * (size_t)ld * (size_t)rank, &st);
-        if (!X) return st;
-        Z = (int32_t *)ws_get(ctx, WS_INV_L, sizeof(int32_t) * (size_t)ld * (size_t)nfree, &st);
-        if (!Z) return st;
-        MODP_TRY(trinv_i32(ctx, true, T, ldt, X, ld, rank, mp));
-        GemmArgs g;
-        g.m = rank; g.n = nfree; g.k = rank;
-        g.A = X; g.lda = ld; g.ka = EK_I32;
-        g.B = Y; g.ldb = ldy; g.kb = EK_I32;
-        g.C = Z; g.ldc = ld; g.kc = EK_I32;
-        g.epi = EPI_STORE;
-        g.mp = mp;
-        MODP_TRY(gemm_run(ctx, g, gemm_default_config(ctx, g, form)));
+        if (blocks)
+            MODP_TRY(kind == EK_F64 ? rref_free_blocks<double>(ctx, form, u, mp, m, (double *)R, ldr)
+                                    : rref_free_blocks<float>(ctx, form, u, mp, m, (float *)R, ldr));
     }
     const unsigned grid = grid_for(m * n);
+    const int64_t ld = rup(rank, 64);
     if (kind == EK_F64)
-        k_write_rref<double><<<grid, 256, 0, ctx->stream>>>(m, n, (int)rank, kinds, Z, ld, (double *)R, ldr);
+        k_write_rref<double><<<grid, 256, 0, ctx->stream>>>(m, n, (int)rank, kinds, blocks, Z, ld, (double *)R, ldr);
     else
-        k_write_rref<float><<<grid, 256, 0, ctx->stream>>>(m, n, (int)rank, kinds, Z, ld, (float *)R, ldr);
+        k_write_rref<float><<<grid, 256, 0, ctx->stream>>>(m, n, (int)rank, kinds, blocks, Z, ld, (float *)R, ldr);
     HIP_TRY(ctx, hipGetLastError());
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     return MODP_OK;
