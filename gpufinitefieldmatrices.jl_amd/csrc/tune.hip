@@ -136,7 +136,7 @@ int gemm_auto(modp_ctx *ctx, const GemmArgs &g)
         MODP_TRY(tune_gemm(ctx, g, &cfg, &ms));
     }
     // shallow products need no workspace in the plain form
-    if (!tuned && cfg.form == MODP_FORM_LIMB_I8 && g.k < 256 && capturing(ctx))
+    if (!tuned && cfg.form != MODP_FORM_PLAIN_F64 && g.k < 256 && capturing(ctx))
         cfg = gemm_default_config(ctx, g, MODP_FORM_PLAIN_F64);
     return gemm_run(ctx, g, cfg);
 }
