@@ -177,14 +177,16 @@ int gemm_rns_run(modp_ctx *ctx, const GemmArgs &g, int tile)
         uint8_t *E = (uint8_t *)ws_get(ctx, WS_SLICES, (size_t)r * Np * Mp, &st);
         if (!E) return st;
         // one modulus fewer where entries spread over their range would do
-        // with it; the rows' sums start and end at zero
+        // with it; the rows' sums start and end at zero.  Not in a graph: their
+        // workspace grows by other sizes than the planes', so one that the
+        // planes were made for beforehand could find none, or lose it later
         const u128 h = (u128)(g.mp.p / 2), kh2 = (u128)(kc > 0 ? kc : 1) * h * h;
         u128 M = 1;
         for (int j = 0; j + 1 < r; ++j) M *= (u128)QLIST[j];
         unsigned long long *rowsum = nullptr;
         int *fewer = nullptr;
         Moduli less = md;
-        if (!md.single && r > 1 && M > kh2 + kh2 / 32) {
+        if (!md.single && r > 1 && M > kh2 + kh2 / 32 && !capturing(ctx)) {
             const size_t had = ctx->ws_size[WS_RNS];
             int *buf = (int *)ws_get(ctx, WS_RNS, 256 + sizeof(unsigned long long) * (size_t)Mp, &st);
             if (!buf) return st;
