@@ -763,14 +763,18 @@ int gemv_t(modp_ctx *ctx, int64_t m, int64_t k, const T *A, int64_t lda, const T
     S = k > 0 ? (k + kslice - 1) / kslice : 1;
     // y over x or within A: nothing of y is written before all of both is read
     const bool over = k > 0 && m > 0 && (meet(y, y + m, x, x + k) || meet(y, y + m, A, A + (k - 1) * lda + m));
+    // the slices' sum in a launch of its own, which is also the way in a graph:
+    // the counts of arrivals would be one more workspace that has to be there
+    // when it is captured and to stay
+    const bool sum_after = over || (S > 1 && capturing(ctx));
     int32_t *P = nullptr;
     int *arrived = nullptr;
-    if (S > 1 || over) {
+    if (S > 1 || sum_after) {
         int st = MODP_OK;
         P = (int32_t *)ws_get(ctx, WS_SLICES, sizeof(int32_t) * (size_t)S * (size_t)m, &st);
         if (!P) return st;
     }
-    if (S > 1 && !over) {
+    if (S > 1 && !sum_after) {
         int st = MODP_OK;
         const size_t had = ctx->ws_size[WS_GEMV];
         arrived = (int *)ws_get(ctx, WS_GEMV, sizeof(int) * (size_t)rb, &st);
@@ -787,7 +791,7 @@ int gemv_t(modp_ctx *ctx, int64_t m, int64_t k, const T *A, int64_t lda, const T
                                                                                cadence, mp);
         HIP_TRY(ctx, hipGetLastError());
     }
-    if (!over) return MODP_OK;
+    if (!sum_after) return MODP_OK;
     GemmArgs g;
     g.m = m; g.n = 1; g.k = k;
     g.C = y; g.ldc = m; g.kc = sizeof(T) == 8 ? EK_F64 : EK_F32;

@@ -32,6 +32,8 @@ def product(g, ctx, m, n, k, p, seed, **how):
 @pytest.mark.parametrize("name,p,before,inside,after", [
     ("multi-modular", 2 ** 26 - 5, (600, 600, 5000, RNS), (1500, 200, 40, RNS), (3000, 100, 30, RNS)),
     ("multi-modular", 65521, (600, 600, 4000, RNS), (1500, 200, 900, RNS), (3000, 100, 300, RNS)),
+    ("vector", 65521, (512, 512, 4096, 1), (3000, 1, 2000, None), (20000, 1, 600, None)),
+    ("vector", 2 ** 26 - 5, (512, 512, 4096, 1), (1001, 1, 515, None), (20000, 1, 600, None)),
 ])
 def test_capture_after_other_shapes(gffm, name, p, before, inside, after):
     g, runtime = gffm, hip()
