@@ -135,10 +135,14 @@ int gemm_auto(modp_ctx *ctx, const GemmArgs &g)
         double ms = 0;
         MODP_TRY(tune_gemm(ctx, g, &cfg, &ms));
     }
-    // shallow products need no workspace in the plain form
-    if (!tuned && cfg.form != MODP_FORM_PLAIN_F64 && g.k < 256 && capturing(ctx))
-        cfg = gemm_default_config(ctx, g, MODP_FORM_PLAIN_F64);
-    return gemm_run(ctx, g, cfg);
+    // shallow products need no workspace in the plain form: taken where they can
+    // have none, in a graph or short of memory (nothing of C is written by then)
+    const bool shallow = !tuned && cfg.form != MODP_FORM_PLAIN_F64 && g.k < 256;
+    if (shallow && capturing(ctx)) return gemm_plain_f64(ctx, g);
+    const int st = gemm_run(ctx, g, cfg);
+    if (st != MODP_ERR_OOM || !shallow) return st;
+    ctx->last_error.clear();
+    return gemm_plain_f64(ctx, g);
 }
 
 // ---- text form of the cache: one entry per line -------------------------

@@ -1,5 +1,6 @@
 """Products of little depth where no workspace may be had: captured into a graph by a
-context that has none yet.  Bit-exact against the oracle."""
+context that has none yet, and with hardly any device memory left.  Bit-exact against
+the oracle."""
 import ctypes
 
 import numpy as np
@@ -47,3 +48,38 @@ def test_capture_large(gffm, m, n, k):
         ctx.synchronize()
         assert np.array_equal(g.Array(C).astype(np.int64), expect), i
     assert runtime.hipGraphExecDestroy(run) == 0 and runtime.hipGraphDestroy(graph) == 0
+
+
+@pytest.mark.parametrize("m,n,k,p", [(20000, 600, 200, 2 ** 26 - 5), (600, 40000, 255, 65521), (6000, 6000, 255, 2 ** 26 - 5)])
+def test_little_memory(gffm, m, n, k, p):
+    # room for less than the digit planes
+    g, runtime = gffm, hip()
+    print(f"little memory {m}x{n}x{k} p={p}", flush=True)
+    ctx = g.Context()
+    Ah, Bh = O.draw_matrix(m, k, p, 81), O.draw_matrix(k, n, p, 82)
+    A, B = g.CuModMatrix(Ah, p, elem_type=np.float64, ctx=ctx), g.CuModMatrix(Bh, p, elem_type=np.float64, ctx=ctx)
+    C = g.zeros(np.float64, m, n, p, ctx=ctx)
+    X = g.rand(np.float64, 200, 200, p, seed=3, ctx=ctx)
+    g.mul_(g.zeros(np.float64, 200, 200, p, ctx=ctx), X, X)  # (the plain form's code is on the device)
+    ctx.synchronize()
+    ctx.release_freed()
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    keep, ballast = 4 << 20, []
+    try:
+        for _ in range(4):  # (what is free is an estimate while much of it is)
+            assert runtime.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+            if free.value <= keep + (4 << 20):
+                break
+            ballast.append(ctypes.c_void_p())
+            if runtime.hipMalloc(ctypes.byref(ballast[-1]), free.value - keep) != 0:
+                runtime.hipGetLastError()
+                break
+        print(f"{free.value} bytes left of {total.value}", flush=True)
+        g.mul_(C, A, B)
+        ctx.synchronize()
+    finally:
+        assert all([runtime.hipFree(x) == 0 for x in ballast if x.value])
+    assert np.array_equal(g.Array(C).astype(np.int64), O.gemm(Ah, Bh, p))
+    C.data.zero()
+    g.mul_(C, A, B)  # with workspaces
+    assert np.array_equal(g.Array(C).astype(np.int64), O.gemm(Ah, Bh, p))
