@@ -942,7 +942,11 @@ static int elim_attempt(modp_ctx *ctx, int mode, int form, int kind, int64_t m, 
         g.mp = mp;
         g.skip = skip;
         const int use_form = form != MODP_FORM_AUTO ? form : choose_form(rows, cols, K, p);
-        if (use_form == MODP_FORM_LIMB_I8) return gemm_limb_i8(ctx, g);
+        if (use_form == MODP_FORM_LIMB_I8) {
+            const int st = gemm_limb_i8(ctx, g);
+            if (st != MODP_ERR_OOM || form != MODP_FORM_AUTO) return st;
+            ctx->last_error.clear();  // no room for the digit planes
+        }
         return gemm_plain_f64(ctx, g);
     };
     auto launch_panel_any = [&](int blk, int t, int64_t KC, int64_t FAR, int64_t rj, int64_t cj, int64_t w) -> int {
