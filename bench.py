@@ -7,7 +7,7 @@ GEMV, batched products, batched eliminations).
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--only gemm|pluq|batched]
 
 One "step" is one C = A*B mod p over 8192^3 residues resident in HBM (the
-residue splits of A and B, the 9 int8 MFMA products and the Chinese-remainder
+residue splits of A and B, the int8 MFMA products and the Chinese-remainder
 recombination all inside the step).  Prints one JSON line.  The 8192^2 operands are generated on the
 device by the library's seeded generator; the batched workloads come from
 the shared host generator (gpufinitefieldmatrices.workloads) and are
@@ -288,6 +288,7 @@ def main():
     # headline: the multi-modular int8 form (the form FORM_AUTO picks here)
     C_rns = g.zeros(np.float64, n, n, p)
     rns_ms, rns_wall, rns_kms, _ = time_gemm(g, ctx, A, B, C_rns, g.FORM_RNS_I8, a.steps, a.warmup, "gemm_rns")
+    made, planes = ctx.rns_products()
     extra = {}
     bg = be = None
     if a.only == "all":
@@ -375,9 +376,8 @@ def main():
     # (all moduli in one launch): algorithmic work 2 m n k per launch over
     # the mean launch time (HIP events around each launch on the library
     # stream)
-    r_mod = 9  # moduli for p = 2^26 - 5 and k = 8192: 4 k floor(p/2)^2 < prod q_j
     achieved = ops / (rns_kms * 1e-3) / 1e12 if rns_kms else None     # TOP/s
-    issued = r_mod * achieved if achieved else None                    # one int8 product per modulus
+    issued = made * achieved if achieved else None                     # int8 products that the kernel made
     traffic, traffic_src = None, None
     tfile = os.path.join(REPO, "profiles", "gemm_rns_8192_traffic.json")
     if os.path.exists(tfile):
@@ -392,17 +392,17 @@ def main():
     except Exception as e:  # reported, never fatal
         measured = {"error": str(e)}
     m32 = measured.get("int8_mfma_32x32x32_tops")
-    roof = {"bound": "mfma", "kernel": "k_rns_gemm2<256x256 tile, 2x4 waves> (9 moduli per launch)",
+    roof = {"bound": "mfma", "kernel": "k_rns_gemm2<256x256 tile, 2x4 waves> (one int8 product per modulus)",
             "achieved": round(achieved, 2) if achieved else None,
             "peak": INT8_PEAK_TOPS, "unit": "TFLOP/s",
             "frac": round(achieved / INT8_PEAK_TOPS, 4) if achieved else None,
             "traffic": traffic, "traffic_source": traffic_src,
-            # the core kernel reads r int8 residue planes of A and of B and
-            # writes r residue planes of C once each
-            "algorithmic_bytes": int(3 * r_mod * n * n),
+            # the core kernel reads an int8 residue plane of A and of B and
+            # writes one of C for each product that it makes
+            "algorithmic_bytes": int(3 * made * n * n),
             "measured_peaks": measured,
             "frac_of_measured": round(achieved / m32, 4) if achieved and m32 else None,
-            "mfma_issue": {"int8_products": r_mod,
+            "mfma_issue": {"int8_products": made, "residue_planes": planes,
                            "issued_tops": round(issued, 1) if issued else None,
                            "issued_frac_of_peak": round(issued / INT8_PEAK_TOPS, 4) if issued else None,
                            "issued_frac_of_measured": round(issued / m32, 4) if issued and m32 else None},
@@ -431,9 +431,10 @@ def main():
         "dtype": "int8",
         "data": "synthetic",
         "config": {"workload": f"mod-p GEMM {n}x{n}x{n}, p=2^26-5, residues uniform from seed 1, int8 MFMA "
-                               "multi-modular limbs (residues modulo 9 pairwise coprime moduli <= 256), int32 "
+                               f"multi-modular limbs (residues modulo {planes} pairwise coprime moduli <= 256), int32 "
                                "accumulation, FP64 Chinese-remainder recombination; each step includes the "
-                               "limb split, the 9 int8 products and the recombination",
+                               f"limb split, {made} int8 products (the last one is left out where the rows of "
+                               "A show that it is not needed) and the recombination",
                    "n": n, "p": p, "form": "rns_i8", "parallelism": "single GPU"},
         "wall_ms_per_step": round(rns_wall, 4),
         "gemm_core_ms": round(rns_kms, 4) if rns_kms else None,

@@ -847,6 +847,19 @@ int modp_kernel_timing_reset(modp_ctx *ctx)
     return MODP_OK;
 }
 
+int modp_rns_products(modp_ctx *ctx, int *made, int *planes)
+{
+    CTX_CHECK(ctx);
+    if (!made || !planes) return set_error(ctx, MODP_ERR_ARG, "null output pointer");
+    int fewer = 0;
+    if (ctx->rns_asked && ctx->ws[WS_RNS])
+        HIP_TRY(ctx, hipMemcpyAsync(&fewer, ctx->ws[WS_RNS], sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    *planes = ctx->rns_planes;
+    *made = ctx->rns_planes - (fewer != 0);
+    return MODP_OK;
+}
+
 int modp_kernel_time(modp_ctx *ctx, const char *prefix, double *total_ms, int64_t *count)
 {
     CTX_CHECK(ctx);

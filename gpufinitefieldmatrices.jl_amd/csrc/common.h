@@ -291,6 +291,10 @@ struct modp_ctx {
     // steps of the elimination panels so far (64 a panel): their exchange tags
     uint32_t panel_tag = 0;
     int64_t panel_rows[3] = {0, 0, 0};  // that a panel on one XCD takes, by its arithmetic (0: not asked yet)
+    // the last multi-modular product: its planes, and whether WS_RNS holds
+    // if one of them was left out
+    int rns_planes = 0;
+    bool rns_asked = false;
     // autotuner: MODP_TUNE_OFF / _CACHED / _ON_MISS and its cache
     int tune_mode = 0;
     std::map<TuneKey, TuneEntry> tune_cache;

@@ -215,6 +215,8 @@ int gemm_rns_run(modp_ctx *ctx, const GemmArgs &g, int tile)
         if (g.kc == EK_F64) MODP_TRY(combine_t<double>(ctx, g, epi, E, Mp, Np * Mp, md, less, fewer));
         else if (g.kc == EK_F32) MODP_TRY(combine_t<float>(ctx, g, epi, E, Mp, Np * Mp, md, less, fewer));
         else MODP_TRY(combine_t<int32_t>(ctx, g, epi, E, Mp, Np * Mp, md, less, fewer));
+        ctx->rns_planes = r;
+        ctx->rns_asked = fewer != nullptr;
         kdone += kc;
         first = false;
     } while (kdone < g.k);

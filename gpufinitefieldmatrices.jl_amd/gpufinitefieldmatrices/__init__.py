@@ -165,6 +165,12 @@ class Context:
         self.check(self.lib.modp_kernel_time(self.h, prefix.encode(), ctypes.byref(tot), ctypes.byref(cnt)))
         return tot.value, cnt.value
 
+    def rns_products(self) -> Tuple[int, int]:
+        """int8 products that the last multi-modular product made, and had planes for."""
+        made, planes = ctypes.c_int(), ctypes.c_int()
+        self.check(self.lib.modp_rns_products(self.h, ctypes.byref(made), ctypes.byref(planes)), "rns_products")
+        return made.value, planes.value
+
     def event_record(self, slot: int):
         self.check(self.lib.modp_event_record(self.h, slot))
 

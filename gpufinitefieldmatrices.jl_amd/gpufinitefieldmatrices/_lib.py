@@ -117,6 +117,7 @@ SIGNATURES = [
     ("modp_kernel_timing", _int, [_vp, _int]),
     ("modp_kernel_time", _int, [_vp, ctypes.c_char_p, ctypes.POINTER(ctypes.c_double), _p64]),
     ("modp_kernel_timing_reset", _int, [_vp]),
+    ("modp_rns_products", _int, [_vp, ctypes.POINTER(_int), ctypes.POINTER(_int)]),
     ("modp_event_record", _int, [_vp, _int]),
     ("modp_event_elapsed", _int, [_vp, _int, _int, ctypes.POINTER(ctypes.c_float)]),
     ("modp_probe_peak", _int, [_vp, _int, ctypes.POINTER(ctypes.c_double)]),

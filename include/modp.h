@@ -345,6 +345,10 @@ int modp_kernel_timing(modp_ctx *ctx, int enable);
  * `prefix`; synchronises. */
 int modp_kernel_time(modp_ctx *ctx, const char *prefix, double *total_ms, int64_t *count);
 int modp_kernel_timing_reset(modp_ctx *ctx);
+/* int8 products that the context's last multi-modular product made (its last K
+ * chunk) and those it had residue planes for: one fewer where the rows of A
+ * allow it.  0 and 0 before there is one; synchronises. */
+int modp_rns_products(modp_ctx *ctx, int *made, int *planes);
 /* events around arbitrary regions on the context's stream */
 int modp_event_record(modp_ctx *ctx, int slot);
 int modp_event_elapsed(modp_ctx *ctx, int slot_start, int slot_end, float *ms);
