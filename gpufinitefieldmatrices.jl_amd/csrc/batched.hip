@@ -348,7 +348,7 @@ __global__ __launch_bounds__(256, 2) void k_batched_limb(const BJob *__restrict_
 // from memory each.  Loads are clamped into the operands instead of
 // predicated: past K the A digits are zero, and nothing reads other rows or
 // columns.  10,000 products of 16 to 256 rows, columns and k, three digits:
-// 1.23 ms, about 4.8 TB/s with the repeated B reads (one stage in flight,
+// 1.25 ms, 4.0 TB/s with the 0.6 GB of B that is read again (one stage in flight,
 // predicated loads, digits by shifts and masks: 1.74 ms).
 constexpr int RP_KMAX = 256;
 template <typename T> struct __attribute__((packed, aligned(sizeof(T)))) BlPair {

@@ -623,9 +623,11 @@ bool gemm_config_valid(const GemmArgs &g, const GemmConfig &cfg)
 // when it issues at most three quarters of the limb form's MFMA work and the
 // product is large enough for its two more launches and its residue planes of
 // C.  Four digits: 2501 x 1203 x 1777 121 us against 111, 2048^3 126 against
-// 159.  One plane (p <= 255) issues what one digit does and is the slower one
-// (float64 mod 127: 6000^3 499 us against 436, 8192^3 942 against 862); from
-// four 256 x 256 output tiles per CU it remains the documented choice.
+// 159.  One plane (p <= 255) issues what one digit does (mod 127, one plane
+// against one digit: float64 6000^3 495 us and 450, 8192^3 920 and 860, 10,000^3
+// 1550 and 1610, 12,000^3 2390 and 2380; float32 8192^3 845 and 750).  From four
+// 256 x 256 output tiles per CU it is what modp_gemm_config_get has always
+// answered, and stays.
 static bool rns_pays(const modp_ctx *ctx, const GemmArgs &g)
 {
     const int L = limb_count(g.mp.p);
