@@ -672,8 +672,15 @@ GemmConfig gemm_default_config(const modp_ctx *ctx, const GemmArgs &g, int form)
     // 18.9) and K is deep enough for the core to outweigh the epilogue, of which
     // 64x64 keeps four workgroups on a CU (4000 x 4000 x 128, two digits: 34.2
     // us against 41.3 with 128x128); three and four digits gain nothing over 64x64
+    // Narrow products would compute padding: up to 64 rows or columns (40,000 x 16
+    // x 2000, one digit: 184 us with 128x128, 169 with 64x64), with two digits
+    // wherever 128x128 pad a fifth more (192 x 20,000 x 2000 143 and 127, 12,000 x
+    // 320 x 700 47 and 40; 420 x 12,000 x 2000, a seventh more, 105 and 103).
     const int L = limb_count(g.mp.p);
-    if (L <= 2 && g.k > 256 && 4 * t128 >= 3 * ctx->num_cus) c.tile_m = c.tile_n = 128;
+    const double pad64 = (double)round_up(g.m, 64) * (double)round_up(g.n, 64);
+    const double pad128 = (double)round_up(g.m, 128) * (double)round_up(g.n, 128);
+    const bool narrow = std::min(g.m, g.n) <= 64 || (L == 2 && 5 * pad128 >= 6 * pad64);
+    if (L <= 2 && g.k > 256 && 4 * t128 >= 3 * ctx->num_cus && !narrow) c.tile_m = c.tile_n = 128;
     // K slices where the tiles leave CUs idle and a slice keeps at least 512 of
     // a long K: the slices' sum costs a launch, about what 1024 of K cost
     // (512 x 512 x 4096, two digits: 45 us unsplit, 24.9 / 26.8 with 4 / 8 slices;

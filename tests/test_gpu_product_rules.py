@@ -1,0 +1,32 @@
+"""What the automatic choice takes where a form or a tile stops being the faster one,
+and the products there, bit-exact against the oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+PLAIN, DIGITS = 1, 2
+P = {1: 127, 2: 65521, 3: 2 ** 23 - 15, 4: 2 ** 26 - 5}  # by digits
+
+
+def check(g, m, n, k, p):
+    Ah, Bh = O.draw_matrix(m, k, p, 51), O.draw_matrix(k, n, p, 52)
+    A, B = g.CuModMatrix(Ah, p, elem_type=np.float64), g.CuModMatrix(Bh, p, elem_type=np.float64)
+    C = g.zeros(np.float64, m, n, p)
+    g.mul_(C, A, B)
+    assert np.array_equal(g.Array(C).astype(np.int64), O.gemm(Ah, Bh, p))
+
+
+# narrow products keep 64 x 64 tiles
+@pytest.mark.parametrize("m,n,k,digits,tile", [
+    (40000, 16, 300, 1, 64), (64, 40000, 300, 1, 64), (65, 40000, 300, 1, 128), (40000, 192, 300, 1, 128),
+    (40000, 64, 300, 2, 64), (40000, 65, 300, 2, 128), (192, 20000, 300, 2, 64), (12000, 320, 300, 2, 64),
+    (12000, 420, 300, 2, 128), (2501, 1203, 300, 2, 128), (2048, 2048, 300, 2, 128)])
+def test_narrow_tiles(gffm, m, n, k, digits, tile):
+    g, p = gffm, P[digits]
+    print(f"tiles {m}x{n}x{k} p={p}", flush=True)
+    cfg, _ = g.context().gemm_config(m, n, k, p)
+    assert cfg["form"] == DIGITS and cfg["tile_m"] == cfg["tile_n"] == tile
+    check(g, m, n, k, p)
