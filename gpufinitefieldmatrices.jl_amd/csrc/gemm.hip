@@ -595,8 +595,16 @@ int choose_form(int64_t m, int64_t n, int64_t k, int64_t p)
     // shallow ones: the digit form's split passes and its epilogue against the
     // plain form's k-steps.  2048^2: at k = 32 13.3, 15.2 and 26 us with one,
     // two and four digits against 15.8, at k = 64 13.4, 15.4 and 26 against 22,
-    // at k = 128 13.8, 16.5 and 28 against 34
-    return k >= (limb_count(p) <= 3 ? 48 : 96) ? MODP_FORM_LIMB_I8 : MODP_FORM_PLAIN_F64;
+    // at k = 128 13.8, 16.5 and 28 against 34.  Up to about 1000 x 1000 the digit
+    // form's second launch weighs more (1000^2 at k = 48 9.6, 10.4 and 10.8 us with
+    // one, two and three digits against 8.9, at k = 72 9.8, 11.0 and 12.0 against
+    // 11.2), and so do the planes of a long thin product while the plain form takes
+    // 64x64 tiles there (64 x 40,000 at k = 48 14.1, 16.4, 20.6 and 24.3 against
+    // 15.5 to 17, at k = 96 17.3, 20.2, 24.9 and 29.1 against 22.7 to 25.8)
+    static const int wide[4] = {48, 48, 56, 96}, few[4] = {56, 64, 88, 96}, thin[4] = {48, 56, 112, 112};
+    auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
+    const int *from = std::min(m, n) <= 64 && tiles(64) > 256 && tiles(128) < 512 ? thin : m * n <= 1 << 20 ? few : wide;
+    return k >= from[std::min(limb_count(p), 4) - 1] ? MODP_FORM_LIMB_I8 : MODP_FORM_PLAIN_F64;
 }
 
 bool gemm_config_valid(const GemmArgs &g, const GemmConfig &cfg)

@@ -30,3 +30,20 @@ def test_narrow_tiles(gffm, m, n, k, digits, tile):
     cfg, _ = g.context().gemm_config(m, n, k, p)
     assert cfg["form"] == DIGITS and cfg["tile_m"] == cfg["tile_n"] == tile
     check(g, m, n, k, p)
+
+
+# shallow products take the plain form: below 1000 x 1000, where they are long and thin,
+# and elsewhere
+@pytest.mark.parametrize("m,n,starts", [
+    (64, 6000, (56, 64, 88, 96)), (1000, 1000, (56, 64, 88, 96)), (1024, 1025, (48, 48, 56, 96)),
+    (40000, 8, (48, 56, 112, 112)), (64, 16400, (48, 56, 112, 112)), (100000, 16, (48, 48, 56, 96)),
+    (65, 40000, (48, 48, 56, 96)), (2000, 2000, (48, 48, 56, 96))])
+def test_digits_from(gffm, m, n, starts):
+    g = gffm
+    for digits, k in zip(P, starts):
+        p = P[digits]
+        print(f"digits from {m}x{n}x{k} p={p}", flush=True)
+        for kk, form in ((k - 1, PLAIN), (k, DIGITS)):
+            cfg, _ = g.context().gemm_config(m, n, kk, p)
+            assert cfg["form"] == form, (p, kk)
+            check(g, m, n, kk, p)
