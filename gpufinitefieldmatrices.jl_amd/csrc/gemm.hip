@@ -357,17 +357,20 @@ int64_t small_work(int64_t m, int64_t n, int64_t k)
     const int64_t blocks = ((m + 15) / 16) * ((n + 15) / 16);
     return blocks <= 1024 && k <= 1024 && k > 0 ? blocks * k : -1;
 }
-// against 64 x 64 tiles it pays up to 512 x 512 x 256 (11.9 us, 23 in tiles)
+// against 64 x 64 tiles it pays up to 512 x 512 x 256 (11.9 us, 23 in tiles), but
+// not while those take one stage of K, or two in a single tile: 6.0 us from 64 x 64
+// to 512 x 512 at k = 16, where this takes 6.5 to 7.3 (one call after the other)
 bool f64_small(const GemmArgs &g)
 {
     const int64_t w = small_work(g.m, g.n, g.k);
-    return w >= 0 && w <= 262144 && g.ka == g.kb && g.ka == g.kc &&
+    const bool short_k = g.k <= PBK || (g.k <= 2 * PBK && g.m <= 64 && g.n <= 64);
+    return w >= 0 && w <= 262144 && !short_k && g.ka == g.kb && g.ka == g.kc &&
            (g.epi == EPI_STORE || (g.epi == EPI_SUB && g.kc == EK_I32));
 }
 int launch_f64_small(modp_ctx *ctx, const GemmArgs &g, int R, int64_t count, int64_t sa, int64_t sb, int64_t sc,
                      const GemmSize &last)
 {
-    TimedLaunch tl(ctx, "gemm_f64");
+    TimedLaunch tl(ctx, "gemm_f64_small");
     const unsigned grid = (unsigned)(((g.m + 15) / 16) * ((g.n + 15) / 16));
 #define SMALL(T_, EPI_)                                                                                             \
     k_gemm_f64_small<T_, T_, EPI_><<<dim3(grid, (unsigned)count), 256, 0, ctx->stream>>>(g.m, g.n, g.k, (const T_ *)g.A, g.lda,             \

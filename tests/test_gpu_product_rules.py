@@ -47,3 +47,23 @@ def test_digits_from(gffm, m, n, starts):
             cfg, _ = g.context().gemm_config(m, n, kk, p)
             assert cfg["form"] == form, (p, kk)
             check(g, m, n, kk, p)
+
+
+# the small plain kernel, and 64 x 64 tiles of one or two stages of K
+@pytest.mark.parametrize("p", [11, 65521, 2 ** 26 - 5])
+@pytest.mark.parametrize("m,n,k,small", [
+    (17, 17, 16, False), (512, 512, 16, False), (512, 512, 17, True), (64, 64, 32, False), (64, 64, 33, True),
+    (65, 64, 32, True), (65, 64, 16, False), (1, 3, 1, False), (513, 512, 40, False)])
+def test_small_plain_from(gffm, m, n, k, small, p):
+    g = gffm
+    ctx = g.context()
+    print(f"small plain {m}x{n}x{k} p={p}", flush=True)
+    ctx.kernel_timing_reset()
+    ctx.kernel_timing(True)
+    try:
+        check(g, m, n, k, p)
+        assert ctx.kernel_time("gemm_f64")[1] == 1
+        assert ctx.kernel_time("gemm_f64_small")[1] == int(small)
+    finally:
+        ctx.kernel_timing(False)
+        ctx.kernel_timing_reset()
