@@ -61,7 +61,8 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
                                                  int32_t *__restrict__ map_src, PanelCtl *__restrict__ ctl,
                                                  int *__restrict__ abort, int KC, int FAR, int32_t *__restrict__ stage,
                                                  int *__restrict__ cursor, int32_t *__restrict__ gpos,
-                                                 int32_t *__restrict__ grow, PanelSolve *__restrict__ solve, int strict)
+                                                 int32_t *__restrict__ grow, PanelSolve *__restrict__ solve, int strict,
+                                                 int *__restrict__ told)
 {
     constexpr int NW = GPT / 64;
     if (abort && *abort) {
@@ -257,7 +258,10 @@ __global__ __launch_bounds__(GPT) void k_panel_g(int32_t *__restrict__ W, int64_
         ctl->nmap = nmap_all;
         ctl->kr0 = kr0;
         if (cursor) *cursor = kr0 + pc;
-        if (abort && (status != 0 || (strict && pc < w))) *abort = 1;
+        if (abort && (status != 0 || (strict && pc < w))) {
+            *abort = 1;
+            tell(told);
+        }
     }
 }
 
@@ -894,8 +898,10 @@ static int elim_attempt(modp_ctx *ctx, int mode, int form, int kind, int64_t m, 
         if (!gpos) return st;
         grow = gpos + m;
     }
-    PanelCtl *hctl = (PanelCtl *)pinned_get(ctx, sizeof(PanelCtl) * NBATCH * MAXPAN + 64, &st);
+    // (what is read back of them, and a word that a panel writes when it stops)
+    PanelCtl *hctl = (PanelCtl *)pinned_get(ctx, sizeof(PanelCtl) * NBATCH * MAXPAN + 128, &st);
     if (!hctl) return st;
+    int *told = reinterpret_cast<int *>(hctl + NBATCH * MAXPAN) + 16;
 
     MODP_TRY(util_convert(ctx, kind, m, n, A, lda, EK_I32, W, ldw, mp));
     if (nt > n) {
@@ -954,7 +960,7 @@ static int elim_attempt(modp_ctx *ctx, int mode, int form, int kind, int64_t m, 
         a.W = W; a.ldw = ldw; a.m = (int)m; a.kr0 = (int)rj; a.c0 = (int)cj; a.w = (int)w;
         a.KC = (int)KC; a.FAR = (int)FAR; a.mp = mp; a.invs = invs;
         a.ipiv = ipiv; a.pivcol = pivcol; a.map_dst = bmap_dst + t * 64; a.map_src = bmap_src + t * 64;
-        a.stage = stage; a.ctl = bctl + blk * MAXPAN + t; a.solve = solve + t; a.abort = abort_flag;
+        a.stage = stage; a.ctl = bctl + blk * MAXPAN + t; a.solve = solve + t; a.abort = abort_flag; a.told = told;
         TimedLaunch tl(ctx, "elim_panel_any");
         k_panel_any<<<1, 64 * PWAVES, 0, ctx->stream>>>(a);
         return hip_check(ctx, hipGetLastError(), "k_panel_any launch");
@@ -970,7 +976,7 @@ static int elim_attempt(modp_ctx *ctx, int mode, int form, int kind, int64_t m, 
         if (width == GNBW) {
             k_panel_g<GNBW><<<1, GPT, 0, ctx->stream>>>(W, ldw, (int)m, (int)rj, (int)cj, (int)w, mp, ple, ipiv,
                                                         pivval, pivinv, pivcol, mdst, msrc, pctl, abort,
-                                                        (int)KC, (int)FAR, stage, cursor, gpos, grow, solve + t, strict);
+                                                        (int)KC, (int)FAR, stage, cursor, gpos, grow, solve + t, strict, told);
             return hip_check(ctx, hipGetLastError(), "k_panel_g launch");
         }
         PanelArgs a = {};
@@ -979,6 +985,7 @@ static int elim_attempt(modp_ctx *ctx, int mode, int form, int kind, int64_t m, 
         a.ipiv = ipiv; a.pivval = pivval; a.pivinv = pivinv; a.pivcol = pivcol;
         a.map_dst = mdst; a.map_src = msrc; a.stage = stage; a.ctl = pctl; a.solve = solve + t; a.abort = abort; a.cursor = cursor;
         a.strict = strict;
+        a.told = told;
         if (m - rj <= PSINGLE) {
             if (arith == 0) k_panel<false, 0><<<1, PSINGLE, 0, ctx->stream>>>(a);
             else if (arith == 1) k_panel<false, 1><<<1, PSINGLE, 0, ctx->stream>>>(a);
@@ -1091,7 +1098,9 @@ static int elim_attempt(modp_ctx *ctx, int mode, int form, int kind, int64_t m, 
     // each of its columns, so that each block's place is known beforehand.  A panel
     // that does not raises the abort flag, which turns the rest of the batch
     // into no-ops, and its block is completed from the host after one
-    // synchronization.  One a block cost 50 us of an idle GPU each (PLUQ of
+    // synchronization; the host enqueues no further blocks once it sees the word
+    // `told` (rref of a 2000^2 matrix of ones 599 -> 349 us, PLUQ 738
+    // -> 503).  One a block cost 50 us of an idle GPU each (PLUQ of
     // 4096^2 10.3 ms, in batches of eight 9.8).  After an abort the batches
     // start again from one block, since the next one may be near.
     struct Block {
@@ -1137,7 +1146,8 @@ static int elim_attempt(modp_ctx *ctx, int mode, int form, int kind, int64_t m, 
                 hold -= std::min(hold, (int)blocks.size());
                 away -= std::min(away, (int)blocks.size());
             }
-            for (int i = 0; i < (int)blocks.size(); ++i) {
+            __atomic_store_n(told, 0, __ATOMIC_RELAXED);  // (nothing is on its way)
+            for (int i = 0; i < (int)blocks.size() && !__atomic_load_n(told, __ATOMIC_RELAXED); ++i) {
                 const Block &b = blocks[i];
                 for (int t = 0; t < (int)b.w.size(); ++t) {
                     if (any) MODP_TRY(launch_panel_any(i, t, b.KC, b.FAR, b.rj[t], b.cj[t], b.w[t]));

@@ -114,6 +114,12 @@ struct PanelSolve {
     int32_t num[PNW];     // pivot of a panel column, or -1
 };
 
+// a word of host memory that shows the host, still enqueuing, that a panel stopped
+__device__ __forceinline__ void tell(int *word)
+{
+    if (word) __hip_atomic_store(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 struct PanelArgs {
     int32_t *W;
     int64_t ldw;
@@ -123,7 +129,7 @@ struct PanelArgs {
     int32_t *ipiv, *pivval, *pivinv, *pivcol, *map_dst, *map_src, *stage;
     PanelCtl *ctl;
     PanelSolve *solve;
-    int *abort, *cursor;
+    int *abort, *cursor, *told;
     int strict;          // a column without a pivot raises the abort flag, too
     PanelExchange *x;
     uint32_t *arrive;
@@ -781,7 +787,10 @@ __global__ __launch_bounds__(64 * PWAVES, MULTI ? 2 : 1) void k_panel(PanelArgs 
     if (gw == 0 && lane == 0) {
         *a.ctl = PanelCtl{pc, status, consumed, pc + (int)__popc(mask), kr0};
         if (a.cursor) *a.cursor = kr0 + pc;
-        if (a.abort && (status != 0 || (a.strict && pc < w))) *a.abort = 1;
+        if (a.abort && (status != 0 || (a.strict && pc < w))) {
+            *a.abort = 1;
+            tell(a.told);
+        }
     }
 }
 
@@ -815,7 +824,7 @@ struct PanelAnyArgs {
     int32_t *ipiv, *pivcol, *map_dst, *map_src, *stage;
     PanelCtl *ctl;
     PanelSolve *solve;
-    int *abort;
+    int *abort, *told;
 };
 constexpr int PAC = PNW / PWAVES;               // panel columns of a wave
 constexpr int PAB = 3;                          // columns updated before a step's barrier, the rest after it
@@ -894,6 +903,7 @@ __global__ __launch_bounds__(64 * PWAVES) void k_panel_any(PanelAnyArgs a)
         if (tid == 0) {
             *a.ctl = PanelCtl{0, 7, 0, 0, kr0};
             *a.abort = 1;
+            tell(a.told);
         }
         return;
     }

@@ -85,3 +85,16 @@ def test_stops(gffm, name, m, n, p):
         assert rank == ref["rank"] and P == ref["row_swaps"] and Q == ref["col_swaps"]
         assert np.array_equal(g.Array(U).astype(np.int64), ref["U"])
         assert np.array_equal(g.Array(L).astype(np.int64), ref["L"])
+
+
+@pytest.mark.parametrize("p", [7, 65521, 2 ** 26 - 5])
+@pytest.mark.parametrize("name", ["rank 1", "zero"])
+def test_blocks_after_a_stop(gffm, name, p):
+    # the host sees that the first panel stopped long before it has enqueued eight blocks
+    g, n = gffm, 2000
+    A = g.CuModMatrix(matrix(name, n, n, p), p, elem_type=np.float64)
+    for what in (g.rref, g.pluq, g.lu, g.is_invertible_with_inverse):
+        # (a first call waits for its allocations, and a busy device is late)
+        counts = [sum(launches(A.ctx, lambda: what(A))[0].values()) for _ in range(6)]
+        print(name, p, what.__name__, counts, flush=True)
+        assert min(counts) <= 24  # of 32 in a batch
