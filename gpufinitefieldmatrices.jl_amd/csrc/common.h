@@ -466,6 +466,6 @@ int elim_inverse(modp_ctx *ctx, int form, int kind, int64_t n, const void *A, in
 int tri_inverse(modp_ctx *ctx, int kind, int upper, int64_t m, int64_t n, const void *A, int64_t lda, void *Ainv,
                 int64_t ldai, int64_t p);
 int trinv_i32(modp_ctx *ctx, bool upper, const int32_t *T, int64_t ldt, int32_t *X, int64_t ldx, int64_t k,
-              const ModP &mp);
+              const ModP &mp, bool unit = false);
 int mat_inverse(modp_ctx *ctx, int form, int kind, int64_t n, const void *A, int64_t lda, void *Ainv, int64_t ldai,
                 int64_t p, int *invertible);

