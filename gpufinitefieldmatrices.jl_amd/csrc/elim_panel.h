@@ -47,7 +47,8 @@
 //
 // All workgroups have to be on the XCD at once.  The rows' own LDS is 66.6 KB,
 // and the scaled rows are int32 there rather than FP64, so that two workgroups
-// fit on a CU and 64 (16,384 rows) on an XCD.
+// fit on a CU and 64 (16,384 rows) on an XCD.  (The panel of one workgroup keeps
+// FP64: the conversions took 0.5 us of its 33 mod 11.)
 //
 // A 32-column panel mod 65521 takes 45 us at 4096 rows and 37 us at 256,
 // mod 2^26 - 5 51 and 48; at 8192 rows, where every CU has one workgroup, 56
@@ -393,7 +394,9 @@ __global__ __launch_bounds__(64 * PWAVES, MULTI ? 2 : 1) void k_panel(PanelArgs 
     // original and reduced columns by local row, a wave's rows of 64 (the odd
     // pitch spreads a row of the panel over the banks)
     __shared__ int32_t s_A[PWAVES][PNW][65], s_L[PWAVES][PNW][65];
-    __shared__ int32_t s_U[PNW][2 * PNW];  // scaled rows (negated, balanced) by column, and the rows of T
+    // scaled rows (negated, balanced) by column, and the rows of T
+    typedef std::conditional_t<MULTI, int32_t, double> scaled_t;
+    __shared__ scaled_t s_U[PNW][2 * PNW];
     __shared__ __attribute__((aligned(16))) double s_key[2][PWAVES];
     __shared__ int s_go;
 
@@ -455,7 +458,7 @@ __global__ __launch_bounds__(64 * PWAVES, MULTI ? 2 : 1) void k_panel(PanelArgs 
     double nl = 0.0, nup = 0.0;
     int Ipp = -2, atp = -2, Vp = 0;
     auto write_down = [&](int jc) __attribute__((always_inline)) {
-        s_U[jc & (PNW - 1)][lane] = (int32_t)nup;
+        s_U[jc & (PNW - 1)][lane] = (scaled_t)nup;
         iq_l = iq_l == Ipp ? -1 : iq_l;
         const bool here = lane == atp;
         ip_l = here ? Ipp : ip_l;
@@ -689,7 +692,7 @@ __global__ __launch_bounds__(64 * PWAVES, MULTI ? 2 : 1) void k_panel(PanelArgs 
         constexpr int RPW = PNW / PWAVES;
         int32_t y[RPW];
 #pragma unroll
-        for (int q = 0; q < RPW; ++q) y[q] = s_U[wave + PWAVES * q][lane < PNW ? lane : PNW + pj_q];
+        for (int q = 0; q < RPW; ++q) y[q] = (int32_t)s_U[wave + PWAVES * q][lane < PNW ? lane : PNW + pj_q];
 #pragma unroll
         for (int q = 0; q < RPW; ++q) {
             const int jc = wave + PWAVES * q, t = __popc(pivcols & ((1u << jc) - 1u));
